@@ -61,6 +61,7 @@ EXPORTED_SYMBOLS = (
     "bitsmoe_unpack_bitplanes",
     "bitsmoe_quantize_tiles",
     "bitsmoe_pack_slabs",
+    "bitsmoe_pack_matrix",
 )
 
 
@@ -189,6 +190,9 @@ def load() -> ctypes.CDLL:
     lib.bitsmoe_quantize_tiles.argtypes = [c_void_p, c_int64, c_int64, c_int64, c_int32, c_int32, c_void_p, c_void_p, c_void_p]
     lib.bitsmoe_pack_slabs.restype = c_int32
     lib.bitsmoe_pack_slabs.argtypes = [c_void_p, c_void_p, c_int64, c_int64, c_int32, c_void_p, c_void_p, c_void_p]
+    lib.bitsmoe_pack_matrix.restype = c_int32
+    lib.bitsmoe_pack_matrix.argtypes = [c_void_p, c_int64, c_int64, c_int64, c_void_p, c_int32, c_int32, c_void_p, c_int32,
+                                        c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]
     _lib = lib
     return lib
 

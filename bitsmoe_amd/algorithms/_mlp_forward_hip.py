@@ -530,6 +530,43 @@ def pack_slabs(levels: torch.Tensor, scale: torch.Tensor, dim: int, bits: int) -
     return payload, scale16
 
 
+def pack_matrix(matrix: torch.Tensor, ranges: Sequence[Tuple[int, int, int]], s_vec: Optional[torch.Tensor] = None,
+                iters: int = 50):
+    """Rows of a CUDA fp32 matrix [rank, dim] (unit column stride), quantised and packed in runtime order in one launch.
+    ranges: (bits, first row, end row) in packed order, ranges of one width next to each other.  Returns (payload uint32,
+    scale fp16) and, with s_vec [rank] given, also (s fp16, rank_idx int32, tile_meta int32 [n, 3], slab_meta int32 [n, 4])."""
+    _check(matrix.dim() == 2 and matrix.is_cuda and matrix.dtype == torch.float32 and (matrix.stride(1) == 1 or matrix.shape[1] <= 1),
+           "matrix must be a CUDA fp32 matrix with unit column stride")
+    rank, dim = int(matrix.shape[0]), int(matrix.shape[1])
+    dev = matrix.device
+    n_tiles = (dim + 127) // 128
+    flat, rows, word_rows, slabs, bucket, width = [], 0, 0, 0, 0, None
+    for bits, first, end in ranges:
+        flat += (bits, first, end)
+        if bits != width:
+            slabs, bucket, width = slabs + (bucket + 63) // 64, 0, bits
+        rows += end - first
+        bucket += end - first
+        word_rows += (end - first) * bits
+    slabs += (bucket + 63) // 64
+    payload = torch.empty((4 * n_tiles * word_rows,), dtype=torch.uint32, device=dev)
+    scale = torch.empty((rows * n_tiles,), dtype=torch.float16, device=dev)
+    tables = ()
+    if s_vec is not None:
+        _check(s_vec.dim() == 1 and int(s_vec.numel()) == rank and s_vec.device == dev, "s_vec must be [rank] on the matrix's device")
+        s_vec = (s_vec if s_vec.dtype in (torch.float16, torch.float32) else s_vec.to(torch.float16)).contiguous()
+        tables = (torch.empty((rows,), dtype=torch.float16, device=dev), torch.empty((rows,), dtype=torch.int32, device=dev),
+                  torch.empty((slabs * n_tiles, 3), dtype=torch.int32, device=dev),
+                  torch.empty((slabs, 4), dtype=torch.int32, device=dev))
+    with torch.cuda.device(dev):
+        _capi.check(_lib.bitsmoe_pack_matrix(
+            matrix.data_ptr(), rank, dim, int(matrix.stride(0)) if rank > 1 else dim, s_vec.data_ptr() if tables else None,
+            1 if tables and s_vec.dtype == torch.float32 else 0, len(flat) // 3, (ctypes.c_int32 * len(flat))(*flat), int(iters),
+            payload.data_ptr(), scale.data_ptr(), *(t.data_ptr() for t in tables), *((None,) * (4 - len(tables))),
+            _stream_ptr(dev)))
+    return (payload, scale) + tables
+
+
 def router_softmax_topk(router_logits: torch.Tensor, top_k: int, renormalize: bool = True,
                         round_dtype: Optional[torch.dtype] = None, weight_scale: float = 1.0) -> Tuple[torch.Tensor, torch.Tensor]:
     """softmax (fp32) -> top-k -> optional renormalisation -> * weight_scale -> optional round trip through

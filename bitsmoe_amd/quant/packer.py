@@ -11,17 +11,18 @@ Produces, for one rank-major matrix `[rank, dim]`, the buffers of the reference'
   s_buffer         fp16   1-D   per-row multiplier in local row order
 
 Rows are grouped by bit-width (descending), cut into slabs of at most 64 rows; rows with
-bits == 0 are dropped.  Everything runs on the GPU the input lives on, bucket-at-a-time
-(one quantiser call and one bit-plane kernel per bit-width, not per slab).
+bits == 0 are dropped.  A matrix on the GPU is packed by one kernel; one on the host bucket-at-a-time
+(one quantiser call per bit-width, not per slab).
 """
 from __future__ import annotations
 
+import bisect
 from typing import Dict, List, Sequence, Tuple
 
 import torch
 from torch import Tensor
 
-from .quantizer import pack_quantized, quantize_symmetric, quantize_tiles, unpack_quantized
+from .quantizer import pack_quantized, quantize_symmetric, unpack_quantized
 
 K_SLAB = 64
 N_TILE = 128
@@ -94,11 +95,10 @@ def _pack_bucket(rows: Tensor, bits: int) -> Tuple[Tensor, Tensor]:
     """rows [k, dim] of one bit bucket -> (payload words uint32 of its slabs in runtime order, scale fp16
     [slab][tile][row]).  Low bit-widths: the quantiser and the slab packer are kernels; 16-bit slabs
     (raw halves, all-ones scale) are laid out with tensor ops."""
-    if bits != 16 and rows.is_cuda:
+    if rows.is_cuda and rows.dtype != torch.float64:
         from bitsmoe_amd.algorithms import mlp_forward_cuda as hip
 
-        levels, scale = quantize_tiles(rows.to(torch.float32).contiguous(), bits)
-        return hip.pack_slabs(levels, scale, int(rows.shape[1]), bits)
+        return hip.pack_matrix(rows.to(torch.float32).contiguous(), [(bits, 0, int(rows.shape[0]))])
     words, scale = _quantise_bucket(rows, bits)
     k_total = int(rows.shape[0])
     pay = [_to_runtime_order(words[r0:r0 + K_SLAB]) for r0 in range(0, k_total, K_SLAB)]
@@ -107,7 +107,7 @@ def _pack_bucket(rows: Tensor, bits: int) -> Tuple[Tensor, Tensor]:
 
 
 def _bucket_segments(segments: Sequence[Tuple[int, Tuple[int, int]]], rank: int) -> Dict[int, List[Tuple[int, int]]]:
-    seen = torch.zeros(rank, dtype=torch.bool)
+    taken: List[Tuple[int, int]] = []      # sorted, disjoint
     buckets: Dict[int, List[Tuple[int, int]]] = {}
     for bits, (s, e) in segments:
         bits, s, e = int(bits), int(s), int(e)
@@ -117,9 +117,10 @@ def _bucket_segments(segments: Sequence[Tuple[int, Tuple[int, int]]], rank: int)
             raise ValueError(f"Invalid segment range (s={s}, e={e}) for rank={rank}")
         if e == s:
             continue
-        if bool(seen[s:e].any()):
+        at = bisect.bisect_left(taken, (s, e))
+        if (at > 0 and taken[at - 1][1] > s) or (at < len(taken) and taken[at][0] < e):
             raise ValueError(f"Overlapping segments in range [{s}, {e})")
-        seen[s:e] = True
+        taken.insert(at, (s, e))
         buckets.setdefault(bits, []).append((s, e))
     for ranges in buckets.values():
         ranges.sort()
@@ -143,6 +144,9 @@ def pack_rank_major(rank_major: Tensor, s_vec: Tensor,
     device = rank_major.device
     n_tiles = (dim + N_TILE - 1) // N_TILE
     buckets = _bucket_segments(segments, rank)
+
+    if rank_major.is_cuda and rank_major.dtype != torch.float64 and any(bits for bits in buckets):
+        return _pack_rank_major_device(rank_major, s_vec, buckets)
 
     payload_parts: List[Tensor] = []
     scale_parts: List[Tensor] = []
@@ -193,6 +197,37 @@ def pack_rank_major(rank_major: Tensor, s_vec: Tensor,
         "segments": torch.tensor(seg_rows, dtype=torch.int32).reshape(-1, 3),
         "original_indices": rank_idx.clone(),
         "original_rank": torch.tensor(rank, dtype=torch.int32),
+        "groupsize": torch.tensor(N_TILE, dtype=torch.int16),
+    }
+
+
+def _pack_rank_major_device(rank_major: Tensor, s_vec: Tensor, buckets: Dict[int, List[Tuple[int, int]]]) -> Dict[str, Tensor]:
+    """pack_rank_major on the GPU: one launch quantises and packs every row and writes the tables (nothing is copied to the
+    device or waited for; the three bookkeeping tensors of the host are made here)."""
+    from bitsmoe_amd.algorithms import mlp_forward_cuda as hip
+
+    ranges = [(bits, s, e) for bits in sorted(buckets, reverse=True) if bits for s, e in buckets[bits]]
+    matrix = rank_major.to(torch.float32)
+    if matrix.stride(1) != 1:
+        matrix = matrix.contiguous()
+    payload, scale, s16, rank_idx, tile_meta, slab_meta = hip.pack_matrix(matrix, ranges, s_vec.to(rank_major.device))
+    seg_rows: List[List[int]] = []
+    cursor = 0
+    for bits, s, e in ranges:
+        if not seg_rows or seg_rows[-1][0] != bits:
+            seg_rows.append([bits, cursor, cursor])
+        cursor += e - s
+        seg_rows[-1][2] = cursor
+    return {
+        "payload_buffer": payload,
+        "rank_idx_buffer": rank_idx,
+        "tile_meta_buffer": tile_meta,
+        "slab_meta_buffer": slab_meta,
+        "scale_buffer": scale,
+        "s_buffer": s16,
+        "segments": torch.tensor(seg_rows, dtype=torch.int32),
+        "original_indices": torch.cat([torch.arange(s, e, dtype=torch.int32) for _, s, e in ranges]),
+        "original_rank": torch.tensor(int(rank_major.shape[0]), dtype=torch.int32),
         "groupsize": torch.tensor(N_TILE, dtype=torch.int16),
     }
 

@@ -387,6 +387,19 @@ int bitsmoe_quantize_tiles(const float* rows, int64_t k, int64_t dim, int64_t ro
  */
 int bitsmoe_pack_slabs(const int8_t* levels, const float* scale, int64_t k, int64_t dim, int32_t bits,
                        uint32_t* payload_out, void* scale_out_f16, void* stream);
+/*
+ * The two steps above for one rank-major matrix [rank, dim] (fp32, row_stride elements apart) with rows of several
+ * widths, in one launch, and its tables.  Replaces pack_single_weight's device work (bitsmoe/quant/packer.py:517-749).
+ * ranges: HOST array of n_ranges x {bits, first row, one past the last row}: the source rows in packed order, ranges of
+ * one width next to each other; 16-bit rows are stored as halves.  payload_out: 4 * words * ceil(dim/128) per row
+ * (words = bits, 16 for 16-bit rows); scale_out_f16: ceil(dim/128) per row.  Tables (all or none; slab_meta_out NULL:
+ * none): s_out_f16 and rank_idx_out per packed row from s_vec [rank] (f16, or fp32 with s_is_f32), tile_meta_out
+ * int32 [slabs * tiles, 3], slab_meta_out int32 [slabs, 4], a bucket of n rows having ceil(n/64) slabs.
+ */
+int bitsmoe_pack_matrix(const float* matrix, int64_t rank, int64_t dim, int64_t row_stride, const void* s_vec,
+                        int32_t s_is_f32, int32_t n_ranges, const int32_t* ranges, int32_t iters,
+                        uint32_t* payload_out, void* scale_out_f16, void* s_out_f16, int32_t* rank_idx_out,
+                        int32_t* tile_meta_out, int32_t* slab_meta_out, void* stream);
 
 #ifdef __cplusplus
 }

@@ -80,6 +80,46 @@ def test_quantiser_and_slab_packer_kernels(cuda_device, bits, k, dim):
     assert np.array_equal(scale16.cpu().numpy(), np.concatenate(sc_ref))
 
 
+@pytest.mark.parametrize("dim,segs", [
+    (128, [(2, (0, 1))]),                                                                    # one row
+    (160, [(16, (0, 3)), (4, (3, 70)), (1, (70, 199)), (3, (210, 211)), (2, (211, 340))]),   # widths mixed in a wavefront, tail tile
+    (96, [((2, 3, 4, 6, 8)[i % 5], (2 * i, 2 * i + 1)) for i in range(150)]),                # more ranges than one launch carries
+])
+def test_whole_matrix_packer_equals_quantiser_and_slab_packer(cuda_device, dim, segs):
+    """bitsmoe_pack_matrix against the two single kernels, width by width: the same words and scales bit for bit."""
+    import torch
+
+    from bitsmoe_amd.algorithms import mlp_forward_cuda as hip
+    from bitsmoe_amd.quant.packer import pack_rank_major
+
+    rng = np.random.default_rng(dim + len(segs))
+    rank = max(e for _, (_, e) in segs) + 2
+    x = torch.from_numpy(rng.normal(0, 0.02, size=(rank, dim)).astype(np.float32)).to(cuda_device)
+    bufs = pack_rank_major(x, torch.ones(rank, device=cuda_device), segs)
+    rows, words, scales = [], [], []
+    for bits in sorted({b for b, _ in segs}, reverse=True):
+        idx = torch.cat([torch.arange(s, e) for b, (s, e) in sorted(segs, key=lambda v: v[1]) if b == bits])
+        rows.append(idx)
+        part = x[idx.to(cuda_device)].contiguous()
+        if bits == 16:      # halves as they are; the other kernels have no 16-bit form
+            words.append(None)
+            scales.append(torch.ones(len(idx) * ((dim + 127) // 128), dtype=torch.float16, device=cuda_device))
+            continue
+        levels, scale = hip.quantize_tiles(part, bits)
+        pay, sc = hip.pack_slabs(levels, scale, dim, bits)
+        words.append(pay.view(torch.int32))
+        scales.append(sc)
+    assert torch.equal(bufs["rank_idx_buffer"].cpu(), torch.cat(rows).to(torch.int32))
+    assert torch.equal(bufs["scale_buffer"], torch.cat(scales))
+    got, at = bufs["payload_buffer"].view(torch.int32), 0
+    for part, idx in zip(words, rows):
+        n = len(idx) * ((dim + 127) // 128) * 64 if part is None else part.numel()
+        if part is not None:
+            assert torch.equal(got[at:at + n], part)
+        at += n
+    assert at == got.numel()
+
+
 def test_batched_uniform_packer_equals_general_packer(cuda_device):
     import torch
 
