@@ -12,9 +12,8 @@
 //   k_combine_tokens rank_accum[t, rank_idx[r]] = sum over the assignments of t of route_w * y
 //
 // Both GEMM kernels use 16x16x32 f16 MFMA with four wavefronts of 128 rows x 64 columns per
-// workgroup.  The activation operand is staged through LDS in 128 x 64 pieces (double
-// buffered, one barrier per piece); the weight operand never touches LDS: every lane loads
-// its words of the prepared payload (wave_layout.h) and expands them to packed f16 pairs
+// workgroup.  Activations, payload words and scales come straight from global memory into a ring of LDS stages; every lane
+// takes its words of the prepared payload (wave_layout.h) from there and expands them to packed f16 pairs
 // (2^w + code) with a rotate and an and-or; a packed add and a packed multiply turn the pair
 // into (code - 2^(w-1)) * scale (gate/up: scale * s, folded once at prepare time) -- the same
 // "weight rounded to half" operand the reference's tensor-core path builds
@@ -242,11 +241,6 @@ __device__ inline int xcd_logical(int bid, int n_tiles_real, int units) {
     return tile * units + slot % units;
 }
 
-// 128 x 64 16-bit activation piece: thread i owns rows i/8 + 32*j (j = 0..3), elements 8*(i%8)..+7.
-// NJ: how many of the four 32-row groups hold assignments (tiles of at most 32 rows: one).
-struct APiece {
-    u32x4 v[4];
-};
 // LDS element offset of the 16-byte chunk c (0..7) of row r of a 128 x 64 stage: rows are 128
 // bytes apart without padding, and the chunks of a row are permuted by the row index so that the
 // sixteen rows an MFMA operand load touches fall into different banks.  (LDS-direct loads fill
@@ -284,13 +278,6 @@ __device__ __forceinline__ void load_to_lds16(const void* src, void* lds_base) {
 }
 
 // ------------------------------------------------------------------------------ gate / up
-
-// Everything one thread fetches from global memory for one slab.
-struct GuFetch {
-    APiece a;          // this thread's part of the 128 x 64 activation piece
-    u32x4 sc[2];       // scale pairs of the eight contraction rows this lane feeds per k-step (its own tile)
-    uint32_t bw[2][4]; // payload words of the wavefront's two column-block pairs (its own tile)
-};
 
 // One slab (64 contraction rows, `bits` wide) for a wavefront's (16 * NMB) x 64 tile.  The weight
 // operand is (code - 2^(bits-1)) * scale_s rounded once to f16 -- the operand the reference
@@ -332,167 +319,30 @@ __device__ __forceinline__ void gateup_slab_mfma(int bits, const uint16_t* __res
 #pragma unroll
             for (int i = 0; i < 4; ++i) b[i] = pk_mul_f16(pk_add_f16(b[i], neg[i]), sc[ks][i]);
 #pragma unroll
-            for (int mb = 0; mb < NMB; ++mb) acc[mb][nb] = mfma16<false>(a[mb], b, acc[mb][nb]);
+            for (int mb = 0; mb < NMB; ++mb) acc[mb][nb] = mfma16<false>(b, a[mb], acc[mb][nb]);
         }
     }
 }
 
-// One workgroup = (assignment tile, projection, PAIR of 128-column tiles):
-// out[a, c] = f16 of sum_k A[a, k] * f16(level[k, c] * scale_s[tile(c), k]) over all slabs of the matrix.
-// Wavefront (tl, wn) owns all assignments of the tile and columns 64*wn .. +63 of tile t0 + tl: a
-// decoded weight operand feeds NMB MFMAs.  The activation piece of a slab (128 x 64) is staged in
-// LDS once for both tiles; the loads of slab s + 2 are issued before slab s is multiplied.
-//
-// DIRECT: the activation rows are read straight from the f16 activations [T, ld] through the
-// token index (possible when every aligned run of 8 local rows is 8 consecutive logical ranks);
-// otherwise Hs is the pre-gathered [A, ld].  WU: the bit-width shared by every slab of the
-// matrix, or 0 (mixed).  NMB: 16-row blocks of the assignment tile that are computed.
-template <bool DIRECT, int WU, int NMB>
-__device__ __forceinline__ void gateup_tile_body(const FastExpert fe, const FastSlab* __restrict__ fs_row, int nslabs,
-                                                 const uint16_t* __restrict__ Hs, int ld,
-                                                 const int32_t* __restrict__ token_indices, int T, int I, int n_tiles,
-                                                 uint16_t* __restrict__ out, int a_begin, int rows, int t0,
-                                                 uint16_t* __restrict__ stage_even, uint16_t* __restrict__ stage_odd,
-                                                 bool fuse_silu) {
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int tl = wave >> 1, wn = wave & 1;
+// The epilogue of both GEMM kernels.  The weights are the MFMA's first operand, so that a lane holds, of assignment
+// 16 mb + lane % 16, outputs 16 nb + 4 (lane / 16) + j: four neighbouring ones.  A wavefront turns its 16 * NMB x 64 block
+// around in 16 KB of LDS of its own (`turn`), so that a store instruction writes eight whole 128-byte rows: stores of the
+// registers as they are touch 32 or 64 cache lines per instruction, and their address work was 8 us of the 205 us gate/up
+// launch (4096 tokens, 128 experts).  put(row, chunk, 8 values) stores one 16-byte piece.
+template <int NMB, class Put>
+__device__ __forceinline__ void store_turned(uint16_t* __restrict__ turn, int rows, int lane, const f32x4 (&acc)[NMB][4], Put&& put) {
     const int n = lane & 15, kg = lane >> 4;
-    const bool two_tiles = t0 + 1 < n_tiles;
-    const bool active = tl == 0 || two_tiles;        // a wavefront without a tile only helps to stage
-    const int t = active ? t0 + tl : t0;             // (it re-reads tile t0: in bounds)
-
-    // this thread's staging rows; DIRECT: their activation rows (invalid tokens read row 0: the
-    // combine drops their outputs).  Element offsets: the launcher checks that they fit 32 bits.
-    constexpr int NJ = (NMB + 1) / 2;      // 32-row groups that hold assignments
-    const int r0 = tid >> 3, kc = (tid & 7) * 8;
-    uint32_t rowbase[NJ];
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-        const int a = a_begin + min(r0 + 32 * j, rows - 1);
-        if constexpr (DIRECT) {
-            const int tk = token_indices[a];
-            rowbase[j] = (uint32_t)((tk >= 0 && tk < T) ? tk : 0) * (uint32_t)ld;
-        } else {
-            rowbase[j] = (uint32_t)a * (uint32_t)ld + (uint32_t)kc;
+    for (int mb = 0; mb < NMB; ++mb)
+#pragma unroll
+        for (int nb = 0; nb < 4; ++nb) {
+            const u32x2 v = {f16_pair(acc[mb][nb][0], acc[mb][nb][1]), f16_pair(acc[mb][nb][2], acc[mb][nb][3])};
+            *reinterpret_cast<u32x2*>(turn + dma_chunk_off(16 * mb + n, 2 * nb + (kg >> 1)) + 4 * (kg & 1)) = v;
         }
-    }
-
-    f32x4 acc[NMB][4];
 #pragma unroll
-    for (int i = 0; i < NMB; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0, 0, 0, 0};
-    gptr<uint32_t> payload = as_global(fe.payload);
-    gptr<__half> scale = as_global(fe.scale_s);
-    gptr<int32_t> rank_idx = as_global(fe.rank_idx);
-    GuFetch F;                 // the one slab in flight
-    auto slab_rec = [&](int s) { return s < nslabs ? load_fast_slab(fs_row, s) : FastSlab{0, 0, 0, 0}; };
-    auto rank_base = [&](int s) { return (DIRECT && s < nslabs) ? rank_idx[s * SLAB_ROWS + kc] : 0; };
-    auto issue = [&](GuFetch& dst, const FastSlab& r, int rbase, int s) {
-        const int wb = WU != 0 ? WU : r.bits;
-        const uint32_t col = DIRECT ? (uint32_t)rbase : (uint32_t)(s * SLAB_ROWS);
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) dst.a.v[j] = *reinterpret_cast<const u32x4*>(Hs + (rowbase[j] + col));
-        // the MFMA operand of k-step ks holds contraction rows 16*kg + 8*ks .. +7 of the slab
-        gptr<__half> sp = scale + (uint32_t)(r.scale_off + t * SLAB_ROWS + 16 * kg);
-        dst.sc[0] = *reinterpret_cast<gptr_u32x4>(sp);
-        dst.sc[1] = *reinterpret_cast<gptr_u32x4>(sp + 8);
-        gptr<uint32_t> blk = payload + (uint32_t)(r.pack_off + t * 256 * wb);
-#pragma unroll
-        for (int p = 0; p < 2; ++p) {
-            const int pair = 2 * wn + p;
-            load_pair_role0(blk, wb, (uint32_t)(pair * 64 + lane), (uint32_t)hi_index0(kg, n, 2 * pair), dst.bw[p]);
-        }
-    };
-    auto stage_piece = [&](const GuFetch& src, uint16_t* __restrict__ stage) {
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) *reinterpret_cast<u32x4*>(stage + dma_chunk_off(r0 + 32 * j, tid & 7)) = src.a.v[j];
-    };
-    if (nslabs > 0) {
-        // prologue: slab 0 is fetched and staged, slab 1 requested
-        uint32_t bw[2][4];       // payload words and scales of the slab being multiplied
-        u32x4 sc[2];
-        FastSlab rec = slab_rec(0);
-        FastSlab pending = slab_rec(1);
-        int pending_rb = rank_base(1);
-        int bits = rec.bits;
-        issue(F, rec, rank_base(0), 0);
-        stage_piece(F, stage_even);
-#pragma unroll
-        for (int p = 0; p < 2; ++p) {
-            sc[p] = F.sc[p];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) bw[p][i] = F.bw[p][i];
-        }
-        int bits_next = pending.bits;
-        if (nslabs > 1) {
-            issue(F, pending, pending_rb, 1);
-            pending = slab_rec(2);
-            pending_rb = rank_base(2);
-        }
-        __syncthreads();
-        // step s: slab s is in LDS stage s % 2 with its words in `bw`; slab s + 1 (in flight in F) is
-        // staged, slab s + 2 requested, then slab s is multiplied
-        for (int s = 0; s < nslabs; ++s) {
-            uint32_t bw_next[2][4];
-            u32x4 sc_next[2];
-            const int bits_after = pending.bits;
-            if (s + 1 < nslabs) {
-                stage_piece(F, (s & 1) ? stage_even : stage_odd);
-#pragma unroll
-                for (int p = 0; p < 2; ++p) {
-                    sc_next[p] = F.sc[p];
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) bw_next[p][i] = F.bw[p][i];
-                }
-                if (s + 2 < nslabs) {
-                    issue(F, pending, pending_rb, s + 2);
-                    pending = slab_rec(s + 3);
-                    pending_rb = rank_base(s + 3);
-                }
-            }
-            if (active && bits != 0)
-                gateup_slab_mfma<WU, NMB>(bits, (s & 1) ? stage_odd : stage_even, bw, sc, lane, acc);
-            __syncthreads();
-            if (s + 1 < nslabs) {
-#pragma unroll
-                for (int p = 0; p < 2; ++p) {
-                    sc[p] = sc_next[p];
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) bw[p][i] = bw_next[p][i];
-                }
-                bits = bits_next;
-                bits_next = bits_after;
-            }
-        }
-    }
-    if (!active) return;
-    // lane holds rows 16*mb + 4*kg + j, column 128*t + 64*wn + 16*nb + n
-#pragma unroll
-    for (int mb = 0; mb < NMB; ++mb) {
-        if (16 * mb >= rows) break;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int row = 16 * mb + 4 * kg + j;
-            if (row >= rows) continue;
-            uint16_t* dst = out + (int64_t)(a_begin + row) * I + N_TILE * t + 64 * wn + n;
-            if (fuse_silu) {
-                // `out` holds the gate sums an earlier launch stored: z = silu(gate) * up takes their place
-                uint16_t gbits[4];
-#pragma unroll
-                for (int nb = 0; nb < 4; ++nb) gbits[nb] = dst[16 * nb];
-#pragma unroll
-                for (int nb = 0; nb < 4; ++nb) {
-                    const float g = __half2float(__ushort_as_half(gbits[nb]));
-                    dst[16 * nb] = z_operand(g, acc[mb][nb][j]);
-                }
-                continue;
-            }
-#pragma unroll
-            for (int nb = 0; nb < 4; ++nb) dst[16 * nb] = __builtin_bit_cast(uint16_t, (_Float16)acc[mb][nb][j]);
-        }
+    for (int k = 0; k < 2 * NMB; ++k) {
+        const int row = 8 * k + (lane >> 3);
+        if (row < rows) put(row, lane & 7, *reinterpret_cast<const u32x4*>(turn + dma_chunk_off(row, lane & 7)));
     }
 }
 
@@ -508,21 +358,30 @@ struct DmaStage {
     uint16_t* sc;    // [DMA_SSTAGE]
 };
 
-// The same workgroup job as gateup_tile_body for experts of one bit-width, with EVERYTHING of a
-// slab -- activation piece, payload words, scales -- loaded straight from global memory into LDS
+// One workgroup = (assignment tile, projection, PAIR of 128-column tiles):
+// out[a, c] = f16 of sum_k A[a, k] * f16(level[k, c] * scale_s[tile(c), k]) over all slabs of the matrix.
+// Wavefront (tl, wn) owns all assignments of the tile and columns 64*wn .. +63 of tile t0 + tl: a
+// decoded weight operand feeds NMB MFMAs.  EVERYTHING of a slab -- the activation piece (128 x 64, shared by both tiles),
+// payload words, scales -- is loaded straight from global memory into LDS
 // (global_load_lds: no registers, no staging instructions), two slabs ahead of the MFMAs in a ring
 // of three stages.  A wavefront's load instruction fills LDS in lane order; which 16-byte chunk of
 // its activation row a lane fetches is chosen so that the stage ends up in the bank-friendly order
 // of dma_chunk_off.  The loop contains no load into registers: the loads of a wavefront complete in
 // order, so "slab s + 1 has landed" is "at most the G loads of slab s + 2 are outstanding", waited
 // for with a bare s_waitcnt, and the workgroup barrier is the bare instruction (__syncthreads would
-// wait for every outstanding load).  Per-slab offsets come from small LDS tables built up front.
+// wait for every outstanding load).  Per-slab offsets come from small LDS tables built up front, for DMA_MAX_SLABS slabs
+// at a time.
+//
+// DIRECT: the activation rows are read straight from the f16 activations [T, ld] through the
+// token index (possible when every aligned run of 8 local rows is 8 consecutive logical ranks);
+// otherwise Hs is the pre-gathered [A, ld].  WU: the bit-width shared by every slab of the
+// matrix, or 0 (mixed).  NMB: 16-row blocks of the assignment tile that are computed.
 template <bool DIRECT, int WU, int NMB>
-__device__ __forceinline__ void gateup_tile_body_dma(const FastExpert fe, const FastSlab* __restrict__ fs_row, int nslabs,
+__device__ __forceinline__ void gateup_tile_body(const FastExpert fe, const FastSlab* __restrict__ fs_row, int all_slabs,
                                                      const uint16_t* __restrict__ Hs, int ld,
                                                      const int32_t* __restrict__ token_indices, int T, int I,
                                                      int n_tiles, uint16_t* __restrict__ out, int a_begin, int rows,
-                                                     int t0, const DmaStage st0, const DmaStage st1, const DmaStage st2,
+                                                     int t0, const DmaStage st0, const DmaStage st1, const DmaStage st2, uint16_t* __restrict__ turn,
                                                      int32_t* __restrict__ pack_tab, int32_t* __restrict__ scale_tab,
                                                      int32_t* __restrict__ rank_tab, int32_t* __restrict__ bits_tab,
                                                      bool fuse_silu) {
@@ -555,18 +414,7 @@ __device__ __forceinline__ void gateup_tile_body_dma(const FastExpert fe, const 
             rowbase[j] = (uint32_t)a * (uint32_t)ld + (uint32_t)(8 * cpos);
         }
     }
-    // per-slab tables (ordinary loads, finished before the first LDS-direct load is issued)
     gptr<int32_t> rank_idx = as_global(fe.rank_idx);
-    for (int i = tid; i < nslabs; i += 256) {
-        const i32x4 r = *reinterpret_cast<const i32x4*>(fs_row + i);     // {bits, pack_off, scale_off, rank_off}
-        pack_tab[i] = r[1];
-        scale_tab[i] = r[2];
-        if constexpr (WU == 0) bits_tab[i] = r[0];
-    }
-    if constexpr (DIRECT)
-        for (int i = tid; i < nslabs * 8; i += 256) rank_tab[i] = rank_idx[(i >> 3) * SLAB_ROWS + (i & 7) * 8];
-    __syncthreads();
-
     f32x4 acc[NMB][4];
 #pragma unroll
     for (int i = 0; i < NMB; ++i)
@@ -574,26 +422,39 @@ __device__ __forceinline__ void gateup_tile_body_dma(const FastExpert fe, const 
         for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0, 0, 0, 0};
     const uint32_t* __restrict__ payload = fe.payload;
     const __half* __restrict__ scale = fe.scale_s;
-    // all loads of slab s into stage `st`: G instructions for every wavefront
-    auto request = [&](const DmaStage& st, int s) {
-        const uint32_t col = DIRECT ? (uint32_t)rank_tab[s * 8 + cpos] : (uint32_t)(s * SLAB_ROWS);
+    // what the loads of a slab need from the tables: read a step before the loads are issued, so that their latency is not
+    // in front of them
+    struct SlabAt {
+        uint32_t col;
+        int32_t pack, scale, bits;
+    };
+    auto locate = [&](int s) {
+        SlabAt at;
+        at.col = DIRECT ? (uint32_t)rank_tab[s * 8 + cpos] : (uint32_t)(rank_tab[0] + s * SLAB_ROWS);
+        at.pack = pack_tab[s];
+        at.scale = scale_tab[s];
+        at.bits = WU == 0 ? bits_tab[s] : WU;
+        return at;
+    };
+    // all loads of a slab into stage `st`: G instructions for every wavefront
+    auto request = [&](const DmaStage& st, const SlabAt& at) {
 #pragma unroll
         for (int j = 0; j < NJ; ++j)
-            load_to_lds16(Hs + (rowbase[j] + col), st.a + j * 2048 + wave * 512);
+            load_to_lds16(Hs + (rowbase[j] + at.col), st.a + j * 2048 + wave * 512);
         // scales of this wavefront's tile: 64 contraction rows, eight lanes of 16 bytes
         if (lane < 8)
-            load_to_lds16(scale + (uint32_t)(scale_tab[s] + t * SLAB_ROWS + lane * 8), st.sc + wave * 64);
+            load_to_lds16(scale + (uint32_t)(at.scale + t * SLAB_ROWS + lane * 8), st.sc + wave * 64);
         // payload of the wavefront's two column-block pairs, in memory order
         if constexpr (WU == 0) {
-            const int W = __builtin_amdgcn_readfirstlane(bits_tab[s]);
-            const uint32_t* blk = payload + (uint32_t)(pack_tab[s] + t * 256 * W);
+            const int W = __builtin_amdgcn_readfirstlane(at.bits);
+            const uint32_t* blk = payload + (uint32_t)(at.pack + t * 256 * W);
             const uint32_t first = W == 4 ? (uint32_t)((2 * wn * 64 + lane) * 4) : (uint32_t)(2 * wn * 128 + lane * 4);
             const uint32_t second = W == 4 ? first + 256u : W == 3 ? (uint32_t)(512 + 2 * wn * 64 + lane * 4) : first;
             load_to_lds16(blk + first, st.w + wave * 512);
             if (W != 3 || lane < 32) load_to_lds16(blk + second, st.w + wave * 512 + 256);
             return;
         }
-        const uint32_t* blk = payload + (uint32_t)(pack_tab[s] + t * 256 * WU);
+        const uint32_t* blk = payload + (uint32_t)(at.pack + t * 256 * WU);
         if constexpr (WU == 4) {
 #pragma unroll
             for (int p = 0; p < 2; ++p)
@@ -627,9 +488,25 @@ __device__ __forceinline__ void gateup_tile_body_dma(const FastExpert fe, const 
         sc[0] = *reinterpret_cast<const u32x4*>(st.sc + wave * 64 + 16 * kg);
         sc[1] = *reinterpret_cast<const u32x4*>(st.sc + wave * 64 + 16 * kg + 8);
     };
-    if (nslabs > 0) {
-        request(st0, 0);
-        if (nslabs > 1) request(st1, 1);
+    for (int c0 = 0; c0 < all_slabs; c0 += DMA_MAX_SLABS) {
+        const int nslabs = min(DMA_MAX_SLABS, all_slabs - c0);
+        // per-slab tables (ordinary loads, finished before the first LDS-direct load is issued)
+        if (c0 > 0) barrier_no_drain();      // (every wavefront has read its last entries)
+        for (int i = tid; i < nslabs; i += 256) {
+            const i32x4 r = *reinterpret_cast<const i32x4*>(fs_row + c0 + i);     // {bits, pack_off, scale_off, rank_off}
+            pack_tab[i] = r[1];
+            scale_tab[i] = r[2];
+            if constexpr (WU == 0) bits_tab[i] = r[0];
+        }
+        if constexpr (DIRECT)
+            for (int i = tid; i < nslabs * 8; i += 256)
+                rank_tab[i] = rank_idx[(c0 + (i >> 3)) * SLAB_ROWS + (i & 7) * 8];
+        else if (tid == 0)
+            rank_tab[0] = c0 * SLAB_ROWS;
+        __syncthreads();
+        request(st0, locate(0));
+        if (nslabs > 1) request(st1, locate(1));
+        SlabAt ahead = locate(min(2, nslabs - 1));
         if (nslabs > 1)
             wait_vmcnt<G>();
         else
@@ -647,7 +524,10 @@ __device__ __forceinline__ void gateup_tile_body_dma(const FastExpert fe, const 
             u32x4 sc[2];
             const int W = WU != 0 ? WU : __builtin_amdgcn_readfirstlane(bits_tab[s]);
             take(cur, W, bw, sc);
-            if (s + 2 < nslabs) request(nxt, s + 2);
+            if (s + 2 < nslabs) {
+                request(nxt, ahead);
+                ahead = locate(min(s + 3, nslabs - 1));
+            }
             if (active) gateup_slab_mfma<WU, NMB>(W, cur.a, bw, sc, lane, acc);
             asm volatile("" ::: "memory");
             if (s + 2 < nslabs)
@@ -664,31 +544,20 @@ __device__ __forceinline__ void gateup_tile_body_dma(const FastExpert fe, const 
     }
     BITSMOE_TLP(g_tl_pf_gateup, 3);
     if (!active) return;
-    // lane holds rows 16*mb + 4*kg + j, column 128*t + 64*wn + 16*nb + n
+    uint16_t* cols = out + (int64_t)a_begin * I + N_TILE * t + 64 * wn;
+    store_turned<NMB>(turn + wave * DMA_STAGE, rows, lane, acc, [&](int row, int c, u32x4 v) {
+        u32x4* dst = reinterpret_cast<u32x4*>(cols + (int64_t)row * I + 8 * c);
+        if (fuse_silu) {
+            // `out` holds the gate sums an earlier launch stored: z = silu(gate) * up takes their place
+            const u32x4 g = *dst;
 #pragma unroll
-    for (int mb = 0; mb < NMB; ++mb) {
-        if (16 * mb >= rows) break;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int row = 16 * mb + 4 * kg + j;
-            if (row >= rows) continue;
-            uint16_t* dst = out + (int64_t)(a_begin + row) * I + N_TILE * t + 64 * wn + n;
-            if (fuse_silu) {
-                // `out` holds the gate sums an earlier launch stored: z = silu(gate) * up takes their place
-                uint16_t gbits[4];
-#pragma unroll
-                for (int nb = 0; nb < 4; ++nb) gbits[nb] = dst[16 * nb];
-#pragma unroll
-                for (int nb = 0; nb < 4; ++nb) {
-                    const float g = __half2float(__ushort_as_half(gbits[nb]));
-                    dst[16 * nb] = z_operand(g, acc[mb][nb][j]);
-                }
-                continue;
+            for (int q = 0; q < 4; ++q) {
+                const h2 gp = __builtin_bit_cast(h2, (uint32_t)g[q]), up = __builtin_bit_cast(h2, (uint32_t)v[q]);
+                v[q] = z_operand((float)gp[0], (float)up[0]) | (uint32_t)z_operand((float)gp[1], (float)up[1]) << 16;
             }
-#pragma unroll
-            for (int nb = 0; nb < 4; ++nb) dst[16 * nb] = __builtin_bit_cast(uint16_t, (_Float16)acc[mb][nb][j]);
         }
-    }
+        *dst = v;
+    });
 }
 
 // grid.x = 32 * ceil(max_mtiles / 32) * (2 or 1 projections) * ceil(n_tiles / 2), 256 threads; G and U are f16 [A, I].
@@ -700,9 +569,9 @@ __global__ __launch_bounds__(256, 2) void k_gateup_mfma(
     const int32_t* __restrict__ token_indices, int T,
     const MTile* __restrict__ mtiles, const int32_t* __restrict__ n_mtiles, int I, int n_tiles,
     uint16_t* __restrict__ G, uint16_t* __restrict__ U, int proj_sel, int fuse) {
-    // The ring of the LDS-direct bodies; the register-staged body uses two of the activation stages.
-    __shared__ __attribute__((aligned(16))) uint16_t sa0[DMA_STAGE], sa1[DMA_STAGE], sa2[DMA_STAGE];
-    __shared__ __attribute__((aligned(16))) uint32_t sw0[DMA_WSTAGE], sw1[DMA_WSTAGE], sw2[DMA_WSTAGE];
+    // the ring (three activation stages, three payload stages), which the epilogue uses again: 16 KB per wavefront
+    __shared__ __attribute__((aligned(16))) uint16_t ring[DMA_STAGES * (DMA_STAGE + 2 * DMA_WSTAGE)];
+    static_assert(sizeof(ring) >= 4 * DMA_STAGE * sizeof(uint16_t), "the epilogue's space");
     __shared__ __attribute__((aligned(16))) uint16_t ss0[DMA_SSTAGE], ss1[DMA_SSTAGE], ss2[DMA_SSTAGE];
     __shared__ int32_t pack_tab[DMA_MAX_SLABS], scale_tab[DMA_MAX_SLABS], rank_tab[DMA_MAX_SLABS * 8], bits_tab[DMA_MAX_SLABS];
     BITSMOE_TLP(g_tl_pf_gateup, 0);
@@ -733,36 +602,26 @@ __global__ __launch_bounds__(256, 2) void k_gateup_mfma(
     // tiles of at most 32 / 64 / 96 assignments (experts that see few tokens, remainders) run a body
     // with a quarter / half / three quarters of the accumulators, MFMAs and staging; complete
     // bodies, so that no accumulator lives across the choice
-    const DmaStage st0 = {sa0, sw0, ss0}, st1 = {sa1, sw1, ss1}, st2 = {sa2, sw2, ss2};
+    uint32_t* sw = reinterpret_cast<uint32_t*>(ring + DMA_STAGES * DMA_STAGE);
+    const DmaStage st0 = {ring, sw, ss0}, st1 = {ring + DMA_STAGE, sw + DMA_WSTAGE, ss1},
+                   st2 = {ring + 2 * DMA_STAGE, sw + 2 * DMA_WSTAGE, ss2};
     BITSMOE_TLP(g_tl_pf_gateup, 1);
 #define BITSMOE_GU_BODY(W)                                                                                           \
     do {                                                                                                             \
         if (rows <= 32)                                                                                              \
-            gateup_tile_body_dma<DIRECT, W, 2>(fe, fs_row, nslabs, Hs, ld, token_indices, T, I, n_tiles, out,         \
-                                               a_begin, rows, 2 * tp, st0, st1, st2, pack_tab, scale_tab, rank_tab, bits_tab, fuse_silu); \
+            gateup_tile_body<DIRECT, W, 2>(fe, fs_row, nslabs, Hs, ld, token_indices, T, I, n_tiles, out,         \
+                                               a_begin, rows, 2 * tp, st0, st1, st2, ring, pack_tab, scale_tab, rank_tab, bits_tab, fuse_silu); \
         else if (rows <= 64)                                                                                         \
-            gateup_tile_body_dma<DIRECT, W, 4>(fe, fs_row, nslabs, Hs, ld, token_indices, T, I, n_tiles, out,         \
-                                               a_begin, rows, 2 * tp, st0, st1, st2, pack_tab, scale_tab, rank_tab, bits_tab, fuse_silu); \
+            gateup_tile_body<DIRECT, W, 4>(fe, fs_row, nslabs, Hs, ld, token_indices, T, I, n_tiles, out,         \
+                                               a_begin, rows, 2 * tp, st0, st1, st2, ring, pack_tab, scale_tab, rank_tab, bits_tab, fuse_silu); \
         else if (rows <= 96)                                                                                         \
-            gateup_tile_body_dma<DIRECT, W, 6>(fe, fs_row, nslabs, Hs, ld, token_indices, T, I, n_tiles, out,         \
-                                               a_begin, rows, 2 * tp, st0, st1, st2, pack_tab, scale_tab, rank_tab, bits_tab, fuse_silu); \
+            gateup_tile_body<DIRECT, W, 6>(fe, fs_row, nslabs, Hs, ld, token_indices, T, I, n_tiles, out,         \
+                                               a_begin, rows, 2 * tp, st0, st1, st2, ring, pack_tab, scale_tab, rank_tab, bits_tab, fuse_silu); \
         else                                                                                                         \
-            gateup_tile_body_dma<DIRECT, W, 8>(fe, fs_row, nslabs, Hs, ld, token_indices, T, I, n_tiles, out,         \
-                                               a_begin, rows, 2 * tp, st0, st1, st2, pack_tab, scale_tab, rank_tab, bits_tab, fuse_silu); \
+            gateup_tile_body<DIRECT, W, 8>(fe, fs_row, nslabs, Hs, ld, token_indices, T, I, n_tiles, out,         \
+                                               a_begin, rows, 2 * tp, st0, st1, st2, ring, pack_tab, scale_tab, rank_tab, bits_tab, fuse_silu); \
     } while (0)
-    // experts with more slabs than the tables hold take the register-staged body
-#define BITSMOE_GU_BODY_MIXED()                                                                                      \
-    do {                                                                                                             \
-        if (rows <= 32)                                                                                              \
-            gateup_tile_body<DIRECT, 0, 2>(fe, fs_row, nslabs, Hs, ld, token_indices, T, I, n_tiles, out, a_begin,    \
-                                           rows, 2 * tp, sa0, sa1, fuse_silu);                                       \
-        else                                                                                                         \
-            gateup_tile_body<DIRECT, 0, 8>(fe, fs_row, nslabs, Hs, ld, token_indices, T, I, n_tiles, out, a_begin,    \
-                                           rows, 2 * tp, sa0, sa1, fuse_silu);                                       \
-    } while (0)
-    if (nslabs > DMA_MAX_SLABS)
-        BITSMOE_GU_BODY_MIXED();
-    else if (w == 2)
+    if (w == 2)
         BITSMOE_GU_BODY(2);
     else if (w == 3)
         BITSMOE_GU_BODY(3);
@@ -771,7 +630,6 @@ __global__ __launch_bounds__(256, 2) void k_gateup_mfma(
     else
         BITSMOE_GU_BODY(0);
 #undef BITSMOE_GU_BODY
-#undef BITSMOE_GU_BODY_MIXED
     BITSMOE_TLP(g_tl_pf_gateup, 6);
 }
 
@@ -831,7 +689,7 @@ __device__ __forceinline__ void down_half_mfma(int bits, const uint16_t* stage, 
             }
             for (int i = 0; i < 4; ++i) b[i] = pk_mul_f16(pk_add_f16(b[i], off), scp[nb]);
 #pragma unroll
-            for (int mb = 0; mb < NMB; ++mb) acc[mb][nb] = mfma16<false>(a[mb], b, acc[mb][nb]);
+            for (int mb = 0; mb < NMB; ++mb) acc[mb][nb] = mfma16<false>(b, a[mb], acc[mb][nb]);
         }
     }
 }
@@ -965,8 +823,8 @@ __device__ __forceinline__ void down_tile_loop(const uint32_t* __restrict__ payl
 
 // grid.x = 32 * ceil(max_mtiles / 32) * n_groups; workgroup = (assignment tile, group of four
 // slabs): wavefront w = all 128 assignments x the 64 output rows of slab 4*group + w.
-// Output: y[a, r] = s[r] * sum_c W_down[r, c] z[a, c] as f16, r in the expert's own row order
-// (row `A` of y takes the stores of a tile's unused rows), and the per-token assignment lists
+// Output: y[a, r] = s[r] * sum_c W_down[r, c] z[a, c] as f16, r in the expert's own row order, and the per-token
+// assignment lists
 // token_list[token_start[tok_a] + slot[a]] = (a, expert) that k_combine_tokens walks.
 __global__ __launch_bounds__(256, 2) void k_down_mfma(const FastExpert* __restrict__ down_fe,
                                                       const FastSlab* __restrict__ down_fs, int max_slabs,
@@ -977,8 +835,11 @@ __global__ __launch_bounds__(256, 2) void k_down_mfma(const FastExpert* __restri
                                                       const int32_t* __restrict__ token_start,
                                                       int2* __restrict__ token_list, int A, int I, int n_tiles,
                                                       int n_groups, _Float16* __restrict__ y, int ldy) {
-    __shared__ __attribute__((aligned(16))) uint16_t sz0[DMA_STAGE], sz1[DMA_STAGE], sz2[DMA_STAGE];
-    __shared__ __attribute__((aligned(16))) uint32_t wbuf[4 * DN_WBUF];
+    // three stages of z and the wavefronts' payload buffers, which the epilogue uses again: 16 KB per wavefront
+    __shared__ __attribute__((aligned(16))) uint16_t lds[3 * DMA_STAGE + 2 * 4 * DN_WBUF];
+    static_assert(sizeof(lds) >= 4 * DMA_STAGE * sizeof(uint16_t), "the epilogue's space");
+    uint16_t *sz0 = lds, *sz1 = lds + DMA_STAGE, *sz2 = lds + 2 * DMA_STAGE;
+    uint32_t* wbuf = reinterpret_cast<uint32_t*>(lds + 3 * DMA_STAGE);
     __shared__ __attribute__((aligned(16))) uint16_t sbuf[4 * DN_SBUF];
     BITSMOE_TLP(g_tl_pf_down, 0);
     const int logical = xcd_logical(blockIdx.x, __builtin_amdgcn_readfirstlane(*n_mtiles), n_groups);
@@ -1000,7 +861,7 @@ __global__ __launch_bounds__(256, 2) void k_down_mfma(const FastExpert* __restri
     if (DN_SLABS_MFMA * grp >= nslabs) return;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int n = lane & 15, kg = lane >> 4;
+    const int kg = lane >> 4;
     const int si = DN_SLABS_MFMA * grp + wave;
     FastSlab fs = FastSlab{0, 0, 0, 0};
     if (si < nslabs) fs = load_fast_slab(down_fs + (int64_t)e * max_slabs, si);
@@ -1020,23 +881,19 @@ __global__ __launch_bounds__(256, 2) void k_down_mfma(const FastExpert* __restri
         BITSMOE_TLP(g_tl_pf_down, 3);
         if (fs.bits == 0) return;
 
-        // lane holds assignments 16*mb + 4*kg + j, output rows 16*nb + n of the slab; the rows'
-        // multipliers s[r] go into y here, so that the combine reads one operand per assignment
-        float srow[4];
+        // the rows' multipliers s[r] go into y here, so that the combine reads one operand per assignment
 #pragma unroll
-        for (int nb = 0; nb < 4; ++nb) srow[nb] = __half2float(fe.s[fs.rank_off + 16 * nb + n]);
-        _Float16* ycol = y + fs.rank_off + n;
+        for (int nb = 0; nb < 4; ++nb) {
+            const u32x2 sw = *reinterpret_cast<const u32x2*>(fe.s + fs.rank_off + 16 * nb + 4 * kg);
+            const h2 s01 = __builtin_bit_cast(h2, (uint32_t)sw[0]), s23 = __builtin_bit_cast(h2, (uint32_t)sw[1]);
+            const f32x4 srow = {(float)s01[0], (float)s01[1], (float)s23[0], (float)s23[1]};
 #pragma unroll
-        for (int mb = 0; mb < NMB; ++mb) {
-            if (16 * mb >= rows) break;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int r = 16 * mb + 4 * kg + j;
-                _Float16* dst = ycol + (int64_t)(r < rows ? a_begin + r : A) * ldy;
-#pragma unroll
-                for (int nb = 0; nb < 4; ++nb) dst[16 * nb] = (_Float16)(acc[mb][nb][j] * srow[nb]);
-            }
+            for (int mb = 0; mb < NMB; ++mb) acc[mb][nb] *= srow;
         }
+        _Float16* block = y + (int64_t)a_begin * ldy + fs.rank_off;
+        store_turned<NMB>(lds + wave * DMA_STAGE, rows, lane, acc, [&](int row, int c, u32x4 v) {
+            *reinterpret_cast<u32x4*>(block + (int64_t)row * ldy + 8 * c) = v;
+        });
     };
     if (rows <= 32)
         run(std::integral_constant<int, 2>{});
@@ -1203,7 +1060,7 @@ static MfmaWorkspace mfma_workspace(const bitsmoe_matset* gate, const bitsmoe_ma
     w.acts = take(std::max(direct_ok(gate, up) ? direct : 0, gathered));
     w.z = take((size_t)A * I * 2);
     w.u = take((size_t)A * I * 2);
-    w.y = take((size_t)(A + 1) * down->prep_max_slabs * SLAB_ROWS * 2);
+    w.y = take((size_t)A * down->prep_max_slabs * SLAB_ROWS * 2);
     w.total = at;
     return w;
 }

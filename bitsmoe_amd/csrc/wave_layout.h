@@ -297,6 +297,12 @@ __device__ inline uint16_t to_operand(float v) {
     }
 }
 
+// two fp32 values as a packed f16 pair, each rounded to nearest even
+__device__ __forceinline__ uint32_t f16_pair(float lo, float hi) {
+    const h2 v = {(_Float16)lo, (_Float16)hi};
+    return __builtin_bit_cast(uint32_t, v);
+}
+
 // z = silu(g) * u as a 16-bit MFMA operand: the product rounded to fp32, THEN to 16 bits -- the two steps of the
 // reference's __float2half(silu(g) * u) (the tensor-core down kernel's operand, bitsmoe/algorithms/cpp/mlp_forward.cu).
 // Left to itself the compiler folds product and conversion into one instruction with a single rounding wherever it sees
