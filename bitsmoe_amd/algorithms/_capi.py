@@ -54,6 +54,8 @@ EXPORTED_SYMBOLS = (
     "bitsmoe_moe_forward_routed",
     "bitsmoe_forward_routed_is_inline",
     "bitsmoe_forward_decode_is_fused",
+    "bitsmoe_block_workspace_bytes",
+    "bitsmoe_block_forward",
     "bitsmoe_profile_create",
     "bitsmoe_profile_destroy",
     "bitsmoe_profile_read",
@@ -80,6 +82,20 @@ class MatrixDesc(Structure):
         ("num_slabs", c_int32),
         ("reserved", c_int32),
     ]
+
+
+ROUTER_LOGITS, ROUTER_LINEAR, ROUTER_CALLER = 0, 1, 2
+BLOCK_PROJECT_IN, BLOCK_PROJECT_OUT = 1, 2
+
+
+class BlockPlan(Structure):
+    _fields_ = [(n, c_void_p) for n in (
+        "gate", "up", "down", "global_to_local", "local_to_global", "super_gate", "super_up", "super_down",
+        "super_global_to_local", "super_local_to_global", "w_in", "w_out", "w_router")] + [(n, c_int32) for n in (
+            "w_in_prepared", "w_out_prepared", "act_dtype", "hidden", "in_features", "rank_gate", "rank_up", "rank_out",
+            "intermediate_size", "super_intermediate", "top_k", "n_global", "router_form", "renormalize", "round_dtype",
+            "col_gate", "col_up", "col_logits", "col_shared_gate", "col_shared_up", "col_shared_logit",
+            "shared_intermediate")] + [("weight_scale", c_float)]
 
 
 _lib = None
@@ -176,6 +192,11 @@ def load() -> ctypes.CDLL:
         c_void_p, c_int32, c_void_p, c_int32, c_void_p, c_int32, c_void_p, c_int32, c_int32, c_int32, c_int32,
         c_void_p, c_void_p, c_size_t, c_void_p, c_void_p,
     ]
+    lib.bitsmoe_block_workspace_bytes.restype = c_size_t
+    lib.bitsmoe_block_workspace_bytes.argtypes = [c_void_p, c_int64]
+    lib.bitsmoe_block_forward.restype = c_int32
+    lib.bitsmoe_block_forward.argtypes = [c_void_p, c_void_p, c_int64, c_int64, c_void_p, c_int32, c_void_p, c_void_p, c_void_p,
+                                          c_void_p, c_void_p, c_size_t, c_void_p, c_void_p]
     lib.bitsmoe_profile_create.restype = c_int32
     lib.bitsmoe_profile_create.argtypes = [POINTER(c_void_p)]
     lib.bitsmoe_profile_destroy.restype = None

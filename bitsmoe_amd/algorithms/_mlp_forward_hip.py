@@ -34,8 +34,24 @@ def set_option(name: str, value: int = -1) -> None:
     _capi.check(_lib.bitsmoe_set_option(name.encode(), int(value)))
 
 
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)      # (without a Stream object per call)
+
+
 def _stream_ptr(device: torch.device) -> int:
+    if _raw_stream is not None and device.index is not None:
+        return _raw_stream(device.index)
     return int(torch.cuda.current_stream(device).cuda_stream)
+
+
+def _on(device: torch.device, fn, *args) -> None:
+    """fn(*args) of the library with `device` current; raises what it reports."""
+    if device.index == torch.cuda.current_device():
+        rc = fn(*args)
+    else:
+        with torch.cuda.device(device):
+            rc = fn(*args)
+    if rc != 0:
+        _capi.check(rc)
 
 
 def _check(cond: bool, msg: str) -> None:
@@ -646,6 +662,8 @@ def prepared_linear_weight_of(owner, weight: torch.Tensor) -> "PreparedLinearWei
 
 
 SKINNY_LINEAR_MAX_ROWS = 64
+ROUTER_LOGITS, ROUTER_LINEAR, ROUTER_CALLER = _capi.ROUTER_LOGITS, _capi.ROUTER_LINEAR, _capi.ROUTER_CALLER
+BLOCK_PROJECT_IN, BLOCK_PROJECT_OUT = _capi.BLOCK_PROJECT_IN, _capi.BLOCK_PROJECT_OUT
 
 
 class PreparedLinearWeight:
@@ -740,6 +758,65 @@ def block_finish(rank_accum: torch.Tensor, dtype: torch.dtype, shared_gate_out: 
             shared_gate_logit.data_ptr() if (i_sh and shared_gate_logit is not None) else None, ld_g,
             _capi.DT_F16 if dtype == torch.float16 else _capi.DT_BF16, out.data_ptr(), r + i_sh, _stream_ptr(dev)))
     return out
+
+
+class BlockPlan:
+    """What one layer keeps for bitsmoe_block_forward: the C structure, and everything it points to."""
+
+    def __init__(self, sets: Sequence[MatrixSet], global_to_local: torch.Tensor, local_to_global: torch.Tensor,
+                 super_sets: Sequence[MatrixSet] = (), super_maps: Sequence[torch.Tensor] = (), **fields):
+        for group in (sets, super_sets):
+            if _AUTO_PREPARE and group and all(ms.role < 0 and ms.fast_capable for ms in group):
+                for ms, role in zip(group, (0, 0, 1)):
+                    ms.prepare(role)
+        self._sets = tuple(sets) + tuple(super_sets)
+        self._handles = tuple(ms._handle for ms in self._sets)
+        self._keep = (global_to_local, local_to_global, tuple(super_maps))
+        self.device = sets[0].device
+        c = _capi.BlockPlan()
+        c.gate, c.up, c.down = (ms.handle.value for ms in sets)
+        c.global_to_local, c.local_to_global = global_to_local.data_ptr(), local_to_global.data_ptr()
+        if super_sets:
+            c.super_gate, c.super_up, c.super_down = (ms.handle.value for ms in super_sets)
+            c.super_global_to_local, c.super_local_to_global = (t.data_ptr() for t in super_maps)
+        for name, value in fields.items():
+            setattr(c, name, value)
+        self.c = c
+        self.address = ctypes.addressof(c)
+        self._bytes: dict = {}
+
+    def is_current(self) -> bool:
+        """False once a matrix set was rebuilt or closed."""
+        return all(ms._handle is h for ms, h in zip(self._sets, self._handles))
+
+    def set_weight(self, name: str, weight) -> None:
+        """w_in / w_out / w_router: a tensor or a PreparedLinearWeight of it."""
+        prepared = isinstance(weight, PreparedLinearWeight)
+        self._keep += (weight,)
+        if name != "w_router":
+            setattr(self.c, name + "_prepared", 1 if prepared else 0)
+        setattr(self.c, name, (weight.data if prepared else weight).data_ptr())
+
+    def workspace_bytes(self, n_tokens: int) -> int:
+        n = self._bytes.get(n_tokens)
+        if n is None:
+            if len(self._bytes) >= 256:
+                self._bytes.clear()
+            n = self._bytes[n_tokens] = int(_lib.bitsmoe_block_workspace_bytes(self.address, n_tokens))
+        return n
+
+
+def block_forward(plan: BlockPlan, x: torch.Tensor, proj: torch.Tensor, stages: int, out: torch.Tensor,
+                  selected: Optional[torch.Tensor] = None, weights: Optional[torch.Tensor] = None,
+                  super_out: Optional[torch.Tensor] = None, side_stream: int = 0) -> None:
+    """bitsmoe_block_forward on x's device and current stream (the tensors are the caller's to check)."""
+    dev = x.device
+    n_tokens = x.shape[0]
+    ws = _workspace(dev, plan.workspace_bytes(n_tokens))
+    _on(dev, _lib.bitsmoe_block_forward, plan.address, x.data_ptr(), x.stride(0) if n_tokens > 1 else x.shape[1], n_tokens,
+        proj.data_ptr(), stages, None if selected is None else selected.data_ptr(), None if weights is None else weights.data_ptr(),
+        out.data_ptr(), None if super_out is None else super_out.data_ptr(), ws.data_ptr(), ws.numel(), side_stream,
+        _stream_ptr(dev))
 
 
 # ----------------------------------------------------------------------------------------

@@ -67,29 +67,11 @@ _SKINNY_LONG_CONTRACTION = 4096   # input features up to which more than 16 rows
 _SKINNY_PREPARED = _os.environ.get("BITSMOE_BLOCK_SKINNY_PREPARED", "1") != "0"
 
 
-def _block_linear(x: torch.Tensor, plan: dict, key: str, addend: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """x [T, K] @ plan[key] [N, K].T (+ addend, fp32 [T, N]) in the weight's dtype.  At a few rows: the library's few-rows
-    kernel against a copy of the weight in MFMA operand order (made on first use, kept with the plan: one more copy of the
-    stacked weights), the addend taken in before the result is rounded."""
-    weight = plan[key]
-    rows = int(x.shape[0])
-    # (from 17 rows on only while there is about one workgroup per CU: every workgroup reads all rows of x)
-    n_out, n_in = int(weight.shape[0]), int(weight.shape[1])
-    few = 0 < rows <= _SKINNY_ROWS and (
+def _few_rows(rows: int, n_in: int, n_out: int) -> bool:
+    """Does the few-rows kernel run this GEMM?  (It takes contractions of whole 128 and an even number of outputs.)"""
+    return (0 < rows <= _SKINNY_ROWS and n_in % 128 == 0 and n_out % 2 == 0 and (
         rows <= 16 or (n_in <= _SKINNY_LONG_CONTRACTION
-                       and n_out <= (_SKINNY_WIDE_FEATURES if rows <= 32 else _SKINNY_NARROW_FEATURES)))
-    if few and _HAS_MLP_FORWARD_CUDA:
-        if _SKINNY_PREPARED:
-            prepared = plan.get(key + "_prepared")
-            if prepared is None and mlp_forward_cuda.skinny_linear_possible(x, weight):
-                prepared = mlp_forward_cuda.PreparedLinearWeight(weight)
-                plan[key + "_prepared"] = prepared
-            if prepared is not None and mlp_forward_cuda.skinny_linear_possible(x, prepared):
-                return mlp_forward_cuda.skinny_linear(x, prepared, addend)
-        if mlp_forward_cuda.skinny_linear_possible(x, weight):
-            return mlp_forward_cuda.skinny_linear(x, weight, addend)
-    out = x @ weight.T
-    return out if addend is None else out.add_(addend)
+                       and n_out <= (_SKINNY_WIDE_FEATURES if rows <= 32 else _SKINNY_NARROW_FEATURES))))
 
 
 _SIDE_STREAMS: Dict[int, "torch.cuda.Stream"] = {}
@@ -366,10 +348,7 @@ class BitsMoE_BaseSparseMoeBlock(nn.Module):
             return None
         dev = hidden_states.device
         g2l = self._super_global_to_local(dev)
-        l2g = self._basis_cache.get(("super_l2g", str(dev)))
-        if l2g is None:
-            l2g = torch.tensor([idx for idx, _ in self._super_expert_items], dtype=torch.int32, device=dev)
-            self._basis_cache[("super_l2g", str(dev))] = l2g
+        l2g = self._super_local_to_global(dev)
         (gate, up, down), inter = self._dense_sets_of("super", [layer for _, layer in self._super_expert_items], dev)
         x = hidden_states.contiguous()
         w32 = weights if weights.dtype == torch.float32 else weights.to(torch.float32)
@@ -385,6 +364,13 @@ class BitsMoE_BaseSparseMoeBlock(nn.Module):
                 g2l[idx] = local
             cached = g2l.to(device)
             self._basis_cache[("super_g2l", str(device))] = cached
+        return cached
+
+    def _super_local_to_global(self, device: torch.device) -> torch.Tensor:
+        cached = self._basis_cache.get(("super_l2g", str(device)))
+        if cached is None:
+            cached = torch.tensor([idx for idx, _ in self._super_expert_items], dtype=torch.int32, device=device)
+            self._basis_cache[("super_l2g", str(device))] = cached
         return cached
 
     def _dense_operator_forward(self, key: str, modules, hidden_states: torch.Tensor, token_indices: torch.Tensor,
@@ -526,41 +512,41 @@ class BitsMoE_BaseSparseMoeBlock(nn.Module):
     _FUSED_BLOCK = _os.environ.get("BITSMOE_FUSED_BLOCK", "1") != "0"
 
     @staticmethod
-    def _plain_linear(mod, in_features: Optional[int] = None) -> bool:
-        return (isinstance(mod, nn.Linear) and mod.bias is None and isinstance(mod.weight, torch.Tensor)
-                and mod.weight.dim() == 2 and (in_features is None or int(mod.weight.shape[1]) == in_features))
+    def _plain_linear(mod) -> bool:
+        return isinstance(mod, nn.Linear) and mod.bias is None and isinstance(mod.weight, torch.Tensor) and mod.weight.dim() == 2
 
     def _fused_plan(self, dtype: torch.dtype, router: Optional[nn.Module], shared: Optional[nn.Module],
                     shared_gate: Optional[nn.Module]):
         """The stacked input / output weights and the column ranges of their parts, or None when a module is not
         a bias-free linear layer of the expected shape.  Cached; rebuilt when a source tensor was rebound or written."""
-        hidden = int(self.shared_vh_gate_proj.shape[1])
-        sources = [self.shared_vh_gate_proj, self.shared_vh_up_proj, self.shared_u_down]
-        if router is not None:
-            if not self._plain_linear(router, hidden):
-                return None
-            sources.append(router.weight)
+        linears = [] if router is None else [router]
         if shared is not None:
-            projs = [getattr(shared, n, None) for n in ("gate_proj", "up_proj", "down_proj")]
-            if not (self._plain_linear(projs[0], hidden) and self._plain_linear(projs[1], hidden) and self._plain_linear(projs[2])
-                    and projs[0].weight.shape == projs[1].weight.shape
-                    and tuple(projs[2].weight.shape) == (hidden, int(projs[0].weight.shape[0]))
-                    and int(projs[0].weight.shape[0]) % 8 == 0):
-                return None
-            sources += [p.weight for p in projs]
-            if shared_gate is not None:
-                if not (self._plain_linear(shared_gate, hidden) and int(shared_gate.weight.shape[0]) == 1):
-                    return None
-                sources.append(shared_gate.weight)
-        elif shared_gate is not None:
+            linears += [getattr(shared, n, None) for n in ("gate_proj", "up_proj", "down_proj")]
+        if shared_gate is not None:
+            linears.append(shared_gate)
+        if not all(map(self._plain_linear, linears)):
             return None
-        if int(self.shared_u_down.shape[1]) % 8 or int(self.shared_vh_gate_proj.shape[0]) % 8 or int(self.shared_vh_up_proj.shape[0]) % 8:
-            return None
+        vh_gate, vh_up, u_down = (self._buffers[k] for k in self._SHARED_BASIS_BUFFER_KEYS)
+        sources = [vh_gate, vh_up, u_down] + [lin.weight for lin in linears]
         stamp = tuple((id(t), t.data_ptr(), -1 if t.is_inference() else t._version) for t in sources)
         key = ("fused_plan", dtype, router is not None, shared is not None, shared_gate is not None)
         cached = self._basis_cache.get(key)
         if cached is not None and cached["stamp"] == stamp:
             return cached
+        hidden = int(vh_gate.shape[1])
+        if router is not None and int(router.weight.shape[1]) != hidden:
+            return None
+        if shared is not None:
+            wg, wu, wd = (getattr(shared, n).weight for n in ("gate_proj", "up_proj", "down_proj"))
+            if not (wg.shape == wu.shape and int(wg.shape[1]) == hidden and tuple(wd.shape) == (hidden, int(wg.shape[0]))
+                    and int(wg.shape[0]) % 8 == 0):
+                return None
+            if shared_gate is not None and tuple(shared_gate.weight.shape) != (1, hidden):
+                return None
+        elif shared_gate is not None:
+            return None
+        if int(u_down.shape[1]) % 8 or int(vh_gate.shape[0]) % 8 or int(vh_up.shape[0]) % 8:
+            return None
         parts, ranges, col = [], {}, 0
 
         def add(name, w):      # (every part starts on a multiple of 8 columns: 16-byte aligned rows of its range)
@@ -573,8 +559,8 @@ class BitsMoE_BaseSparseMoeBlock(nn.Module):
             ranges[name] = (col, col + int(w.shape[0]) - pad)
             col += int(w.shape[0])
 
-        add("h_gate", self.shared_vh_gate_proj)
-        add("h_up", self.shared_vh_up_proj)
+        add("h_gate", vh_gate)
+        add("h_up", vh_up)
         if router is not None:
             add("logits", router.weight)
         i_sh = 0
@@ -585,7 +571,7 @@ class BitsMoE_BaseSparseMoeBlock(nn.Module):
             if shared_gate is not None:
                 add("sh_logit", shared_gate.weight)
         w_in = torch.cat(parts, dim=0).contiguous()
-        outs = [self.shared_u_down.detach().to(dtype)]
+        outs = [u_down.detach().to(dtype)]
         if shared is not None:
             outs.append(shared.down_proj.weight.detach().to(dtype))
         w_out = torch.cat(outs, dim=1).contiguous()      # [hidden, rank_out + I_sh]
@@ -593,78 +579,122 @@ class BitsMoE_BaseSparseMoeBlock(nn.Module):
         self._basis_cache[key] = cached
         return cached
 
-    def _fused_block_forward(self, hidden_states: torch.Tensor, *, router: Optional[nn.Module] = None, route_fn=None,
+    def _native_plan(self, plan: dict, dtype: torch.dtype, form: int, round_weights: bool, renormalize: bool, weight_scale: float,
+                     router_weight) -> "mlp_forward_cuda.BlockPlan":
+        """The library's plan of this block (bitsmoe_block_forward), kept with the stacked weights and remade when a
+        matrix set, the id maps or the routing's form changed."""
+        sets = self._ensure_matsets()
+        stamp = (sets, self._packed_global_to_local, form, round_weights, renormalize, weight_scale, router_weight,
+                 self.top_k, _super_via_operator())
+        native, seen = plan.get("native", (None, ()))
+        if native is not None and len(seen) == len(stamp) and all(
+                a is b or (not isinstance(a, (tuple, torch.Tensor)) and a == b) for a, b in zip(seen, stamp)) and native.is_current():
+            return native
+        rng = plan["ranges"]
+        dev = self._packed_global_to_local.device
+        super_sets, super_maps, super_inter = (), (), 0
+        if self._super_expert_items and _super_via_operator():
+            super_sets, super_inter = self._dense_sets_of("super", [layer for _, layer in self._super_expert_items], dev)
+            super_maps = (self._super_global_to_local(dev), self._super_local_to_global(dev))
+        native = mlp_forward_cuda.BlockPlan(
+            sets, self._packed_global_to_local, self._packed_local_to_global, super_sets, super_maps,
+            act_dtype=0 if dtype == torch.float16 else 1, hidden=int(plan["w_in"].shape[1]), in_features=int(plan["w_in"].shape[0]),
+            rank_gate=rng["h_gate"][1] - rng["h_gate"][0], rank_up=rng["h_up"][1] - rng["h_up"][0],
+            rank_out=int(plan["w_out"].shape[1]) - plan["i_sh"], intermediate_size=int(self._packed_intermediate_size),
+            super_intermediate=super_inter, top_k=int(self.top_k), n_global=int(self._packed_global_to_local.numel()),
+            router_form=form, renormalize=1 if renormalize else 0,
+            round_dtype=-1 if not round_weights else 0 if dtype == torch.float16 else 1, weight_scale=float(weight_scale),
+            col_gate=rng["h_gate"][0], col_up=rng["h_up"][0], col_logits=rng.get("logits", (0,))[0],
+            col_shared_gate=rng.get("sh_gate", (0,))[0], col_shared_up=rng.get("sh_up", (0,))[0],
+            col_shared_logit=rng.get("sh_logit", (-1,))[0], shared_intermediate=plan["i_sh"])
+        if router_weight is not None:
+            native.set_weight("w_router", router_weight)
+        plan["native"] = (native, stamp)
+        plan["few_rows_weights"] = {}
+        return native
+
+    def _few_rows_weight(self, plan: dict, native, key: str) -> None:
+        """The weight the few-rows kernel reads: a copy in MFMA operand order, made on first use and kept with the plan."""
+        if key not in plan["few_rows_weights"]:
+            weight = plan.get(key + "_prepared")
+            if weight is None:
+                weight = mlp_forward_cuda.PreparedLinearWeight(plan[key]) if _SKINNY_PREPARED else plan[key]
+                plan[key + "_prepared"] = weight
+            native.set_weight(key, weight)
+            plan["few_rows_weights"][key] = weight
+
+    def _fused_block_forward(self, hidden_states: torch.Tensor, *, router: Optional[nn.Module] = None, linear_gate=None, route_fn=None,
                              renormalize: bool = True, round_weights: bool = True, weight_scale: float = 1.0,
                              shared: Optional[nn.Module] = None, shared_gate: Optional[nn.Module] = None):
         """hidden [T, H] -> (output [T, H], router logits [T, E] or None), or None when this block cannot take the
         fused form (the caller then runs the module-by-module form).  `router`: the bias-free linear layer whose
         logits go through softmax / top-k (renormalize, weight_scale, round trip through the activation dtype);
-        otherwise `route_fn(hidden) -> (selected [T, k], weights fp32 [T, k])`."""
+        `linear_gate`: the prepared weight of a gate with fp32 logits (mlp_forward_cuda.router_linear_topk; the weights are
+        not rounded); otherwise `route_fn(hidden) -> (selected [T, k], weights fp32 [T, k])`."""
+        dtype = hidden_states.dtype
         if not (self._FUSED_BLOCK and hidden_states.is_cuda and _HAS_MLP_FORWARD_CUDA and self._packed_expert_count > 0
-                and self._packed_global_to_local is not None and hidden_states.dtype in (torch.float16, torch.bfloat16)
-                and not _dense_via_operator()):
+                and self._packed_global_to_local is not None and (dtype is torch.float16 or dtype is torch.bfloat16)
+                and self._packed_intermediate_size > 0 and not _dense_via_operator()):
             return None
-        if self.shared_vh_gate_proj.numel() == 0 or self.shared_vh_up_proj.numel() == 0 or self.shared_u_down.numel() == 0:
+        buffers = self._buffers
+        if any(buffers[k].numel() == 0 for k in self._SHARED_BASIS_BUFFER_KEYS):
             return None
         if router is not None and not (int(router.weight.shape[0]) <= 1024 and self.top_k <= 64):
             return None
-        dtype = hidden_states.dtype
+        self._act_type()
         plan = self._fused_plan(dtype, router, shared, shared_gate)
         if plan is None:
             return None
-        token_count = int(hidden_states.shape[0])
-        big = _block_linear(hidden_states, plan, "w_in")
-        rng = plan["ranges"]
-        h_gate = big[:, rng["h_gate"][0]:rng["h_gate"][1]]
-        h_up = big[:, rng["h_up"][0]:rng["h_up"][1]]
-        logits = None
-        if router is not None:
-            logits = big[:, rng["logits"][0]:rng["logits"][1]]
-            selected, weights = mlp_forward_cuda.router_softmax_topk(logits, self.top_k, renormalize,
-                                                                     round_dtype=dtype if round_weights else None,
-                                                                     weight_scale=weight_scale)
+        x = hidden_states
+        rows, hidden = x.shape
+        if x.stride(1) != 1 or (rows > 1 and x.stride(0) % 8 != 0) or x.data_ptr() % 16 != 0:
+            x = x.clone(memory_format=torch.contiguous_format)
+        form = (mlp_forward_cuda.ROUTER_LOGITS if router is not None else
+                mlp_forward_cuda.ROUTER_LINEAR if linear_gate is not None else mlp_forward_cuda.ROUTER_CALLER)
+        native = self._native_plan(plan, dtype, form, round_weights and linear_gate is None, renormalize, weight_scale, linear_gate)
+        w_in, w_out = plan["w_in"], plan["w_out"]
+        dev = x.device
+        stages = 0
+        if _few_rows(rows, hidden, w_in.shape[0]):
+            self._few_rows_weight(plan, native, "w_in")
+            proj = torch.empty((rows, w_in.shape[0]), dtype=dtype, device=dev)
+            stages |= mlp_forward_cuda.BLOCK_PROJECT_IN
         else:
+            proj = x @ w_in.T
+        selected = weights = sup = None
+        if form == mlp_forward_cuda.ROUTER_CALLER:
             selected, weights = route_fn(hidden_states)
-            selected = selected.reshape(token_count, self.top_k)
-            weights = weights.reshape(token_count, self.top_k).to(torch.float32)
-        rank_out = int(self.shared_u_down.shape[1])
-        gate, up, down = self._ensure_matsets()
+            selected = selected.reshape(rows, self.top_k).to(torch.int64).contiguous()
+            weights = weights.reshape(rows, self.top_k).to(torch.float32).contiguous()
+        super_modules = bool(self._super_expert_items) and not _super_via_operator()
+        if super_modules and selected is None:
+            selected = torch.empty((rows, self.top_k), dtype=torch.int64, device=dev)
+            weights = torch.empty((rows, self.top_k), dtype=torch.float32, device=dev)
+        if _few_rows(rows, w_out.shape[1], hidden):
+            self._few_rows_weight(plan, native, "w_out")
+            out = torch.empty((rows, hidden), dtype=dtype, device=dev)
+            stages |= mlp_forward_cuda.BLOCK_PROJECT_OUT
+        else:
+            out = torch.empty((rows, w_out.shape[1]), dtype=dtype, device=dev)
+            if self._super_expert_items and not super_modules:
+                sup = torch.empty((rows, hidden), dtype=torch.float32, device=dev)
         # The super experts' operator call needs the router's output and the hidden states only: it runs on a side
         # stream beside the packed experts' call (its small launches fill what the packed kernels leave idle).
-        sup, side = None, None
-        if self._super_expert_items and _SUPER_SIDE_STREAM and _super_via_operator():
-            side = _side_stream(hidden_states.device)
-            side.wait_stream(torch.cuda.current_stream(hidden_states.device))
-            with torch.cuda.stream(side):
-                sup = self._super_operator_output(hidden_states, selected, weights)
-        rank_accum = mlp_forward_cuda.moe_forward_routed(h_gate, h_up, selected, weights, self._packed_global_to_local,
-                                                         self._packed_local_to_global, gate, up, down, rank_out,
-                                                         int(self._packed_intermediate_size), self._act_type())
-        if shared is not None:
-            sh_logit = big[:, rng["sh_logit"][0]:rng["sh_logit"][1]] if shared_gate is not None else None
-            operand = mlp_forward_cuda.block_finish(rank_accum, dtype, big[:, rng["sh_gate"][0]:rng["sh_gate"][1]],
-                                                    big[:, rng["sh_up"][0]:rng["sh_up"][1]], sh_logit)
-        elif 0 < token_count <= min(_SKINNY_ROWS, 16) and mlp_forward_cuda.skinny_linear_possible(rank_accum, plan["w_out"]):
-            operand = rank_accum      # (fp32: the few-rows kernel rounds it to the activation dtype on its way in)
-        else:
-            operand = mlp_forward_cuda.block_finish(rank_accum, dtype)
-        if self._super_expert_items:
-            # (the super experts' share is ready long before the packed experts' call ends: joined here, it goes into the
-            # output GEMM's epilogue where the few-rows kernel runs, else it is added behind the GEMM)
-            if side is not None:
-                cur = torch.cuda.current_stream(hidden_states.device)
-                cur.wait_stream(side)
-                if sup is not None:
-                    sup.record_stream(cur)
-            else:
-                sup = self._super_operator_output(hidden_states, selected, weights)
-        out = _block_linear(operand, plan, "w_out", addend=sup)
-        if self._super_expert_items and sup is None:
+        side = _side_stream(dev).cuda_stream if self._super_expert_items and _SUPER_SIDE_STREAM and not super_modules else 0
+        mlp_forward_cuda.block_forward(native, x, proj, stages, out, selected, weights, sup, side)
+        if not stages & mlp_forward_cuda.BLOCK_PROJECT_OUT:
+            out = out @ w_out.T
+            if sup is not None:
+                out.add_(sup)
+        if super_modules:
             extra = torch.zeros_like(out)
-            self._run_super_experts(hidden_states, extra, selected.reshape(-1),
-                                    self._get_flat_token_ids(token_count, hidden_states.device),
+            self._run_super_experts(hidden_states, extra, selected.reshape(-1), self._get_flat_token_ids(rows, dev),
                                     weights.reshape(-1).to(dtype))
             out = out + extra
+        logits = None
+        if router is not None:
+            lo, hi = plan["ranges"]["logits"]
+            logits = proj[:, lo:hi]
         return out, logits
 
     # ---- shared forward body --------------------------------------------------------------

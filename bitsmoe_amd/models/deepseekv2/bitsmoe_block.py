@@ -32,24 +32,22 @@ class BitsMoE_DeepSeekSparseMoeBlock(BitsMoE_BaseSparseMoeBlock):
                 setattr(self, attr, int(getattr(source_block, attr)))
         self._init_bitsmoe_common_state(super_experts=super_experts, track_super_projected_weights=True)
 
-    def _gate_route(self, hidden_states: torch.Tensor):
+    def _linear_gate(self, x: torch.Tensor):
+        """(prepared weight, renormalise, scale) of a gate of the plain form -- fp32 logits, softmax, greedy top-k, then
+        renormalisation or the scaling factor (the defaults of bitsmoe/models/deepseekv2/configuration_deepseek.py:125-139;
+        "gready" is that file's spelling) -- in evaluation mode: linear layer, softmax and top-k are then ONE kernel.  None
+        for any other gate: the module routes."""
         gate = self.gate
-        # A gate of the plain form -- fp32 logits, softmax, greedy top-k, then renormalisation or the scaling factor
-        # (the defaults of bitsmoe/models/deepseekv2/configuration_deepseek.py:125-139; "gready" is that file's
-        # spelling) -- in evaluation mode: linear layer, softmax and top-k as ONE kernel.  Any other gate: the module.
-        if (not getattr(gate, "training", False) and getattr(gate, "scoring_func", "softmax") == "softmax"
-                and getattr(gate, "topk_method", "greedy") in ("greedy", "gready") and hasattr(gate, "top_k")
-                and hasattr(gate, "norm_topk_prob") and hasattr(gate, "routed_scaling_factor")
-                and isinstance(getattr(gate, "weight", None), torch.Tensor) and hidden_states.is_cuda and _HAS_MLP_FORWARD_CUDA):
-            x = hidden_states.reshape(-1, hidden_states.shape[-1])
-            top_k = int(gate.top_k)
-            if mlp_forward_cuda.router_linear_topk_possible(x, gate.weight, top_k):
-                renorm = top_k > 1 and bool(gate.norm_topk_prob)
-                return mlp_forward_cuda.router_linear_topk(x, mlp_forward_cuda.prepared_linear_weight_of(gate, gate.weight), top_k,
-                                                           renorm, round_dtype=None,
-                                                           weight_scale=1.0 if renorm else float(gate.routed_scaling_factor))
-        topk_idx, topk_weight, _aux = self.gate(hidden_states)
-        return topk_idx.reshape(-1, topk_idx.shape[-1]), topk_weight.reshape(-1, topk_weight.shape[-1]).to(torch.float32)
+        weight = getattr(gate, "weight", None)
+        if (getattr(gate, "training", False) or getattr(gate, "scoring_func", "softmax") != "softmax"
+                or getattr(gate, "topk_method", "greedy") not in ("greedy", "gready") or not hasattr(gate, "top_k")
+                or not hasattr(gate, "norm_topk_prob") or not hasattr(gate, "routed_scaling_factor")
+                or not isinstance(weight, torch.Tensor) or int(gate.top_k) != self.top_k
+                or not mlp_forward_cuda.router_linear_topk_possible(x, weight, self.top_k)):
+            return None
+        renorm = self.top_k > 1 and bool(gate.norm_topk_prob)
+        return (mlp_forward_cuda.prepared_linear_weight_of(gate, weight), renorm,
+                1.0 if renorm else float(gate.routed_scaling_factor))
 
     def forward(self, hidden_states: torch.Tensor):
         identity = hidden_states
@@ -57,9 +55,12 @@ class BitsMoE_DeepSeekSparseMoeBlock(BitsMoE_BaseSparseMoeBlock):
         flat = hidden_states.reshape(-1, orig_shape[-1])
         self._ensure_runtime_cache(flat.device)
         has_shared = getattr(self.config, "n_shared_experts", None) is not None and hasattr(self, "shared_experts")
-        # (the model's own gate module picks; the shared-basis projections, the shared experts and the output
+        # (the model's own gate picks; the shared-basis projections, the shared experts and the output
         # projection take the one-GEMM-in, one-GEMM-out form)
-        fused = self._fused_block_forward(flat, route_fn=lambda h2d: self._gate_route(h2d.reshape(orig_shape)),
+        plain = self._linear_gate(flat) if flat.is_cuda and _HAS_MLP_FORWARD_CUDA else None
+        fused = self._fused_block_forward(flat, linear_gate=plain[0] if plain else None,
+                                          route_fn=lambda h2d: self.gate(h2d.reshape(orig_shape))[:2],
+                                          renormalize=plain[1] if plain else False, weight_scale=plain[2] if plain else 1.0,
                                           shared=self.shared_experts if has_shared else None)
         if fused is not None:
             return fused[0].reshape(*orig_shape)

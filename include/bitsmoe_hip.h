@@ -313,6 +313,41 @@ int bitsmoe_moe_forward_routed(const bitsmoe_matset* gate, const bitsmoe_matset*
                                size_t workspace_bytes, bitsmoe_profile* profile, void* stream);
 
 /*
+ * The block's forward between its two projections (bitsmoe/models/qwen3moe/bitsmoe_block.py:45-98 and its two siblings:
+ * router, bitsmoe/models/base_block.py:258-289 and :381-414, shared and super experts), and the projections themselves
+ * where the few-rows kernel runs them, in one call on the caller's stream.  A plan names what a layer keeps; it is only
+ * read, so several threads may share one.
+ *   x [T, hidden] in act_dtype, rows ld_x elements apart;  proj [T, in_features]: x times the row-stacked input weights
+ *   (columns col_gate / col_up: the shared-basis projections, col_logits: the router's logits, col_shared_gate /
+ *   col_shared_up / col_shared_logit: the shared expert's), written here with BITSMOE_BLOCK_PROJECT_IN, else given.
+ *   selected int64 / weights fp32 [T, top_k]: given with BITSMOE_ROUTER_CALLER, else written (may then be null).
+ *   out: with BITSMOE_BLOCK_PROJECT_OUT the block output [T, hidden], else the output projection's operand
+ *   [T, rank_out + shared_intermediate]; super experts' share: in the output, or (fp32 [T, hidden]) in super_out.
+ *   side_stream (may be null): a stream for the super experts' call beside the packed experts'; joined before the call ends.
+ */
+#define BITSMOE_ROUTER_LOGITS 0     /* softmax and top-k of proj's logits columns */
+#define BITSMOE_ROUTER_LINEAR 1     /* fp32 logits from x and w_router (bitsmoe_router_linear_topk, prepared weight) */
+#define BITSMOE_ROUTER_CALLER 2
+#define BITSMOE_BLOCK_PROJECT_IN 1
+#define BITSMOE_BLOCK_PROJECT_OUT 2
+typedef struct {
+    const bitsmoe_matset *gate, *up, *down;
+    const int32_t *global_to_local, *local_to_global;
+    const bitsmoe_matset *super_gate, *super_up, *super_down;      /* dense experts' sets, or null */
+    const int32_t *super_global_to_local, *super_local_to_global;
+    const void *w_in, *w_out, *w_router;                           /* for the stages that run here */
+    int32_t w_in_prepared, w_out_prepared;
+    int32_t act_dtype, hidden, in_features, rank_gate, rank_up, rank_out, intermediate_size, super_intermediate;
+    int32_t top_k, n_global, router_form, renormalize, round_dtype;
+    int32_t col_gate, col_up, col_logits, col_shared_gate, col_shared_up, col_shared_logit, shared_intermediate;
+    float weight_scale;
+} bitsmoe_block_plan;
+size_t bitsmoe_block_workspace_bytes(const bitsmoe_block_plan* plan, int64_t n_tokens);
+int bitsmoe_block_forward(const bitsmoe_block_plan* plan, const void* x, int64_t ld_x, int64_t n_tokens, void* proj,
+                          int32_t stages, void* selected, float* weights, void* out, float* super_out, void* workspace,
+                          size_t workspace_bytes, void* side_stream, void* stream);
+
+/*
  * The forward for callers that cannot allocate device memory (code under HIP graph capture,
  * tight serving loops, harnesses that forbid hipMalloc): bitsmoe_moe_forward_strided without the
  * workspace argument.  No counterpart in the reference, whose operator allocates its

@@ -270,3 +270,52 @@ def test_block_with_super_and_shared_experts(cuda_device, family, kw, dense, mon
         graph.replay()
         torch.cuda.synchronize()
         assert float((yg.float() - y.float()).abs().max()) <= 2e-2 * float(y.float().abs().max())
+
+
+@pytest.mark.parametrize("tokens", [16, 17, 33, 65])      # both sides of where either projection leaves the few-rows kernel
+@pytest.mark.parametrize("family,kw", [("qwen3moe", {}), ("qwen3next", {"shared_intermediate": 128}), ("deepseekv2", {})])
+@pytest.mark.parametrize("super_experts", [(), (1, 6)])
+def test_block_in_one_call_equals_module_by_module(cuda_device, family, kw, tokens, super_experts, monkeypatch):
+    """bitsmoe_block_forward against the module-by-module form on the same block (both round to bf16 along the way: 1e-2),
+    and from two threads on streams of their own at once against itself alone: one plan, intermediates per stream."""
+    import threading
+
+    import torch
+
+    from bitsmoe_amd.models.base_block import BitsMoE_BaseSparseMoeBlock
+    from bitsmoe_amd.synth import make_layer
+
+    block = make_layer(_small_spec(family, **kw), device=cuda_device, dtype=torch.bfloat16, seed=31, s_mode="rand",
+                       super_experts=super_experts)
+    block.prepare_runtime_fastpath(warmup=True)
+    g = torch.Generator().manual_seed(tokens)
+    xs = [torch.randn((1, tokens, block.spec.hidden_size), generator=g).to(torch.bfloat16).to(cuda_device) for _ in range(2)]
+    first = lambda out: (out[0] if isinstance(out, tuple) else out).float()
+    with torch.no_grad():
+        alone = [first(block(x)) for x in xs]
+        with monkeypatch.context() as m:
+            m.setattr(BitsMoE_BaseSparseMoeBlock, "_FUSED_BLOCK", False)
+            apart = [first(block(x)) for x in xs]
+    torch.cuda.synchronize()
+    for a, b in zip(alone, apart):
+        assert float((a - b).abs().max()) <= 1e-2 * float(b.abs().max())
+    got, errors = [None, None], []
+
+    def work(i):
+        try:
+            st = torch.cuda.Stream(device=cuda_device)
+            with torch.no_grad(), torch.cuda.stream(st):
+                for _ in range(20):
+                    got[i] = first(block(xs[i]))
+            st.synchronize()
+        except Exception as exc:      # noqa: BLE001 - reported below
+            errors.append(exc)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
+    for a, b in zip(got, alone):      # (fp32 atomics in another order, then one bf16 rounding)
+        assert float((a - b).abs().max()) <= 1e-2 * float(b.abs().max())
