@@ -5,11 +5,25 @@
 // i.e. a stream of W at HBM speed, which general GEMM kernels tiled for square problems reach a fraction of.
 // W stays in the framework's [out_features, in_features] layout: a lane's 16 bytes of a weight row are eight
 // consecutive contraction indices, which is what the 16x16x32 MFMA takes as its second operand.
-// A workgroup owns 16 * NBW output columns; its four wavefronts contract a quarter of K each, two batches of four
-// k-steps in flight (every load of a batch is out before the previous batch's MFMAs run), and add up in LDS.
+// A workgroup owns 16 output columns; each of its wavefronts contracts a share of K and they add up in LDS.
+//
+// What bounds it: one trip to memory for W, and x, which EVERY workgroup reads in full (T / 16 bytes of x per byte of W,
+// from L2).  So (a) a wavefront requests its whole share of W -- up to MAXS steps, 1 KB each -- before it multiplies anything:
+// with batches of four steps the trips followed each other; (b) x is fetched in pieces of whole cache lines (a wavefront
+// reads G * 64 consecutive bytes of a row, several rows per instruction), turned in LDS and read from there as operands:
+// fetched in operand order a load touched 64 bytes of sixteen rows, and the launch grew by 4 us per sixteen rows.
+// Longer contractions take eight wavefronts, so that a share stays within MAXS steps (beyond that: several passes).
+// Prepared weights, graph of launches over 600 MB of weights, us per launch (batches of four steps and x in operand order ->
+// now; the library GEMM) at 1, 16, 32, 48, 64 rows:
+//   2048 -> 4224 features: 6.1 -> 6.2, 8.3 -> 7.3 (11.4), 12.1 -> 8.8 (11.5), 16.0 -> 10.4 (11.9), 19.4 -> 12.4 (12.2)
+//   2048 -> 2048 features: 4.5 -> 4.2, 5.4 -> 4.7 (11.0), 7.4 -> 5.7 (11.2), 9.6 -> 6.5 (11.2), 11.5 -> 7.6 (11.7)
+//   4864 -> 2048 features: 7.7 -> 7.1, 9.8 -> 8.2 (16.3), 14.1 -> 10.1 (12.8), 19.7 -> 12.4 (13.0), 24.6 -> 14.9 (15.2)
+//   2048 -> 9728 features: 9.9 -> 9.6, 12.6 -> 11.0 (15.7), 18.1 -> 12.9 (15.8), 23.5 -> 15.8 (16.8), 28.6 -> 18.7 (17.1)
 #include "common.h"
 
 #include <algorithm>
+#include <type_traits>
+#include <utility>
 
 namespace bitsmoe {
 
@@ -18,135 +32,161 @@ typedef uint32_t sk_u32x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 sk_f16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 sk_bf16x8 __attribute__((ext_vector_type(8)));
 
-constexpr int SK_U = 4;      // k-steps per batch of loads
+template <class F, int... P>
+__device__ __forceinline__ void static_for_pieces(F&& f, std::integer_sequence<int, P...>) {
+    (f(std::integral_constant<int, P>{}), ...);
+}
 
 // XF32: x is fp32 and is rounded to the 16-bit type on its way into the MFMA (the cast of the operator's fp32 output in
 // front of the output projection, bitsmoe/models/base_block.py:414, without a pass of its own); one 16-row block only.
 // PREP: W was re-laid out once (bitsmoe_prepare_linear_weight) into the order the MFMA takes it: [16-column block]
 // [k-step of 32][lane][8 values], so that a wavefront's load is 1 KB of consecutive memory instead of sixteen 64-byte
 // pieces of sixteen rows.
-template <bool BF16, int NMB, int NBW, bool XF32 = false, bool PREP = false>
-__global__ __launch_bounds__(256) void k_skinny_linear(const void* __restrict__ x_any, int64_t ld_x, const uint16_t* __restrict__ w,
-                                                       int T, int K, int N, uint16_t* __restrict__ out, int64_t ld_out,
-                                                       const float* __restrict__ addend, int64_t ld_add) {
-    static_assert(!XF32 || NMB == 1, "fp32 rows: one block of 16 rows");
-    const uint16_t* __restrict__ x = reinterpret_cast<const uint16_t*>(x_any);
-    const float* __restrict__ xf = reinterpret_cast<const float*>(x_any);
-    __shared__ float part[4][NMB * 16][NBW * 16 + 1];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int n0 = blockIdx.x * (NBW * 16);
-    const int kq = K >> 2;                       // contraction range of this wavefront (a multiple of 32)
-    const int kbase = wv * kq + (lane >> 4) * 8;
-    const uint16_t* xp[NMB];
-    const uint16_t* wp[NBW];
-    const float* xfp = xf + (int64_t)min(lane & 15, T - 1) * ld_x + kbase;
+// TURN: x by way of LDS; else (a few rows: nothing to gain from whole lines) every step's operand straight from x.
+template <bool BF16, int NMB, int NW, int MAXS, bool XF32, bool PREP, bool TURN>
+__global__ __launch_bounds__(64 * NW) void k_skinny_linear(const void* __restrict__ x, int64_t ld_x, const uint16_t* __restrict__ w,
+                                                           int T, int K, int N, uint16_t* __restrict__ out, int64_t ld_out,
+                                                           const float* __restrict__ addend, int64_t ld_add) {
+    static_assert((!XF32 && TURN) || NMB == 1, "fp32 rows and few rows: one block of 16 rows");
+    constexpr int G = NMB <= 2 ? 4 : 2;                // k-steps per piece of x
+    static_assert(MAXS % G == 0, "whole pieces");
+    constexpr int EB = XF32 ? 4 : 2;                   // bytes of an element of x
+    constexpr int CPR = 32 * G * EB / 16;              // 16-byte chunks per row of a piece
+    constexpr int RPI = 64 / CPR;                      // rows per load instruction
+    constexpr int NI = 16 * NMB / RPI;                 // load instructions per piece
+    constexpr int PIECE = TURN ? 16 * NMB * CPR * 16 : 0;      // bytes
+    constexpr int PART = NW * NMB * 16 * 17 * 4;
+    __shared__ __attribute__((aligned(16))) unsigned char lds[NW * PIECE > PART ? NW * PIECE : PART];
+    const int lane = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n = lane & 15, kg = lane >> 4;
+    const int n0 = blockIdx.x * 16;
+    const int steps = K >> 5;
+    const int first = wv * steps / NW, end = (wv + 1) * steps / NW;
+    // chunk c of row r sits at chunk position c ^ swz(r) of its row: the sixteen rows of an operand read hit different banks
+    auto swz = [](int r) { return CPR == 8 ? (r >> 1) & 7 : r & 15; };
+    unsigned char* piece = lds + wv * PIECE;
+    const unsigned char* xrow[NI];
 #pragma unroll
-    for (int mb = 0; mb < NMB; ++mb) xp[mb] = x + (int64_t)min(mb * 16 + (lane & 15), T - 1) * ld_x + kbase;
-#pragma unroll
-    for (int nb = 0; nb < NBW; ++nb) {
-        if constexpr (PREP)      // (N is a multiple of 16 * NBW there; step ks of this wavefront: + (ks / 32) * 512 elements)
-            wp[nb] = w + ((int64_t)(blockIdx.x * NBW + nb) * (K >> 5) + wv * (kq >> 5)) * 512 + lane * 8;
-        else
-            wp[nb] = w + (int64_t)min(n0 + nb * 16 + (lane & 15), N - 1) * K + kbase;
+    for (int i = 0; i < NI; ++i) {
+        const int r = i * RPI + lane / CPR;
+        xrow[i] = (const unsigned char*)x + (int64_t)min(r, T - 1) * ld_x * EB + ((lane % CPR) ^ swz(r)) * 16;
     }
-    sk_f32x4 acc[NMB][NBW];
+    const uint16_t* wp = PREP ? w + ((int64_t)blockIdx.x * steps) * 512 + lane * 8 : w + (int64_t)min(n0 + n, N - 1) * K + kg * 8;
+    sk_f32x4 acc[NMB];
 #pragma unroll
-    for (int mb = 0; mb < NMB; ++mb)
-#pragma unroll
-        for (int nb = 0; nb < NBW; ++nb) acc[mb][nb] = sk_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    sk_u32x4 a[2][SK_U][NMB], b[2][SK_U][NBW];
-    sk_f32x4 af[2][SK_U][XF32 ? 2 : 1];      // (fp32 rows as loaded: eight values per lane and k-step)
-    auto request = [&](auto buf_c, int s0) {
-        constexpr int B = decltype(buf_c)::value;
-#pragma unroll
-        for (int u = 0; u < SK_U; ++u) {
-            const int ks = min(s0 + 32 * u, kq - 32);      // (a short last batch repeats its final step: masked below)
-#pragma unroll
-            for (int nb = 0; nb < NBW; ++nb)
-                b[B][u][nb] = *reinterpret_cast<const sk_u32x4*>(wp[nb] + (PREP ? ks * 16 : ks));
-            if constexpr (XF32) {
-                af[B][u][0] = *reinterpret_cast<const sk_f32x4*>(xfp + ks);
-                af[B][u][1] = *reinterpret_cast<const sk_f32x4*>(xfp + ks + 4);
-            } else {
-#pragma unroll
-                for (int mb = 0; mb < NMB; ++mb) a[B][u][mb] = *reinterpret_cast<const sk_u32x4*>(xp[mb] + ks);
-            }
-        }
-    };
+    for (int mb = 0; mb < NMB; ++mb) acc[mb] = sk_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     auto round16 = [](float v) -> uint32_t {
         if constexpr (BF16)
             return (uint32_t)__builtin_bit_cast(uint16_t, (__bf16)v);
         else
             return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)v);
     };
-    auto multiply = [&](auto buf_c, int s0) {
-        constexpr int B = decltype(buf_c)::value;
+    auto multiply = [&](sk_f32x4& c, sk_u32x4 av, sk_u32x4 bv) {
+        if constexpr (BF16)
+            c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(sk_bf16x8, av), __builtin_bit_cast(sk_bf16x8, bv), c, 0, 0, 0);
+        else
+            c = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(sk_f16x8, av), __builtin_bit_cast(sk_f16x8, bv), c, 0, 0, 0);
+    };
+    auto rounded = [&](sk_f32x4 lo, sk_f32x4 hi) {
+        return sk_u32x4{round16(lo[0]) | (round16(lo[1]) << 16), round16(lo[2]) | (round16(lo[3]) << 16),
+                        round16(hi[0]) | (round16(hi[1]) << 16), round16(hi[2]) | (round16(hi[3]) << 16)};
+    };
+    for (int s0 = first; s0 < end; s0 += MAXS) {
+        // (no branches: steps past the end repeat the last one and count as zeros)
+        const int ns = end - s0;
+        sk_u32x4 b[MAXS];
+        auto request_w = [&](int u) {
+            b[u] = *reinterpret_cast<const sk_u32x4*>(wp + (int64_t)(s0 + min(u, ns - 1)) * (PREP ? 512 : 32));
+        };
+        auto weights = [&](int u) {
+            sk_u32x4 bv = b[u];
+            const bool live = u < ns;
 #pragma unroll
-        for (int u = 0; u < SK_U; ++u) {
-            const bool live = s0 + 32 * u < kq;      // (no branch between the steps: a step past the end contributes zeros)
-            if constexpr (XF32) {
+            for (int c = 0; c < 4; ++c) bv[c] = live ? bv[c] : 0u;
+            return bv;
+        };
+        if constexpr (!TURN) {
+            sk_u32x4 xr[MAXS][XF32 ? 2 : 1];
+            const unsigned char* row = (const unsigned char*)x + ((int64_t)min(n, T - 1) * ld_x + kg * 8) * EB;
 #pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    const sk_f32x4 v = af[B][u][c >> 1];
-                    a[B][u][0][c] = round16(v[2 * (c & 1)]) | (round16(v[2 * (c & 1) + 1]) << 16);
-                }
+            for (int u = 0; u < MAXS; ++u) {
+#pragma unroll
+                for (int q = 0; q < (XF32 ? 2 : 1); ++q)
+                    xr[u][q] = *reinterpret_cast<const sk_u32x4*>(row + (int64_t)(s0 + min(u, ns - 1)) * (32 * EB) + 16 * q);
+                request_w(u);
             }
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int nb = 0; nb < NBW; ++nb) {
-                sk_u32x4 bv = b[B][u][nb];
+            for (int u = 0; u < MAXS; ++u) {
+                if constexpr (XF32)
+                    multiply(acc[0], rounded(__builtin_bit_cast(sk_f32x4, xr[u][0]), __builtin_bit_cast(sk_f32x4, xr[u][1])), weights(u));
+                else
+                    multiply(acc[0], xr[u][0], weights(u));
+            }
+            continue;
+        }
+        sk_u32x4 xr[2][NI];
+        auto request_x = [&](auto p_c) {
+            constexpr int P = decltype(p_c)::value;
+            // (a piece that would stick out of the row is moved back: its steps are found `shift` further up, or count as zeros)
+            const int at = min(s0 + P * G, steps - G);
 #pragma unroll
-                for (int c = 0; c < 4; ++c) bv[c] = live ? bv[c] : 0u;
+            for (int i = 0; i < NI; ++i) xr[P & 1][i] = *reinterpret_cast<const sk_u32x4*>(xrow[i] + (int64_t)at * (32 * EB));
+        };
+        // (x first: loads return in the order they are asked for, and x is the one that comes from L2)
+        request_x(std::integral_constant<int, 0>{});
+        if constexpr (MAXS > G) request_x(std::integral_constant<int, 1>{});
+#pragma unroll
+        for (int u = 0; u < MAXS; ++u) request_w(u);
+        __builtin_amdgcn_sched_barrier(0);
+        static_for_pieces([&](auto p_c) {
+            constexpr int P = decltype(p_c)::value;
+#pragma unroll
+            for (int i = 0; i < NI; ++i) *reinterpret_cast<sk_u32x4*>(piece + (i * 64 + lane) * 16) = xr[P & 1][i];
+            if constexpr ((P + 2) * G < MAXS) request_x(std::integral_constant<int, P + 2>{});
+            __builtin_amdgcn_sched_barrier(0);
+            const int shift = s0 + P * G - min(s0 + P * G, steps - G);
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                const sk_u32x4 bv = weights(P * G + g);
+                const int gs = min(g + shift, G - 1);
 #pragma unroll
                 for (int mb = 0; mb < NMB; ++mb) {
-                    if constexpr (BF16)
-                        acc[mb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(sk_bf16x8, a[B][u][mb]),
-                                                                              __builtin_bit_cast(sk_bf16x8, bv), acc[mb][nb], 0, 0, 0);
+                    const int r = 16 * mb + n;
+                    const unsigned char* row = piece + r * (CPR * 16);
+                    if constexpr (XF32)
+                        multiply(acc[mb], rounded(*reinterpret_cast<const sk_f32x4*>(row + (((gs * 8 + 2 * kg) ^ swz(r)) << 4)),
+                                                  *reinterpret_cast<const sk_f32x4*>(row + (((gs * 8 + 2 * kg + 1) ^ swz(r)) << 4))), bv);
                     else
-                        acc[mb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(sk_f16x8, a[B][u][mb]),
-                                                                             __builtin_bit_cast(sk_f16x8, bv), acc[mb][nb], 0, 0, 0);
+                        multiply(acc[mb], *reinterpret_cast<const sk_u32x4*>(row + (((gs * 4 + kg) ^ swz(r)) << 4)), bv);
                 }
             }
-        }
-    };
-    using B0 = std::integral_constant<int, 0>;
-    using B1 = std::integral_constant<int, 1>;
-    constexpr int STEP = 32 * SK_U;
-    request(B0{}, 0);
-    for (int s0 = 0; s0 < kq; s0 += 2 * STEP) {
-        if (s0 + STEP < kq) request(B1{}, s0 + STEP);
-        __builtin_amdgcn_sched_barrier(0);
-        multiply(B0{}, s0);
-        if (s0 + STEP < kq) {
-            if (s0 + 2 * STEP < kq) request(B0{}, s0 + 2 * STEP);
-            __builtin_amdgcn_sched_barrier(0);
-            multiply(B1{}, s0 + STEP);
-        }
+        }, std::make_integer_sequence<int, MAXS / G>{});
     }
-    // lane holds rows 16 mb + 4 (lane / 16) + j, column 16 nb + lane % 16
+    // lane holds rows 16 mb + 4 kg + j, column n; the partial sums take the place of the pieces of x
+    auto part = [&](int w_, int row, int col) -> float& { return reinterpret_cast<float*>(lds)[(w_ * (NMB * 16) + row) * 17 + col]; };
+    __syncthreads();
 #pragma unroll
     for (int mb = 0; mb < NMB; ++mb)
 #pragma unroll
-        for (int nb = 0; nb < NBW; ++nb)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) part[wv][mb * 16 + 4 * (lane >> 4) + j][nb * 16 + (lane & 15)] = acc[mb][nb][j];
+        for (int j = 0; j < 4; ++j) part(wv, mb * 16 + 4 * kg + j, n) = acc[mb][j];
     __syncthreads();
-    // the four partial sums in a fixed order, two neighbouring columns per thread
-    constexpr int PAIRS = NMB * 16 * NBW * 8;
-    for (int i = threadIdx.x; i < PAIRS; i += 256) {
-        const int row = i / (NBW * 8), c = (i - row * (NBW * 8)) * 2;
+    // the partial sums in a fixed order, two neighbouring columns per thread
+    for (int i = threadIdx.x; i < NMB * 16 * 8; i += 64 * NW) {
+        const int row = i / 8, c = (i % 8) * 2;
         if (row >= T || n0 + c >= N) continue;
-        float v0 = part[0][row][c] + part[1][row][c] + part[2][row][c] + part[3][row][c];
-        float v1 = part[0][row][c + 1] + part[1][row][c + 1] + part[2][row][c + 1] + part[3][row][c + 1];
+        float v0 = 0.0f, v1 = 0.0f;
+#pragma unroll
+        for (int q = 0; q < NW; ++q) {
+            v0 += part(q, row, c);
+            v1 += part(q, row, c + 1);
+        }
         if (addend) {      // (fp32 [T, N] added to the sums before the one rounding of the result)
             v0 += addend[(int64_t)row * ld_add + n0 + c];
             v1 += addend[(int64_t)row * ld_add + n0 + c + 1];
         }
-        uint32_t packed;
-        if constexpr (BF16)
-            packed = (uint32_t)__builtin_bit_cast(uint16_t, (__bf16)v0) | ((uint32_t)__builtin_bit_cast(uint16_t, (__bf16)v1) << 16);
-        else
-            packed = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)v0) | ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)v1) << 16);
-        *reinterpret_cast<uint32_t*>(out + (int64_t)row * ld_out + n0 + c) = packed;
+        *reinterpret_cast<uint32_t*>(out + (int64_t)row * ld_out + n0 + c) = round16(v0) | (round16(v1) << 16);
     }
 }
 
@@ -204,48 +244,53 @@ extern "C" int bitsmoe_skinny_linear(const void* x, int32_t dtype, int32_t x_is_
     BITSMOE_REQUIRE((((uintptr_t)x | (uintptr_t)weight) & 15) == 0 && ((uintptr_t)out & 3) == 0,
                     "x and weight must be 16-byte aligned, out 4-byte aligned");
     hipStream_t st = (hipStream_t)stream;
-    const bool bf16 = dtype == BITSMOE_DT_BF16;
-    // two 16-column blocks per wavefront once that still leaves a workgroup per CU and more (half the re-reads of x)
-    const bool two = out_features >= 32 * 512;
     const int nmb = (int)((n_rows + 15) / 16);
-    const unsigned grid = (unsigned)((out_features + (two ? 32 : 16) - 1) / (two ? 32 : 16));
-#define BITSMOE_SKINNY(B, NMB, NBW)                                                                                     \
-    hipLaunchKernelGGL((k_skinny_linear<B, NMB, NBW>), dim3(grid), dim3(256), 0, st, x, ld_x,           \
-                       (const uint16_t*)weight, (int)n_rows, in_features, out_features, (uint16_t*)out, ld_out, (const float*)addend, ld_addend)
-#define BITSMOE_SKINNY_M(B, NBW)                                      \
-    do {                                                              \
-        if (nmb == 1) BITSMOE_SKINNY(B, 1, NBW);                      \
-        else if (nmb == 2) BITSMOE_SKINNY(B, 2, NBW);                 \
-        else if (nmb == 3) BITSMOE_SKINNY(B, 3, NBW);                 \
-        else BITSMOE_SKINNY(B, 4, NBW);                               \
-    } while (0)
-    if (x_is_f32 || weight_is_prepared) {
-        // (the forms the block uses at a few tokens: one column block per wavefront)
-        BITSMOE_REQUIRE(!x_is_f32 || n_rows <= 16, "fp32 rows: at most 16 rows");
-        const dim3 g1((unsigned)((out_features + 15) / 16));
-        const int nmb1 = (int)((n_rows + 15) / 16);
-#define BITSMOE_SKINNY_1(B, NMB, XF, PR)                                                                                   \
-        hipLaunchKernelGGL((k_skinny_linear<B, NMB, 1, XF, PR>), g1, dim3(256), 0, st, x, ld_x, (const uint16_t*)weight,   \
-                           (int)n_rows, in_features, out_features, (uint16_t*)out, ld_out, (const float*)addend, ld_addend)
-#define BITSMOE_SKINNY_P(B)                                                                  \
-        do {                                                                                 \
-            if (x_is_f32 && weight_is_prepared) BITSMOE_SKINNY_1(B, 1, true, true);          \
-            else if (x_is_f32) BITSMOE_SKINNY_1(B, 1, true, false);                          \
-            else if (nmb1 == 1) BITSMOE_SKINNY_1(B, 1, false, true);                         \
-            else if (nmb1 == 2) BITSMOE_SKINNY_1(B, 2, false, true);                         \
-            else if (nmb1 == 3) BITSMOE_SKINNY_1(B, 3, false, true);                         \
-            else BITSMOE_SKINNY_1(B, 4, false, true);                                        \
-        } while (0)
-        if (bf16) BITSMOE_SKINNY_P(true); else BITSMOE_SKINNY_P(false);
-#undef BITSMOE_SKINNY_P
-#undef BITSMOE_SKINNY_1
-    } else if (bf16) {
-        if (two) BITSMOE_SKINNY_M(true, 2); else BITSMOE_SKINNY_M(true, 1);
-    } else {
-        if (two) BITSMOE_SKINNY_M(false, 2); else BITSMOE_SKINNY_M(false, 1);
-    }
-#undef BITSMOE_SKINNY_M
-#undef BITSMOE_SKINNY
+    const dim3 grid((unsigned)((out_features + 15) / 16));
+    // a wavefront's share of the contraction, with four wavefronts or (shares of more than twenty steps) eight
+    const int steps = in_features / 32;
+    const int nw = steps > 80 ? 8 : 4;
+    const int share = (steps + nw - 1) / nw;
+    auto run = [&](auto bf_c, auto nmb_c, auto nw_c, auto s_c, auto xf_c, auto pr_c, auto turn_c) {
+        hipLaunchKernelGGL((k_skinny_linear<decltype(bf_c)::value, decltype(nmb_c)::value, decltype(nw_c)::value, decltype(s_c)::value,
+                                            decltype(xf_c)::value, decltype(pr_c)::value, decltype(turn_c)::value>),
+                           grid, dim3(64 * decltype(nw_c)::value), 0, st, x, ld_x, (const uint16_t*)weight, (int)n_rows, in_features,
+                           out_features, (uint16_t*)out, ld_out, addend, ld_addend);
+    };
+    using std::integral_constant;
+    using Yes = std::true_type;
+    using No = std::false_type;
+    using W4 = integral_constant<int, 4>;
+    using W8 = integral_constant<int, 8>;
+    using S8 = integral_constant<int, 8>;
+    using S16 = integral_constant<int, 16>;
+    using S20 = integral_constant<int, 20>;
+    auto by_share = [&](auto bf_c, auto nmb_c, auto xf_c, auto turn_c) {
+        constexpr bool twenty = !(decltype(xf_c)::value && !decltype(turn_c)::value);      // (fp32 operands of twenty steps do not fit the registers)
+        if (!weight_is_prepared) {      // (in passes of sixteen steps: the same sums in the same order)
+            if (nw == 8) run(bf_c, nmb_c, W8{}, S16{}, xf_c, No{}, turn_c); else run(bf_c, nmb_c, W4{}, S16{}, xf_c, No{}, turn_c);
+        } else if (nw == 8) {
+            if (share <= 16 || !twenty) run(bf_c, nmb_c, W8{}, S16{}, xf_c, Yes{}, turn_c);
+            else if constexpr (twenty) run(bf_c, nmb_c, W8{}, S20{}, xf_c, Yes{}, turn_c);
+        } else if (share <= 8) {
+            run(bf_c, nmb_c, W4{}, S8{}, xf_c, Yes{}, turn_c);
+        } else {
+            if (share <= 16 || !twenty) run(bf_c, nmb_c, W4{}, S16{}, xf_c, Yes{}, turn_c);
+            else if constexpr (twenty) run(bf_c, nmb_c, W4{}, S20{}, xf_c, Yes{}, turn_c);
+        }
+    };
+    auto by_rows = [&](auto bf_c) {
+        using One = integral_constant<int, 1>;
+        // x by way of LDS from five rows on: 2048 -> 4224 features at one row 6.2 us straight from x, 7.0 through LDS; 4864 -> 2048
+        // features at eight rows 8.9 against 7.9
+        if (n_rows <= 4 && x_is_f32 && share <= 16) by_share(bf_c, One{}, Yes{}, No{});
+        else if (n_rows <= 4 && !x_is_f32) by_share(bf_c, One{}, No{}, No{});
+        else if (x_is_f32) by_share(bf_c, One{}, Yes{}, Yes{});
+        else if (nmb == 1) by_share(bf_c, One{}, No{}, Yes{});
+        else if (nmb == 2) by_share(bf_c, integral_constant<int, 2>{}, No{}, Yes{});
+        else if (nmb == 3) by_share(bf_c, integral_constant<int, 3>{}, No{}, Yes{});
+        else by_share(bf_c, integral_constant<int, 4>{}, No{}, Yes{});
+    };
+    if (dtype == BITSMOE_DT_BF16) by_rows(Yes{}); else by_rows(No{});
     BITSMOE_HIP_TRY(hipGetLastError());
     return BITSMOE_OK;
 }

@@ -50,19 +50,16 @@ def _super_via_operator() -> bool:
 
 
 # Rows up to which the block's two stacked GEMMs run the library's own few-rows kernel (against a copy of the stacked
-# weights in MFMA operand order) instead of the framework's GEMM.  Whole block under graph replay, cold weights,
-# 128-expert layer of hidden size 2048 (4224 stacked input features): 1 token 30.4 vs 40.6 us, 8 tokens 51.8 vs 65.5,
-# 16 tokens 67.1 vs 77.3, 24 tokens 76.9 vs 83.2, 32 tokens 79.2 vs 83.3, 48 tokens 88.9 vs 87.4, 64 tokens 97.4 vs 91.0.
-# Every workgroup of the kernel reads all rows of x, so from 17 rows on it is used only while there is about one workgroup
-# per CU and the contraction is short: the 64-expert layer with two shared experts (9728 stacked input features, 4864
-# output-side contraction) at 32 tokens ran 111.3 vs 108.2 us with the kernel for both GEMMs, 108.5 with it for the output
-# GEMM alone.  From 33 to 64 rows only the narrow output GEMM (2048 features) takes it: 40 tokens 85.0 vs 87.5 (both GEMMs:
-# 87.2), 48 tokens 87.0 vs 88.7 (90.4), 64 tokens 92.2 vs 93.1 (99.1).  BITSMOE_BLOCK_SKINNY_ROWS caps the rows, 0 switches
-# the kernel off.
+# weights in MFMA operand order) instead of the framework's GEMM.  Up to 48 rows it is the faster one at every shape
+# measured (us per launch, kernel against framework: 2048 -> 4224 features 8.8 vs 11.5 at 32 rows, 10.4 vs 11.9 at 48; 2048 -> 9728
+# 12.9 vs 15.8, 15.8 vs 16.8; 4864 -> 2048 10.1 vs 12.8, 12.4 vs 13.0).  Every workgroup reads all rows of x, so from 49 to 64 rows only
+# GEMMs of about one workgroup per CU and a contraction of at most 4096 take it: 2048 -> 2048 7.6 vs 11.7 at 64 rows, 2560 -> 2048
+# 9.0 vs 13.6, 2048 -> 4224 12.4 vs 12.2; but 2048 -> 9728 18.7 vs 17.1, and 4864 -> 2048 14.6 vs 12.9 at 56.
+# BITSMOE_BLOCK_SKINNY_ROWS caps the rows, 0 switches the kernel off.
 _SKINNY_ROWS = int(_os.environ.get("BITSMOE_BLOCK_SKINNY_ROWS", "64"))
-_SKINNY_WIDE_FEATURES = 5120      # output features up to which 17 to 32 rows still take the few-rows kernel
-_SKINNY_NARROW_FEATURES = 2048    # ... and 33 to 64 rows
-_SKINNY_LONG_CONTRACTION = 4096   # input features up to which more than 16 rows take it
+_SKINNY_ANY_SHAPE_ROWS = 48
+_SKINNY_NARROW_FEATURES = 4352    # output features, and
+_SKINNY_SHORT_CONTRACTION = 4096  # input features up to which 49 to 64 rows take it
 # BITSMOE_BLOCK_SKINNY_PREPARED=0: the few-rows kernel reads the stacked weights in the framework's layout (no extra copy)
 _SKINNY_PREPARED = _os.environ.get("BITSMOE_BLOCK_SKINNY_PREPARED", "1") != "0"
 
@@ -70,8 +67,7 @@ _SKINNY_PREPARED = _os.environ.get("BITSMOE_BLOCK_SKINNY_PREPARED", "1") != "0"
 def _few_rows(rows: int, n_in: int, n_out: int) -> bool:
     """Does the few-rows kernel run this GEMM?  (It takes contractions of whole 128 and an even number of outputs.)"""
     return (0 < rows <= _SKINNY_ROWS and n_in % 128 == 0 and n_out % 2 == 0 and (
-        rows <= 16 or (n_in <= _SKINNY_LONG_CONTRACTION
-                       and n_out <= (_SKINNY_WIDE_FEATURES if rows <= 32 else _SKINNY_NARROW_FEATURES))))
+        rows <= _SKINNY_ANY_SHAPE_ROWS or (n_in <= _SKINNY_SHORT_CONTRACTION and n_out <= _SKINNY_NARROW_FEATURES)))
 
 
 _SIDE_STREAMS: Dict[int, "torch.cuda.Stream"] = {}

@@ -722,3 +722,13 @@ def test_skinny_linear_matches_float64(cuda_device, rows, k, n, dtype_name):
     if rows <= 16:
         assert torch.equal(hip.skinny_linear(xf, wd), hip.skinny_linear(xf.to(dt), wd))
         assert torch.equal(hip.skinny_linear(xf, hip.PreparedLinearWeight(wd)), hip.skinny_linear(xf.to(dt), wd))
+
+
+@pytest.mark.parametrize("rows,k,n", [
+    (4, 2560, 48), (5, 2560, 48),      # x straight into the operands / by way of LDS; shares of twenty steps
+    (17, 896, 34), (64, 128, 16),      # shares that are no whole pieces of x, one step per wavefront
+    (49, 5248, 48), (3, 11008, 18),    # eight wavefronts, several passes over a share
+])
+@pytest.mark.parametrize("dtype_name", ["bf16", "f16"])
+def test_skinny_linear_edges(cuda_device, rows, k, n, dtype_name):
+    test_skinny_linear_matches_float64(cuda_device, rows, k, n, dtype_name)
