@@ -359,7 +359,6 @@ extern "C" int bitsmoe_pack_matrix(const float* matrix, int64_t rank, int64_t di
     BITSMOE_REQUIRE(n_tiles < ((int64_t)1 << 24), "too many columns");
     PackTables tab = {};
     int64_t row = 0, pay = 0, sc = 0, slab = 0;
-    std::vector<PackRange> all;
     for (int i = 0; i < n_ranges; ++i) {
         const int bits = ranges[3 * i], from = ranges[3 * i + 1], to = ranges[3 * i + 2];
         BITSMOE_REQUIRE(bits_supported(bits), "Unsupported bit width: %d", bits);
@@ -375,7 +374,6 @@ extern "C" int bitsmoe_pack_matrix(const float* matrix, int64_t rank, int64_t di
             BITSMOE_REQUIRE(tab.n_buckets < PACK_MAX_BUCKETS, "rows of one width must be neighbouring ranges");
             tab.bucket[tab.n_buckets++] = PackBucket{pay, sc, bits, (int32_t)row, 0, (int32_t)slab};
         }
-        all.push_back(PackRange{(int32_t)row, from, tab.n_buckets - 1});
         tab.bucket[tab.n_buckets - 1].rows += to - from;
         row += to - from;
         BITSMOE_REQUIRE(row < ((int64_t)1 << 31), "too many rows");
@@ -387,11 +385,17 @@ extern "C" int bitsmoe_pack_matrix(const float* matrix, int64_t rank, int64_t di
     BITSMOE_REQUIRE(!tables || (pay < ((int64_t)1 << 31) && slab * n_tiles < ((int64_t)1 << 31)),
                     "the tables' 32-bit offsets do not reach over %lld payload words", (long long)pay);
     // (a launch carries PACK_MAX_RANGES ranges by value; more of them take more launches)
-    for (size_t r0 = 0; r0 < all.size(); r0 += PACK_MAX_RANGES) {
-        const size_t r1 = std::min(all.size(), r0 + PACK_MAX_RANGES);
-        std::copy(all.begin() + r0, all.begin() + r1, tab.range);
-        tab.n_ranges = (int32_t)(r1 - r0);
-        tab.row_end = r1 < all.size() ? all[r1].first : (int32_t)row;
+    int32_t at = 0;      // packed rows so far, and the bucket of the range before
+    int bucket = -1;
+    for (int r0 = 0; r0 < n_ranges; r0 += PACK_MAX_RANGES) {
+        tab.n_ranges = std::min(n_ranges - r0, PACK_MAX_RANGES);
+        for (int k = 0; k < tab.n_ranges; ++k) {
+            const int32_t* rg = ranges + 3 * (int64_t)(r0 + k);
+            if (r0 + k == 0 || rg[0] != rg[-3]) ++bucket;
+            tab.range[k] = PackRange{at, rg[1], bucket};
+            at += rg[2] - rg[1];
+        }
+        tab.row_end = at;
         const bool first = r0 == 0;
         const int64_t rows_here = tab.row_end - tab.range[0].first;
         const int64_t unit_blocks = std::min<int64_t>((rows_here * n_tiles + 15) / 16, 1 << 20);

@@ -95,7 +95,7 @@ def _pack_bucket(rows: Tensor, bits: int) -> Tuple[Tensor, Tensor]:
     """rows [k, dim] of one bit bucket -> (payload words uint32 of its slabs in runtime order, scale fp16
     [slab][tile][row]).  Low bit-widths: the quantiser and the slab packer are kernels; 16-bit slabs
     (raw halves, all-ones scale) are laid out with tensor ops."""
-    if rows.is_cuda and rows.dtype != torch.float64:
+    if rows.is_cuda and (bits != 16 or rows.dtype != torch.float64):      # (a double becomes a half in one rounding)
         from bitsmoe_amd.algorithms import mlp_forward_cuda as hip
 
         return hip.pack_matrix(rows.to(torch.float32).contiguous(), [(bits, 0, int(rows.shape[0]))])
@@ -145,7 +145,8 @@ def pack_rank_major(rank_major: Tensor, s_vec: Tensor,
     n_tiles = (dim + N_TILE - 1) // N_TILE
     buckets = _bucket_segments(segments, rank)
 
-    if rank_major.is_cuda and rank_major.dtype != torch.float64 and any(bits for bits in buckets):
+    if (rank_major.is_cuda and rank_major.dtype != torch.float64 and any(bits for bits in buckets)
+            and s_vec.dim() == 1 and s_vec.device == rank_major.device):
         return _pack_rank_major_device(rank_major, s_vec, buckets)
 
     payload_parts: List[Tensor] = []
@@ -208,9 +209,9 @@ def _pack_rank_major_device(rank_major: Tensor, s_vec: Tensor, buckets: Dict[int
 
     ranges = [(bits, s, e) for bits in sorted(buckets, reverse=True) if bits for s, e in buckets[bits]]
     matrix = rank_major.to(torch.float32)
-    if matrix.stride(1) != 1:
+    if matrix.stride(1) != 1 or matrix.stride(0) < int(matrix.shape[1]):      # (overlapping rows: an expanded one)
         matrix = matrix.contiguous()
-    payload, scale, s16, rank_idx, tile_meta, slab_meta = hip.pack_matrix(matrix, ranges, s_vec.to(rank_major.device))
+    payload, scale, s16, rank_idx, tile_meta, slab_meta = hip.pack_matrix(matrix, ranges, s_vec)
     seg_rows: List[List[int]] = []
     cursor = 0
     for bits, s, e in ranges:

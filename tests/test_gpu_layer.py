@@ -120,6 +120,32 @@ def test_whole_matrix_packer_equals_quantiser_and_slab_packer(cuda_device, dim, 
     assert at == got.numel()
 
 
+def test_whole_matrix_packer_forms_of_input(cuda_device):
+    """Inputs beside a plain fp32 matrix: a double one (low widths as its fp32 values, halves rounded once), one whose rows
+    overlap (expanded), s on another device (refused) and as a column (kept as it comes)."""
+    import torch
+
+    from bitsmoe_amd.quant.packer import pack_rank_major
+
+    rng = np.random.default_rng(77)
+    x64 = torch.from_numpy(rng.normal(0, 0.02, size=(70, 96))).to(cuda_device)
+    x64[0, 0] = 1.0 + 2.0 ** -11 + 2.0 ** -40      # a half-way case once it went through fp32
+    s = torch.from_numpy(rng.uniform(0.5, 2.0, size=70)).to(cuda_device)
+    segs = [(16, (0, 2)), (3, (2, 20)), (2, (20, 70))]
+    a, b = pack_rank_major(x64, s, segs), pack_rank_major(x64.float(), s.float(), segs)
+    low = 2 * 4 * 16      # the halves' words: rows x micro-tiles x words
+    assert torch.equal(a["payload_buffer"].view(torch.int32)[low:], b["payload_buffer"].view(torch.int32)[low:])
+    assert torch.equal(a["scale_buffer"], b["scale_buffer"])
+    assert int(a["payload_buffer"].view(torch.int32)[0]) & 0xFFFF == int(x64[0, 0].half().view(torch.int16)) & 0xFFFF
+    one = x64.float()[:1].expand(70, 96)
+    e, f = pack_rank_major(one, s, segs), pack_rank_major(one.contiguous(), s, segs)
+    assert all(torch.equal(e[k], f[k]) for k in ("scale_buffer", "s_buffer", "rank_idx_buffer", "tile_meta_buffer", "slab_meta_buffer"))
+    assert torch.equal(e["payload_buffer"].view(torch.int32), f["payload_buffer"].view(torch.int32))
+    with pytest.raises(RuntimeError):
+        pack_rank_major(x64.float(), s.cpu(), segs)
+    assert pack_rank_major(x64.float(), s[:, None], segs)["s_buffer"].shape == (70, 1)
+
+
 def test_batched_uniform_packer_equals_general_packer(cuda_device):
     import torch
 
