@@ -93,18 +93,21 @@ __global__ __launch_bounds__(64 * NW) void k_skinny_linear(const void* __restric
                         round16(hi[0]) | (round16(hi[1]) << 16), round16(hi[2]) | (round16(hi[3]) << 16)};
     };
     for (int s0 = first; s0 < end; s0 += MAXS) {
-        // (no branches: steps past the end repeat the last one and count as zeros)
+        // (no branches: steps past the end repeat the last one and count as zeros -- both operands, or an infinite x would
+        // make a NaN of its row)
         const int ns = end - s0;
         sk_u32x4 b[MAXS];
         auto request_w = [&](int u) {
             b[u] = *reinterpret_cast<const sk_u32x4*>(wp + (int64_t)(s0 + min(u, ns - 1)) * (PREP ? 512 : 32));
         };
-        auto weights = [&](int u) {
-            sk_u32x4 bv = b[u];
+        auto step = [&](int u, sk_f32x4& c, sk_u32x4 av, sk_u32x4 bv) {
             const bool live = u < ns;
 #pragma unroll
-            for (int c = 0; c < 4; ++c) bv[c] = live ? bv[c] : 0u;
-            return bv;
+            for (int i = 0; i < 4; ++i) {
+                av[i] = live ? av[i] : 0u;
+                bv[i] = live ? bv[i] : 0u;
+            }
+            multiply(c, av, bv);
         };
         if constexpr (!TURN) {
             sk_u32x4 xr[MAXS][XF32 ? 2 : 1];
@@ -120,16 +123,16 @@ __global__ __launch_bounds__(64 * NW) void k_skinny_linear(const void* __restric
 #pragma unroll
             for (int u = 0; u < MAXS; ++u) {
                 if constexpr (XF32)
-                    multiply(acc[0], rounded(__builtin_bit_cast(sk_f32x4, xr[u][0]), __builtin_bit_cast(sk_f32x4, xr[u][1])), weights(u));
+                    step(u, acc[0], rounded(__builtin_bit_cast(sk_f32x4, xr[u][0]), __builtin_bit_cast(sk_f32x4, xr[u][1])), b[u]);
                 else
-                    multiply(acc[0], xr[u][0], weights(u));
+                    step(u, acc[0], xr[u][0], b[u]);
             }
             continue;
         }
         sk_u32x4 xr[2][NI];
         auto request_x = [&](auto p_c) {
             constexpr int P = decltype(p_c)::value;
-            // (a piece that would stick out of the row is moved back: its steps are found `shift` further up, or count as zeros)
+            // (a piece that would stick out of the row is moved back: its steps are found `shift` further up)
             const int at = min(s0 + P * G, steps - G);
 #pragma unroll
             for (int i = 0; i < NI; ++i) xr[P & 1][i] = *reinterpret_cast<const sk_u32x4*>(xrow[i] + (int64_t)at * (32 * EB));
@@ -149,17 +152,16 @@ __global__ __launch_bounds__(64 * NW) void k_skinny_linear(const void* __restric
             const int shift = s0 + P * G - min(s0 + P * G, steps - G);
 #pragma unroll
             for (int g = 0; g < G; ++g) {
-                const sk_u32x4 bv = weights(P * G + g);
                 const int gs = min(g + shift, G - 1);
 #pragma unroll
                 for (int mb = 0; mb < NMB; ++mb) {
                     const int r = 16 * mb + n;
                     const unsigned char* row = piece + r * (CPR * 16);
                     if constexpr (XF32)
-                        multiply(acc[mb], rounded(*reinterpret_cast<const sk_f32x4*>(row + (((gs * 8 + 2 * kg) ^ swz(r)) << 4)),
-                                                  *reinterpret_cast<const sk_f32x4*>(row + (((gs * 8 + 2 * kg + 1) ^ swz(r)) << 4))), bv);
+                        step(P * G + g, acc[mb], rounded(*reinterpret_cast<const sk_f32x4*>(row + (((gs * 8 + 2 * kg) ^ swz(r)) << 4)),
+                                                      *reinterpret_cast<const sk_f32x4*>(row + (((gs * 8 + 2 * kg + 1) ^ swz(r)) << 4))), b[P * G + g]);
                     else
-                        multiply(acc[mb], *reinterpret_cast<const sk_u32x4*>(row + (((gs * 4 + kg) ^ swz(r)) << 4)), bv);
+                        step(P * G + g, acc[mb], *reinterpret_cast<const sk_u32x4*>(row + (((gs * 4 + kg) ^ swz(r)) << 4)), b[P * G + g]);
                 }
             }
         }, std::make_integer_sequence<int, MAXS / G>{});

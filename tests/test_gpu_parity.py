@@ -732,3 +732,22 @@ def test_skinny_linear_matches_float64(cuda_device, rows, k, n, dtype_name):
 @pytest.mark.parametrize("dtype_name", ["bf16", "f16"])
 def test_skinny_linear_edges(cuda_device, rows, k, n, dtype_name):
     test_skinny_linear_matches_float64(cuda_device, rows, k, n, dtype_name)
+
+
+@pytest.mark.parametrize("rows,k,x_dtype", [(1, 896, "bf16"), (16, 896, "bf16"), (40, 1536, "bf16"), (2, 896, "f32"), (9, 896, "f32")])
+def test_skinny_linear_infinite_activation(cuda_device, rows, k, x_dtype):
+    """An infinite activation gives an infinite output, not a NaN: shares of 7 and 12 steps, fewer than are requested."""
+    import torch
+
+    from bitsmoe_amd.algorithms import mlp_forward_cuda as hip
+
+    x = torch.ones((rows, k), device=cuda_device, dtype=torch.bfloat16 if x_dtype == "bf16" else torch.float32)
+    w = torch.ones((32, k), device=cuda_device, dtype=torch.bfloat16)
+    for at in (k // 4 - 1, k - 1):      # the step that the first and the last wavefront end with
+        xi = x.clone()
+        xi[rows // 2, at] = float("inf")
+        for weight in (w, hip.PreparedLinearWeight(w)):
+            y = hip.skinny_linear(xi, weight).float()
+            assert bool(torch.isinf(y[rows // 2]).all())
+            others = [r for r in range(rows) if r != rows // 2]
+            assert bool((y[others] == torch.tensor(float(k), dtype=torch.bfloat16).item()).all())
