@@ -783,6 +783,7 @@ class BlockPlan:
             setattr(c, name, value)
         self.c = c
         self.address = ctypes.addressof(c)
+        self._weights: dict = {}      # (kept alive; an entry is made once its field is set)
         self._bytes: dict = {}
 
     def is_current(self) -> bool:
@@ -792,10 +793,13 @@ class BlockPlan:
     def set_weight(self, name: str, weight) -> None:
         """w_in / w_out / w_router: a tensor or a PreparedLinearWeight of it."""
         prepared = isinstance(weight, PreparedLinearWeight)
-        self._keep += (weight,)
         if name != "w_router":
             setattr(self.c, name + "_prepared", 1 if prepared else 0)
         setattr(self.c, name, (weight.data if prepared else weight).data_ptr())
+        self._weights[name] = weight
+
+    def has_weight(self, name: str) -> bool:
+        return name in self._weights
 
     def workspace_bytes(self, n_tokens: int) -> int:
         n = self._bytes.get(n_tokens)

@@ -28,6 +28,7 @@ _BUFFER_NAMES = ("payload", "rank_idx", "tile_meta", "slab_meta", "scale", "s")
 
 
 import os as _os
+import threading as _threading
 
 _CHECK_VERSIONS = _os.environ.get("BITSMOE_BLOCK_CHECK_VERSIONS", "0") == "1"
 # BITSMOE_SUPER_SIDE_STREAM=0: the super experts' operator call on the caller's stream, after the packed experts'
@@ -62,6 +63,9 @@ _SKINNY_NARROW_FEATURES = 4352    # output features, and
 _SKINNY_SHORT_CONTRACTION = 4096  # input features up to which 49 to 64 rows take it
 # BITSMOE_BLOCK_SKINNY_PREPARED=0: the few-rows kernel reads the stacked weights in the framework's layout (no extra copy)
 _SKINNY_PREPARED = _os.environ.get("BITSMOE_BLOCK_SKINNY_PREPARED", "1") != "0"
+
+
+_FEW_ROWS_LOCK = _threading.Lock()      # (held while a layer's copy is made, once; never during a forward)
 
 
 def _few_rows(rows: int, n_in: int, n_out: int) -> bool:
@@ -511,10 +515,10 @@ class BitsMoE_BaseSparseMoeBlock(nn.Module):
     def _plain_linear(mod) -> bool:
         return isinstance(mod, nn.Linear) and mod.bias is None and isinstance(mod.weight, torch.Tensor) and mod.weight.dim() == 2
 
-    def _fused_plan(self, dtype: torch.dtype, router: Optional[nn.Module], shared: Optional[nn.Module],
+    def _fused_plan(self, dtype: torch.dtype, bases, router: Optional[nn.Module], shared: Optional[nn.Module],
                     shared_gate: Optional[nn.Module]):
-        """The stacked input / output weights and the column ranges of their parts, or None when a module is not
-        a bias-free linear layer of the expected shape.  Cached; rebuilt when a source tensor was rebound or written."""
+        """The stacked input / output weights (`bases`: the three shared bases) and the column ranges of their parts, or
+        None when a module is not a bias-free linear layer of the expected shape.  Cached; rebuilt when a source tensor was rebound or written."""
         linears = [] if router is None else [router]
         if shared is not None:
             linears += [getattr(shared, n, None) for n in ("gate_proj", "up_proj", "down_proj")]
@@ -522,7 +526,7 @@ class BitsMoE_BaseSparseMoeBlock(nn.Module):
             linears.append(shared_gate)
         if not all(map(self._plain_linear, linears)):
             return None
-        vh_gate, vh_up, u_down = (self._buffers[k] for k in self._SHARED_BASIS_BUFFER_KEYS)
+        vh_gate, vh_up, u_down = bases
         sources = [vh_gate, vh_up, u_down] + [lin.weight for lin in linears]
         stamp = tuple((id(t), t.data_ptr(), -1 if t.is_inference() else t._version) for t in sources)
         key = ("fused_plan", dtype, router is not None, shared is not None, shared_gate is not None)
@@ -530,7 +534,7 @@ class BitsMoE_BaseSparseMoeBlock(nn.Module):
         if cached is not None and cached["stamp"] == stamp:
             return cached
         hidden = int(vh_gate.shape[1])
-        if router is not None and int(router.weight.shape[1]) != hidden:
+        if router is not None and tuple(router.weight.shape) != (int(self._packed_global_to_local.numel()), hidden):
             return None
         if shared is not None:
             wg, wu, wd = (getattr(shared, n).weight for n in ("gate_proj", "up_proj", "down_proj"))
@@ -606,18 +610,22 @@ class BitsMoE_BaseSparseMoeBlock(nn.Module):
         if router_weight is not None:
             native.set_weight("w_router", router_weight)
         plan["native"] = (native, stamp)
-        plan["few_rows_weights"] = {}
         return native
 
-    def _few_rows_weight(self, plan: dict, native, key: str) -> None:
-        """The weight the few-rows kernel reads: a copy in MFMA operand order, made on first use and kept with the plan."""
-        if key not in plan["few_rows_weights"]:
+    @staticmethod
+    def _few_rows_weight(plan: dict, native, key: str) -> None:
+        """The weight the few-rows kernel reads: a copy in MFMA operand order, made on first use and kept with the plan.
+        (Two threads may come here at once, each with a native plan of its own or both with one: one of them makes it.)"""
+        if native.has_weight(key):
+            return
+        with _FEW_ROWS_LOCK:
+            if native.has_weight(key):
+                return
             weight = plan.get(key + "_prepared")
             if weight is None:
                 weight = mlp_forward_cuda.PreparedLinearWeight(plan[key]) if _SKINNY_PREPARED else plan[key]
                 plan[key + "_prepared"] = weight
             native.set_weight(key, weight)
-            plan["few_rows_weights"][key] = weight
 
     def _fused_block_forward(self, hidden_states: torch.Tensor, *, router: Optional[nn.Module] = None, linear_gate=None, route_fn=None,
                              renormalize: bool = True, round_weights: bool = True, weight_scale: float = 1.0,
@@ -632,13 +640,13 @@ class BitsMoE_BaseSparseMoeBlock(nn.Module):
                 and self._packed_global_to_local is not None and (dtype is torch.float16 or dtype is torch.bfloat16)
                 and self._packed_intermediate_size > 0 and not _dense_via_operator()):
             return None
-        buffers = self._buffers
-        if any(buffers[k].numel() == 0 for k in self._SHARED_BASIS_BUFFER_KEYS):
+        bases = tuple(getattr(self, k) for k in self._SHARED_BASIS_BUFFER_KEYS)
+        if any(b.numel() == 0 for b in bases):
             return None
         if router is not None and not (int(router.weight.shape[0]) <= 1024 and self.top_k <= 64):
             return None
         self._act_type()
-        plan = self._fused_plan(dtype, router, shared, shared_gate)
+        plan = self._fused_plan(dtype, bases, router, shared, shared_gate)
         if plan is None:
             return None
         x = hidden_states

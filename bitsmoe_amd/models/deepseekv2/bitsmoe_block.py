@@ -43,6 +43,7 @@ class BitsMoE_DeepSeekSparseMoeBlock(BitsMoE_BaseSparseMoeBlock):
                 or getattr(gate, "topk_method", "greedy") not in ("greedy", "gready") or not hasattr(gate, "top_k")
                 or not hasattr(gate, "norm_topk_prob") or not hasattr(gate, "routed_scaling_factor")
                 or not isinstance(weight, torch.Tensor) or int(gate.top_k) != self.top_k
+                or self._packed_global_to_local is None or int(weight.shape[0]) != int(self._packed_global_to_local.numel())
                 or not mlp_forward_cuda.router_linear_topk_possible(x, weight, self.top_k)):
             return None
         renorm = self.top_k > 1 and bool(gate.norm_topk_prob)

@@ -345,3 +345,36 @@ def test_block_in_one_call_equals_module_by_module(cuda_device, family, kw, toke
     assert not errors, errors
     for a, b in zip(got, alone):      # (fp32 atomics in another order, then one bf16 rounding)
         assert float((a - b).abs().max()) <= 1e-2 * float(b.abs().max())
+
+
+def test_block_plan_made_twice_at_once(cuda_device, monkeypatch):
+    """Two first forwards of one block at the same time may each make a native plan: both get both projections' weights
+    (the second forward runs here in the middle of the first, where a thread switch would put it).  And a router whose
+    width is not the number of experts is not taken into the stacked weights."""
+    import torch
+
+    from bitsmoe_amd.synth import make_layer
+
+    block = make_layer(_small_spec("qwen3moe"), device=cuda_device, dtype=torch.bfloat16, seed=5, s_mode="rand")
+    block.prepare_runtime_fastpath(warmup=True)
+    x = torch.randn((1, 8, block.spec.hidden_size), generator=torch.Generator().manual_seed(3)).to(torch.bfloat16).to(cuda_device)
+    first = lambda out: (out[0] if isinstance(out, tuple) else out).float()
+    real, inner = block._few_rows_weight, []
+
+    def between(plan, native, key):
+        if not inner:
+            inner.append(None)
+            plan.pop("native")
+            inner[0] = first(block(x))
+        return real(plan, native, key)
+
+    with torch.no_grad():
+        monkeypatch.setattr(block, "_few_rows_weight", between)
+        outer = first(block(x))
+        monkeypatch.undo()
+        again = first(block(x))
+    for y in (inner[0], outer):      # (fp32 atomics in another order, then one bf16 rounding)
+        assert float((y - again).abs().max()) <= 1e-2 * float(again.abs().max())
+    wide = torch.nn.Linear(block.spec.hidden_size, block.spec.num_experts + 8, bias=False).to(cuda_device)
+    bases = tuple(getattr(block, k) for k in block._SHARED_BASIS_BUFFER_KEYS)
+    assert block._fused_plan(torch.bfloat16, bases, wide, None, None) is None
