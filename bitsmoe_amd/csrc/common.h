@@ -151,6 +151,7 @@ struct RouteSideJobs {
     MTile* mtiles = nullptr;             // [max_mtiles]; null: not wanted
     int32_t* n_mtiles = nullptr;
     int max_mtiles = 0;
+    int mtile_rows = 0;                  // assignments per tile at most
     const FastExpert* gate_fe = nullptr;
     const FastExpert* up_fe = nullptr;
 };

@@ -25,6 +25,7 @@
 #include <type_traits>
 
 #include "fast_helpers.h"
+#include "launch_policy.h"
 #include "mtiles.h"
 
 // ---- optional in-kernel time stamps (timeline build: -DBITSMOE_TIMELINE) of k_gateup_mfma / k_down_mfma: thread 0 of a
@@ -74,7 +75,7 @@ __global__ __launch_bounds__(256) void k_token_count(const int32_t* __restrict__
 // One workgroup: the list of (expert, first assignment, rows <= 128) tiles from
 // expert_offsets (build_mtile_list), then token_start = exclusive scan of token_count (T + 1 entries).
 __global__ __launch_bounds__(256) void k_build_mtiles(const int32_t* __restrict__ expert_offsets, int E, int A,
-                                                      int max_tiles, MTile* __restrict__ tiles,
+                                                      int tile_rows, int max_tiles, MTile* __restrict__ tiles,
                                                       int32_t* __restrict__ n_tiles_out,
                                                       const int32_t* __restrict__ token_count, int T,
                                                       int32_t* __restrict__ token_start,
@@ -83,7 +84,7 @@ __global__ __launch_bounds__(256) void k_build_mtiles(const int32_t* __restrict_
     __shared__ int scan[256];
     __shared__ MTileLds mt_lds;
     const int tid = threadIdx.x;
-    build_mtile_list(expert_offsets, E, A, max_tiles, tiles, n_tiles_out, gate_fe, up_fe, mt_lds);
+    build_mtile_list(expert_offsets, E, A, tile_rows, max_tiles, tiles, n_tiles_out, gate_fe, up_fe, mt_lds);
 
     if (token_count == nullptr) return;
     // every thread scans one contiguous run of tokens (a multiple of four: 16-byte loads)
@@ -264,7 +265,7 @@ __device__ __forceinline__ void barrier_no_drain() {
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
 }
-constexpr int DMA_STAGE = PF_M * 64;    // 16-bit elements of one unpadded 128 x 64 activation piece
+constexpr int dma_stage(int tile_rows) { return tile_rows * 64; }    // 16-bit elements of an unpadded rows x 64 activation piece
 
 // LDS-direct load: every active lane fetches 16 bytes from `src`, and the wavefront's data lands in
 // LDS at lds_base + 16 * lane (lds_base is wave-uniform).  Issued from an asm statement, so the
@@ -353,7 +354,7 @@ constexpr int DMA_SSTAGE = 4 * 64;      // 16-bit scales: 64 contraction rows pe
 
 // One stage of the ring: everything a workgroup needs for one slab.
 struct DmaStage {
-    uint16_t* a;     // [DMA_STAGE]
+    uint16_t* a;     // [dma_stage(PFM)]
     uint32_t* w;     // [DMA_WSTAGE]
     uint16_t* sc;    // [DMA_SSTAGE]
 };
@@ -376,7 +377,7 @@ struct DmaStage {
 // token index (possible when every aligned run of 8 local rows is 8 consecutive logical ranks);
 // otherwise Hs is the pre-gathered [A, ld].  WU: the bit-width shared by every slab of the
 // matrix, or 0 (mixed).  NMB: 16-row blocks of the assignment tile that are computed.
-template <bool DIRECT, int WU, int NMB>
+template <bool DIRECT, int PFM, int WU, int NMB>
 __device__ __forceinline__ void gateup_tile_body(const FastExpert fe, const FastSlab* __restrict__ fs_row, int all_slabs,
                                                      const uint16_t* __restrict__ Hs, int ld,
                                                      const int32_t* __restrict__ token_indices, int T, int I,
@@ -545,7 +546,7 @@ __device__ __forceinline__ void gateup_tile_body(const FastExpert fe, const Fast
     BITSMOE_TLP(g_tl_pf_gateup, 3);
     if (!active) return;
     uint16_t* cols = out + (int64_t)a_begin * I + N_TILE * t + 64 * wn;
-    store_turned<NMB>(turn + wave * DMA_STAGE, rows, lane, acc, [&](int row, int c, u32x4 v) {
+    store_turned<NMB>(turn + wave * dma_stage(PFM), rows, lane, acc, [&](int row, int c, u32x4 v) {
         u32x4* dst = reinterpret_cast<u32x4*>(cols + (int64_t)row * I + 8 * c);
         if (fuse_silu) {
             // `out` holds the gate sums an earlier launch stored: z = silu(gate) * up takes their place
@@ -561,8 +562,11 @@ __device__ __forceinline__ void gateup_tile_body(const FastExpert fe, const Fast
 }
 
 // grid.x = 32 * ceil(max_mtiles / 32) * (2 or 1 projections) * ceil(n_tiles / 2), 256 threads; G and U are f16 [A, I].
-template <bool DIRECT>
-__global__ __launch_bounds__(256, 2) void k_gateup_mfma(
+// PFM: assignments per tile at most.  With 128 the ring takes 78 KB of LDS and a wavefront up to 247 registers: two workgroups
+// per CU.  With 64 (53 KB, 145 registers: three) a short tile's step -- a quarter or half of the MFMAs behind the same loads,
+// waits and barrier -- is hidden by one more workgroup (rule and measurements: launch_policy.h); k_down_mfma likewise.
+template <bool DIRECT, int PFM>
+__global__ __launch_bounds__(256, PFM == 128 ? 2 : 3) void k_gateup_mfma(
     const FastExpert* __restrict__ gate_fe, const FastSlab* __restrict__ gate_fs, int gate_max_slabs,
     const FastExpert* __restrict__ up_fe, const FastSlab* __restrict__ up_fs, int up_max_slabs,
     const uint16_t* __restrict__ Hs_g, const uint16_t* __restrict__ Hs_u, int ldg, int ldu,
@@ -570,8 +574,8 @@ __global__ __launch_bounds__(256, 2) void k_gateup_mfma(
     const MTile* __restrict__ mtiles, const int32_t* __restrict__ n_mtiles, int I, int n_tiles,
     uint16_t* __restrict__ G, uint16_t* __restrict__ U, int proj_sel, int fuse) {
     // the ring (three activation stages, three payload stages), which the epilogue uses again: 16 KB per wavefront
-    __shared__ __attribute__((aligned(16))) uint16_t ring[DMA_STAGES * (DMA_STAGE + 2 * DMA_WSTAGE)];
-    static_assert(sizeof(ring) >= 4 * DMA_STAGE * sizeof(uint16_t), "the epilogue's space");
+    __shared__ __attribute__((aligned(16))) uint16_t ring[DMA_STAGES * (dma_stage(PFM) + 2 * DMA_WSTAGE)];
+    static_assert(sizeof(ring) >= 4 * dma_stage(PFM) * sizeof(uint16_t), "the epilogue's space");
     __shared__ __attribute__((aligned(16))) uint16_t ss0[DMA_SSTAGE], ss1[DMA_SSTAGE], ss2[DMA_SSTAGE];
     __shared__ int32_t pack_tab[DMA_MAX_SLABS], scale_tab[DMA_MAX_SLABS], rank_tab[DMA_MAX_SLABS * 8], bits_tab[DMA_MAX_SLABS];
     BITSMOE_TLP(g_tl_pf_gateup, 0);
@@ -602,34 +606,36 @@ __global__ __launch_bounds__(256, 2) void k_gateup_mfma(
     // tiles of at most 32 / 64 / 96 assignments (experts that see few tokens, remainders) run a body
     // with a quarter / half / three quarters of the accumulators, MFMAs and staging; complete
     // bodies, so that no accumulator lives across the choice
-    uint32_t* sw = reinterpret_cast<uint32_t*>(ring + DMA_STAGES * DMA_STAGE);
-    const DmaStage st0 = {ring, sw, ss0}, st1 = {ring + DMA_STAGE, sw + DMA_WSTAGE, ss1},
-                   st2 = {ring + 2 * DMA_STAGE, sw + 2 * DMA_WSTAGE, ss2};
+    constexpr int STAGE = dma_stage(PFM);
+    uint32_t* sw = reinterpret_cast<uint32_t*>(ring + DMA_STAGES * STAGE);
+    const DmaStage st0 = {ring, sw, ss0}, st1 = {ring + STAGE, sw + DMA_WSTAGE, ss1},
+                   st2 = {ring + 2 * STAGE, sw + 2 * DMA_WSTAGE, ss2};
     BITSMOE_TLP(g_tl_pf_gateup, 1);
-#define BITSMOE_GU_BODY(W)                                                                                           \
-    do {                                                                                                             \
-        if (rows <= 32)                                                                                              \
-            gateup_tile_body<DIRECT, W, 2>(fe, fs_row, nslabs, Hs, ld, token_indices, T, I, n_tiles, out,         \
-                                               a_begin, rows, 2 * tp, st0, st1, st2, ring, pack_tab, scale_tab, rank_tab, bits_tab, fuse_silu); \
-        else if (rows <= 64)                                                                                         \
-            gateup_tile_body<DIRECT, W, 4>(fe, fs_row, nslabs, Hs, ld, token_indices, T, I, n_tiles, out,         \
-                                               a_begin, rows, 2 * tp, st0, st1, st2, ring, pack_tab, scale_tab, rank_tab, bits_tab, fuse_silu); \
-        else if (rows <= 96)                                                                                         \
-            gateup_tile_body<DIRECT, W, 6>(fe, fs_row, nslabs, Hs, ld, token_indices, T, I, n_tiles, out,         \
-                                               a_begin, rows, 2 * tp, st0, st1, st2, ring, pack_tab, scale_tab, rank_tab, bits_tab, fuse_silu); \
-        else                                                                                                         \
-            gateup_tile_body<DIRECT, W, 8>(fe, fs_row, nslabs, Hs, ld, token_indices, T, I, n_tiles, out,         \
-                                               a_begin, rows, 2 * tp, st0, st1, st2, ring, pack_tab, scale_tab, rank_tab, bits_tab, fuse_silu); \
-    } while (0)
+    auto body = [&](auto w_c, auto nmb_c) {
+        gateup_tile_body<DIRECT, PFM, decltype(w_c)::value, decltype(nmb_c)::value>(
+            fe, fs_row, nslabs, Hs, ld, token_indices, T, I, n_tiles, out, a_begin, rows, 2 * tp, st0, st1, st2, ring, pack_tab,
+            scale_tab, rank_tab, bits_tab, fuse_silu);
+    };
+    auto by_rows = [&](auto w_c) {
+        if (rows <= 32)
+            body(w_c, std::integral_constant<int, 2>{});
+        else if (rows <= 64)
+            body(w_c, std::integral_constant<int, 4>{});
+        else if constexpr (PFM > 64) {
+            if (rows <= 96)
+                body(w_c, std::integral_constant<int, 6>{});
+            else
+                body(w_c, std::integral_constant<int, 8>{});
+        }
+    };
     if (w == 2)
-        BITSMOE_GU_BODY(2);
+        by_rows(std::integral_constant<int, 2>{});
     else if (w == 3)
-        BITSMOE_GU_BODY(3);
+        by_rows(std::integral_constant<int, 3>{});
     else if (w == 4)
-        BITSMOE_GU_BODY(4);
+        by_rows(std::integral_constant<int, 4>{});
     else
-        BITSMOE_GU_BODY(0);
-#undef BITSMOE_GU_BODY
+        by_rows(std::integral_constant<int, 0>{});
     BITSMOE_TLP(g_tl_pf_gateup, 6);
 }
 
@@ -826,7 +832,8 @@ __device__ __forceinline__ void down_tile_loop(const uint32_t* __restrict__ payl
 // Output: y[a, r] = s[r] * sum_c W_down[r, c] z[a, c] as f16, r in the expert's own row order, and the per-token
 // assignment lists
 // token_list[token_start[tok_a] + slot[a]] = (a, expert) that k_combine_tokens walks.
-__global__ __launch_bounds__(256, 2) void k_down_mfma(const FastExpert* __restrict__ down_fe,
+template <int PFM>
+__global__ __launch_bounds__(256, PFM == 128 ? 2 : 3) void k_down_mfma(const FastExpert* __restrict__ down_fe,
                                                       const FastSlab* __restrict__ down_fs, int max_slabs,
                                                       const uint16_t* __restrict__ z, const MTile* __restrict__ mtiles,
                                                       const int32_t* __restrict__ n_mtiles,
@@ -836,10 +843,11 @@ __global__ __launch_bounds__(256, 2) void k_down_mfma(const FastExpert* __restri
                                                       int2* __restrict__ token_list, int A, int I, int n_tiles,
                                                       int n_groups, _Float16* __restrict__ y, int ldy) {
     // three stages of z and the wavefronts' payload buffers, which the epilogue uses again: 16 KB per wavefront
-    __shared__ __attribute__((aligned(16))) uint16_t lds[3 * DMA_STAGE + 2 * 4 * DN_WBUF];
-    static_assert(sizeof(lds) >= 4 * DMA_STAGE * sizeof(uint16_t), "the epilogue's space");
-    uint16_t *sz0 = lds, *sz1 = lds + DMA_STAGE, *sz2 = lds + 2 * DMA_STAGE;
-    uint32_t* wbuf = reinterpret_cast<uint32_t*>(lds + 3 * DMA_STAGE);
+    __shared__ __attribute__((aligned(16))) uint16_t lds[3 * dma_stage(PFM) + 2 * 4 * DN_WBUF];
+    constexpr int STAGE = dma_stage(PFM);
+    static_assert(sizeof(lds) >= 4 * STAGE * sizeof(uint16_t), "the epilogue's space");
+    uint16_t *sz0 = lds, *sz1 = lds + STAGE, *sz2 = lds + 2 * STAGE;
+    uint32_t* wbuf = reinterpret_cast<uint32_t*>(lds + 3 * STAGE);
     __shared__ __attribute__((aligned(16))) uint16_t sbuf[4 * DN_SBUF];
     BITSMOE_TLP(g_tl_pf_down, 0);
     const int logical = xcd_logical(blockIdx.x, __builtin_amdgcn_readfirstlane(*n_mtiles), n_groups);
@@ -891,7 +899,7 @@ __global__ __launch_bounds__(256, 2) void k_down_mfma(const FastExpert* __restri
             for (int mb = 0; mb < NMB; ++mb) acc[mb][nb] *= srow;
         }
         _Float16* block = y + (int64_t)a_begin * ldy + fs.rank_off;
-        store_turned<NMB>(lds + wave * DMA_STAGE, rows, lane, acc, [&](int row, int c, u32x4 v) {
+        store_turned<NMB>(lds + wave * STAGE, rows, lane, acc, [&](int row, int c, u32x4 v) {
             *reinterpret_cast<u32x4*>(block + (int64_t)row * ldy + 8 * c) = v;
         });
     };
@@ -899,10 +907,12 @@ __global__ __launch_bounds__(256, 2) void k_down_mfma(const FastExpert* __restri
         run(std::integral_constant<int, 2>{});
     else if (rows <= 64)
         run(std::integral_constant<int, 4>{});
-    else if (rows <= 96)
-        run(std::integral_constant<int, 6>{});
-    else
-        run(std::integral_constant<int, 8>{});
+    else if constexpr (PFM > 64) {
+        if (rows <= 96)
+            run(std::integral_constant<int, 6>{});
+        else
+            run(std::integral_constant<int, 8>{});
+    }
     BITSMOE_TLP(g_tl_pf_down, 6);
 }
 
@@ -1037,13 +1047,18 @@ static bool direct_ok(const bitsmoe_matset* gate, const bitsmoe_matset* up) {
 // (columns of the f16 copy of bf16 activations: every rank the prepared rank table names, padding rows included)
 static inline int direct_ld(const bitsmoe_matset* set) { return (set->pad_rank_plus1 + 7) / 8 * 8; }
 
+// Assignments per tile at most: low tiles while experts have few assignments (launch_policy.h).
+static inline int mtile_rows(int64_t A, int E) {
+    return A <= (int64_t)policy::LOW_TILES_MAX_ASSIGN_PER_EXPERT * E ? PF_M / 2 : PF_M;
+}
+
 // Carving of the workspace, shared by the size query and the launcher.
 struct MfmaWorkspace {
     size_t mtiles, n_mtiles, token_count, token_start, slot, token_list, acts, z, u, y, total;
 };
 static MfmaWorkspace mfma_workspace(const bitsmoe_matset* gate, const bitsmoe_matset* up, const bitsmoe_matset* down,
                                     int64_t T, int64_t A, int I) {
-    const int64_t max_mtiles = A / PF_M + gate->n_experts;
+    const int64_t max_mtiles = A / (PF_M / 2) + gate->n_experts;      // (of the lower tiles: never less for more assignments)
     const size_t direct = align256((size_t)T * direct_ld(gate) * 2) + align256((size_t)T * direct_ld(up) * 2);
     const size_t gathered = align256((size_t)A * gate->prep_max_slabs * SLAB_ROWS * 2) + align256((size_t)A * up->prep_max_slabs * SLAB_ROWS * 2);
     MfmaWorkspace w;
@@ -1118,7 +1133,8 @@ bool mfma_front_jobs(const bitsmoe_matset* gate, const bitsmoe_matset* up, const
     jobs->token_start = (int32_t*)(ws + w.token_start);
     jobs->mtiles = (MTile*)(ws + w.mtiles);
     jobs->n_mtiles = (int32_t*)(ws + w.n_mtiles);
-    jobs->max_mtiles = (int)(A / PF_M + gate->n_experts);
+    jobs->mtile_rows = mtile_rows(A, gate->n_experts);
+    jobs->max_mtiles = (int)(A / jobs->mtile_rows + gate->n_experts);
     jobs->gate_fe = gate->d_fast_experts;
     jobs->up_fe = up->d_fast_experts;
     return true;
@@ -1130,7 +1146,8 @@ int launch_forward_mfma(const bitsmoe_matset* gate, const bitsmoe_matset* up, co
                         int I, float* rank_accum, void* workspace, int front_done, bitsmoe_profile* prof, hipStream_t st) {
     const int E = gate->n_experts;
     const int n_tiles = gate->n_tiles;
-    const int64_t max_mtiles = A / PF_M + E;
+    const int tile_rows = mtile_rows(A, E);
+    const int64_t max_mtiles = A / tile_rows + E;
     const ActsPlan plan = acts_plan(gate, up, h_gate, h_up, act_dtype, T, Rg, Ru, ldg_in, ldu_in);
     const bool direct = plan.direct;
     const int ldg = plan.ldg, ldu = plan.ldu;
@@ -1167,7 +1184,7 @@ int launch_forward_mfma(const bitsmoe_matset* gate, const bitsmoe_matset* up, co
         hipLaunchKernelGGL(k_token_count, dim3((unsigned)((A + 255) / 256)), dim3(256), 0, st, tok, off, E, (int)A, (int)T,
                            token_count, slot);
     if (!counted)
-        hipLaunchKernelGGL(k_build_mtiles, dim3(1), dim3(256), 0, st, off, E, (int)A, (int)max_mtiles, mtiles, n_mtiles,
+        hipLaunchKernelGGL(k_build_mtiles, dim3(1), dim3(256), 0, st, off, E, (int)A, tile_rows, (int)max_mtiles, mtiles, n_mtiles,
                            token_count, (int)T, token_start, gate->d_fast_experts, up->d_fast_experts);
     BITSMOE_HIP_TRY(hipGetLastError());
     if (direct) {
@@ -1204,12 +1221,14 @@ int launch_forward_mfma(const bitsmoe_matset* gate, const bitsmoe_matset* up, co
                                (int)T, mtiles, n_mtiles, I, n_tiles, z, Ubuf, proj_sel, fuse);
             return hipGetLastError();
         };
+        const auto kernel = tile_rows == PF_M ? (direct ? k_gateup_mfma<true, PF_M> : k_gateup_mfma<false, PF_M>)
+                                              : (direct ? k_gateup_mfma<true, PF_M / 2> : k_gateup_mfma<false, PF_M / 2>);
         if (split) {
-            BITSMOE_HIP_TRY(direct ? launch(k_gateup_mfma<true>, 0, 0) : launch(k_gateup_mfma<false>, 0, 0));
-            BITSMOE_HIP_TRY(direct ? launch(k_gateup_mfma<true>, 1, 1) : launch(k_gateup_mfma<false>, 1, 1));
+            BITSMOE_HIP_TRY(launch(kernel, 0, 0));
+            BITSMOE_HIP_TRY(launch(kernel, 1, 1));
             record(prof, 2, st);
         } else {
-            BITSMOE_HIP_TRY(direct ? launch(k_gateup_mfma<true>, -1, 0) : launch(k_gateup_mfma<false>, -1, 0));
+            BITSMOE_HIP_TRY(launch(kernel, -1, 0));
             if (wide_gu) {      // rows of 6-, 8- and 16-bit slabs: their share of the (f16) gate and up sums
                 const int rc = launch_wide_gateup(gate, up, h_gate, h_up, act_dtype, Rg, Ru, ldg_in, ldu_in, tok, off, A, I, z, Ubuf,
                                                   true, st);
@@ -1226,8 +1245,8 @@ int launch_forward_mfma(const bitsmoe_matset* gate, const bitsmoe_matset* up, co
     {
         const int n_pairs = (down->prep_max_slabs + DN_SLABS_MFMA - 1) / DN_SLABS_MFMA;
         const int64_t wgs = (max_mtiles + 31) / 32 * 32 * n_pairs;
-        hipLaunchKernelGGL(k_down_mfma, dim3((unsigned)wgs), dim3(256), 0, st, down->d_fast_experts, down->d_fast_slabs,
-                           down->prep_max_slabs, z, mtiles, n_mtiles, tok, slot, token_start, token_list, (int)A, I, n_tiles,
+        hipLaunchKernelGGL((tile_rows == PF_M ? k_down_mfma<PF_M> : k_down_mfma<PF_M / 2>), dim3((unsigned)wgs), dim3(256), 0, st,
+                           down->d_fast_experts, down->d_fast_slabs, down->prep_max_slabs, z, mtiles, n_mtiles, tok, slot, token_start, token_list, (int)A, I, n_tiles,
                            n_pairs, y, ldy);
         record(prof, 4, st);
         if (down->rank_identity)

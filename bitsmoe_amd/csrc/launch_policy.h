@@ -14,6 +14,14 @@ namespace policy {
 // assignments, the grouped GEMM pays for a longer launch chain: routing, conversion, SiLU pass, combine).
 constexpr int MFMA_MIN_ASSIGN_PER_EXPERT = 14;
 
+// Grouped GEMM: tiles of at most 64 assignments (three workgroups per CU: half the accumulators and half the activation
+// stages) instead of 128 (two) up to this many assignments per expert on average.  Most tiles are that low there anyway, and
+// their steps are short: what a CU needs is more of them.  Operator, us, 128 -> 64 rows, at 15 / 20 / 32 / 48 / 64
+// assignments per expert: 128-expert layer 118 -> 109, 120 -> 112, 131 -> 126, 151 -> 147, 168 -> 177; 64-expert layer 113 -> 103,
+// 109 -> 102, 123 -> 116, 135 -> 133, 150 -> 163; 512-expert layer 250 -> 222, 257 -> 229, 300 -> 273, 344 -> 315, 392 -> 402.
+// (Experts above 64 assignments read their payload twice.)
+constexpr int LOW_TILES_MAX_ASSIGN_PER_EXPERT = 48;
+
 // Decode grids.  The expert coordinate counts 16-assignment CHUNKS from this many assignments per expert on average
 // (most experts then have several chunks; below, the chunk search -- one more dependent round trip per workgroup,
 // +10 % -- costs more than walking an expert's few chunks in a loop) ...

@@ -1,4 +1,4 @@
-// Tile list of the grouped-GEMM path: (expert, first assignment, rows <= 128) tiles of the expert-sorted
+// Tile list of the grouped-GEMM path: (expert, first assignment, rows <= tile_rows) tiles of the expert-sorted
 // assignment list, ordered by decreasing cost.  Built by the workgroup that has the expert offsets at hand:
 // the grouped-GEMM launcher's own kernel, or the routing scan when the forward starts from the router's output.
 #pragma once
@@ -6,7 +6,7 @@
 
 namespace bitsmoe {
 
-constexpr int PF_M = 128;        // assignments per workgroup tile
+constexpr int PF_M = 128;        // assignments per workgroup tile at most
 
 struct MTile {
     int32_t expert;   // -1: unused slot
@@ -33,8 +33,8 @@ struct MTileLds {
 
 // Whole workgroup (every thread calls it; `offsets` holds E + 1 entries in global memory or LDS, written before
 // a barrier the caller has passed).  Writes tiles[0 .. max_tiles) and *n_tiles_out.
-__device__ inline void build_mtile_list(const int32_t* offsets, int E, int A, int max_tiles, MTile* __restrict__ tiles,
-                                        int32_t* __restrict__ n_tiles_out, const FastExpert* __restrict__ gate_fe,
+__device__ inline void build_mtile_list(const int32_t* offsets, int E, int A, int tile_rows, int max_tiles,
+                                        MTile* __restrict__ tiles, int32_t* __restrict__ n_tiles_out, const FastExpert* __restrict__ gate_fe,
                                         const FastExpert* __restrict__ up_fe, MTileLds& lds) {
     const int tid = threadIdx.x, nthreads = blockDim.x;
     if (tid < MT_KEYS) lds.hist[tid] = 0;
@@ -51,14 +51,14 @@ __device__ inline void build_mtile_list(const int32_t* offsets, int E, int A, in
         if (*cnt == 0) return;
         const int wg = gate_fe ? gate_fe[e].uniform_bits : 2, wu = up_fe ? up_fe[e].uniform_bits : 2;
         const int wsum = (wg == 0 || wu == 0) ? 8 : wg + wu;
-        *k_full = mtile_key(PF_M, wsum);
-        *k_last = mtile_key(*cnt - (*cnt - 1) / PF_M * PF_M, wsum);
+        *k_full = mtile_key(tile_rows, wsum);
+        *k_last = mtile_key(*cnt - (*cnt - 1) / tile_rows * tile_rows, wsum);
     };
     // pass 1: tiles per cost class
     for (int e0 = 0; e0 < E; e0 += nthreads) {
         int begin, cnt, k_full, k_last;
         expert_tiles(e0 + tid, &begin, &cnt, &k_full, &k_last);
-        const int nt = (cnt + PF_M - 1) / PF_M;
+        const int nt = (cnt + tile_rows - 1) / tile_rows;
         if (nt > 1) atomicAdd(&lds.hist[k_full], nt - 1);
         if (nt > 0) atomicAdd(&lds.hist[k_last], 1);
     }
@@ -77,15 +77,15 @@ __device__ inline void build_mtile_list(const int32_t* offsets, int E, int A, in
         const int e = e0 + tid;
         int begin, cnt, k_full, k_last;
         expert_tiles(e, &begin, &cnt, &k_full, &k_last);
-        const int nt = (cnt + PF_M - 1) / PF_M;
+        const int nt = (cnt + tile_rows - 1) / tile_rows;
         if (nt > 1) {
             const int at = atomicAdd(&lds.cursor[k_full], nt - 1);
             for (int j = 0; j < nt - 1; ++j)
-                if (at + j < max_tiles) tiles[at + j] = MTile{e, begin + j * PF_M, PF_M, 0};
+                if (at + j < max_tiles) tiles[at + j] = MTile{e, begin + j * tile_rows, tile_rows, 0};
         }
         if (nt > 0) {
             const int at = atomicAdd(&lds.cursor[k_last], 1);
-            if (at < max_tiles) tiles[at] = MTile{e, begin + (nt - 1) * PF_M, cnt - (nt - 1) * PF_M, 0};
+            if (at < max_tiles) tiles[at] = MTile{e, begin + (nt - 1) * tile_rows, cnt - (nt - 1) * tile_rows, 0};
         }
     }
     __syncthreads();

@@ -303,7 +303,7 @@ __global__ __launch_bounds__(1024) void k_route_scan(int32_t* __restrict__ chunk
     }
     if (jobs.mtiles != nullptr) {
         __syncthreads();
-        build_mtile_list(totals, n_packed, n_flat, jobs.max_mtiles, jobs.mtiles, jobs.n_mtiles, jobs.gate_fe, jobs.up_fe,
+        build_mtile_list(totals, n_packed, n_flat, jobs.mtile_rows, jobs.max_mtiles, jobs.mtiles, jobs.n_mtiles, jobs.gate_fe, jobs.up_fe,
                          mt_lds);
     }
 }

@@ -288,3 +288,36 @@ def test_sweep_across_launcher_thresholds(cuda_device, n_experts, inter):
                                           block._packed_local_to_global, gate, up, down, rank_out, isz, 0)
         err = float(np.abs(one_call.cpu().numpy() - ref).max()) / scale
         assert err <= 1e-2, f"{case}: from the router's output, normalised error {err:.3e}"
+
+
+@pytest.mark.parametrize("counts", [
+    (63, 64, 65, 1, 0, 31, 32, 33),              # 36 per expert: tiles of at most 64, edges of their bodies and one of two tiles
+    (129, 2, 128, 0, 1, 64, 17, 40),             # 47.6: three low tiles in one expert
+    (48, 48, 48, 48, 48, 48, 48, 48),            # the last that takes the low tiles
+    (48, 48, 48, 48, 48, 48, 48, 49),            # the first that takes 128 rows
+])
+@pytest.mark.parametrize("layout", ["uniform", "checkpoint"])
+def test_grouped_gemm_low_and_high_tiles(cuda_device, counts, layout):
+    """The grouped GEMM on both sides of where it changes its tile height, against the C oracle: assignments dealt so that
+    expert e gets counts[e]."""
+    import torch
+
+    from bitsmoe_amd.synth import LayerSpec, make_layer
+
+    spec = LayerSpec("tiles", "qwen3moe", len(counts), 1, 512, 288, (0.6, 0.25, 0.15), "normal", True, 0)
+    block = make_layer(spec, device=cuda_device, dtype=torch.bfloat16, seed=11, layout=layout)
+    block._ensure_runtime_cache(cuda_device)
+    order = torch.randperm(sum(counts), generator=torch.Generator().manual_seed(1))
+    picks = torch.repeat_interleave(torch.arange(len(counts)), torch.tensor(counts))[order]
+    h_gate, h_up, selected, weights = _inputs(block, spec, sum(counts), 12, cuda_device)
+    selected = picks[:, None].to(device=selected.device, dtype=selected.dtype)
+    tok, off, rw, out = _run(block, h_gate, h_up, selected, weights)
+    assert tuple((off[1:] - off[:-1]).tolist()) == counts
+    ref = _oracle(block, h_gate, h_up, *(t.cpu().numpy() for t in (tok, off, rw)))
+    scale = float(np.abs(ref).max())
+    assert float(np.abs(out.cpu().numpy() - ref).max()) <= 1e-2 * scale
+    from bitsmoe_amd.algorithms import mlp_forward_cuda as hip
+    gate, up, down = block._ensure_matsets()
+    one = hip.moe_forward_routed(h_gate, h_up, selected, weights, block._packed_global_to_local, block._packed_local_to_global,
+                                 gate, up, down, int(block.shared_u_down.shape[1]), int(block._packed_intermediate_size), 0)
+    assert float(np.abs(one.cpu().numpy() - ref).max()) <= 1e-2 * scale
