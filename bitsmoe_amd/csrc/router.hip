@@ -29,8 +29,34 @@ __device__ inline float wave_sum(float v) {
     return v;
 }
 
-// grid = ceil(T / 4), 256 threads (four tokens per workgroup)
-template <int DT>
+// The value N lanes away inside a row of sixteen, and reductions of a wavefront to a uniform value by it: a row's in four
+// rotations, the four rows' through scalar registers (the LDS crossbar's permutes: six dependent round trips).
+template <int N>
+__device__ __forceinline__ int row_ror(int v) {
+    return __builtin_amdgcn_update_dpp(0, v, 0x120 + N, 0xF, 0xF, false);
+}
+template <class F>
+__device__ __forceinline__ int wave_fold(int v, F&& f) {
+    v = f(v, row_ror<8>(v));
+    v = f(v, row_ror<4>(v));
+    v = f(v, row_ror<2>(v));
+    v = f(v, row_ror<1>(v));
+    return f(f(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)),
+             f(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
+}
+__device__ __forceinline__ float wave_max(float v) {
+    return __int_as_float(wave_fold(__float_as_int(v), [](int a, int b) { return __float_as_int(fmaxf(__int_as_float(a), __int_as_float(b))); }));
+}
+__device__ __forceinline__ int wave_min(int v) {
+    return wave_fold(v, [](int a, int b) { return min(a, b); });
+}
+
+// grid = ceil(T / 4), 256 threads (four tokens per workgroup); PER: logits a lane holds, E <= 64 * PER.
+// Bound by the chain of the k arg-max rounds: a round is PER compares, two reductions by row rotations, PER compares to take
+// the pick out; exponentials and divisions come once, behind the rounds.  (With permutes, both parts of the pair in every
+// step, sixteen logits per lane whatever E, and an exponential and a division per round: 512 experts, top-10, 256 tokens
+// 12.6 -> 5.6 us; 4096 tokens 16.7 -> 10.2.)
+template <int DT, int PER>
 __global__ __launch_bounds__(256) void k_router_softmax_topk(const void* __restrict__ logits, int64_t ld, float wscale,
                                                              int T, int E, int k,
                                                              int renorm, int round_dt, int32_t* __restrict__ sel32,
@@ -38,58 +64,47 @@ __global__ __launch_bounds__(256) void k_router_softmax_topk(const void* __restr
     const int lane = threadIdx.x & 63;
     const int tkn = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (tkn >= T) return;
-    const int per = (E + 63) >> 6;
-    float v[ROUTER_MAX_PER_LANE];
+    float v[PER];
     float vmax = -INFINITY;
 #pragma unroll
-    for (int i = 0; i < ROUTER_MAX_PER_LANE; ++i) {
+    for (int i = 0; i < PER; ++i) {
         const int e = lane + 64 * i;
-        v[i] = (i < per && e < E) ? load_logit<DT>(logits, (int64_t)tkn * ld + e) : -INFINITY;
+        v[i] = e < E ? load_logit<DT>(logits, (int64_t)tkn * ld + e) : -INFINITY;
         vmax = fmaxf(vmax, v[i]);
     }
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) vmax = fmaxf(vmax, __shfl_xor(vmax, d));
+    vmax = wave_max(vmax);
     float part = 0.0f;
 #pragma unroll
-    for (int i = 0; i < ROUTER_MAX_PER_LANE; ++i)
-        if (i < per) part += (v[i] == -INFINITY) ? 0.0f : expf(v[i] - vmax);
+    for (int i = 0; i < PER; ++i) part += (v[i] == -INFINITY) ? 0.0f : expf(v[i] - vmax);
     const float denom = wave_sum(part);
 
     // k rounds of arg-max over what is left; ties go to the lower expert index
-    float my_w = 0.0f;      // lane j < k keeps the j-th pick
+    float my_v = -INFINITY;      // lane j < k keeps the j-th pick
     int my_e = 0;
-    float picked_sum = 0.0f;
     for (int j = 0; j < k; ++j) {
         float best = -INFINITY;
         int best_e = 0x7fffffff;
 #pragma unroll
-        for (int i = 0; i < ROUTER_MAX_PER_LANE; ++i) {
-            const int e = lane + 64 * i;
-            if (i < per && (v[i] > best)) {      // ascending e inside a lane: strict > keeps the lower index
+        for (int i = 0; i < PER; ++i) {
+            if (v[i] > best) {      // ascending e inside a lane: strict > keeps the lower index (and a NaN is never picked)
                 best = v[i];
-                best_e = e;
+                best_e = lane + 64 * i;
             }
         }
-#pragma unroll
-        for (int d = 32; d >= 1; d >>= 1) {
-            const float ob = __shfl_xor(best, d);
-            const int oe = __shfl_xor(best_e, d);
-            if (ob > best || (ob == best && oe < best_e)) {
-                best = ob;
-                best_e = oe;
-            }
-        }
+        const float top = wave_max(best);
+        const int top_e = wave_min(best == top ? best_e : 0x7fffffff);
         // remove the pick from its owner
 #pragma unroll
-        for (int i = 0; i < ROUTER_MAX_PER_LANE; ++i)
-            if (lane + 64 * i == best_e) v[i] = -INFINITY;
-        const float p = (best == -INFINITY) ? 0.0f : expf(best - vmax) / denom;
-        picked_sum += p;
+        for (int i = 0; i < PER; ++i)
+            if (lane + 64 * i == top_e) v[i] = -INFINITY;
         if (lane == j) {
-            my_w = p;
-            my_e = best_e < E ? best_e : 0;
+            my_v = top;
+            my_e = top_e < E ? top_e : 0;
         }
     }
+    const float my_w = my_v == -INFINITY ? 0.0f : expf(my_v - vmax) / denom;
+    float picked_sum = 0.0f;
+    for (int j = 0; j < k; ++j) picked_sum += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(my_w), j));
     if (lane < k) {
         float w = (renorm ? my_w / picked_sum : my_w) * wscale;
         if (round_dt == BITSMOE_DT_F16)
@@ -367,13 +382,16 @@ extern "C" int bitsmoe_router_softmax_topk_strided(const void* logits, int32_t l
 #define BITSMOE_ROUTER_LAUNCH(KERNEL)                                                                              \
     hipLaunchKernelGGL(KERNEL, grid, dim3(256), 0, st, logits, ld_logits, weight_scale, (int)n_tokens, n_experts, top_k, \
                        renormalize, round_dtype, s32, s64, weights)
-    if (logits_dtype == 0) {
-        if (by_rank) BITSMOE_ROUTER_LAUNCH(k_router_rank_topk<0>); else BITSMOE_ROUTER_LAUNCH(k_router_softmax_topk<0>);
-    } else if (logits_dtype == 1) {
-        if (by_rank) BITSMOE_ROUTER_LAUNCH(k_router_rank_topk<1>); else BITSMOE_ROUTER_LAUNCH(k_router_softmax_topk<1>);
-    } else {
-        if (by_rank) BITSMOE_ROUTER_LAUNCH(k_router_rank_topk<2>); else BITSMOE_ROUTER_LAUNCH(k_router_softmax_topk<2>);
-    }
+#define BITSMOE_ROUTER_FORM(DT)                                                                                    \
+    do {                                                                                                           \
+        if (by_rank) BITSMOE_ROUTER_LAUNCH((k_router_rank_topk<DT>));                                              \
+        else if (n_experts <= 512) BITSMOE_ROUTER_LAUNCH((k_router_softmax_topk<DT, 8>));                          \
+        else BITSMOE_ROUTER_LAUNCH((k_router_softmax_topk<DT, ROUTER_MAX_PER_LANE>));                              \
+    } while (0)
+    if (logits_dtype == 0) BITSMOE_ROUTER_FORM(0);
+    else if (logits_dtype == 1) BITSMOE_ROUTER_FORM(1);
+    else BITSMOE_ROUTER_FORM(2);
+#undef BITSMOE_ROUTER_FORM
 #undef BITSMOE_ROUTER_LAUNCH
     BITSMOE_HIP_TRY(hipGetLastError());
     return BITSMOE_OK;

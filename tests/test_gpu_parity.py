@@ -751,3 +751,27 @@ def test_skinny_linear_infinite_activation(cuda_device, rows, k, x_dtype):
             assert bool(torch.isinf(y[rows // 2]).all())
             others = [r for r in range(rows) if r != rows // 2]
             assert bool((y[others] == torch.tensor(float(k), dtype=torch.bfloat16).item()).all())
+
+
+@pytest.mark.parametrize("n_experts,top_k", [(257, 1), (512, 64), (513, 10), (1024, 64)])
+def test_router_rounds_with_ties_and_masked_logits(cuda_device, n_experts, top_k):
+    """More than 256 experts (arg-max rounds; eight or sixteen logits per lane): equal logits go to the lower index, across
+    lanes and inside one, -0 equals 0, masked experts (-inf) are picked never: positions they leave are expert 0, weight 0."""
+    import torch
+
+    hip = _hip()
+    rng = np.random.default_rng(n_experts + top_k)
+    logits = rng.integers(-3, 4, size=(9, n_experts)).astype(np.float32)      # about n / 7 of a kind
+    logits[1][logits[1] == 0] = -0.0
+    logits[2] = np.where(rng.uniform(size=n_experts) < 0.98, -np.inf, logits[2])
+    logits[2, n_experts - 1] = 7.0
+    logits[3] = 0.0
+    sel, w = hip.router_softmax_topk(torch.from_numpy(logits).to(cuda_device), top_k, True)
+    sel, w = sel.cpu().numpy(), w.cpu().numpy()
+    for t in range(logits.shape[0]):
+        v = logits[t].astype(np.float64)
+        order = [e for e in np.lexsort((np.arange(n_experts), -v)) if v[e] > -np.inf][:top_k]
+        p = np.exp(v[order] - v.max())
+        assert list(sel[t][:len(order)]) == order and not sel[t][len(order):].any()
+        # (each weight: one exponential, one division, a sum of at most 64 terms in fp32)
+        assert np.allclose(w[t][:len(order)], p / p.sum(), rtol=1e-5, atol=0) and not w[t][len(order):].any()
