@@ -43,7 +43,7 @@ __device__ __forceinline__ void static_for_pieces(F&& f, std::integer_sequence<i
 // [k-step of 32][lane][8 values], so that a wavefront's load is 1 KB of consecutive memory instead of sixteen 64-byte
 // pieces of sixteen rows.
 // TURN: x by way of LDS; else (a few rows: nothing to gain from whole lines) every step's operand straight from x.
-template <bool BF16, int NMB, int NW, int MAXS, bool XF32, bool PREP, bool TURN>
+template <bool BF16, int NMB, int NW, int MAXS, bool XF32, bool PREP, bool TURN, bool WHOLE>
 __global__ __launch_bounds__(64 * NW) void k_skinny_linear(const void* __restrict__ x, int64_t ld_x, const uint16_t* __restrict__ w,
                                                            int T, int K, int N, uint16_t* __restrict__ out, int64_t ld_out,
                                                            const float* __restrict__ addend, int64_t ld_add) {
@@ -57,10 +57,12 @@ __global__ __launch_bounds__(64 * NW) void k_skinny_linear(const void* __restric
     constexpr int PIECE = TURN ? 16 * NMB * CPR * 16 : 0;      // bytes
     constexpr int PART = NW * NMB * 16 * 17 * 4;
     __shared__ __attribute__((aligned(16))) unsigned char lds[NW * PIECE > PART ? NW * PIECE : PART];
+    __shared__ __attribute__((aligned(16))) unsigned char zero_piece[16];
     const int lane = threadIdx.x & 63;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n = lane & 15, kg = lane >> 4;
     const int n0 = blockIdx.x * 16;
+    if (TURN && lane == 0) *reinterpret_cast<sk_u32x4*>(zero_piece) = sk_u32x4{0u, 0u, 0u, 0u};      // (by every wavefront: no barrier)
     const int steps = K >> 5;
     const int first = wv * steps / NW, end = (wv + 1) * steps / NW;
     // chunk c of row r sits at chunk position c ^ swz(r) of its row: the sixteen rows of an operand read hit different banks
@@ -93,21 +95,21 @@ __global__ __launch_bounds__(64 * NW) void k_skinny_linear(const void* __restric
                         round16(hi[0]) | (round16(hi[1]) << 16), round16(hi[2]) | (round16(hi[3]) << 16)};
     };
     for (int s0 = first; s0 < end; s0 += MAXS) {
-        // (no branches: steps past the end repeat the last one and count as zeros -- both operands, or an infinite x would
-        // make a NaN of its row)
+        // (no branches between the steps: those past the end repeat the last one and count as zeros -- both operands, or an
+        // infinite x would make a NaN of its row; from LDS, x comes from a zero piece there: one select per operand, not four.
+        // WHOLE: every share is whole passes of MAXS steps, no selects: with four per operand and step they were 0.3 to 1 us of a
+        // launch.  A choice between the two bodies inside the kernel cost 1 to 3 us at 64 rows, in registers.)
         const int ns = end - s0;
         sk_u32x4 b[MAXS];
         auto request_w = [&](int u) {
             b[u] = *reinterpret_cast<const sk_u32x4*>(wp + (int64_t)(s0 + min(u, ns - 1)) * (PREP ? 512 : 32));
         };
-        auto step = [&](int u, sk_f32x4& c, sk_u32x4 av, sk_u32x4 bv) {
-            const bool live = u < ns;
+        auto live_or_zero = [&](int u, sk_u32x4 v) {
+            if constexpr (!WHOLE) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                av[i] = live ? av[i] : 0u;
-                bv[i] = live ? bv[i] : 0u;
+                for (int i = 0; i < 4; ++i) v[i] = u < ns ? v[i] : 0u;
             }
-            multiply(c, av, bv);
+            return v;
         };
         if constexpr (!TURN) {
             sk_u32x4 xr[MAXS][XF32 ? 2 : 1];
@@ -122,10 +124,9 @@ __global__ __launch_bounds__(64 * NW) void k_skinny_linear(const void* __restric
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int u = 0; u < MAXS; ++u) {
-                if constexpr (XF32)
-                    step(u, acc[0], rounded(__builtin_bit_cast(sk_f32x4, xr[u][0]), __builtin_bit_cast(sk_f32x4, xr[u][1])), b[u]);
-                else
-                    step(u, acc[0], xr[u][0], b[u]);
+                sk_u32x4 av = xr[u][0];
+                if constexpr (XF32) av = rounded(__builtin_bit_cast(sk_f32x4, xr[u][0]), __builtin_bit_cast(sk_f32x4, xr[u][1]));
+                multiply(acc[0], live_or_zero(u, av), live_or_zero(u, b[u]));
             }
             continue;
         }
@@ -149,19 +150,23 @@ __global__ __launch_bounds__(64 * NW) void k_skinny_linear(const void* __restric
             for (int i = 0; i < NI; ++i) *reinterpret_cast<sk_u32x4*>(piece + (i * 64 + lane) * 16) = xr[P & 1][i];
             if constexpr ((P + 2) * G < MAXS) request_x(std::integral_constant<int, P + 2>{});
             __builtin_amdgcn_sched_barrier(0);
-            const int shift = s0 + P * G - min(s0 + P * G, steps - G);
+            const int shift = WHOLE ? 0 : s0 + P * G - min(s0 + P * G, steps - G);
 #pragma unroll
             for (int g = 0; g < G; ++g) {
+                const sk_u32x4 bv = live_or_zero(P * G + g, b[P * G + g]);
                 const int gs = min(g + shift, G - 1);
+                auto chunk = [&](int r, int c) -> const unsigned char* {
+                    const unsigned char* at = piece + r * (CPR * 16) + ((c ^ swz(r)) << 4);
+                    return WHOLE || P * G + g < ns ? at : zero_piece;
+                };
 #pragma unroll
                 for (int mb = 0; mb < NMB; ++mb) {
                     const int r = 16 * mb + n;
-                    const unsigned char* row = piece + r * (CPR * 16);
                     if constexpr (XF32)
-                        step(P * G + g, acc[mb], rounded(*reinterpret_cast<const sk_f32x4*>(row + (((gs * 8 + 2 * kg) ^ swz(r)) << 4)),
-                                                      *reinterpret_cast<const sk_f32x4*>(row + (((gs * 8 + 2 * kg + 1) ^ swz(r)) << 4))), b[P * G + g]);
+                        multiply(acc[mb], rounded(*reinterpret_cast<const sk_f32x4*>(chunk(r, gs * 8 + 2 * kg)),
+                                                  *reinterpret_cast<const sk_f32x4*>(chunk(r, gs * 8 + 2 * kg + 1))), bv);
                     else
-                        step(P * G + g, acc[mb], *reinterpret_cast<const sk_u32x4*>(row + (((gs * 4 + kg) ^ swz(r)) << 4)), b[P * G + g]);
+                        multiply(acc[mb], *reinterpret_cast<const sk_u32x4*>(chunk(r, gs * 4 + kg)), bv);
                 }
             }
         }, std::make_integer_sequence<int, MAXS / G>{});
@@ -253,10 +258,17 @@ extern "C" int bitsmoe_skinny_linear(const void* x, int32_t dtype, int32_t x_is_
     const int nw = steps > 80 ? 8 : 4;
     const int share = (steps + nw - 1) / nw;
     auto run = [&](auto bf_c, auto nmb_c, auto nw_c, auto s_c, auto xf_c, auto pr_c, auto turn_c) {
-        hipLaunchKernelGGL((k_skinny_linear<decltype(bf_c)::value, decltype(nmb_c)::value, decltype(nw_c)::value, decltype(s_c)::value,
-                                            decltype(xf_c)::value, decltype(pr_c)::value, decltype(turn_c)::value>),
-                           grid, dim3(64 * decltype(nw_c)::value), 0, st, x, ld_x, (const uint16_t*)weight, (int)n_rows, in_features,
-                           out_features, (uint16_t*)out, ld_out, addend, ld_addend);
+        auto launch = [&](auto whole_c) {
+            hipLaunchKernelGGL((k_skinny_linear<decltype(bf_c)::value, decltype(nmb_c)::value, decltype(nw_c)::value, decltype(s_c)::value,
+                                                decltype(xf_c)::value, decltype(pr_c)::value, decltype(turn_c)::value, decltype(whole_c)::value>),
+                               grid, dim3(64 * decltype(nw_c)::value), 0, st, x, ld_x, (const uint16_t*)weight, (int)n_rows, in_features,
+                               out_features, (uint16_t*)out, ld_out, addend, ld_addend);
+        };
+        // (hidden sizes 1024, 1536, 2048 and 2560 are four whole shares of prepared weights)
+        if constexpr (decltype(pr_c)::value && decltype(nw_c)::value == 4) {
+            if (steps % (4 * decltype(s_c)::value) == 0) return launch(std::true_type{});
+        }
+        launch(std::false_type{});
     };
     using std::integral_constant;
     using Yes = std::true_type;
@@ -264,6 +276,7 @@ extern "C" int bitsmoe_skinny_linear(const void* x, int32_t dtype, int32_t x_is_
     using W4 = integral_constant<int, 4>;
     using W8 = integral_constant<int, 8>;
     using S8 = integral_constant<int, 8>;
+    using S12 = integral_constant<int, 12>;
     using S16 = integral_constant<int, 16>;
     using S20 = integral_constant<int, 20>;
     auto by_share = [&](auto bf_c, auto nmb_c, auto xf_c, auto turn_c) {
@@ -275,6 +288,8 @@ extern "C" int bitsmoe_skinny_linear(const void* x, int32_t dtype, int32_t x_is_
             else if constexpr (twenty) run(bf_c, nmb_c, W8{}, S20{}, xf_c, Yes{}, turn_c);
         } else if (share <= 8) {
             run(bf_c, nmb_c, W4{}, S8{}, xf_c, Yes{}, turn_c);
+        } else if (share <= 12) {      // (1536 -> 4224 features at one row 6.0 us as sixteen steps, 5.6 as twelve)
+            run(bf_c, nmb_c, W4{}, S12{}, xf_c, Yes{}, turn_c);
         } else {
             if (share <= 16 || !twenty) run(bf_c, nmb_c, W4{}, S16{}, xf_c, Yes{}, turn_c);
             else if constexpr (twenty) run(bf_c, nmb_c, W4{}, S20{}, xf_c, Yes{}, turn_c);

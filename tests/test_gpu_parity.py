@@ -728,22 +728,23 @@ def test_skinny_linear_matches_float64(cuda_device, rows, k, n, dtype_name):
     (4, 2560, 48), (5, 2560, 48),      # x straight into the operands / by way of LDS; shares of twenty steps
     (17, 896, 34), (64, 128, 16),      # shares that are no whole pieces of x, one step per wavefront
     (49, 5248, 48), (3, 11008, 18),    # eight wavefronts, several passes over a share
+    (1, 1536, 34), (50, 1536, 32), (4, 1280, 48), (33, 1280, 16),      # shares of twelve steps, whole and not
 ])
 @pytest.mark.parametrize("dtype_name", ["bf16", "f16"])
 def test_skinny_linear_edges(cuda_device, rows, k, n, dtype_name):
     test_skinny_linear_matches_float64(cuda_device, rows, k, n, dtype_name)
 
 
-@pytest.mark.parametrize("rows,k,x_dtype", [(1, 896, "bf16"), (16, 896, "bf16"), (40, 1536, "bf16"), (2, 896, "f32"), (9, 896, "f32")])
+@pytest.mark.parametrize("rows,k,x_dtype", [(1, 896, "bf16"), (16, 896, "bf16"), (40, 1280, "bf16"), (64, 4864, "bf16"), (2, 896, "f32"), (9, 896, "f32")])
 def test_skinny_linear_infinite_activation(cuda_device, rows, k, x_dtype):
-    """An infinite activation gives an infinite output, not a NaN: shares of 7 and 12 steps, fewer than are requested."""
+    """An infinite activation gives an infinite output, not a NaN: shares of 7, 10 and 19 steps, fewer than are requested."""
     import torch
 
     from bitsmoe_amd.algorithms import mlp_forward_cuda as hip
 
     x = torch.ones((rows, k), device=cuda_device, dtype=torch.bfloat16 if x_dtype == "bf16" else torch.float32)
     w = torch.ones((32, k), device=cuda_device, dtype=torch.bfloat16)
-    for at in (k // 4 - 1, k - 1):      # the step that the first and the last wavefront end with
+    for at in (k // 4 - 1, k // 8 - 1, k - 1):      # steps that the first and the last wavefront end with
         xi = x.clone()
         xi[rows // 2, at] = float("inf")
         for weight in (w, hip.PreparedLinearWeight(w)):
