@@ -534,6 +534,8 @@ class BitsMoE_BaseSparseMoeBlock(nn.Module):
         if cached is not None and cached["stamp"] == stamp:
             return cached
         hidden = int(vh_gate.shape[1])
+        if int(u_down.shape[0]) != hidden:
+            return None
         if router is not None and tuple(router.weight.shape) != (int(self._packed_global_to_local.numel()), hidden):
             return None
         if shared is not None:
@@ -651,6 +653,9 @@ class BitsMoE_BaseSparseMoeBlock(nn.Module):
             return None
         x = hidden_states
         rows, hidden = x.shape
+        # (the library gets a pointer and a row stride: the width is known here only)
+        if hidden != plan["w_in"].shape[1]:
+            raise RuntimeError(f"hidden states of width {hidden}, but this block's input projections take {plan['w_in'].shape[1]}")
         if x.stride(1) != 1 or (rows > 1 and x.stride(0) % 8 != 0) or x.data_ptr() % 16 != 0:
             x = x.clone(memory_format=torch.contiguous_format)
         form = (mlp_forward_cuda.ROUTER_LOGITS if router is not None else

@@ -378,3 +378,28 @@ def test_block_plan_made_twice_at_once(cuda_device, monkeypatch):
     wide = torch.nn.Linear(block.spec.hidden_size, block.spec.num_experts + 8, bias=False).to(cuda_device)
     bases = tuple(getattr(block, k) for k in block._SHARED_BASIS_BUFFER_KEYS)
     assert block._fused_plan(torch.bfloat16, bases, wide, None, None) is None
+
+
+_FAMILIES = [("qwen3moe", {}), ("qwen3next", {"shared_intermediate": 128}), ("deepseekv2", {})]
+
+
+@pytest.mark.parametrize("tokens", [1, 16, 40, 100])      # the few-rows kernel for both projections, and the framework's GEMMs
+@pytest.mark.parametrize("family,kw", _FAMILIES)
+def test_block_refuses_hidden_states_of_another_width(cuda_device, family, kw, tokens):
+    """The library takes a pointer and a row stride: wider hidden states, and columns cut from rows that are wide enough, are
+    refused where the width is known.  And a down basis that does not lead back to the hidden size is not stacked."""
+    import torch
+
+    from bitsmoe_amd.synth import make_layer
+
+    block = make_layer(_small_spec(family, hidden_size=256, **kw), device=cuda_device, dtype=torch.bfloat16, seed=41)
+    block.prepare_runtime_fastpath(warmup=True)
+    hidden = block.spec.hidden_size
+    x = torch.zeros((1, tokens, hidden + 128), dtype=torch.bfloat16, device=cuda_device)
+    with torch.no_grad():
+        block(x[..., :hidden])
+        for bad in (x, x[..., :hidden - 128]):
+            with pytest.raises(RuntimeError):
+                block(bad)
+    vh_gate, vh_up, u_down = (getattr(block, k) for k in block._SHARED_BASIS_BUFFER_KEYS)
+    assert block._fused_plan(torch.bfloat16, (vh_gate, vh_up, u_down[:-16]), None, None, None) is None
