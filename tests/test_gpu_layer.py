@@ -403,3 +403,24 @@ def test_block_refuses_hidden_states_of_another_width(cuda_device, family, kw, t
                 block(bad)
     vh_gate, vh_up, u_down = (getattr(block, k) for k in block._SHARED_BASIS_BUFFER_KEYS)
     assert block._fused_plan(torch.bfloat16, (vh_gate, vh_up, u_down[:-16]), None, None, None) is None
+
+
+@pytest.mark.parametrize("tokens", [8, 32, 100])
+@pytest.mark.parametrize("family,kw", _FAMILIES)
+@pytest.mark.parametrize("super_experts", [(), (1, 6)])
+def test_block_takes_overlapping_rows(cuda_device, family, kw, tokens, super_experts):
+    """Hidden states whose rows overlap in memory (one row expanded, windows of a signal) give what their copy gives."""
+    import torch
+
+    from bitsmoe_amd.synth import make_layer
+
+    block = make_layer(_small_spec(family, **kw), device=cuda_device, dtype=torch.bfloat16, seed=43, super_experts=super_experts)
+    block.prepare_runtime_fastpath(warmup=True)
+    hidden = block.spec.hidden_size
+    signal = torch.randn(64 * tokens + hidden, generator=torch.Generator().manual_seed(tokens)).to(torch.bfloat16).to(cuda_device)
+    first = lambda out: (out[0] if isinstance(out, tuple) else out).float()
+    with torch.no_grad():
+        for x in (signal[:hidden].expand(1, tokens, hidden), signal.unfold(0, hidden, 64)[None, :tokens]):
+            got, ref = first(block(x)), first(block(x.contiguous()))
+            # (fp32 atomics in another order, then one bf16 rounding)
+            assert float((got - ref).abs().max()) <= 1e-2 * float(ref.abs().max())
