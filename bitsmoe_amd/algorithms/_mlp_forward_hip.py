@@ -619,7 +619,7 @@ def router_linear_topk_possible(hidden: torch.Tensor, weight, top_k: int) -> boo
         w_dtype, e, k = weight.dtype, int(weight.shape[0]), int(weight.shape[1])
     return (hidden.is_cuda and hidden.dim() == 2 and hidden.dtype in (torch.float16, torch.bfloat16) and w_dtype == hidden.dtype
             and hidden.stride(1) == 1 and int(hidden.shape[1]) == k and k % 128 == 0
-            and (int(hidden.shape[0]) <= 1 or int(hidden.stride(0)) % 8 == 0) and hidden.data_ptr() % 16 == 0
+            and (int(hidden.shape[0]) <= 1 or (int(hidden.stride(0)) % 8 == 0 and int(hidden.stride(0)) >= k)) and hidden.data_ptr() % 16 == 0
             and 1 <= int(top_k) <= min(64, e) and e <= 256)
 
 
@@ -700,6 +700,8 @@ def skinny_linear_possible(x: torch.Tensor, weight) -> bool:
     if not (x.is_cuda and x.dim() == 2 and x.stride(1) == 1 and int(x.shape[1]) == k and k % 128 == 0 and x.data_ptr() % 16 == 0):
         return False
     rows = int(x.shape[0])
+    if rows > 1 and int(x.stride(0)) < k:      # (rows that overlap)
+        return False
     if x.dtype == torch.float32:
         return 1 <= rows <= 16 and (rows <= 1 or int(x.stride(0)) % 4 == 0)
     return x.dtype == w_dtype and 1 <= rows <= SKINNY_LINEAR_MAX_ROWS and (rows <= 1 or int(x.stride(0)) % 8 == 0)

@@ -415,6 +415,7 @@ def test_block_takes_overlapping_rows(cuda_device, family, kw, tokens, super_exp
     from bitsmoe_amd.synth import make_layer
 
     block = make_layer(_small_spec(family, **kw), device=cuda_device, dtype=torch.bfloat16, seed=43, super_experts=super_experts)
+    block.train(tokens == 8)      # (a DeepSeek gate in training mode is called as a module)
     block.prepare_runtime_fastpath(warmup=True)
     hidden = block.spec.hidden_size
     signal = torch.randn(64 * tokens + hidden, generator=torch.Generator().manual_seed(tokens)).to(torch.bfloat16).to(cuda_device)
