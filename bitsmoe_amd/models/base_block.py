@@ -58,6 +58,7 @@ def _super_via_operator() -> bool:
 # 9.0 vs 13.6, 2048 -> 4224 12.4 vs 12.2; but 2048 -> 9728 18.7 vs 17.1, and 4864 -> 2048 14.6 vs 12.9 at 56.
 # BITSMOE_BLOCK_SKINNY_ROWS caps the rows, 0 switches the kernel off.
 _SKINNY_ROWS = int(_os.environ.get("BITSMOE_BLOCK_SKINNY_ROWS", "64"))
+_SKINNY_MOST_ROWS = 64            # that the kernel takes at all
 _SKINNY_ANY_SHAPE_ROWS = 48
 _SKINNY_NARROW_FEATURES = 4352    # output features, and
 _SKINNY_SHORT_CONTRACTION = 4096  # input features up to which 49 to 64 rows take it
@@ -70,7 +71,7 @@ _FEW_ROWS_LOCK = _threading.Lock()      # (held while a layer's copy is made, on
 
 def _few_rows(rows: int, n_in: int, n_out: int) -> bool:
     """Does the few-rows kernel run this GEMM?  (It takes contractions of whole 128 and an even number of outputs.)"""
-    return (0 < rows <= _SKINNY_ROWS and n_in % 128 == 0 and n_out % 2 == 0 and (
+    return (0 < rows <= min(_SKINNY_ROWS, _SKINNY_MOST_ROWS) and n_in % 128 == 0 and n_out % 2 == 0 and (
         rows <= _SKINNY_ANY_SHAPE_ROWS or (n_in <= _SKINNY_SHORT_CONTRACTION and n_out <= _SKINNY_NARROW_FEATURES)))
 
 

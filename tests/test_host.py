@@ -236,3 +236,13 @@ def test_set_option_names():
         hip.set_option(name, -1)
     with pytest.raises(RuntimeError, match="unknown option"):
         hip.set_option("no_such_switch", 1)
+
+
+def test_few_rows_rule_stays_inside_the_kernel(monkeypatch):
+    """However many rows the environment variable asks for, the rule sends no more than the kernel takes."""
+    from bitsmoe_amd.models import base_block
+
+    for rows in (200, 64, 10, 0):
+        monkeypatch.setattr(base_block, "_SKINNY_ROWS", rows)
+        taken = [t for t in range(300) if base_block._few_rows(t, 2048, 2048)]
+        assert taken == list(range(1, min(rows, 64) + 1))
