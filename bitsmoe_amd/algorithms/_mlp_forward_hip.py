@@ -21,6 +21,7 @@ from typing import List, Optional, Sequence, Tuple
 import torch
 
 from . import _capi
+from ._streams import settled
 
 _lib = _capi.load()
 # BITSMOE_NO_PREPARE=1 keeps every matrix set on the generic kernels (no wave-native copy)
@@ -654,10 +655,11 @@ def prepared_linear_weight_of(owner, weight: torch.Tensor) -> "PreparedLinearWei
     cached = getattr(owner, "_bitsmoe_prepared_weight", None)
     if cached is None or cached[0] != stamp:
         cached = (stamp, PreparedLinearWeight(weight.detach()))
-        try:
-            object.__setattr__(owner, "_bitsmoe_prepared_weight", cached)
-        except (AttributeError, TypeError):
-            pass
+        if settled(weight.device):
+            try:
+                object.__setattr__(owner, "_bitsmoe_prepared_weight", cached)
+            except (AttributeError, TypeError):
+                pass
     return cached[1]
 
 
@@ -668,7 +670,7 @@ BLOCK_PROJECT_IN, BLOCK_PROJECT_OUT = _capi.BLOCK_PROJECT_IN, _capi.BLOCK_PROJEC
 
 class PreparedLinearWeight:
     """A weight [N, K] re-laid out once into the order the few-rows kernel's MFMAs take it (every load of a wavefront
-    is then 1 KB of consecutive memory).  A snapshot of the weight's values."""
+    is then 1 KB of consecutive memory).  A snapshot of the weight's values, made on the stream that is current then."""
 
     def __init__(self, weight: torch.Tensor):
         _check(weight.is_cuda and weight.dim() == 2 and weight.dtype in (torch.float16, torch.bfloat16) and weight.is_contiguous()
@@ -802,6 +804,15 @@ class BlockPlan:
 
     def has_weight(self, name: str) -> bool:
         return name in self._weights
+
+    def copy(self) -> "BlockPlan":
+        """The same plan in a structure of its own, whose weights are set apart from this one's."""
+        other = object.__new__(BlockPlan)
+        other.__dict__.update(self.__dict__)
+        other.c = _capi.BlockPlan.from_buffer_copy(self.c)
+        other.address = ctypes.addressof(other.c)
+        other._weights = dict(self._weights)
+        return other
 
     def workspace_bytes(self, n_tokens: int) -> int:
         n = self._bytes.get(n_tokens)

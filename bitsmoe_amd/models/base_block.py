@@ -22,6 +22,7 @@ import torch
 import torch.nn as nn
 
 from bitsmoe_amd.algorithms import _HAS_MLP_FORWARD_CUDA, mlp_forward_cuda
+from bitsmoe_amd.algorithms._streams import settled
 from bitsmoe_amd.models.base_mlp import buffer_generation
 
 _BUFFER_NAMES = ("payload", "rank_idx", "tile_meta", "slab_meta", "scale", "s")
@@ -273,7 +274,8 @@ class BitsMoE_BaseSparseMoeBlock(nn.Module):
         cached = self._basis_cache.get(dtype)
         if cached is None:
             cached = tuple(getattr(self, k).to(dtype).contiguous() for k in self._SHARED_BASIS_BUFFER_KEYS)
-            self._basis_cache[dtype] = cached
+            if settled(cached[0].device):
+                self._basis_cache[dtype] = cached
         return cached
 
     def _shared_basis_stacked(self, dtype: torch.dtype) -> torch.Tensor:
@@ -283,7 +285,8 @@ class BitsMoE_BaseSparseMoeBlock(nn.Module):
         if cached is None:
             vh_gate, vh_up, _ = self._shared_basis(dtype)
             cached = torch.cat([vh_gate, vh_up], dim=0).contiguous()
-            self._basis_cache[key] = cached
+            if settled(cached.device):
+                self._basis_cache[key] = cached
         return cached
 
     def _get_flat_token_ids(self, token_count: int, device: torch.device) -> torch.Tensor:
@@ -413,7 +416,8 @@ class BitsMoE_BaseSparseMoeBlock(nn.Module):
         if cached is None:
             cached = (torch.arange(t, dtype=torch.int32, device=dev), torch.tensor([0, t], dtype=torch.int32, device=dev),
                       torch.ones((t,), dtype=torch.float32, device=dev))
-            self._basis_cache[("always_on", t, str(dev))] = cached
+            if settled(dev):
+                self._basis_cache[("always_on", t, str(dev))] = cached
         tok, off, ones = cached
         rw = ones if token_weights is None else token_weights.reshape(-1).to(torch.float32).contiguous()
         return self._dense_operator_forward(key, [module], hidden_states, tok, off, rw).to(hidden_states.dtype)
@@ -519,7 +523,8 @@ class BitsMoE_BaseSparseMoeBlock(nn.Module):
     def _fused_plan(self, dtype: torch.dtype, bases, router: Optional[nn.Module], shared: Optional[nn.Module],
                     shared_gate: Optional[nn.Module]):
         """The stacked input / output weights (`bases`: the three shared bases) and the column ranges of their parts, or
-        None when a module is not a bias-free linear layer of the expected shape.  Cached; rebuilt when a source tensor was rebound or written."""
+        None when a module is not a bias-free linear layer of the expected shape.  Rebuilt when a source tensor was rebound or
+        written; the forward that asked for a new one keeps it, once it is made."""
         linears = [] if router is None else [router]
         if shared is not None:
             linears += [getattr(shared, n, None) for n in ("gate_proj", "up_proj", "down_proj")]
@@ -578,9 +583,7 @@ class BitsMoE_BaseSparseMoeBlock(nn.Module):
         if shared is not None:
             outs.append(shared.down_proj.weight.detach().to(dtype))
         w_out = torch.cat(outs, dim=1).contiguous()      # [hidden, rank_out + I_sh]
-        cached = {"stamp": stamp, "w_in": w_in, "w_out": w_out, "ranges": ranges, "i_sh": i_sh}
-        self._basis_cache[key] = cached
-        return cached
+        return {"key": key, "kept": False, "stamp": stamp, "w_in": w_in, "w_out": w_out, "ranges": ranges, "i_sh": i_sh}
 
     def _native_plan(self, plan: dict, dtype: torch.dtype, form: int, round_weights: bool, renormalize: bool, weight_scale: float,
                      router_weight) -> "mlp_forward_cuda.BlockPlan":
@@ -616,19 +619,25 @@ class BitsMoE_BaseSparseMoeBlock(nn.Module):
         return native
 
     @staticmethod
-    def _few_rows_weight(plan: dict, native, key: str) -> None:
-        """The weight the few-rows kernel reads: a copy in MFMA operand order, made on first use and kept with the plan.
-        (Two threads may come here at once, each with a native plan of its own or both with one: one of them makes it.)"""
+    def _few_rows_weight(plan: dict, native, key: str) -> "mlp_forward_cuda.BlockPlan":
+        """The native plan with the weight the few-rows kernel reads: a copy in MFMA operand order, made on first use and
+        kept with the plan -- of a kept plan (other threads and streams may hold it) only once it is made, so that under
+        capture it goes into a native plan of that call's own.  Two threads may come here at once, each with a native plan
+        of its own or both with one: one of them makes the copy."""
         if native.has_weight(key):
-            return
+            return native
         with _FEW_ROWS_LOCK:
             if native.has_weight(key):
-                return
+                return native
             weight = plan.get(key + "_prepared")
             if weight is None:
                 weight = mlp_forward_cuda.PreparedLinearWeight(plan[key]) if _SKINNY_PREPARED else plan[key]
-                plan[key + "_prepared"] = weight
+                if plan["kept"] and not settled(weight.device):
+                    native = native.copy()
+                else:
+                    plan[key + "_prepared"] = weight
             native.set_weight(key, weight)
+            return native
 
     def _fused_block_forward(self, hidden_states: torch.Tensor, *, router: Optional[nn.Module] = None, linear_gate=None, route_fn=None,
                              renormalize: bool = True, round_weights: bool = True, weight_scale: float = 1.0,
@@ -666,7 +675,7 @@ class BitsMoE_BaseSparseMoeBlock(nn.Module):
         dev = x.device
         stages = 0
         if _few_rows(rows, hidden, w_in.shape[0]):
-            self._few_rows_weight(plan, native, "w_in")
+            native = self._few_rows_weight(plan, native, "w_in")
             proj = torch.empty((rows, w_in.shape[0]), dtype=dtype, device=dev)
             stages |= mlp_forward_cuda.BLOCK_PROJECT_IN
         else:
@@ -681,7 +690,7 @@ class BitsMoE_BaseSparseMoeBlock(nn.Module):
             selected = torch.empty((rows, self.top_k), dtype=torch.int64, device=dev)
             weights = torch.empty((rows, self.top_k), dtype=torch.float32, device=dev)
         if _few_rows(rows, w_out.shape[1], hidden):
-            self._few_rows_weight(plan, native, "w_out")
+            native = self._few_rows_weight(plan, native, "w_out")
             out = torch.empty((rows, hidden), dtype=dtype, device=dev)
             stages |= mlp_forward_cuda.BLOCK_PROJECT_OUT
         else:
@@ -691,6 +700,9 @@ class BitsMoE_BaseSparseMoeBlock(nn.Module):
         # The super experts' operator call needs the router's output and the hidden states only: it runs on a side
         # stream beside the packed experts' call (its small launches fill what the packed kernels leave idle).
         side = _side_stream(dev).cuda_stream if self._super_expert_items and _SUPER_SIDE_STREAM and not super_modules else 0
+        if not plan["kept"] and settled(dev):      # (one wait for the stacked weights and their copies)
+            plan["kept"] = True
+            self._basis_cache[plan["key"]] = plan
         mlp_forward_cuda.block_forward(native, x, proj, stages, out, selected, weights, sup, side)
         if not stages & mlp_forward_cuda.BLOCK_PROJECT_OUT:
             out = out @ w_out.T

@@ -9,6 +9,8 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from bitsmoe_amd.algorithms._streams import settled
+
 
 class DenseSwiGLUMLP(nn.Module):
     """down(silu(gate(x)) * up(x)) with bias-free linears."""
@@ -43,7 +45,8 @@ class SoftmaxGreedyGate(nn.Module):
         cached = getattr(self, "_w32_cache", None)
         if cached is None or cached[0] != stamp:
             cached = (stamp, w.detach().float().contiguous())
-            self._w32_cache = cached
+            if settled(w.device):
+                self._w32_cache = cached
         return cached[1]
 
     def forward(self, hidden_states: torch.Tensor):

@@ -425,3 +425,72 @@ def test_block_takes_overlapping_rows(cuda_device, family, kw, tokens, super_exp
             got, ref = first(block(x)), first(block(x.contiguous()))
             # (fp32 atomics in another order, then one bf16 rounding)
             assert float((got - ref).abs().max()) <= 1e-2 * float(ref.abs().max())
+
+
+@pytest.mark.parametrize("warm_tokens", [0, 100])      # nothing made before; the stacked weights, but not their few-rows copies
+@pytest.mark.parametrize("family,kw", _FAMILIES)
+def test_block_weights_made_on_one_stream_taken_on_another(cuda_device, family, kw, warm_tokens):
+    """A first forward behind other work on its stream, and a second one on another stream right after it: what the first made
+    (stacked weights, copies in operand order, the gate's copy) is there for the second."""
+    import torch
+
+    from bitsmoe_amd.synth import make_layer
+
+    blocks = [make_layer(_small_spec(family, **kw), device=cuda_device, dtype=torch.bfloat16, seed=47).eval() for _ in range(2)]
+    g = torch.Generator().manual_seed(5)
+    x, warm = (torch.randn((1, t, 128), generator=g).to(torch.bfloat16).to(cuda_device) for t in (8, max(warm_tokens, 1)))
+    busy = torch.randn((4096, 4096), device=cuda_device)
+    first = lambda out: (out[0] if isinstance(out, tuple) else out).float()
+    with torch.no_grad():
+        for b in blocks:
+            b.prepare_runtime_fastpath(warmup=True)
+            if warm_tokens:
+                b(warm)
+        ref = first(blocks[0](x))
+        del blocks[0]
+        rest = [torch.full((1 << k,), float("nan"), device=cuda_device) for k in range(8, 22)]      # (what new memory then holds)
+        del rest
+        torch.cuda.synchronize()
+        streams = [torch.cuda.Stream(device=cuda_device) for _ in range(2)]
+        got = []
+        for i, s in enumerate(streams):
+            with torch.cuda.stream(s):
+                if i == 0:
+                    for _ in range(20):
+                        busy @ busy
+                got.append(first(blocks[0](x)))
+        torch.cuda.synchronize()
+    for y in got:      # (fp32 atomics in another order, then one bf16 rounding)
+        assert float((y - ref).abs().max()) <= 1e-2 * float(ref.abs().max())
+
+
+@pytest.mark.parametrize("warm_tokens", [0, 100])
+@pytest.mark.parametrize("family,kw", _FAMILIES)
+def test_block_first_forward_under_capture(cuda_device, family, kw, warm_tokens):
+    """What a capture makes is the graph's: an eager forward before any replay makes its own, and every replay agrees."""
+    import torch
+
+    from bitsmoe_amd.synth import make_layer
+
+    block = make_layer(_small_spec(family, **kw), device=cuda_device, dtype=torch.bfloat16, seed=49).eval()
+    block.prepare_runtime_fastpath(warmup=True)
+    g = torch.Generator().manual_seed(6)
+    x, warm = (torch.randn((1, t, 128), generator=g).to(torch.bfloat16).to(cuda_device) for t in (8, max(warm_tokens, 1)))
+    first = lambda out: out[0] if isinstance(out, tuple) else out
+    with torch.no_grad():
+        if warm_tokens:
+            block(warm)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            y = first(block(x))
+        eager = first(block(x)).float()
+        again = first(block(x)).float()
+        torch.cuda.synchronize()
+        top = float(again.abs().max())
+        assert 0 < top < float("inf") and float((eager - again).abs().max()) <= 1e-2 * top
+        for _ in range(3):
+            y.fill_(float("nan"))
+            graph.replay()
+            torch.cuda.synchronize()
+            assert float((y.float() - again).abs().max()) <= 1e-2 * top
+            block(x)
