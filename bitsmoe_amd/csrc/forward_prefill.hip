@@ -377,15 +377,14 @@ struct DmaStage {
 // token index (possible when every aligned run of 8 local rows is 8 consecutive logical ranks);
 // otherwise Hs is the pre-gathered [A, ld].  WU: the bit-width shared by every slab of the
 // matrix, or 0 (mixed).  NMB: 16-row blocks of the assignment tile that are computed.
-template <bool DIRECT, int PFM, int WU, int NMB>
+template <bool DIRECT, int PFM, bool FUSE, int WU, int NMB>
 __device__ __forceinline__ void gateup_tile_body(const FastExpert fe, const FastSlab* __restrict__ fs_row, int all_slabs,
                                                      const uint16_t* __restrict__ Hs, int ld,
                                                      const int32_t* __restrict__ token_indices, int T, int I,
                                                      int n_tiles, uint16_t* __restrict__ out, int a_begin, int rows,
                                                      int t0, const DmaStage st0, const DmaStage st1, const DmaStage st2, uint16_t* __restrict__ turn,
                                                      int32_t* __restrict__ pack_tab, int32_t* __restrict__ scale_tab,
-                                                     int32_t* __restrict__ rank_tab, int32_t* __restrict__ bits_tab,
-                                                     bool fuse_silu) {
+                                                     int32_t* __restrict__ rank_tab, int32_t* __restrict__ bits_tab) {
     static_assert(WU == 0 || WU == 2 || WU == 3 || WU == 4, "a bit-width, or 0 for widths that differ from slab to slab");
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -546,18 +545,31 @@ __device__ __forceinline__ void gateup_tile_body(const FastExpert fe, const Fast
     BITSMOE_TLP(g_tl_pf_gateup, 3);
     if (!active) return;
     uint16_t* cols = out + (int64_t)a_begin * I + N_TILE * t + 64 * wn;
-    store_turned<NMB>(turn + wave * dma_stage(PFM), rows, lane, acc, [&](int row, int c, u32x4 v) {
-        u32x4* dst = reinterpret_cast<u32x4*>(cols + (int64_t)row * I + 8 * c);
-        if (fuse_silu) {
-            // `out` holds the gate sums an earlier launch stored: z = silu(gate) * up takes their place
-            const u32x4 g = *dst;
+    uint16_t* mine = turn + wave * dma_stage(PFM);
+    if constexpr (FUSE) {
+        // `out` holds the gate sums an earlier launch stored: z = silu(gate) * up takes their place.  The gate sums are turned
+        // into the accumulators' order: up enters the product in fp32.
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const h2 gp = __builtin_bit_cast(h2, (uint32_t)g[q]), up = __builtin_bit_cast(h2, (uint32_t)v[q]);
-                v[q] = z_operand((float)gp[0], (float)up[0]) | (uint32_t)z_operand((float)gp[1], (float)up[1]) << 16;
-            }
+        for (int k = 0; k < 2 * NMB; ++k) {
+            const int row = 8 * k + (lane >> 3);
+            if (row < rows)
+                *reinterpret_cast<u32x4*>(mine + dma_chunk_off(row, lane & 7)) =
+                    *reinterpret_cast<const u32x4*>(cols + (int64_t)row * I + 8 * (lane & 7));
         }
-        *dst = v;
+#pragma unroll
+        for (int mb = 0; mb < NMB; ++mb)
+#pragma unroll
+            for (int nb = 0; nb < 4; ++nb) {
+                const u32x2 g = *reinterpret_cast<const u32x2*>(mine + dma_chunk_off(16 * mb + n, 2 * nb + (kg >> 1)) + 4 * (kg & 1));
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const uint16_t gate = (uint16_t)((uint32_t)g[j >> 1] >> (16 * (j & 1)));
+                    acc[mb][nb][j] = __half2float(__ushort_as_half(z_operand(__half2float(__ushort_as_half(gate)), acc[mb][nb][j])));
+                }
+            }
+    }
+    store_turned<NMB>(mine, rows, lane, acc, [&](int row, int c, u32x4 v) {
+        *reinterpret_cast<u32x4*>(cols + (int64_t)row * I + 8 * c) = v;
     });
 }
 
@@ -565,14 +577,14 @@ __device__ __forceinline__ void gateup_tile_body(const FastExpert fe, const Fast
 // PFM: assignments per tile at most.  With 128 the ring takes 78 KB of LDS and a wavefront up to 247 registers: two workgroups
 // per CU.  With 64 (53 KB, 145 registers: three) a short tile's step -- a quarter or half of the MFMAs behind the same loads,
 // waits and barrier -- is hidden by one more workgroup (rule and measurements: launch_policy.h); k_down_mfma likewise.
-template <bool DIRECT, int PFM>
+template <bool DIRECT, int PFM, bool FUSE>
 __global__ __launch_bounds__(256, PFM == 128 ? 2 : 3) void k_gateup_mfma(
     const FastExpert* __restrict__ gate_fe, const FastSlab* __restrict__ gate_fs, int gate_max_slabs,
     const FastExpert* __restrict__ up_fe, const FastSlab* __restrict__ up_fs, int up_max_slabs,
     const uint16_t* __restrict__ Hs_g, const uint16_t* __restrict__ Hs_u, int ldg, int ldu,
     const int32_t* __restrict__ token_indices, int T,
     const MTile* __restrict__ mtiles, const int32_t* __restrict__ n_mtiles, int I, int n_tiles,
-    uint16_t* __restrict__ G, uint16_t* __restrict__ U, int proj_sel, int fuse) {
+    uint16_t* __restrict__ G, uint16_t* __restrict__ U, int proj_sel) {
     // the ring (three activation stages, three payload stages), which the epilogue uses again: 16 KB per wavefront
     __shared__ __attribute__((aligned(16))) uint16_t ring[DMA_STAGES * (dma_stage(PFM) + 2 * DMA_WSTAGE)];
     static_assert(sizeof(ring) >= 4 * dma_stage(PFM) * sizeof(uint16_t), "the epilogue's space");
@@ -580,7 +592,7 @@ __global__ __launch_bounds__(256, PFM == 128 ? 2 : 3) void k_gateup_mfma(
     __shared__ int32_t pack_tab[DMA_MAX_SLABS], scale_tab[DMA_MAX_SLABS], rank_tab[DMA_MAX_SLABS * 8], bits_tab[DMA_MAX_SLABS];
     BITSMOE_TLP(g_tl_pf_gateup, 0);
     const int n_tp = (n_tiles + 1) >> 1;
-    // proj_sel < 0: both projections in this launch; 0 / 1: the gate / the up projection alone.  fuse (up alone, after
+    // proj_sel < 0: both projections in this launch; 0 / 1: the gate / the up projection alone.  FUSE (up alone, after
     // a gate launch): the epilogue stores z = silu(gate) * up over the gate sums instead of the up sums.
     const int units = proj_sel < 0 ? 2 * n_tp : n_tp;
     const int logical = xcd_logical(blockIdx.x, __builtin_amdgcn_readfirstlane(*n_mtiles), units);
@@ -589,7 +601,6 @@ __global__ __launch_bounds__(256, PFM == 128 ? 2 : 3) void k_gateup_mfma(
     const int tp = logical % n_tp;
     const int proj = proj_sel < 0 ? (logical / n_tp) & 1 : proj_sel;
     const int mt_i = logical / units;
-    const bool fuse_silu = fuse != 0 && proj == 1;
     const i32x4 tv = *reinterpret_cast<const i32x4*>(mtiles + mt_i);
     const int e = __builtin_amdgcn_readfirstlane(tv[0]);
     const int a_begin = __builtin_amdgcn_readfirstlane(tv[1]);
@@ -601,7 +612,7 @@ __global__ __launch_bounds__(256, PFM == 128 ? 2 : 3) void k_gateup_mfma(
     const int nslabs = __builtin_amdgcn_readfirstlane(min(fe.num_slabs, max_slabs));
     const uint16_t* __restrict__ Hs = proj ? Hs_u : Hs_g;
     const int ld = proj ? ldu : ldg;
-    uint16_t* __restrict__ out = (proj && !fuse_silu) ? U : G;
+    uint16_t* __restrict__ out = (proj && !FUSE) ? U : G;
     const int w = __builtin_amdgcn_readfirstlane(fe.uniform_bits);
     // tiles of at most 32 / 64 / 96 assignments (experts that see few tokens, remainders) run a body
     // with a quarter / half / three quarters of the accumulators, MFMAs and staging; complete
@@ -612,9 +623,9 @@ __global__ __launch_bounds__(256, PFM == 128 ? 2 : 3) void k_gateup_mfma(
                    st2 = {ring + 2 * STAGE, sw + 2 * DMA_WSTAGE, ss2};
     BITSMOE_TLP(g_tl_pf_gateup, 1);
     auto body = [&](auto w_c, auto nmb_c) {
-        gateup_tile_body<DIRECT, PFM, decltype(w_c)::value, decltype(nmb_c)::value>(
+        gateup_tile_body<DIRECT, PFM, FUSE, decltype(w_c)::value, decltype(nmb_c)::value>(
             fe, fs_row, nslabs, Hs, ld, token_indices, T, I, n_tiles, out, a_begin, rows, 2 * tp, st0, st1, st2, ring, pack_tab,
-            scale_tab, rank_tab, bits_tab, fuse_silu);
+            scale_tab, rank_tab, bits_tab);
     };
     auto by_rows = [&](auto w_c) {
         if (rows <= 32)
@@ -1214,21 +1225,24 @@ int launch_forward_mfma(const bitsmoe_matset* gate, const bitsmoe_matset* up, co
         // off unless asked for.
         const bool wide_gu = has_wide_rows(gate) || has_wide_rows(up);
         const bool split = options().prefill_split > 0 && !wide_gu;      // (the side kernel adds to the sums before SiLU)
-        auto launch = [&](auto kernel, int proj_sel, int fuse) -> hipError_t {
+        auto launch = [&](auto kernel, int proj_sel) -> hipError_t {
             const int64_t wgs = (max_mtiles + 31) / 32 * 32 * (proj_sel < 0 ? 2 : 1) * n_tp;
             hipLaunchKernelGGL(kernel, dim3((unsigned)wgs), dim3(256), 0, st, gate->d_fast_experts, gate->d_fast_slabs,
                                gate->prep_max_slabs, up->d_fast_experts, up->d_fast_slabs, up->prep_max_slabs, Hs_g, Hs_u, ldg, ldu, tok,
-                               (int)T, mtiles, n_mtiles, I, n_tiles, z, Ubuf, proj_sel, fuse);
+                               (int)T, mtiles, n_mtiles, I, n_tiles, z, Ubuf, proj_sel);
             return hipGetLastError();
         };
-        const auto kernel = tile_rows == PF_M ? (direct ? k_gateup_mfma<true, PF_M> : k_gateup_mfma<false, PF_M>)
-                                              : (direct ? k_gateup_mfma<true, PF_M / 2> : k_gateup_mfma<false, PF_M / 2>);
+        auto kernel = [&](auto fuse_c) {
+            constexpr bool F = decltype(fuse_c)::value;
+            return tile_rows == PF_M ? (direct ? k_gateup_mfma<true, PF_M, F> : k_gateup_mfma<false, PF_M, F>)
+                                     : (direct ? k_gateup_mfma<true, PF_M / 2, F> : k_gateup_mfma<false, PF_M / 2, F>);
+        };
         if (split) {
-            BITSMOE_HIP_TRY(launch(kernel, 0, 0));
-            BITSMOE_HIP_TRY(launch(kernel, 1, 1));
+            BITSMOE_HIP_TRY(launch(kernel(std::false_type{}), 0));
+            BITSMOE_HIP_TRY(launch(kernel(std::true_type{}), 1));
             record(prof, 2, st);
         } else {
-            BITSMOE_HIP_TRY(launch(kernel, -1, 0));
+            BITSMOE_HIP_TRY(launch(kernel(std::false_type{}), -1));
             if (wide_gu) {      // rows of 6-, 8- and 16-bit slabs: their share of the (f16) gate and up sums
                 const int rc = launch_wide_gateup(gate, up, h_gate, h_up, act_dtype, Rg, Ru, ldg_in, ldu_in, tok, off, A, I, z, Ubuf,
                                                   true, st);

@@ -70,19 +70,23 @@ def test_routing_tables_bit_exact(cuda_device, tokens, top_k, n_global, n_super,
 
 
 def _forward_case(cuda_device, seed, n_experts, tokens, top_k, rank_in, rank_out, dim, dtype_name, choices,
-                  path=None, tol=1e-2, uniform_bits=False, slab_multiple=None, scramble_ranks=False, expect_fused=None):
+                  path=None, tol=1e-2, uniform_bits=False, slab_multiple=None, scramble_ranks=False, expect_fused=None,
+                  times=(1.0, 1.0, 1.0)):
     import torch
 
     hip = _hip()
     rng = np.random.default_rng(seed)
     gate, up, down = helpers.make_experts(seed, n_experts, rank_in, rank_out, dim, choices=choices,
                                           uniform_bits=uniform_bits, slab_multiple=slab_multiple)
+    for lst, t in ((gate, times[0]), (up, times[1])):      # (of the gate and up weights, and of the up activations)
+        for m in lst:
+            m["scale"] = (m["scale"].astype(np.float32) * t).astype(np.float16)
     if scramble_ranks:       # rows of gate / up read arbitrary columns of h instead of runs of eight
         for m in gate + up:
             m["rank_idx"] = rng.permutation(rank_in).astype(np.int32)[m["rank_idx"]]
     dt = torch.float16 if dtype_name == "f16" else torch.bfloat16
     h_gate = torch.from_numpy(rng.normal(size=(tokens, rank_in)).astype(np.float32)).to(dt)
-    h_up = torch.from_numpy(rng.normal(size=(tokens, rank_in)).astype(np.float32)).to(dt)
+    h_up = torch.from_numpy((rng.normal(size=(tokens, rank_in)) * times[2]).astype(np.float32)).to(dt)
     logits = rng.normal(size=(tokens, n_experts)).astype(np.float32)
     idx, w = o.router_qwen(logits, top_k)
     tok, off, rw = o.build_routing(idx, w, np.arange(n_experts, dtype=np.int32), n_experts)
@@ -297,8 +301,8 @@ def test_forward_mfma_path_one_width_per_expert(cuda_device, bits, slabs, tokens
 @pytest.mark.parametrize("split", [0, 1])
 def test_forward_mfma_path_silu_pass_or_up_epilogue(cuda_device, split, lib_option):
     """Option prefill_split: 0 (default) one launch for both projections and a SiLU pass behind it; 1 gate and up as two
-    launches, z = silu(gate) * up stored by the up launch's epilogue over the gate sums.  Ragged tiles, two
-    widths-per-expert layouts (LDS-direct bodies and the register-staged one)."""
+    launches, z = silu(gate) * up stored by the up launch's epilogue over the gate sums.  Ragged tiles, experts of one
+    width and of several."""
     from bitsmoe_amd.algorithms import _capi
 
     lib_option("prefill_split", split)
@@ -306,6 +310,18 @@ def test_forward_mfma_path_silu_pass_or_up_epilogue(cuda_device, split, lib_opti
         err = _forward_case(cuda_device, 900 + split, 4, 300, 2, 256, 128, 384, "bf16", (2, 3, 4), path=_capi.PATH_MFMA,
                             tol=1e-2, uniform_bits=uniform, slab_multiple=None if uniform else 64)
         assert err < 3e-3
+
+
+@pytest.mark.parametrize("tokens", [40, 300])      # tiles of at most 64 rows, and of 128
+def test_forward_mfma_path_up_epilogue_takes_fp32_sums(cuda_device, tokens, lib_option):
+    """Option prefill_split = 1: the up sums enter silu(gate) * up in fp32.  Here they have a deviation of 8e4, past the f16 range
+    in every second value, beside gate sums of 0.04, so that z stays in range."""
+    from bitsmoe_amd.algorithms import _capi
+
+    lib_option("prefill_split", 1)
+    err = _forward_case(cuda_device, 940, 4, tokens, 2, 256, 128, 384, "bf16", (2, 3, 4), path=_capi.PATH_MFMA, tol=1e-2,
+                        slab_multiple=64, times=(2.0 ** -3, 2.0 ** 6, 2.0 ** 12))
+    assert err < 3e-3
 
 
 def test_forward_mfma_path_more_slabs_than_the_slab_tables_hold(cuda_device):
