@@ -11,6 +11,9 @@ using namespace bitsmoe;
 
 static inline size_t align256(size_t v) { return (v + 255) / 256 * 256; }
 
+// Rows that the few-rows kernel takes: a call of more ends with the projection's operand (and super_out), in the caller's memory.
+constexpr int64_t PROJECT_OUT_MAX_ROWS = 64;
+
 // Where the intermediates of a call sit in the workspace.
 struct BlockWorkspace {
     size_t selected, weights, rank_accum, operand, forward, forward_bytes, super_forward, super_bytes, super_out, total;
@@ -22,13 +25,14 @@ static BlockWorkspace carve(const bitsmoe_block_plan* p, int64_t T) {
     w.selected = take((size_t)T * p->top_k * 8);
     w.weights = take((size_t)T * p->top_k * 4);
     w.rank_accum = take((size_t)T * p->rank_out * 4);
-    w.operand = take((size_t)T * (p->rank_out + p->shared_intermediate) * 2);
+    const bool may_project = T <= PROJECT_OUT_MAX_ROWS;
+    w.operand = take(may_project ? (size_t)T * (p->rank_out + p->shared_intermediate) * 2 : 0);
     w.forward_bytes = align256(bitsmoe_forward_routed_workspace_bytes(p->gate, p->up, p->down, T, p->top_k, BITSMOE_PATH_AUTO));
     w.forward = take(w.forward_bytes);
     w.super_bytes = p->super_gate ? align256(bitsmoe_forward_routed_workspace_bytes(p->super_gate, p->super_up, p->super_down, T,
                                                                                     p->top_k, BITSMOE_PATH_AUTO)) : 0;
     w.super_forward = take(w.super_bytes);
-    w.super_out = take(p->super_gate ? (size_t)T * p->hidden * 4 : 0);
+    w.super_out = take(p->super_gate && may_project ? (size_t)T * p->hidden * 4 : 0);
     w.total = at;
     return w;
 }
@@ -58,6 +62,7 @@ extern "C" int bitsmoe_block_forward(const bitsmoe_block_plan* p, const void* x,
     BITSMOE_REQUIRE(x && proj && out, "null pointer");
     BITSMOE_REQUIRE(p->router_form != BITSMOE_ROUTER_CALLER || (selected && weights), "the caller's routing is missing");
     const bool project_in = (stages & BITSMOE_BLOCK_PROJECT_IN) != 0, project_out = (stages & BITSMOE_BLOCK_PROJECT_OUT) != 0;
+    BITSMOE_REQUIRE(!project_out || n_tokens <= PROJECT_OUT_MAX_ROWS, "the output projection takes at most 64 tokens");
     const bool super = p->super_gate != nullptr;
     BITSMOE_REQUIRE(!super || project_out || super_out, "super_out must not be null where the caller projects");
     const BlockWorkspace w = carve(p, n_tokens);

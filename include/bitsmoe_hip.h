@@ -323,6 +323,7 @@ int bitsmoe_moe_forward_routed(const bitsmoe_matset* gate, const bitsmoe_matset*
  *   selected int64 / weights fp32 [T, top_k]: given with BITSMOE_ROUTER_CALLER, else written (may then be null).
  *   out: with BITSMOE_BLOCK_PROJECT_OUT the block output [T, hidden], else the output projection's operand
  *   [T, rank_out + shared_intermediate]; super experts' share: in the output, or (fp32 [T, hidden]) in super_out.
+ *   The projections run here at up to 64 tokens; a larger call's workspace has no room for their operand and is refused.
  *   side_stream (may be null): a stream for the super experts' call beside the packed experts'; joined before the call ends.
  */
 #define BITSMOE_ROUTER_LOGITS 0     /* softmax and top-k of proj's logits columns */

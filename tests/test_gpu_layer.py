@@ -494,3 +494,33 @@ def test_block_first_forward_under_capture(cuda_device, family, kw, warm_tokens)
             torch.cuda.synchronize()
             assert float((y.float() - again).abs().max()) <= 1e-2 * top
             block(x)
+
+
+def test_block_workspace_holds_no_projection_past_the_few_rows_kernel(cuda_device):
+    """Past 64 tokens the caller projects, from an operand and super experts' share in memory of its own: the workspace (which
+    outlives the call) holds the routing, the rank-space sums and the two operators' own, and a call that asks for the
+    projection all the same is refused before anything is launched."""
+    import torch
+
+    from bitsmoe_amd.algorithms import mlp_forward_cuda as hip
+    from bitsmoe_amd.synth import make_layer
+
+    block = make_layer(_small_spec("qwen3moe"), device=cuda_device, dtype=torch.bfloat16, seed=51, super_experts=(1, 6)).eval()
+    block.prepare_runtime_fastpath(warmup=True)
+    hidden, k = block.spec.hidden_size, block.top_k
+    with torch.no_grad():
+        block(torch.randn((1, 8, hidden), device=cuda_device, dtype=torch.bfloat16))
+    plan = next(v for v in block._basis_cache.values() if isinstance(v, dict) and "native" in v)
+    native, rank_out = plan["native"][0], int(block.shared_u_down.shape[1])
+    up256 = lambda n: (n + 255) // 256 * 256
+    for t in (64, 65, 4096):
+        operators = sum(up256(hip._lib.bitsmoe_forward_routed_workspace_bytes(*(s.handle for s in native._sets[i:i + 3]), t, k, 0))
+                        for i in (0, 3))
+        projection = up256(2 * t * rank_out) + up256(4 * t * hidden) if t <= 64 else 0
+        assert native.workspace_bytes(t) == up256(8 * t * k) + up256(4 * t * k) + up256(4 * t * rank_out) + operators + projection
+    x = torch.zeros((65, hidden), device=cuda_device, dtype=torch.bfloat16)
+    proj, out = x @ plan["w_in"].T, torch.full_like(x, 3.0)
+    with pytest.raises(RuntimeError, match="at most 64 tokens"):
+        hip.block_forward(native, x, proj, hip.BLOCK_PROJECT_OUT, out)
+    torch.cuda.synchronize()
+    assert bool((out == 3.0).all())
