@@ -663,9 +663,11 @@ class BitsMoE_BaseSparseMoeBlock(nn.Module):
             return None
         x = hidden_states
         rows, hidden = x.shape
-        # (the library gets a pointer and a row stride: the width is known here only)
+        # (the library gets a pointer and a row stride: width and device are known here only)
         if hidden != plan["w_in"].shape[1]:
             raise RuntimeError(f"hidden states of width {hidden}, but this block's input projections take {plan['w_in'].shape[1]}")
+        if x.device != plan["w_in"].device:
+            raise RuntimeError(f"hidden states on {x.device}, but this block's projections are on {plan['w_in'].device}")
         if x.stride(1) != 1 or (rows > 1 and (x.stride(0) % 8 != 0 or x.stride(0) < hidden)) or x.data_ptr() % 16 != 0:
             x = x.clone(memory_format=torch.contiguous_format)
         form = (mlp_forward_cuda.ROUTER_LOGITS if router is not None else

@@ -405,6 +405,25 @@ def test_block_refuses_hidden_states_of_another_width(cuda_device, family, kw, t
     assert block._fused_plan(torch.bfloat16, (vh_gate, vh_up, u_down[:-16]), None, None, None) is None
 
 
+@pytest.mark.parametrize("tokens", [1, 40])      # (both projections by the few-rows kernel)
+def test_block_refuses_hidden_states_of_another_device(cuda_device, tokens):
+    """As the framework's GEMMs do.  (One card: the plan's stacked weights are swapped for a copy on the host, the copies the
+    kernels read stay where they are.)"""
+    import torch
+
+    from bitsmoe_amd.synth import make_layer
+
+    block = make_layer(_small_spec("qwen3moe"), device=cuda_device, dtype=torch.bfloat16, seed=42).eval()
+    block.prepare_runtime_fastpath(warmup=True)
+    x = torch.zeros((1, tokens, block.spec.hidden_size), dtype=torch.bfloat16, device=cuda_device)
+    with torch.no_grad():
+        block(x)
+        plan = next(v for v in block._basis_cache.values() if isinstance(v, dict) and "native" in v)
+        plan["w_in"] = plan["w_in"].cpu()
+        with pytest.raises(RuntimeError):
+            block(x)
+
+
 @pytest.mark.parametrize("tokens", [8, 32, 100])
 @pytest.mark.parametrize("family,kw", _FAMILIES)
 @pytest.mark.parametrize("super_experts", [(), (1, 6)])
