@@ -685,6 +685,8 @@ class BitsMoE_BaseSparseMoeBlock(nn.Module):
         selected = weights = sup = None
         if form == mlp_forward_cuda.ROUTER_CALLER:
             selected, weights = route_fn(hidden_states)
+            if selected.dtype not in (torch.int32, torch.int64):
+                raise RuntimeError("selected must be int32 or int64")
             selected = selected.reshape(rows, self.top_k).to(torch.int64).contiguous()
             weights = weights.reshape(rows, self.top_k).to(torch.float32).contiguous()
         super_modules = bool(self._super_expert_items) and not _super_via_operator()

@@ -424,6 +424,38 @@ def test_block_refuses_hidden_states_of_another_device(cuda_device, tokens):
             block(x)
 
 
+@pytest.mark.parametrize("ids", ["int32", "int64", "int16", "float32"])
+def test_block_takes_the_picks_of_a_gate_module_as_the_operator_does(cuda_device, ids):
+    """A gate of the model's own: ids int32 or int64, anything else is refused."""
+    import torch
+
+    from bitsmoe_amd.synth import make_layer
+
+    block = make_layer(_small_spec("deepseekv2"), device=cuda_device, dtype=torch.bfloat16, seed=45).eval()
+    block.prepare_runtime_fastpath(warmup=True)
+    x = torch.randn((1, 8, block.spec.hidden_size), generator=torch.Generator().manual_seed(9)).to(torch.bfloat16).to(cuda_device)
+    with torch.no_grad():
+        ref = block(x).float()
+        real = block.gate
+
+        class Gate(torch.nn.Module):
+            def __init__(self):
+                super().__init__()
+                self.weight = real.weight
+
+            def forward(self, h):
+                idx, w, aux = real(h)
+                return idx.to(getattr(torch, ids)), w, aux
+
+        block.gate = Gate()
+        if ids in ("int32", "int64"):
+            got = block(x).float()      # (fp32 atomics in another order, then one bf16 rounding)
+            assert float((got - ref).abs().max()) <= 1e-2 * float(ref.abs().max())
+        else:
+            with pytest.raises(RuntimeError):
+                block(x)
+
+
 @pytest.mark.parametrize("tokens", [8, 32, 100])
 @pytest.mark.parametrize("family,kw", _FAMILIES)
 @pytest.mark.parametrize("super_experts", [(), (1, 6)])
