@@ -1062,6 +1062,11 @@ static inline int direct_ld(const bitsmoe_matset* set) { return (set->pad_rank_p
 static inline int mtile_rows(int64_t A, int E) {
     return A <= (int64_t)policy::LOW_TILES_MAX_ASSIGN_PER_EXPERT * E ? PF_M / 2 : PF_M;
 }
+// Tiles of any call of at most A assignments (a workspace taken for one size serves the smaller ones).
+static inline int64_t max_mtiles_up_to(int64_t A, int E) {
+    const int64_t low = std::min(A, (int64_t)policy::LOW_TILES_MAX_ASSIGN_PER_EXPERT * E);
+    return std::max(low / (PF_M / 2), A / PF_M) + E;
+}
 
 // Carving of the workspace, shared by the size query and the launcher.
 struct MfmaWorkspace {
@@ -1069,7 +1074,7 @@ struct MfmaWorkspace {
 };
 static MfmaWorkspace mfma_workspace(const bitsmoe_matset* gate, const bitsmoe_matset* up, const bitsmoe_matset* down,
                                     int64_t T, int64_t A, int I) {
-    const int64_t max_mtiles = A / (PF_M / 2) + gate->n_experts;      // (of the lower tiles: never less for more assignments)
+    const int64_t max_mtiles = max_mtiles_up_to(A, gate->n_experts);
     const size_t direct = align256((size_t)T * direct_ld(gate) * 2) + align256((size_t)T * direct_ld(up) * 2);
     const size_t gathered = align256((size_t)A * gate->prep_max_slabs * SLAB_ROWS * 2) + align256((size_t)A * up->prep_max_slabs * SLAB_ROWS * 2);
     MfmaWorkspace w;

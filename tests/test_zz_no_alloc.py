@@ -86,6 +86,23 @@ def test_static_scratch_forward_rejects_oversized_call(cuda_device):
     torch.cuda.synchronize()
 
 
+def test_grouped_gemm_workspace_counts_the_tiles_it_takes(cuda_device):
+    """What a call needs decides whether it fits the static scratch: past the low tiles' range a tile entry (16 bytes) per 128
+    assignments, and never less room for fewer assignments."""
+    from bitsmoe_amd.algorithms import _capi as capi, mlp_forward_cuda as hip
+
+    n_experts, rank, dim = 2, 64, 128
+    gate, up, down = helpers.make_experts(3, n_experts, rank, rank, dim, uniform_bits=True)
+    sets = [hip.MatrixSet(*helpers.to_device_lists(m, cuda_device), intermediate_size=dim) for m in (gate, up, down)]
+    assert sets[0].prepare(0) and sets[1].prepare(0) and sets[2].prepare(1)
+    need = lambda a: int(capi.load().bitsmoe_forward_workspace_bytes_sets(*[s.handle for s in sets], 4096, a, capi.PATH_MFMA))
+    # slot and list entry, z and u, y, the activations gathered for gate and up (a group of eight 64-row slabs at least)
+    per_assignment = 4 + 8 + 2 * 2 * dim + 2 * rank + 2 * 2 * 512
+    assert need(36864) - need(32768) == 4096 * per_assignment + 4096 // 128 * 16
+    sizes = [need(a) for a in range(1, 48 * n_experts * 3)]
+    assert sizes == sorted(sizes)
+
+
 def test_static_scratch_forward_under_graph_capture(cuda_device):
     """The static entry point captured into a HIP graph (its scratch address was located when the matrix sets
     were created, so nothing but launches happens during capture): two sizes in one graph, the second smaller,
