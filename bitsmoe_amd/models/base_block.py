@@ -704,9 +704,6 @@ class BitsMoE_BaseSparseMoeBlock(nn.Module):
         # The super experts' operator call needs the router's output and the hidden states only: it runs on a side
         # stream beside the packed experts' call (its small launches fill what the packed kernels leave idle).
         side = _side_stream(dev).cuda_stream if self._super_expert_items and _SUPER_SIDE_STREAM and not super_modules else 0
-        if not plan["kept"] and settled(dev):      # (one wait for the stacked weights and their copies)
-            plan["kept"] = True
-            self._basis_cache[plan["key"]] = plan
         mlp_forward_cuda.block_forward(native, x, proj, stages, out, selected, weights, sup, side)
         if not stages & mlp_forward_cuda.BLOCK_PROJECT_OUT:
             out = out @ w_out.T
@@ -721,6 +718,9 @@ class BitsMoE_BaseSparseMoeBlock(nn.Module):
         if router is not None:
             lo, hi = plan["ranges"]["logits"]
             logits = proj[:, lo:hi]
+        if not plan["kept"] and settled(dev):      # (one wait for the stacked weights and their copies, behind the launches)
+            plan["kept"] = True
+            self._basis_cache[plan["key"]] = plan
         return out, logits
 
     # ---- shared forward body --------------------------------------------------------------
