@@ -515,6 +515,53 @@ def test_block_weights_made_on_one_stream_taken_on_another(cuda_device, family, 
         assert float((y - ref).abs().max()) <= 1e-2 * float(ref.abs().max())
 
 
+@pytest.mark.parametrize("family,kw", _FAMILIES)
+@pytest.mark.parametrize("super_experts", [(), (1, 6)])
+def test_block_first_forwards_on_two_threads(cuda_device, family, kw, super_experts):
+    """Two threads on streams of their own, each with the block's first forward: what either of them makes and keeps is there
+    for both, and for a third stream behind them."""
+    import threading
+
+    import torch
+
+    from bitsmoe_amd.synth import make_layer
+
+    made = lambda: make_layer(_small_spec(family, **kw), device=cuda_device, dtype=torch.bfloat16, seed=53, super_experts=super_experts)
+    g = torch.Generator().manual_seed(8)
+    xs = [torch.randn((1, 8, 128), generator=g).to(torch.bfloat16).to(cuda_device) for _ in range(2)]
+    first = lambda out: (out[0] if isinstance(out, tuple) else out).float()
+    with torch.no_grad():
+        warm = made().eval()
+        refs = [first(warm(x)) for x in xs]
+    for _ in range(4):
+        block = made().eval()
+        block.prepare_runtime_fastpath(warmup=True)
+        torch.cuda.synchronize()
+        got, errors, start = [None, None], [], threading.Barrier(2)
+
+        def work(i):
+            try:
+                st = torch.cuda.Stream(device=cuda_device)
+                with torch.no_grad(), torch.cuda.stream(st):
+                    start.wait()
+                    got[i] = first(block(xs[i]))
+                st.synchronize()
+            except Exception as exc:      # noqa: BLE001 - reported below
+                errors.append(exc)
+
+        threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert not errors, errors
+        with torch.no_grad(), torch.cuda.stream(torch.cuda.Stream(device=cuda_device)):
+            got.append(first(block(xs[0])))
+        torch.cuda.synchronize()
+        for y, ref in zip(got, refs + refs[:1]):      # (fp32 atomics in another order, then one bf16 rounding)
+            assert float((y - ref).abs().max()) <= 1e-2 * float(ref.abs().max())
+
+
 @pytest.mark.parametrize("warm_tokens", [0, 100])
 @pytest.mark.parametrize("family,kw", _FAMILIES)
 def test_block_first_forward_under_capture(cuda_device, family, kw, warm_tokens):

@@ -324,12 +324,16 @@ def test_forward_mfma_path_up_epilogue_takes_fp32_sums(cuda_device, tokens, lib_
     assert err < 3e-3
 
 
-def test_forward_mfma_path_more_slabs_than_the_slab_tables_hold(cuda_device):
-    """65 slabs of one width: past the per-slab tables of the LDS-direct body, the register-staged body runs."""
+@pytest.mark.parametrize("scramble", [False, True])      # activations through the token index, and gathered
+@pytest.mark.parametrize("choices", [(3,), (2, 3, 4)])
+@pytest.mark.parametrize("tokens", [40, 300])             # tiles of at most 64 rows, and of 128
+def test_forward_mfma_path_more_slabs_than_the_slab_tables_hold(cuda_device, tokens, choices, scramble):
+    """70 slabs of one or several widths: more than the per-slab tables of the loop hold, which are filled again for the six that
+    are left (twice the three stages of its ring)."""
     from bitsmoe_amd.algorithms import _capi
 
-    err = _forward_case(cuda_device, 650, 2, 40, 1, 65 * 64, 64, 128, "bf16", (3,), path=_capi.PATH_MFMA, tol=1e-2,
-                        uniform_bits=True)
+    err = _forward_case(cuda_device, 650, 2, tokens, 1, 70 * 64, 64, 128, "bf16", choices, path=_capi.PATH_MFMA, tol=1e-2,
+                        uniform_bits=len(choices) == 1, slab_multiple=None if len(choices) == 1 else 64, scramble_ranks=scramble)
     assert err < 3e-3
 
 
