@@ -21,7 +21,7 @@ from typing import List, Optional, Sequence, Tuple
 import torch
 
 from . import _capi
-from ._streams import settled
+from ._streams import keep_first
 
 _lib = _capi.load()
 # BITSMOE_NO_PREPARE=1 keeps every matrix set on the generic kernels (no wave-native copy)
@@ -654,12 +654,7 @@ def prepared_linear_weight_of(owner, weight: torch.Tensor) -> "PreparedLinearWei
     stamp = (weight.data_ptr(), -1 if weight.is_inference() else weight._version, tuple(weight.shape), weight.dtype)
     cached = getattr(owner, "_bitsmoe_prepared_weight", None)
     if cached is None or cached[0] != stamp:
-        cached = (stamp, PreparedLinearWeight(weight.detach()))
-        if settled(weight.device):
-            try:
-                object.__setattr__(owner, "_bitsmoe_prepared_weight", cached)
-            except (AttributeError, TypeError):
-                pass
+        cached = keep_first(owner, "_bitsmoe_prepared_weight", (stamp, PreparedLinearWeight(weight.detach())))
     return cached[1]
 
 

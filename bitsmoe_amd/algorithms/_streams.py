@@ -1,5 +1,9 @@
 """What one stream makes and every other may take."""
+import threading
+
 import torch
+
+_KEEPING = threading.Lock()
 
 
 def settled(device: torch.device) -> bool:
@@ -13,3 +17,20 @@ def settled(device: torch.device) -> bool:
             return False
         torch.cuda.current_stream().synchronize()
     return True
+
+
+def keep_first(owner, name: str, made: tuple) -> tuple:
+    """Keeps made = (stamp, value) as an attribute of `owner` once it is settled, and returns it.  Where another thread has kept
+    one of the same stamp meanwhile, that one stays and is returned: a third stream may read it already, and memory that is let
+    go is used again behind its own stream's work only."""
+    if not settled(made[1].device):
+        return made
+    with _KEEPING:
+        kept = getattr(owner, name, None)
+        if kept is not None and kept[0] == made[0]:
+            return kept
+        try:
+            object.__setattr__(owner, name, made)
+        except (AttributeError, TypeError):
+            pass
+    return made

@@ -67,7 +67,7 @@ _SKINNY_SHORT_CONTRACTION = 4096  # input features up to which 49 to 64 rows tak
 _SKINNY_PREPARED = _os.environ.get("BITSMOE_BLOCK_SKINNY_PREPARED", "1") != "0"
 
 
-_FEW_ROWS_LOCK = _threading.Lock()      # (held while a layer's copy is made, once; never during a forward)
+_FEW_ROWS_LOCK = _threading.Lock()      # (held while a layer's copy is made or its plan kept, once; never during a forward)
 
 
 def _few_rows(rows: int, n_in: int, n_out: int) -> bool:
@@ -275,7 +275,7 @@ class BitsMoE_BaseSparseMoeBlock(nn.Module):
         if cached is None:
             cached = tuple(getattr(self, k).to(dtype).contiguous() for k in self._SHARED_BASIS_BUFFER_KEYS)
             if settled(cached[0].device):
-                self._basis_cache[dtype] = cached
+                return self._basis_cache.setdefault(dtype, cached)
         return cached
 
     def _shared_basis_stacked(self, dtype: torch.dtype) -> torch.Tensor:
@@ -286,7 +286,7 @@ class BitsMoE_BaseSparseMoeBlock(nn.Module):
             vh_gate, vh_up, _ = self._shared_basis(dtype)
             cached = torch.cat([vh_gate, vh_up], dim=0).contiguous()
             if settled(cached.device):
-                self._basis_cache[key] = cached
+                return self._basis_cache.setdefault(key, cached)
         return cached
 
     def _get_flat_token_ids(self, token_count: int, device: torch.device) -> torch.Tensor:
@@ -417,7 +417,7 @@ class BitsMoE_BaseSparseMoeBlock(nn.Module):
             cached = (torch.arange(t, dtype=torch.int32, device=dev), torch.tensor([0, t], dtype=torch.int32, device=dev),
                       torch.ones((t,), dtype=torch.float32, device=dev))
             if settled(dev):
-                self._basis_cache[("always_on", t, str(dev))] = cached
+                cached = self._basis_cache.setdefault(("always_on", t, str(dev)), cached)
         tok, off, ones = cached
         rw = ones if token_weights is None else token_weights.reshape(-1).to(torch.float32).contiguous()
         return self._dense_operator_forward(key, [module], hidden_states, tok, off, rw).to(hidden_states.dtype)
@@ -719,8 +719,12 @@ class BitsMoE_BaseSparseMoeBlock(nn.Module):
             lo, hi = plan["ranges"]["logits"]
             logits = proj[:, lo:hi]
         if not plan["kept"] and settled(dev):      # (one wait for the stacked weights and their copies, behind the launches)
-            plan["kept"] = True
-            self._basis_cache[plan["key"]] = plan
+            with _FEW_ROWS_LOCK:
+                # (of two first forwards at once the first one's plan stays: a third stream may read its weights already)
+                kept = self._basis_cache.get(plan["key"])
+                if kept is None or kept["stamp"] != plan["stamp"]:
+                    plan["kept"] = True
+                    self._basis_cache[plan["key"]] = plan
         return out, logits
 
     # ---- shared forward body --------------------------------------------------------------

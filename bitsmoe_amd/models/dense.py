@@ -9,7 +9,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from bitsmoe_amd.algorithms._streams import settled
+from bitsmoe_amd.algorithms._streams import keep_first
 
 
 class DenseSwiGLUMLP(nn.Module):
@@ -44,9 +44,7 @@ class SoftmaxGreedyGate(nn.Module):
         stamp = (w.data_ptr(), -1 if w.is_inference() else w._version)
         cached = getattr(self, "_w32_cache", None)
         if cached is None or cached[0] != stamp:
-            cached = (stamp, w.detach().float().contiguous())
-            if settled(w.device):
-                self._w32_cache = cached
+            cached = keep_first(self, "_w32_cache", (stamp, w.detach().float().contiguous()))
         return cached[1]
 
     def forward(self, hidden_states: torch.Tensor):

@@ -562,6 +562,38 @@ def test_block_first_forwards_on_two_threads(cuda_device, family, kw, super_expe
             assert float((y - ref).abs().max()) <= 1e-2 * float(ref.abs().max())
 
 
+@pytest.mark.parametrize("family,kw", _FAMILIES)
+def test_block_keeps_what_the_first_of_two_forwards_made(cuda_device, family, kw, monkeypatch):
+    """A forward that finds its plan kept by another one meanwhile does not put its own in its place: a third stream may be
+    reading those weights.  (The second forward runs here in the middle of the first.)"""
+    import torch
+
+    from bitsmoe_amd.algorithms import mlp_forward_cuda as hip
+    from bitsmoe_amd.synth import make_layer
+
+    block = make_layer(_small_spec(family, **kw), device=cuda_device, dtype=torch.bfloat16, seed=57).eval()
+    block.prepare_runtime_fastpath(warmup=True)
+    x = torch.randn((1, 8, 128), generator=torch.Generator().manual_seed(4)).to(torch.bfloat16).to(cuda_device)
+    kept = lambda: [v for v in block._basis_cache.values() if isinstance(v, dict) and "native" in v] + [
+        getattr(block.gate, "_bitsmoe_prepared_weight", None)]
+    real, inner = hip.PreparedLinearWeight, []
+
+    def between(weight):
+        if not inner:
+            inner.append(None)
+            with torch.no_grad():
+                block(x)
+            inner[0] = kept()
+        return real(weight)
+
+    monkeypatch.setattr(block, "_few_rows_weight", lambda plan, native, key, f=block._few_rows_weight: (between(plan["w_in"]), f(plan, native, key))[1])
+    if family == "deepseekv2":
+        monkeypatch.setattr(hip, "PreparedLinearWeight", type("Made", (real,), {"__init__": lambda self, w: (between(w), real.__init__(self, w))[1]}))
+    with torch.no_grad():
+        block(x)
+    assert len(inner[0]) == 2 and all(a is b for a, b in zip(inner[0], kept()))
+
+
 @pytest.mark.parametrize("warm_tokens", [0, 100])
 @pytest.mark.parametrize("family,kw", _FAMILIES)
 def test_block_first_forward_under_capture(cuda_device, family, kw, warm_tokens):
