@@ -683,7 +683,7 @@ class PreparedLinearWeight:
 def skinny_linear_possible(x: torch.Tensor, weight) -> bool:
     """Can skinny_linear take these tensors?  (at most 64 rows of x [T, K] in the weight's 16-bit dtype -- or at most 16
     rows of fp32, rounded to that dtype inside the kernel -- with unit column stride and 16-byte aligned rows, a
-    contiguous weight [N, K], K a multiple of 128, N even; a PreparedLinearWeight: at most 16 rows.)"""
+    contiguous weight [N, K] or a PreparedLinearWeight of it, K a multiple of 128, N even.)"""
     prepared = isinstance(weight, PreparedLinearWeight)
     if prepared:
         w_dtype, n, k = weight.dtype, weight.out_features, weight.in_features

@@ -327,9 +327,11 @@ __device__ __forceinline__ void gateup_slab_mfma(int bits, const uint16_t* __res
 
 // The epilogue of both GEMM kernels.  The weights are the MFMA's first operand, so that a lane holds, of assignment
 // 16 mb + lane % 16, outputs 16 nb + 4 (lane / 16) + j: four neighbouring ones.  A wavefront turns its 16 * NMB x 64 block
-// around in 16 KB of LDS of its own (`turn`), so that a store instruction writes eight whole 128-byte rows: stores of the
-// registers as they are touch 32 or 64 cache lines per instruction, and their address work was 8 us of the 205 us gate/up
-// launch (4096 tokens, 128 experts).  put(row, chunk, 8 values) stores one 16-byte piece.
+// around in LDS of its own (`turn`: 128 bytes per row of the tile, 16 KB or 8), so that a store instruction writes eight whole
+// 128-byte rows: stores of the registers as they are touch 32 or 64 cache lines per instruction.  Kernel times under the tracer,
+// two runs of each on one card, before -> after this and the slab tables read a step ahead (one build): 4096 tokens, 128 experts,
+// gate/up 229, 225 -> 216, 219 us and down 156, 154 -> 151, 153; 1500 tokens, 64 checkpoint-shaped experts: 117, 118 -> 119, 115 and
+// 58, 59 -> 60, 58, no difference.  put(row, chunk, 8 values) stores one 16-byte piece.
 template <int NMB, class Put>
 __device__ __forceinline__ void store_turned(uint16_t* __restrict__ turn, int rows, int lane, const f32x4 (&acc)[NMB][4], Put&& put) {
     const int n = lane & 15, kg = lane >> 4;
@@ -585,7 +587,7 @@ __global__ __launch_bounds__(256, PFM == 128 ? 2 : 3) void k_gateup_mfma(
     const int32_t* __restrict__ token_indices, int T,
     const MTile* __restrict__ mtiles, const int32_t* __restrict__ n_mtiles, int I, int n_tiles,
     uint16_t* __restrict__ G, uint16_t* __restrict__ U, int proj_sel) {
-    // the ring (three activation stages, three payload stages), which the epilogue uses again: 16 KB per wavefront
+    // the ring (three activation stages, three payload stages), which the epilogue uses again: 128 bytes per row and wavefront
     __shared__ __attribute__((aligned(16))) uint16_t ring[DMA_STAGES * (dma_stage(PFM) + 2 * DMA_WSTAGE)];
     static_assert(sizeof(ring) >= 4 * dma_stage(PFM) * sizeof(uint16_t), "the epilogue's space");
     __shared__ __attribute__((aligned(16))) uint16_t ss0[DMA_SSTAGE], ss1[DMA_SSTAGE], ss2[DMA_SSTAGE];
@@ -853,7 +855,7 @@ __global__ __launch_bounds__(256, PFM == 128 ? 2 : 3) void k_down_mfma(const Fas
                                                       const int32_t* __restrict__ token_start,
                                                       int2* __restrict__ token_list, int A, int I, int n_tiles,
                                                       int n_groups, _Float16* __restrict__ y, int ldy) {
-    // three stages of z and the wavefronts' payload buffers, which the epilogue uses again: 16 KB per wavefront
+    // three stages of z and the wavefronts' payload buffers, which the epilogue uses again: 128 bytes per row and wavefront
     __shared__ __attribute__((aligned(16))) uint16_t lds[3 * dma_stage(PFM) + 2 * 4 * DN_WBUF];
     constexpr int STAGE = dma_stage(PFM);
     static_assert(sizeof(lds) >= 4 * STAGE * sizeof(uint16_t), "the epilogue's space");

@@ -13,12 +13,13 @@
 // reads G * 64 consecutive bytes of a row, several rows per instruction), turned in LDS and read from there as operands:
 // fetched in operand order a load touched 64 bytes of sixteen rows, and the launch grew by 4 us per sixteen rows.
 // Longer contractions take eight wavefronts, so that a share stays within MAXS steps (beyond that: several passes).
-// Prepared weights, graph of launches over 600 MB of weights, us per launch (batches of four steps and x in operand order ->
-// now; the library GEMM) at 1, 16, 32, 48, 64 rows:
-//   2048 -> 4224 features: 6.1 -> 6.2, 8.3 -> 7.3 (11.4), 12.1 -> 8.8 (11.5), 16.0 -> 10.4 (11.9), 19.4 -> 12.4 (12.2)
-//   2048 -> 2048 features: 4.5 -> 4.2, 5.4 -> 4.7 (11.0), 7.4 -> 5.7 (11.2), 9.6 -> 6.5 (11.2), 11.5 -> 7.6 (11.7)
-//   4864 -> 2048 features: 7.7 -> 7.1, 9.8 -> 8.2 (16.3), 14.1 -> 10.1 (12.8), 19.7 -> 12.4 (13.0), 24.6 -> 14.9 (15.2)
-//   2048 -> 9728 features: 9.9 -> 9.6, 12.6 -> 11.0 (15.7), 18.1 -> 12.9 (15.8), 23.5 -> 15.8 (16.8), 28.6 -> 18.7 (17.1)
+// Prepared weights, graph of launches over 600 MB of weights, us per launch (the library GEMM on the same card; before, with
+// batches of four steps and x in operand order, on another) at 1, 16, 32, 48, 64 rows:
+//   2048 -> 4224 features: 6.4 (12.0;  6.1),  7.4 (11.9;  8.3),  9.0 (11.9; 12.1), 10.3 (12.3; 16.0), 12.4 (12.5; 19.4)
+//   2048 -> 2048 features: 4.4 (11.0;  4.5),  4.7 (11.0;  5.4),  5.7 (11.2;  7.4),  6.3 (11.1;  9.6),  7.4 (11.6; 11.5)
+//   4864 -> 2048 features: 7.9 (17.4;  7.7),  8.2 (17.4;  9.8), 10.3 (13.8; 14.1), 13.4 (13.9; 19.7), 15.8 (16.3; 24.6)
+//   2048 -> 9728 features: 9.7 (15.9;  9.9), 11.1 (14.4; 12.6), 13.0 (14.4; 18.1), 15.2 (15.5; 23.5), 17.6 (15.5; 28.6)
+// (Shares that are no whole passes -- 4864 features are eight of nineteen steps -- pay for their selects: 0.5 to 1 us.)
 #include "common.h"
 
 #include <algorithm>

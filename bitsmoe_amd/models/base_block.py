@@ -52,11 +52,13 @@ def _super_via_operator() -> bool:
 
 
 # Rows up to which the block's two stacked GEMMs run the library's own few-rows kernel (against a copy of the stacked
-# weights in MFMA operand order) instead of the framework's GEMM.  Up to 48 rows it is the faster one at every shape
-# measured (us per launch, kernel against framework: 2048 -> 4224 features 8.8 vs 11.5 at 32 rows, 10.4 vs 11.9 at 48; 2048 -> 9728
-# 12.9 vs 15.8, 15.8 vs 16.8; 4864 -> 2048 10.1 vs 12.8, 12.4 vs 13.0).  Every workgroup reads all rows of x, so from 49 to 64 rows only
-# GEMMs of about one workgroup per CU and a contraction of at most 4096 take it: 2048 -> 2048 7.6 vs 11.7 at 64 rows, 2560 -> 2048
-# 9.0 vs 13.6, 2048 -> 4224 12.4 vs 12.2; but 2048 -> 9728 18.7 vs 17.1, and 4864 -> 2048 14.6 vs 12.9 at 56.
+# weights in MFMA operand order) instead of the framework's GEMM.  us per launch, kernel against framework on one card, seventeen
+# shapes of hidden sizes 1024 to 2048 with and without shared experts: up to 32 rows it is the faster one at all of them (at 32:
+# 2048 -> 4224 features 9.0 vs 11.9, 2048 -> 9728 13.0 vs 14.4, 4864 -> 2048 10.3 vs 13.8, 4352 -> 1536 9.7 vs 12.6); from 33 to 48 at
+# all but one (at 48: 10.3 vs 12.3, 15.2 vs 15.5, 13.4 vs 13.9; but 4352 -> 1536 12.9 vs 12.6).  Every workgroup reads all
+# rows of x, so from 49 to 64 rows only GEMMs of about one workgroup per CU and a contraction of at most 4096 take it (at 64: 2048 -> 2048
+# 7.4 vs 11.6, 2560 -> 2048 8.4 vs 13.6, 2048 -> 4224 12.4 vs 12.5); 2048 -> 9728 17.6 vs 15.5 and, at 56, 4864 -> 2048 15.4 vs 13.8,
+# 4352 -> 1536 14.8 vs 12.6.
 # BITSMOE_BLOCK_SKINNY_ROWS caps the rows, 0 switches the kernel off.
 _SKINNY_ROWS = int(_os.environ.get("BITSMOE_BLOCK_SKINNY_ROWS", "64"))
 _SKINNY_MOST_ROWS = 64            # that the kernel takes at all

@@ -184,7 +184,7 @@ int bitsmoe_router_linear_topk(const void* hidden, int32_t dtype, int64_t ld_hid
  * x_is_f32 = 1: x is fp32 (at most 16 rows, ld_x a multiple of 4) and is rounded to `dtype` on its way into the MFMA:
  * the cast of the operator's fp32 rank_accum in front of the output projection (bitsmoe/models/base_block.py:414)
  * without a pass of its own.
- * weight_is_prepared = 1 (at most 16 rows): `weight` is the copy bitsmoe_prepare_linear_weight made of W, in the order the
+ * weight_is_prepared = 1: `weight` is the copy bitsmoe_prepare_linear_weight made of W, in the order the
  * MFMA takes it ([16-column block][k-step of 32][lane][8 values]; bitsmoe_prepared_linear_weight_elements 16-bit elements):
  * every load of a wavefront is 1 KB of consecutive memory.
  * addend (may be null): fp32 [n_rows, out_features], rows ld_addend elements apart, added to the sums before the one
