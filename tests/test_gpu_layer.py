@@ -349,7 +349,8 @@ def test_block_in_one_call_equals_module_by_module(cuda_device, family, kw, toke
 
 def test_block_plan_made_twice_at_once(cuda_device, monkeypatch):
     """Two first forwards of one block at the same time may each make a native plan: both get both projections' weights
-    (the second forward runs here in the middle of the first, where a thread switch would put it).  And a router whose
+    (the second forward runs here in the middle of the first, where a thread switch would put it, and on its stream: what other
+    streams may take is for the tests of two streams and two threads below).  And a router whose
     width is not the number of experts is not taken into the stacked weights."""
     import torch
 
