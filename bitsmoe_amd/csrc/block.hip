@@ -14,6 +14,11 @@ static inline size_t align256(size_t v) { return (v + 255) / 256 * 256; }
 // Rows that the few-rows kernel takes: a call of more ends with the projection's operand (and super_out), in the caller's memory.
 constexpr int64_t PROJECT_OUT_MAX_ROWS = 64;
 
+// Rows that go into the output projection as the operator's fp32 sums (layers without a shared expert): no pass that rounds them, but
+// twice the bytes of x for every workgroup of the projection.  Graph of four 128-expert layers, us per layer, pass -> fp32 rows:
+// 20 tokens 70.5 -> 68.7, 32 tokens 72.9 -> 71.1, 48 tokens 78.4 either way, 64 tokens 83.8 -> 84.7.
+constexpr int F32_ROWS_MAX = 32;
+
 // Where the intermediates of a call sit in the workspace.
 struct BlockWorkspace {
     size_t selected, weights, rank_accum, operand, forward, forward_bytes, super_forward, super_bytes, super_out, total;
@@ -107,22 +112,24 @@ extern "C" int bitsmoe_block_forward(const bitsmoe_block_plan* p, const void* x,
         super_rc = run_super((hipStream_t)side_stream);      // (reported after the join)
     }
     float* rank_accum = (float*)(ws + w.rank_accum);
-    const int rc = bitsmoe_moe_forward_routed(p->gate, p->up, p->down, big + p->col_gate, big + p->col_up, p->act_dtype, n_tokens,
-                                              p->rank_gate, p->rank_up, ld, ld, selected, 1, weights, p->top_k, p->global_to_local,
-                                              p->n_global, p->local_to_global, p->rank_out, p->intermediate_size, 0,
-                                              BITSMOE_PATH_AUTO, rank_accum, ws + w.forward, w.forward_bytes, nullptr, stream);
     // what the output projection reads: the cast sums beside the shared expert's activations; a few fp32 rows without a
     // shared expert go into it as they are
-    const bool f32_rows = project_out && p->shared_intermediate == 0 && n_tokens <= 16;
+    const bool f32_rows = project_out && p->shared_intermediate == 0 && n_tokens <= F32_ROWS_MAX &&
+                          skinny_f32_rows_possible(n_tokens, p->rank_out, p->w_out_prepared);
     void* operand = project_out ? (void*)(ws + w.operand) : out;
     const int k_out = p->rank_out + p->shared_intermediate;
+    CastRows cast = {operand, k_out, false};
+    const int rc = forward_routed_cast(p->gate, p->up, p->down, big + p->col_gate, big + p->col_up, p->act_dtype, n_tokens, p->rank_gate,
+                                       p->rank_up, ld, ld, selected, 1, weights, p->top_k, p->global_to_local, p->n_global,
+                                       p->local_to_global, p->rank_out, p->intermediate_size, rank_accum, ws + w.forward,
+                                       w.forward_bytes, f32_rows ? nullptr : &cast, stream);
     int finish_rc = BITSMOE_OK;
-    if (rc == BITSMOE_OK && !f32_rows) {
+    if (rc == BITSMOE_OK && !f32_rows && !(cast.done && p->shared_intermediate == 0)) {
         const bool shared = p->shared_intermediate > 0;
-        finish_rc = bitsmoe_block_finish(rank_accum, n_tokens, p->rank_out, shared ? big + p->col_shared_gate : nullptr,
-                                         shared ? big + p->col_shared_up : nullptr, ld, p->shared_intermediate,
-                                         shared && p->col_shared_logit >= 0 ? big + p->col_shared_logit : nullptr, ld, p->act_dtype,
-                                         operand, k_out, stream);
+        finish_rc = block_finish(rank_accum, n_tokens, p->rank_out, shared ? big + p->col_shared_gate : nullptr,
+                                 shared ? big + p->col_shared_up : nullptr, ld, p->shared_intermediate,
+                                 shared && p->col_shared_logit >= 0 ? big + p->col_shared_logit : nullptr, ld, p->act_dtype,
+                                 operand, k_out, cast.done, stream);
     }
     if (super && side_stream)      // (joined whatever happened in between: the side stream may hold launches)
         BITSMOE_TRY(stream_after(st, (hipStream_t)side_stream));
@@ -131,9 +138,9 @@ extern "C" int bitsmoe_block_forward(const bitsmoe_block_plan* p, const void* x,
     BITSMOE_TRY(super_rc);
     if (super && !side_stream) BITSMOE_TRY(run_super(st));
     if (project_out)
-        BITSMOE_TRY(bitsmoe_skinny_linear(f32_rows ? (const void*)rank_accum : operand, p->act_dtype, f32_rows ? 1 : 0, k_out, p->w_out,
-                                          p->w_out_prepared, n_tokens, k_out, p->hidden, out, p->hidden, super ? sup : nullptr,
-                                          p->hidden, stream));
+        BITSMOE_TRY(skinny_linear(f32_rows ? (const void*)rank_accum : operand, p->act_dtype, f32_rows ? 1 : 0, k_out, p->w_out,
+                                  p->w_out_prepared, n_tokens, k_out, p->hidden, out, p->hidden, super ? sup : nullptr, p->hidden,
+                                  F32_ROWS_MAX, stream));
 #undef BITSMOE_TRY
     return BITSMOE_OK;
 }

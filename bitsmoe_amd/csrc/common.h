@@ -168,11 +168,33 @@ int route_with_jobs(const void* selected, int32_t ids_are_i64, const float* weig
                     int32_t n_global, int64_t n_tokens, int32_t top_k, int32_t n_packed, int32_t* token_indices,
                     int32_t* expert_offsets, float* route_flat, void* workspace, size_t workspace_bytes,
                     const RouteSideJobs* jobs, int* jobs_done, hipStream_t st);
+// Where a caller that only goes on with the sums rounded to the activation dtype takes them: rows of `rank_out` 16-bit values, `ld`
+// apart.  The grouped GEMM's combine then writes these instead of rank_accum and says so (`done`).
+struct CastRows {
+    void* out;
+    int64_t ld;
+    bool done;
+};
 // front_done: MFMA_FRONT_* bits of what an earlier launch on the stream has already produced in `workspace`.
 int launch_forward_mfma(const bitsmoe_matset* gate, const bitsmoe_matset* up, const bitsmoe_matset* down,
                         const void* h_gate, const void* h_up, int act_dtype, int64_t T, int Rg, int Ru, int64_t ldg_in,
                         int64_t ldu_in, const int32_t* tok, const int32_t* off, const float* rw, int64_t A, int rank_out,
-                        int I, float* rank_accum, void* workspace, int front_done, bitsmoe_profile* prof, hipStream_t st);
+                        int I, float* rank_accum, void* workspace, int front_done, CastRows* cast, bitsmoe_profile* prof, hipStream_t st);
+// bitsmoe_moe_forward_routed with `cast` (may be null); `path` is AUTO, the activation SiLU, no profile.
+int forward_routed_cast(const bitsmoe_matset* gate, const bitsmoe_matset* up, const bitsmoe_matset* down, const void* h_gate, const void* h_up,
+                        int32_t act_dtype, int64_t n_tokens, int32_t rank_gate, int32_t rank_up, int64_t ld_gate, int64_t ld_up,
+                        const void* selected, int32_t ids_are_i64, const float* weights, int32_t top_k, const int32_t* global_to_local,
+                        int32_t n_global, const int32_t* local_to_global, int32_t rank_out, int32_t intermediate_size,
+                        float* rank_accum, void* workspace, size_t workspace_bytes, CastRows* cast, void* stream);
+// bitsmoe_block_finish; shared_only: the shared expert's columns alone (the others are there already).
+int block_finish(const float* rank_accum, int64_t n_tokens, int32_t rank_out, const void* shared_gate_out, const void* shared_up_out,
+                 int64_t ld_shared, int32_t shared_intermediate, const void* shared_gate_logit, int64_t ld_gate_logit, int32_t act_dtype,
+                 void* out, int64_t ld_out, bool shared_only, void* stream);
+// bitsmoe_skinny_linear; fp32 rows up to `f32_rows` of them where skinny_f32_rows_possible says so.
+int skinny_linear(const void* x, int32_t dtype, int32_t x_is_f32, int64_t ld_x, const void* weight, int32_t weight_is_prepared,
+                  int64_t n_rows, int32_t in_features, int32_t out_features, void* out, int64_t ld_out, const float* addend,
+                  int64_t ld_addend, int f32_rows, void* stream);
+bool skinny_f32_rows_possible(int64_t n_rows, int32_t in_features, int32_t weight_is_prepared);
 
 // bf16 -> f16, eight elements at a time: group `i` of `total = T * (ld / 8)` groups of one projection.
 __device__ inline void convert_bf16_group(const uint16_t* __restrict__ src, uint16_t* __restrict__ dst, int64_t stride,

@@ -115,7 +115,7 @@ static int forward_strided_impl(const bitsmoe_matset* gate, const bitsmoe_matset
                                 const int32_t* token_indices, const int32_t* expert_offsets, const float* route_w,
                                 int64_t n_assign, int32_t rank_out, int32_t intermediate_size, int32_t act_type,
                                 int32_t path, float* rank_accum, void* workspace, size_t workspace_bytes, int front_done,
-                                bitsmoe_profile* profile, hipStream_t st);
+                                CastRows* cast, bitsmoe_profile* profile, hipStream_t st);
 
 extern "C" int bitsmoe_moe_forward_strided(const bitsmoe_matset* gate, const bitsmoe_matset* up,
                                            const bitsmoe_matset* down, const void* h_gate, const void* h_up,
@@ -128,7 +128,7 @@ extern "C" int bitsmoe_moe_forward_strided(const bitsmoe_matset* gate, const bit
                                            bitsmoe_profile* profile, void* stream) {
     return forward_strided_impl(gate, up, down, h_gate, h_up, act_dtype, n_tokens, rank_gate, rank_up, ld_gate, ld_up,
                                 token_indices, expert_offsets, route_w, n_assign, rank_out, intermediate_size, act_type, path,
-                                rank_accum, workspace, workspace_bytes, 0, profile, (hipStream_t)stream);
+                                rank_accum, workspace, workspace_bytes, 0, nullptr, profile, (hipStream_t)stream);
 }
 
 static int forward_strided_impl(const bitsmoe_matset* gate, const bitsmoe_matset* up, const bitsmoe_matset* down,
@@ -137,7 +137,7 @@ static int forward_strided_impl(const bitsmoe_matset* gate, const bitsmoe_matset
                                 const int32_t* token_indices, const int32_t* expert_offsets, const float* route_w,
                                 int64_t n_assign, int32_t rank_out, int32_t intermediate_size, int32_t act_type,
                                 int32_t path, float* rank_accum, void* workspace, size_t workspace_bytes, int front_done,
-                                bitsmoe_profile* profile, hipStream_t st) {
+                                CastRows* cast, bitsmoe_profile* profile, hipStream_t st) {
     BITSMOE_REQUIRE(gate && up && down, "matrix sets must not be null");
     BITSMOE_REQUIRE(act_type == 0, "only SiLU act_type=0 is currently supported");
     BITSMOE_REQUIRE(act_dtype == BITSMOE_DT_F16 || act_dtype == BITSMOE_DT_BF16, "act_dtype must be f16 (0) or bf16 (1)");
@@ -190,7 +190,7 @@ static int forward_strided_impl(const bitsmoe_matset* gate, const bitsmoe_matset
     if (chosen == BITSMOE_PATH_MFMA)
         return launch_forward_mfma(gate, up, down, h_gate, h_up, act_dtype, n_tokens, rank_gate, rank_up, ld_gate, ld_up,
                                    token_indices, expert_offsets, route_w, n_assign, rank_out, cols, rank_accum,
-                                   workspace, front_done, profile, st);
+                                   workspace, front_done, cast, profile, st);
     const size_t inter = align_up((size_t)n_assign * (size_t)cols * sizeof(float), 256);
     float* G = (float*)workspace;
     float* U = (float*)((char*)workspace + inter);
@@ -244,14 +244,14 @@ extern "C" int bitsmoe_forward_decode_is_fused(const bitsmoe_matset* gate, const
                ? 1 : 0;
 }
 
-extern "C" int bitsmoe_moe_forward_routed(const bitsmoe_matset* gate, const bitsmoe_matset* up, const bitsmoe_matset* down,
-                                          const void* h_gate, const void* h_up, int32_t act_dtype, int64_t n_tokens,
-                                          int32_t rank_gate, int32_t rank_up, int64_t ld_gate, int64_t ld_up,
-                                          const void* selected, int32_t ids_are_i64, const float* weights, int32_t top_k,
-                                          const int32_t* global_to_local, int32_t n_global,
-                                          const int32_t* local_to_global, int32_t rank_out, int32_t intermediate_size,
-                                          int32_t act_type, int32_t path, float* rank_accum, void* workspace,
-                                          size_t workspace_bytes, bitsmoe_profile* profile, void* stream) {
+static int forward_routed_impl(const bitsmoe_matset* gate, const bitsmoe_matset* up, const bitsmoe_matset* down,
+                               const void* h_gate, const void* h_up, int32_t act_dtype, int64_t n_tokens,
+                               int32_t rank_gate, int32_t rank_up, int64_t ld_gate, int64_t ld_up,
+                               const void* selected, int32_t ids_are_i64, const float* weights, int32_t top_k,
+                               const int32_t* global_to_local, int32_t n_global,
+                               const int32_t* local_to_global, int32_t rank_out, int32_t intermediate_size,
+                               int32_t act_type, int32_t path, float* rank_accum, void* workspace,
+                               size_t workspace_bytes, CastRows* cast, bitsmoe_profile* profile, void* stream) {
     hipStream_t st = (hipStream_t)stream;
     BITSMOE_REQUIRE(gate && up && down, "matrix sets must not be null");
     BITSMOE_REQUIRE(top_k > 0 && n_tokens >= 0, "n_tokens must be >= 0 and top_k > 0");
@@ -320,7 +320,31 @@ extern "C" int bitsmoe_moe_forward_routed(const bitsmoe_matset* gate, const bits
     if (rc != BITSMOE_OK) return rc;
     return forward_strided_impl(gate, up, down, h_gate, h_up, act_dtype, n_tokens, rank_gate, rank_up, ld_gate, ld_up, tok, off,
                                 rw, n_flat, rank_out, intermediate_size, act_type, path, rank_accum, workspace,
-                                align_up(fwd, 256), front_done, profile, st);
+                                align_up(fwd, 256), front_done, cast, profile, st);
+}
+
+extern "C" int bitsmoe_moe_forward_routed(const bitsmoe_matset* gate, const bitsmoe_matset* up, const bitsmoe_matset* down,
+                                          const void* h_gate, const void* h_up, int32_t act_dtype, int64_t n_tokens,
+                                          int32_t rank_gate, int32_t rank_up, int64_t ld_gate, int64_t ld_up,
+                                          const void* selected, int32_t ids_are_i64, const float* weights, int32_t top_k,
+                                          const int32_t* global_to_local, int32_t n_global,
+                                          const int32_t* local_to_global, int32_t rank_out, int32_t intermediate_size,
+                                          int32_t act_type, int32_t path, float* rank_accum, void* workspace,
+                                          size_t workspace_bytes, bitsmoe_profile* profile, void* stream) {
+    return forward_routed_impl(gate, up, down, h_gate, h_up, act_dtype, n_tokens, rank_gate, rank_up, ld_gate, ld_up, selected, ids_are_i64,
+                               weights, top_k, global_to_local, n_global, local_to_global, rank_out, intermediate_size, act_type, path,
+                               rank_accum, workspace, workspace_bytes, nullptr, profile, stream);
+}
+
+int bitsmoe::forward_routed_cast(const bitsmoe_matset* gate, const bitsmoe_matset* up, const bitsmoe_matset* down, const void* h_gate,
+                                 const void* h_up, int32_t act_dtype, int64_t n_tokens, int32_t rank_gate, int32_t rank_up,
+                                 int64_t ld_gate, int64_t ld_up, const void* selected, int32_t ids_are_i64, const float* weights,
+                                 int32_t top_k, const int32_t* global_to_local, int32_t n_global, const int32_t* local_to_global,
+                                 int32_t rank_out, int32_t intermediate_size, float* rank_accum, void* workspace,
+                                 size_t workspace_bytes, CastRows* cast, void* stream) {
+    return forward_routed_impl(gate, up, down, h_gate, h_up, act_dtype, n_tokens, rank_gate, rank_up, ld_gate, ld_up, selected, ids_are_i64,
+                               weights, top_k, global_to_local, n_global, local_to_global, rank_out, intermediate_size, 0,
+                               BITSMOE_PATH_AUTO, rank_accum, workspace, workspace_bytes, cast, nullptr, stream);
 }
 
 extern "C" size_t bitsmoe_static_scratch_bytes(void) { return (size_t)BITSMOE_STATIC_SCRATCH_BYTES; }

@@ -927,6 +927,9 @@ constexpr int CB_SORT = 256;     // list entries ordered at a time
 // row, so rank_accum needs no zero fill.  IDENTITY: rank_idx_e[r] == r in every expert, and a
 // thread keeps its eight columns in registers; otherwise the row is accumulated in LDS, one
 // assignment after the other.
+// `cast`: the sums go there, rounded to bf16 (cast_bf16) or f16, eight columns at a time, and not into rank_accum: a block's output
+// projection reads them in the activation dtype (at 4096 tokens of 2048 ranks: 34 MB less written here, and no
+// pass that reads 34 MB and writes 17: the 128-expert layer 558 -> 541 us).
 template <bool IDENTITY>
 __global__ __launch_bounds__(256) void k_combine_tokens(const FastExpert* __restrict__ down_fe, int max_slabs,
                                                         const _Float16* __restrict__ y, int ldy,
@@ -934,7 +937,8 @@ __global__ __launch_bounds__(256) void k_combine_tokens(const FastExpert* __rest
                                                         const int32_t* __restrict__ token_count,
                                                         const int2* __restrict__ token_list,
                                                         const float* __restrict__ route_w, int rank_out,
-                                                        float* __restrict__ rank_accum) {
+                                                        float* __restrict__ rank_accum, uint16_t* __restrict__ cast, int64_t ld_cast,
+                                                        int cast_bf16) {
     __shared__ __attribute__((aligned(16))) float out_s[IDENTITY ? 4 : CB_COLS];
     __shared__ int2 raw_s[CB_SORT];
     __shared__ const _Float16* y_s[CB_SORT];
@@ -1018,13 +1022,34 @@ __global__ __launch_bounds__(256) void k_combine_tokens(const FastExpert* __rest
                 }
             }
         }
-        if (IDENTITY) {
+        auto put_cast = [&](int c, const float (&v)[8]) {
+            u32x4 o;
 #pragma unroll
-            for (int k = 0; k < 8; ++k)
-                if (tid * 8 + k < cols) out_row[c0 + tid * 8 + k] = acc[k];
+            for (int k = 0; k < 4; ++k)
+                o[k] = cast_bf16 ? (uint32_t)to_operand<true>(v[2 * k]) | ((uint32_t)to_operand<true>(v[2 * k + 1]) << 16)
+                                 : f16_pair(v[2 * k], v[2 * k + 1]);
+            *reinterpret_cast<u32x4*>(cast + (int64_t)t * ld_cast + c) = o;
+        };
+        if (IDENTITY) {
+            if (cast) {      // (rank_out is a multiple of eight then)
+                if (tid * 8 < cols) put_cast(c0 + tid * 8, acc);
+            } else {
+#pragma unroll
+                for (int k = 0; k < 8; ++k)
+                    if (tid * 8 + k < cols) out_row[c0 + tid * 8 + k] = acc[k];
+            }
         } else {
             __syncthreads();
-            for (int i = tid; i < cols; i += 256) out_row[c0 + i] = out_s[i];
+            if (cast) {
+                for (int i = 8 * tid; i < cols; i += 8 * 256) {
+                    float v[8];
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) v[k] = out_s[i + k];
+                    put_cast(c0 + i, v);
+                }
+            } else {
+                for (int i = tid; i < cols; i += 256) out_row[c0 + i] = out_s[i];
+            }
             __syncthreads();
         }
     }
@@ -1150,7 +1175,7 @@ bool mfma_front_jobs(const bitsmoe_matset* gate, const bitsmoe_matset* up, const
 int launch_forward_mfma(const bitsmoe_matset* gate, const bitsmoe_matset* up, const bitsmoe_matset* down,
                         const void* h_gate, const void* h_up, int act_dtype, int64_t T, int Rg, int Ru, int64_t ldg_in,
                         int64_t ldu_in, const int32_t* tok, const int32_t* off, const float* rw, int64_t A, int rank_out,
-                        int I, float* rank_accum, void* workspace, int front_done, bitsmoe_profile* prof, hipStream_t st) {
+                        int I, float* rank_accum, void* workspace, int front_done, CastRows* cast, bitsmoe_profile* prof, hipStream_t st) {
     const int E = gate->n_experts;
     const int n_tiles = gate->n_tiles;
     const int tile_rows = mtile_rows(A, E);
@@ -1258,14 +1283,13 @@ int launch_forward_mfma(const bitsmoe_matset* gate, const bitsmoe_matset* up, co
                            down->d_fast_experts, down->d_fast_slabs, down->prep_max_slabs, z, Ubuf, mtiles, n_mtiles, tok, slot, token_start,
                            token_list, I, n_tiles, n_groups, y, ldy);
         record(prof, 4, st);
-        if (down->rank_identity)
-            hipLaunchKernelGGL(k_combine_tokens<true>, dim3((unsigned)T), dim3(256), 0, st, down->d_fast_experts,
-                               down->prep_max_slabs, y, ldy, token_start, counted ? token_count : nullptr, token_list, rw,
-                               rank_out, rank_accum);
-        else
-            hipLaunchKernelGGL(k_combine_tokens<false>, dim3((unsigned)T), dim3(256), 0, st, down->d_fast_experts,
-                               down->prep_max_slabs, y, ldy, token_start, counted ? token_count : nullptr, token_list, rw,
-                               rank_out, rank_accum);
+        // (wide rows add to the fp32 sums behind the combine)
+        const bool to_cast = cast && !has_wide_rows(down) && rank_out % 8 == 0 && cast->ld % 8 == 0 && ((uintptr_t)cast->out & 15) == 0;
+        hipLaunchKernelGGL((down->rank_identity ? k_combine_tokens<true> : k_combine_tokens<false>), dim3((unsigned)T), dim3(256), 0, st,
+                           down->d_fast_experts, down->prep_max_slabs, y, ldy, token_start, counted ? token_count : nullptr, token_list, rw,
+                           rank_out, rank_accum, to_cast ? (uint16_t*)cast->out : nullptr, to_cast ? cast->ld : 0,
+                           act_dtype == BITSMOE_DT_BF16 ? 1 : 0);
+        if (to_cast) cast->done = true;
         BITSMOE_HIP_TRY(hipGetLastError());
         if (has_wide_rows(down)) {      // (behind the combine, which writes every element of rank_accum)
             const int rc = launch_wide_down(down, z, reinterpret_cast<const float*>(Ubuf), WIDE_Z_RECORDS, 1, 0, tok, off, rw, A, I, rank_out, rank_accum, st);

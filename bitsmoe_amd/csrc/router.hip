@@ -466,8 +466,8 @@ template <bool BF16>
 __global__ __launch_bounds__(256) void k_block_finish(const float* __restrict__ rank_accum, int64_t T, int R,
                                                       const uint16_t* __restrict__ a, const uint16_t* __restrict__ b,
                                                       int64_t ld_ab, int I_sh, const uint16_t* __restrict__ g, int64_t ld_g,
-                                                      uint16_t* __restrict__ out, int64_t ld_out) {
-    const int per_row = (R + I_sh) >> 3;
+                                                      uint16_t* __restrict__ out, int64_t ld_out, int c_first) {
+    const int per_row = (R + I_sh - c_first) >> 3;      // (columns from c_first on)
     const int64_t total = T * per_row;
     auto to_f32 = [](uint16_t v) {
         if constexpr (BF16) return __uint_as_float((uint32_t)v << 16);
@@ -481,7 +481,7 @@ __global__ __launch_bounds__(256) void k_block_finish(const float* __restrict__ 
     typedef float f4 __attribute__((ext_vector_type(4)));
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256) {
         const int64_t t = i / per_row;
-        const int c = (int)(i - t * per_row) * 8;
+        const int c = c_first + (int)(i - t * per_row) * 8;
         uint16_t o[8];
         if (c < R) {
             const f4 lo = *reinterpret_cast<const f4*>(rank_accum + t * R + c);
@@ -517,6 +517,13 @@ extern "C" int bitsmoe_block_finish(const float* rank_accum, int64_t n_tokens, i
                                     const void* shared_up_out, int64_t ld_shared, int32_t shared_intermediate,
                                     const void* shared_gate_logit, int64_t ld_gate_logit, int32_t act_dtype, void* out,
                                     int64_t ld_out, void* stream) {
+    return bitsmoe::block_finish(rank_accum, n_tokens, rank_out, shared_gate_out, shared_up_out, ld_shared, shared_intermediate,
+                                 shared_gate_logit, ld_gate_logit, act_dtype, out, ld_out, false, stream);
+}
+
+int bitsmoe::block_finish(const float* rank_accum, int64_t n_tokens, int32_t rank_out, const void* shared_gate_out,
+                          const void* shared_up_out, int64_t ld_shared, int32_t shared_intermediate, const void* shared_gate_logit,
+                          int64_t ld_gate_logit, int32_t act_dtype, void* out, int64_t ld_out, bool shared_only, void* stream) {
     BITSMOE_REQUIRE(n_tokens >= 0 && rank_out > 0 && shared_intermediate >= 0, "negative size");
     BITSMOE_REQUIRE(rank_out % 8 == 0 && shared_intermediate % 8 == 0, "rank_out and shared_intermediate must be multiples of 8");
     BITSMOE_REQUIRE(act_dtype == BITSMOE_DT_F16 || act_dtype == BITSMOE_DT_BF16, "act_dtype must be f16 (0) or bf16 (1)");
@@ -531,16 +538,18 @@ extern "C" int bitsmoe_block_finish(const float* rank_accum, int64_t n_tokens, i
                         "shared expert operands must be 16-byte aligned");
     }
     hipStream_t st = (hipStream_t)stream;
-    const int64_t total = n_tokens * ((rank_out + shared_intermediate) / 8);
+    const int c_first = shared_only ? rank_out : 0;
+    const int64_t total = n_tokens * ((rank_out + shared_intermediate - c_first) / 8);
+    if (total == 0) return BITSMOE_OK;
     const unsigned blocks = (unsigned)std::min<int64_t>((total + 255) / 256, 4096);
     if (act_dtype == BITSMOE_DT_BF16)
         hipLaunchKernelGGL(k_block_finish<true>, dim3(blocks), dim3(256), 0, st, rank_accum, n_tokens, rank_out,
                            (const uint16_t*)shared_gate_out, (const uint16_t*)shared_up_out, ld_shared, shared_intermediate,
-                           (const uint16_t*)shared_gate_logit, ld_gate_logit, (uint16_t*)out, ld_out);
+                           (const uint16_t*)shared_gate_logit, ld_gate_logit, (uint16_t*)out, ld_out, c_first);
     else
         hipLaunchKernelGGL(k_block_finish<false>, dim3(blocks), dim3(256), 0, st, rank_accum, n_tokens, rank_out,
                            (const uint16_t*)shared_gate_out, (const uint16_t*)shared_up_out, ld_shared, shared_intermediate,
-                           (const uint16_t*)shared_gate_logit, ld_gate_logit, (uint16_t*)out, ld_out);
+                           (const uint16_t*)shared_gate_logit, ld_gate_logit, (uint16_t*)out, ld_out, c_first);
     BITSMOE_HIP_TRY(hipGetLastError());
     return BITSMOE_OK;
 }

@@ -39,7 +39,7 @@ __device__ __forceinline__ void static_for_pieces(F&& f, std::integer_sequence<i
 }
 
 // XF32: x is fp32 and is rounded to the 16-bit type on its way into the MFMA (the cast of the operator's fp32 output in
-// front of the output projection, bitsmoe/models/base_block.py:414, without a pass of its own); one 16-row block only.
+// front of the output projection, bitsmoe/models/base_block.py:414, without a pass of its own).
 // PREP: W was re-laid out once (bitsmoe_prepare_linear_weight) into the order the MFMA takes it: [16-column block]
 // [k-step of 32][lane][8 values], so that a wavefront's load is 1 KB of consecutive memory instead of sixteen 64-byte
 // pieces of sixteen rows.
@@ -48,8 +48,8 @@ template <bool BF16, int NMB, int NW, int MAXS, bool XF32, bool PREP, bool TURN,
 __global__ __launch_bounds__(64 * NW) void k_skinny_linear(const void* __restrict__ x, int64_t ld_x, const uint16_t* __restrict__ w,
                                                            int T, int K, int N, uint16_t* __restrict__ out, int64_t ld_out,
                                                            const float* __restrict__ addend, int64_t ld_add) {
-    static_assert((!XF32 && TURN) || NMB == 1, "fp32 rows and few rows: one block of 16 rows");
-    constexpr int G = NMB <= 2 ? 4 : 2;                // k-steps per piece of x
+    static_assert(TURN || NMB == 1, "few rows: one block of 16 rows");
+    constexpr int G = NMB <= (XF32 ? 1 : 2) ? 4 : 2;   // k-steps per piece of x
     static_assert(MAXS % G == 0, "whole pieces");
     constexpr int EB = XF32 ? 4 : 2;                   // bytes of an element of x
     constexpr int CPR = 32 * G * EB / 16;              // 16-byte chunks per row of a piece
@@ -239,8 +239,21 @@ extern "C" int bitsmoe_prepare_linear_weight(const void* weight, int32_t in_feat
 extern "C" int bitsmoe_skinny_linear(const void* x, int32_t dtype, int32_t x_is_f32, int64_t ld_x, const void* weight,
                                      int32_t weight_is_prepared, int64_t n_rows, int32_t in_features, int32_t out_features,
                                      void* out, int64_t ld_out, const float* addend, int64_t ld_addend, void* stream) {
+    return bitsmoe::skinny_linear(x, dtype, x_is_f32, ld_x, weight, weight_is_prepared, n_rows, in_features, out_features, out, ld_out,
+                                  addend, ld_addend, 16, stream);
+}
+
+// More than sixteen fp32 rows: prepared weights and four wavefronts (their pieces of x fill the LDS).
+bool bitsmoe::skinny_f32_rows_possible(int64_t n_rows, int32_t in_features, int32_t weight_is_prepared) {
+    return n_rows <= 16 || (n_rows <= 64 && weight_is_prepared != 0 && in_features <= 80 * 32);
+}
+
+int bitsmoe::skinny_linear(const void* x, int32_t dtype, int32_t x_is_f32, int64_t ld_x, const void* weight, int32_t weight_is_prepared,
+                           int64_t n_rows, int32_t in_features, int32_t out_features, void* out, int64_t ld_out, const float* addend,
+                           int64_t ld_addend, int f32_rows, void* stream) {
     BITSMOE_REQUIRE(dtype == BITSMOE_DT_F16 || dtype == BITSMOE_DT_BF16, "dtype must be f16 (0) or bf16 (1)");
-    BITSMOE_REQUIRE(n_rows >= 0 && n_rows <= (x_is_f32 ? 16 : 64), "n_rows must be in [0, 64] (fp32 rows: [0, 16])");
+    BITSMOE_REQUIRE(n_rows >= 0 && n_rows <= (x_is_f32 ? f32_rows : 64), "n_rows must be in [0, 64] (fp32 rows: [0, %d])", f32_rows);
+    BITSMOE_REQUIRE(!x_is_f32 || skinny_f32_rows_possible(n_rows, in_features, weight_is_prepared), "fp32 rows past 16 need prepared weights");
     BITSMOE_REQUIRE(in_features >= 128 && in_features % 128 == 0, "in_features must be a positive multiple of 128");
     BITSMOE_REQUIRE(out_features >= 2 && out_features % 2 == 0, "out_features must be even");
     BITSMOE_REQUIRE(ld_x >= in_features && ld_x % (x_is_f32 ? 4 : 8) == 0,
@@ -282,7 +295,13 @@ extern "C" int bitsmoe_skinny_linear(const void* x, int32_t dtype, int32_t x_is_
     using S20 = integral_constant<int, 20>;
     auto by_share = [&](auto bf_c, auto nmb_c, auto xf_c, auto turn_c) {
         constexpr bool twenty = !(decltype(xf_c)::value && !decltype(turn_c)::value);      // (fp32 operands of twenty steps do not fit the registers)
-        if (!weight_is_prepared) {      // (in passes of sixteen steps: the same sums in the same order)
+        constexpr bool many_f32 = decltype(xf_c)::value && decltype(nmb_c)::value > 1;
+        if constexpr (many_f32) {       // (prepared, four wavefronts: skinny_f32_rows_possible)
+            if (share <= 8) run(bf_c, nmb_c, W4{}, S8{}, xf_c, Yes{}, turn_c);
+            else if (share <= 12) run(bf_c, nmb_c, W4{}, S12{}, xf_c, Yes{}, turn_c);
+            else if (share <= 16) run(bf_c, nmb_c, W4{}, S16{}, xf_c, Yes{}, turn_c);
+            else run(bf_c, nmb_c, W4{}, S20{}, xf_c, Yes{}, turn_c);
+        } else if (!weight_is_prepared) {      // (in passes of sixteen steps: the same sums in the same order)
             if (nw == 8) run(bf_c, nmb_c, W8{}, S16{}, xf_c, No{}, turn_c); else run(bf_c, nmb_c, W4{}, S16{}, xf_c, No{}, turn_c);
         } else if (nw == 8) {
             if (share <= 16 || !twenty) run(bf_c, nmb_c, W8{}, S16{}, xf_c, Yes{}, turn_c);
@@ -302,7 +321,10 @@ extern "C" int bitsmoe_skinny_linear(const void* x, int32_t dtype, int32_t x_is_
         // features at eight rows 8.9 against 7.9
         if (n_rows <= 4 && x_is_f32 && share <= 16) by_share(bf_c, One{}, Yes{}, No{});
         else if (n_rows <= 4 && !x_is_f32) by_share(bf_c, One{}, No{}, No{});
-        else if (x_is_f32) by_share(bf_c, One{}, Yes{}, Yes{});
+        else if (x_is_f32 && nmb == 1) by_share(bf_c, One{}, Yes{}, Yes{});
+        else if (x_is_f32 && nmb == 2) by_share(bf_c, integral_constant<int, 2>{}, Yes{}, Yes{});
+        else if (x_is_f32 && nmb == 3) by_share(bf_c, integral_constant<int, 3>{}, Yes{}, Yes{});
+        else if (x_is_f32) by_share(bf_c, integral_constant<int, 4>{}, Yes{}, Yes{});
         else if (nmb == 1) by_share(bf_c, One{}, No{}, Yes{});
         else if (nmb == 2) by_share(bf_c, integral_constant<int, 2>{}, No{}, Yes{});
         else if (nmb == 3) by_share(bf_c, integral_constant<int, 3>{}, No{}, Yes{});

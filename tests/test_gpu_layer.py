@@ -347,6 +347,31 @@ def test_block_in_one_call_equals_module_by_module(cuda_device, family, kw, toke
         assert float((a - b).abs().max()) <= 1e-2 * float(b.abs().max())
 
 
+@pytest.mark.parametrize("tokens", [17, 32, 33, 200])      # fp32 rows into the output projection, the cast pass, the combine's cast
+@pytest.mark.parametrize("layout", ["uniform", "checkpoint"])      # output ranks in order, and scattered (the row summed in LDS)
+@pytest.mark.parametrize("family,kw", [("qwen3moe", {}), ("qwen3next", {"shared_intermediate": 128})])
+@pytest.mark.parametrize("dtype_name", ["bfloat16", "float16"])
+def test_block_sums_reach_the_output_projection_in_the_activation_type(cuda_device, dtype_name, family, kw, layout, tokens, monkeypatch):
+    """However the operator's fp32 sums are rounded on their way into the output projection, the block equals its module-by-module
+    form (both round along the way: 1e-2, as in the test above)."""
+    import torch
+
+    from bitsmoe_amd.models.base_block import BitsMoE_BaseSparseMoeBlock
+    from bitsmoe_amd.synth import make_layer
+
+    dtype = getattr(torch, dtype_name)
+    block = make_layer(_small_spec(family, **kw), device=cuda_device, dtype=dtype, seed=33, s_mode="rand", layout=layout)
+    block.prepare_runtime_fastpath(warmup=True)
+    g = torch.Generator().manual_seed(tokens)
+    x = torch.randn((1, tokens, block.spec.hidden_size), generator=g).to(dtype).to(cuda_device)
+    first = lambda out: (out[0] if isinstance(out, tuple) else out).float()
+    with torch.no_grad():
+        got = first(block(x))
+        monkeypatch.setattr(BitsMoE_BaseSparseMoeBlock, "_FUSED_BLOCK", False)
+        apart = first(block(x))
+    assert float((got - apart).abs().max()) <= 1e-2 * float(apart.abs().max())
+
+
 def test_block_plan_made_twice_at_once(cuda_device, monkeypatch):
     """Two first forwards of one block at the same time may each make a native plan: both get both projections' weights
     (the second forward runs here in the middle of the first, where a thread switch would put it, and on its stream: what other
