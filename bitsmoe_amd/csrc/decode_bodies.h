@@ -850,9 +850,13 @@ __device__ __forceinline__ void build_z_records(const float* __restrict__ G, con
     const uint32_t pieces = (uint32_t)(nt + 1) >> 1, units = (uint32_t)n_a * pieces;
     struct Batch {
         int row[ZUNITS], col[ZUNITS];      // assignment and first column of the units
-        f32x4 g[ZUNITS], u[ZUNITS];
+        f32x4 g0, g1, g2, g3, u0, u1, u2, u3;      // sums of the units, or partial results 0, 1, 2 and 3 of ONE unit
         u32x2 hi[ZUNITS], lo[ZUNITS];
     };
+    // (the gate/up kernel split the contraction where there are few workgroups: then a batch is one unit, and its partial results come
+    // together instead of one round trip after the other)
+    const bool parts = !ZREADY && n_part > 1;
+    const uint32_t batch = parts ? 1u : (uint32_t)ZUNITS;
     auto request = [&](Batch& b, uint32_t u0) {
 #pragma unroll
         for (int k = 0; k < ZUNITS; ++k) {
@@ -861,48 +865,59 @@ __device__ __forceinline__ void build_z_records(const float* __restrict__ G, con
             b.row[k] = __builtin_amdgcn_readfirstlane(r);
             b.col[k] = __builtin_amdgcn_readfirstlane(256 * (u - r * pieces));
         }
+        auto column = [&](int k) { return c_begin + min(b.col[k] + 4 * lane, cols - 4); };      // (past the end: the last four again)
+        if constexpr (ZREADY) {
 #pragma unroll
-        for (int k = 0; k < ZUNITS; ++k) {
-            const int c = c_begin + min(b.col[k] + 4 * lane, cols - 4);      // (past the end: the last four again)
-            if constexpr (ZREADY) {
-                const int64_t at = (int64_t)(a0 + b.row[k]) * I + c;
+            for (int k = 0; k < ZUNITS; ++k) {
+                const int64_t at = (int64_t)(a0 + b.row[k]) * I + column(k);
                 b.hi[k] = *reinterpret_cast<const u32x2*>(reinterpret_cast<const uint16_t*>(G) + at);
                 b.lo[k] = *reinterpret_cast<const u32x2*>(reinterpret_cast<const uint16_t*>(U) + at);
-            } else {
-                const int64_t at = (int64_t)as.row(a0 + b.row[k]) * I + c;
-                b.g[k] = *reinterpret_cast<const f32x4*>(G + at);
-                b.u[k] = *reinterpret_cast<const f32x4*>(U + at);
             }
-        }
-        if constexpr (!ZREADY) {
-            // (the gate/up kernel split the contraction: the sums are totals of partial results)
-            for (int p = 1; p < n_part; ++p) {
-                f32x4 g[ZUNITS], u[ZUNITS];
-#pragma unroll
-                for (int k = 0; k < ZUNITS; ++k) {
-                    const int c = c_begin + min(b.col[k] + 4 * lane, cols - 4);
-                    const int64_t at = (int64_t)as.row(a0 + b.row[k]) * I + c + p * part_stride;
-                    g[k] = *reinterpret_cast<const f32x4*>(G + at);
-                    u[k] = *reinterpret_cast<const f32x4*>(U + at);
-                }
-#pragma unroll
-                for (int k = 0; k < ZUNITS; ++k) {
-                    b.g[k] += g[k];
-                    b.u[k] += u[k];
-                }
-            }
+        } else if (parts) {
+            const float* gp = G + (int64_t)as.row(a0 + b.row[0]) * I + column(0);
+            const float* up = U + (gp - G);
+            const int64_t third = n_part > 2 ? 2 * part_stride : 0;      // (two or four of them)
+            b.g0 = *reinterpret_cast<const f32x4*>(gp);
+            b.u0 = *reinterpret_cast<const f32x4*>(up);
+            b.g1 = *reinterpret_cast<const f32x4*>(gp + part_stride);
+            b.u1 = *reinterpret_cast<const f32x4*>(up + part_stride);
+            b.g2 = *reinterpret_cast<const f32x4*>(gp + third);
+            b.u2 = *reinterpret_cast<const f32x4*>(up + third);
+            b.g3 = *reinterpret_cast<const f32x4*>(gp + third + part_stride);
+            b.u3 = *reinterpret_cast<const f32x4*>(up + third + part_stride);
+        } else {
+            auto sums = [&](int k, f32x4& g, f32x4& u) {
+                const int64_t at = (int64_t)as.row(a0 + b.row[k]) * I + column(k);
+                g = *reinterpret_cast<const f32x4*>(G + at);
+                u = *reinterpret_cast<const f32x4*>(U + at);
+            };
+            sums(0, b.g0, b.u0);
+            sums(1, b.g1, b.u1);
+            sums(2, b.g2, b.u2);
         }
     };
+    static_assert(ZUNITS == 3, "partial results 0 to 2 take the units' places");
     auto make = [&](const Batch& bt, uint32_t u0) {
+        f32x4 g0 = bt.g0, v0 = bt.u0;
+        if (parts) {
+            g0 += bt.g1;
+            v0 += bt.u1;
+            if (n_part > 2) {
+                g0 = (g0 + bt.g2) + bt.g3;
+                v0 = (v0 + bt.u2) + bt.u3;
+            }
+        }
+        const uint32_t end = min(u0 + batch, units);
 #pragma unroll
         for (int k = 0; k < ZUNITS; ++k) {
-            if (u0 + k >= units) break;      // (wave-uniform)
+            if (u0 + k >= end) break;      // (wave-uniform)
             u32x2 hi, lo;
             if constexpr (ZREADY) {
                 hi = bt.hi[k];
                 lo = bt.lo[k];
             } else {
-                const ZPair a = z_pair(bt.g[k][0], bt.u[k][0], bt.g[k][1], bt.u[k][1]), b = z_pair(bt.g[k][2], bt.u[k][2], bt.g[k][3], bt.u[k][3]);
+                const f32x4 g = k == 0 ? g0 : k == 1 ? bt.g1 : bt.g2, v = k == 0 ? v0 : k == 1 ? bt.u1 : bt.u2;
+                const ZPair a = z_pair(g[0], v[0], g[1], v[1]), b = z_pair(g[2], v[2], g[3], v[3]);
                 hi = u32x2{a.hi, b.hi};
                 lo = u32x2{a.lo, b.lo};
             }
@@ -924,7 +939,7 @@ __device__ __forceinline__ void build_z_records(const float* __restrict__ G, con
             c = k == q ? bt.col[q] : c;
         }
         c += Z_BLOCK * b;
-        if (k < ZUNITS && u0 + k < units && c < cols) {
+        if (u0 + k < end && c < cols) {
             const u32x4* src = reinterpret_cast<const u32x4*>(stage + 256 * k + Z_BLOCK * b);
             unsigned char* dst = zrec + (c / N_TILE) * ZB_BYTES + (16 * (b & 3) + r) * 16;
             const u32x4* low = reinterpret_cast<const u32x4*>(dst);
@@ -939,13 +954,13 @@ __device__ __forceinline__ void build_z_records(const float* __restrict__ G, con
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
         __builtin_amdgcn_wave_barrier();
     };
-    uint32_t u0 = (uint32_t)wave * ZUNITS;
+    uint32_t u0 = (uint32_t)wave * batch;
     if (u0 < units) {
         Batch first;
         request(first, u0);
         behind();
         make(first, u0);
-        for (u0 += 4 * ZUNITS; u0 < units; u0 += 4 * ZUNITS) {
+        for (u0 += 4 * batch; u0 < units; u0 += 4 * batch) {
             Batch next;
             request(next, u0);
             make(next, u0);
