@@ -854,7 +854,11 @@ __device__ __forceinline__ void build_z_records(const float* __restrict__ G, con
         u32x2 hi[ZUNITS], lo[ZUNITS];
     };
     // (the gate/up kernel split the contraction where there are few workgroups: then a batch is one unit, and its partial results come
-    // together instead of one round trip after the other)
+    // together instead of one round trip after the other.  Layer in a graph, medians of four, us per layer, one after the other ->
+    // together.  Four partial results: 128 experts 28.8 -> 28.2 (1 token), 31.8 -> 31.3 (2); 64 experts 44.6 -> 43.7 (1);
+    // 512 experts 32.1 -> 32.2 (1), 36.6 -> 35.4 (2).  Two: 128 experts 37.1 -> 37.6 (4), 64 experts 52.1 -> 53.1 (2), 512
+    // experts 41.4 -> 40.9 (4).  Left to four partial results only, the sums that are whole lost 1 to 3 % (512 experts, 8 tokens:
+    // 51.2 -> 52.9) with another register allocation.)
     const bool parts = !ZREADY && n_part > 1;
     const uint32_t batch = parts ? 1u : (uint32_t)ZUNITS;
     auto request = [&](Batch& b, uint32_t u0) {
