@@ -104,7 +104,7 @@ int launch_forward_decode_fused(const bitsmoe_matset* gate, const bitsmoe_matset
 // The side kernels for the wide rows of prepared sets (forward_wide.hip).  Gate/up: adds the wide rows' share to the
 // gate and up sums the fast kernel has written -- fp32 sums [A, I] by atomics (part 0 of the decode path's partial
 // results), or f16 sums (the grouped-GEMM path) by a plain read-add-write.  Down: reads z = silu(G) * U as f16
-// [A, I] or as records, or forms it from `n_part` fp32 partial sums, and adds the wide rows' outputs, scaled by the
+// [A, I] (z_f16) or forms it from `n_part` fp32 partial sums, and adds the wide rows' outputs, scaled by the
 // routing weight, into rank_accum by atomics: after whatever writes or clears rank_accum.  Both need the routing
 // tables.  No-ops for sets without wide rows.
 bool has_wide_rows(const bitsmoe_matset* set);
@@ -113,8 +113,7 @@ bool only_wide_rows(const bitsmoe_matset* gate, const bitsmoe_matset* up, const 
 int launch_wide_gateup(const bitsmoe_matset* gate, const bitsmoe_matset* up, const void* h_gate, const void* h_up,
                        int act_dtype, int Rg, int Ru, int64_t ldg, int64_t ldu, const int32_t* tok, const int32_t* off,
                        int64_t A, int I, void* G, void* U, bool sums_f16, hipStream_t st);
-constexpr int WIDE_Z_SUMS = 0, WIDE_Z_F16 = 1, WIDE_Z_RECORDS = 2;      // where launch_wide_down takes z from
-int launch_wide_down(const bitsmoe_matset* down, const void* g_or_z, const float* u, int z_source, int n_part,
+int launch_wide_down(const bitsmoe_matset* down, const void* g_or_z, const float* u, bool z_f16, int n_part,
                      int64_t part_stride, const int32_t* tok, const int32_t* off, const float* rw, int64_t A, int I,
                      int rank_out, float* rank_accum, hipStream_t st);
 
@@ -358,9 +357,7 @@ __device__ inline float to_f32<__half>(__half v) { return __half2float(v); }
 template <>
 __device__ inline float to_f32<__hip_bfloat16>(__hip_bfloat16 v) { return __bfloat162float(v); }
 
-// (the hardware's reciprocal, 1 ulp: an exactly rounded division is nine more vector instructions per element, most of what the
-// SiLU passes issued; the reference compiles this with --use_fast_math)
-__device__ inline float silu_f32(float x) { return x * __builtin_amdgcn_rcpf(1.0f + __expf(-x)); }
+__device__ inline float silu_f32(float x) { return x / (1.0f + __expf(-x)); }
 
 // launchers implemented in the kernel translation units
 int launch_fill_zero(float* p, int64_t n, hipStream_t st);

@@ -8,7 +8,6 @@
 #include <utility>
 
 #include "fast_helpers.h"
-#include "z_planes.h"
 
 #ifndef BITSMOE_TL_DOWN_STAMP
 #define BITSMOE_TL_DOWN_STAMP(i) do {} while (0)      // (time stamps of the timeline build, forward_decode.hip)
@@ -18,9 +17,9 @@ namespace bitsmoe {
 constexpr int GU_STRIDE = GU_SLABS * SLAB_ROWS + 8;  // 16-bit elements; +8 staggers LDS banks
 constexpr int DN_SLABS_PER_WG = 4;                 // one slab per wavefront
 constexpr int MAX_A = 16;                          // assignments per MFMA pass
-constexpr int ZUNITS = 3;                          // pieces of 256 columns of G / U a wavefront of the down kernel has in flight
-constexpr int DOWN_RING2 = 3, DOWN_RING3 = 2, DOWN_RING4 = 2;      // tiles of payload a wavefront of the down kernel has in flight, by width
-constexpr int MAX_DECODE_TILES = 15;               // column tiles of the sets the decode kernels take (I <= 1920)
+constexpr int ZROWS = 2;                           // assignment rows of G / U the down kernel's z build fetches together
+constexpr int ZROWS_WIDE = 6;                      // ... where z is so large that only three workgroups fit a CU anyway
+constexpr int ZSUM_STRIDE = 16;                    // tiles per assignment row of the down kernel's z sums (I <= 1920)
 
 // With few assignments most experts are idle; launching a workgroup per (expert, ...) then
 // costs more than the work.  The kernels can instead be launched over `slots` and let every
@@ -627,12 +626,14 @@ __device__ __forceinline__ void gateup_walk_item_mixed(gptr<uint32_t> payload, g
 // slab groups of the gate matrix, then all of the up matrix; the payload stream of a wavefront runs on
 // from the one into the other), for sets in which the two matrices of every expert share one bit-width
 // and one slab count.  The tile's gate sums stay in registers while the up sums are formed, and the item
-// writes what the down projection needs:
-//     Z[a, c]      = f16(silu(G[a, c]) * U[a, c]), Zlow[a, c] what f16 leaves of it     ([A, I])
+// writes what the down projection needs, ready-made:
+//     Z[a, c]      = f16(silu(G[a, c]) * U[a, c])                    (16-bit MFMA operand, [A, I])
+//     Zsum[a, t]   = sum over the tile's 128 columns of Z as rounded  ([A, n_tiles] fp32; the constant term
+//                                                                      of the down projection's decode)
 // so the fp32 G / U round trip (8 bytes per element written, then read by every slab group of the expert)
 // and the SiLU leave the down kernel, and the gate/up launch is one round of (expert, tile) workgroups
 // instead of two rounds of (expert, tile, projection) ones.
-// `cterm_lds`: 2 * MAX_A floats (LDS).
+// `cterm_lds`: 2 * MAX_A floats, `zs_lds`: 4 * MAX_A floats (LDS).
 struct WalkMatrix {     // one projection's operands (wave-uniform)
     gptr<uint32_t> payload;
     gptr<__half> scale_s;
@@ -646,8 +647,8 @@ template <bool BF16, bool IDENT, int W>
 __device__ __forceinline__ void gateup_walk_z_item(const WalkMatrix& mg, const WalkMatrix& mu,
                                                    const int32_t* __restrict__ token_indices, int a0, int n_a, int A, int T,
                                                    int I, int n_tiles, int t, int n_groups, uint16_t* __restrict__ Z,
-                                                   uint16_t* __restrict__ Zlow, uint16_t* __restrict__ hs_all,
-                                                   float* __restrict__ cterm_lds, int tid) {
+                                                   float* __restrict__ Zsum, uint16_t* __restrict__ hs_all,
+                                                   float* __restrict__ cterm_lds, float* __restrict__ zs_lds, int tid) {
     const int pair = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform
     const int lane = tid & 63;
     const int n = lane & 15, kg = lane >> 4;
@@ -772,6 +773,7 @@ __device__ __forceinline__ void gateup_walk_z_item(const WalkMatrix& mg, const W
     }
     __syncthreads();
     // lane holds rows a = 4*kg + j of columns 32*pair + 16*nbl + n
+    float zpart[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const int a = 4 * kg + j;
@@ -779,279 +781,274 @@ __device__ __forceinline__ void gateup_walk_z_item(const WalkMatrix& mg, const W
 #pragma unroll
         for (int nbl = 0; nbl < 2; ++nbl) {
             const int c = t * N_TILE + 32 * pair + 16 * nbl + n;
-            if (a < n_a && c < I) {
-                const ZPair z = z_pair(acc_g[nbl][j] - cg, acc[nbl][j] - cu, 0.0f, 0.0f);
-                Z[(int64_t)(a0 + a) * I + c] = (uint16_t)z.hi;
-                Zlow[(int64_t)(a0 + a) * I + c] = (uint16_t)z.lo;
-            }
+            const uint16_t zb = z_operand(acc_g[nbl][j] - cg, acc[nbl][j] - cu);
+            if (a < n_a && c < I) Z[(int64_t)(a0 + a) * I + c] = zb;
+            zpart[j] += __half2float(__ushort_as_half(zb));
         }
     }
+    // row sums over this wavefront's 32 columns: the 16 lanes that share kg (one DPP row) hold one row
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        float v = zpart[j];
+        v = dpp_add_f32<0x111>(v);
+        v = dpp_add_f32<0x112>(v);
+        v = dpp_add_f32<0x114>(v);
+        v = dpp_add_f32<0x118>(v);
+        if (n == 15) zs_lds[pair * MAX_A + 4 * kg + j] = v;
+    }
+    __syncthreads();
+    if (tid < n_a)
+        Zsum[(int64_t)(a0 + tid) * n_tiles + t] = zs_lds[tid] + zs_lds[MAX_A + tid] + zs_lds[2 * MAX_A + tid] + zs_lds[3 * MAX_A + tid];
 }
 
 // ----------------------------------------------------------------------------------- down
-// One (slab, tile) block of a down matrix: 4 row blocks of 16 output rows x 128 columns against the tile's z records.
-// `c0`: minus 2^(W-1) times the sum of the tile's z planes, per assignment row of the lane (the codes are the levels plus
-// 2^(W-1)); three MFMAs against an operand of ones make it, in the layout the products start from (down_constant).
-// put(nb, sums): called for every row block.
+// One (slab, tile) block of a down matrix: 4 row blocks x 4 k-steps (micro-tiles).
+// `corr`: 1.5 * 2^W times the sum of the tile's z over its 128 columns, per assignment row of the
+// lane (the constant term of the decoded operands 2^W + code; the z rows are summed once, when z
+// is built, instead of by four more MFMAs per block).
 template <int W>
-__device__ __forceinline__ f32x4 down_constant(const ZOperand& z) {
-    const i32x8 ones = minus_ones();
-    f32x4 t = {0.0f, 0.0f, 0.0f, 0.0f};
-    t = mfma_plane<Z_FMT_FP4, 0, false>(z, ones, minus_ones_scale(W), t);
-    t = mfma_plane<Z_FMT_FP4, 1, false>(z, ones, minus_ones_scale(W), t);
-    return mfma_plane<Z_FMT_FP4, 2, false>(z, ones, minus_ones_scale(W), t);
-}
-template <int W, class Put>
-__device__ __forceinline__ void down_block(const Block16& b, const ZOperand& z, f32x4 c0, Put&& put) {
-    using F = CodeFormat<W>;
-    const u32x4 q0 = opaque(b.q0), q1 = opaque(b.q1), q2 = W >= 3 ? opaque(b.q2) : q0, q3 = W >= 4 ? opaque(b.q3) : q0;
-    // (two row blocks' chains of three or six MFMAs side by side: all four at once need more registers than there are)
-    auto half = [&](auto nb_c) {
-        constexpr int NB = decltype(nb_c)::value;
-        i32x8 x0, x1, y0, y1;      // low, high
-        code_operands<W, NB>(q0, q1, q2, q3, x0, y0);
-        code_operands<W, NB + 1>(q0, q1, q2, q3, x1, y1);
-        f32x4 t0 = c0, t1 = c0;
-        static_for([&](auto pc) {
-            constexpr int P = decltype(pc)::value;
-            t0 = mfma_plane<F::FMT, P, false>(z, x0, F::SCALE, t0);
-            t1 = mfma_plane<F::FMT, P, false>(z, x1, F::SCALE, t1);
-            if constexpr (W == 4) {
-                t0 = mfma_plane<F::FMT, P, false>(z, y0, W_SCALE_FP4_HI, t0);
-                t1 = mfma_plane<F::FMT, P, false>(z, y1, W_SCALE_FP4_HI, t1);
-            }
-        }, std::make_integer_sequence<int, 3>{});
-        put(NB, t0);
-        put(NB + 1, t1);
-    };
-    half(std::integral_constant<int, 0>{});
-    half(std::integral_constant<int, 2>{});
-}
-
-// z of a chunk's assignments for the workgroup's tiles tb .. tb + nt - 1, as records in operand order in LDS (`zrec`, ZB_BYTES
-// per tile, [piece][lane 16 kg + row]; rows without an assignment stay whatever they were: they feed output rows that are never
-// stored).
-// The work comes in units of one assignment x 256 columns, in batches of ZUNITS dealt to the wavefronts in turn (`wave`: this
-// one's place): a wavefront requests a batch together -- four columns of each unit per lane --, forms
-// z = silu(G) * U, puts the f16 values into its own `stage` (ZUNITS x 256), their remainders where the records will be, and makes
-// the records of them, one lane per 32 columns.  One memory round trip for 12 units (an assignment has 3 at 768 columns), however they are spread over
-// assignments, and wavefronts without a unit issue nothing: at one or two assignments per expert what the pass costs
-// is the instructions the four workgroups of a CU issue side by side.
-// ZREADY: `G` holds z as f16 [A, I] and U the remainders likewise (k_gateup_walk_z, k_decode_silu).  Otherwise G and U are the first of `n_part` partial
-// results, part_stride floats apart, that are added up.
-// `behind()` is called once, when the first batch has been requested: what it requests comes in behind the sums (loads return in
-// the order they were asked for) while z is made of them.  So that the wait for the sums is not one for all of that, the first
-// batch is a copy of the code of its own, and behind() requests the same number of loads on every path.
-template <bool ZREADY, class AS, class Behind>
-__device__ __forceinline__ void build_z_records(const float* __restrict__ G, const float* __restrict__ U, int n_part,
-                                                int64_t part_stride, const AS& as, int a0, int n_a, int I, int tb, int nt,
-                                                unsigned char* __restrict__ zrec, uint16_t* __restrict__ stage, int wave, int lane, Behind&& behind) {
-    const int c_begin = tb * N_TILE, cols = min(nt * N_TILE, I - c_begin);
-    const uint32_t pieces = (uint32_t)(nt + 1) >> 1, units = (uint32_t)n_a * pieces;
-    struct Batch {
-        int row[ZUNITS], col[ZUNITS];      // assignment and first column of the units
-        f32x4 g0, g1, g2, g3, u0, u1, u2, u3;      // sums of the units, or partial results 0, 1, 2 and 3 of ONE unit
-        u32x2 hi[ZUNITS], lo[ZUNITS];
-    };
-    // (the gate/up kernel split the contraction where there are few workgroups: then a batch is one unit, and its partial results come
-    // together instead of one round trip after the other.  Layer in a graph, medians of four, us per layer, one after the other ->
-    // together.  Four partial results: 128 experts 28.8 -> 28.2 (1 token), 31.8 -> 31.3 (2); 64 experts 44.6 -> 43.7 (1);
-    // 512 experts 32.1 -> 32.2 (1), 36.6 -> 35.4 (2).  Two: 128 experts 37.1 -> 37.6 (4), 64 experts 52.1 -> 53.1 (2), 512
-    // experts 41.4 -> 40.9 (4).  Left to four partial results only, the sums that are whole lost 1 to 3 % (512 experts, 8 tokens:
-    // 51.2 -> 52.9) with another register allocation.)
-    const bool parts = !ZREADY && n_part > 1;
-    const uint32_t batch = parts ? 1u : (uint32_t)ZUNITS;
-    auto request = [&](Batch& b, uint32_t u0) {
+__device__ __forceinline__ void down_block(const Block16& b, const u32x4 (&az)[4], const float (&sc)[4], f32x4 corr, f32x4 (&acc)[4]) {
 #pragma unroll
-        for (int k = 0; k < ZUNITS; ++k) {
-            const uint32_t u = min(u0 + k, units - 1);      // (a unit past the end: the last again)
-            const uint32_t r = u / pieces;
-            b.row[k] = __builtin_amdgcn_readfirstlane(r);
-            b.col[k] = __builtin_amdgcn_readfirstlane(256 * (u - r * pieces));
-        }
-        auto column = [&](int k) { return c_begin + min(b.col[k] + 4 * lane, cols - 4); };      // (past the end: the last four again)
-        if constexpr (ZREADY) {
+    for (int nb = 0; nb < 4; ++nb) {
+        f32x4 t = {0, 0, 0, 0};
 #pragma unroll
-            for (int k = 0; k < ZUNITS; ++k) {
-                const int64_t at = (int64_t)(a0 + b.row[k]) * I + column(k);
-                b.hi[k] = *reinterpret_cast<const u32x2*>(reinterpret_cast<const uint16_t*>(G) + at);
-                b.lo[k] = *reinterpret_cast<const u32x2*>(reinterpret_cast<const uint16_t*>(U) + at);
-            }
-        } else if (parts) {
-            const float* gp = G + (int64_t)as.row(a0 + b.row[0]) * I + column(0);
-            const float* up = U + (gp - G);
-            const int64_t third = n_part > 2 ? 2 * part_stride : 0;      // (two or four of them)
-            b.g0 = *reinterpret_cast<const f32x4*>(gp);
-            b.u0 = *reinterpret_cast<const f32x4*>(up);
-            b.g1 = *reinterpret_cast<const f32x4*>(gp + part_stride);
-            b.u1 = *reinterpret_cast<const f32x4*>(up + part_stride);
-            b.g2 = *reinterpret_cast<const f32x4*>(gp + third);
-            b.u2 = *reinterpret_cast<const f32x4*>(up + third);
-            b.g3 = *reinterpret_cast<const f32x4*>(gp + third + part_stride);
-            b.u3 = *reinterpret_cast<const f32x4*>(up + third + part_stride);
-        } else {
-            auto sums = [&](int k, f32x4& g, f32x4& u) {
-                const int64_t at = (int64_t)as.row(a0 + b.row[k]) * I + column(k);
-                g = *reinterpret_cast<const f32x4*>(G + at);
-                u = *reinterpret_cast<const f32x4*>(U + at);
-            };
-            sums(0, b.g0, b.u0);
-            sums(1, b.g1, b.u1);
-            sums(2, b.g2, b.u2);
+        for (int m = 0; m < 4; ++m) {
+            u32x4 bw;
+            if constexpr (W == 2)
+                bw = decode_fields2<2, false>(b.w[nb * 2 + (m >> 1)], 8 * (m & 1));
+            else if constexpr (W == 4)
+                bw = decode_fields4<false>(b.w[nb * 4 + m]);
+            else
+                bw = decode_r1w3<false>(b.w, nb, m);
+            t = mfma16<false>(az[m], bw, t);
         }
-    };
-    static_assert(ZUNITS == 3, "partial results 0 to 2 take the units' places");
-    auto make = [&](const Batch& bt, uint32_t u0) {
-        f32x4 g0 = bt.g0, v0 = bt.u0;
-        if (parts) {
-            g0 += bt.g1;
-            v0 += bt.u1;
-            if (n_part > 2) {
-                g0 = (g0 + bt.g2) + bt.g3;
-                v0 = (v0 + bt.u2) + bt.u3;
-            }
-        }
-        const uint32_t end = min(u0 + batch, units);
-#pragma unroll
-        for (int k = 0; k < ZUNITS; ++k) {
-            if (u0 + k >= end) break;      // (wave-uniform)
-            u32x2 hi, lo;
-            if constexpr (ZREADY) {
-                hi = bt.hi[k];
-                lo = bt.lo[k];
-            } else {
-                const f32x4 g = k == 0 ? g0 : k == 1 ? bt.g1 : bt.g2, v = k == 0 ? v0 : k == 1 ? bt.u1 : bt.u2;
-                const ZPair a = z_pair(g[0], v[0], g[1], v[1]), b = z_pair(g[2], v[2], g[3], v[3]);
-                hi = u32x2{a.hi, b.hi};
-                lo = u32x2{a.lo, b.lo};
-            }
-            *reinterpret_cast<u32x2*>(stage + 256 * k + 4 * lane) = hi;
-            const int c = bt.col[k] + 4 * lane;      // (pieces a to d of the record, in the order of its columns)
-            if (c < cols)
-                *reinterpret_cast<u32x2*>(zrec + (c / N_TILE) * ZB_BYTES + ((c & 31) >> 3) * 1024 + (16 * ((c >> 5) & 3) + bt.row[k]) * 16 +
-                                          2 * (c & 7)) = lo;
-        }
-        // (the stage is the wavefront's own, and its LDS accesses complete in order: no barrier, but neither may the compiler
-        // move the reads across the writes)
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
-        __builtin_amdgcn_wave_barrier();
-        const int k = lane >> 3, b = lane & 7;       // unit and 32-column block of this lane's record
-        int r = bt.row[0], c = bt.col[0];
-#pragma unroll
-        for (int q = 1; q < ZUNITS; ++q) {
-            r = k == q ? bt.row[q] : r;
-            c = k == q ? bt.col[q] : c;
-        }
-        c += Z_BLOCK * b;
-        if (u0 + k < end && c < cols) {
-            const u32x4* src = reinterpret_cast<const u32x4*>(stage + 256 * k + Z_BLOCK * b);
-            unsigned char* dst = zrec + (c / N_TILE) * ZB_BYTES + (16 * (b & 3) + r) * 16;
-            const u32x4* low = reinterpret_cast<const u32x4*>(dst);
-            float none;
-            const ZRecord rec = z_record<false>(F16x32{src[0], src[1], src[2], src[3]}, F16x32{low[0], low[64], low[128], low[192]}, none);
-            *reinterpret_cast<u32x4*>(dst) = rec.a;
-            *reinterpret_cast<u32x4*>(dst + 1024) = rec.b;
-            *reinterpret_cast<u32x4*>(dst + 2048) = rec.c;
-            *reinterpret_cast<u32x4*>(dst + 3072) = rec.d;
-            *reinterpret_cast<u32x4*>(dst + 4096) = rec.e;
-        }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
-        __builtin_amdgcn_wave_barrier();
-    };
-    uint32_t u0 = (uint32_t)wave * batch;
-    if (u0 < units) {
-        Batch first;
-        request(first, u0);
-        behind();
-        make(first, u0);
-        for (u0 += 4 * batch; u0 < units; u0 += 4 * batch) {
-            Batch next;
-            request(next, u0);
-            make(next, u0);
-        }
-    } else {
-        behind();
+        acc[nb] += (t - corr) * sc[nb];
     }
 }
 
 // Everything one wavefront of the down kernel does after the metadata has arrived, compiled
 // per bit-width of the wavefront's slab (W == 0: no slab, the wavefront only helps to build z).
-// The payload goes through a ring of register buffers, three tiles for 2-bit slabs, two for 3- and 4-bit ones (one more each: two
-// to twenty registers spilled).  All of
-// them are requested right BEHIND the first sums that z is made of: the sums come first (loads return in the order they
-// were asked for; payload in front of them holds them up, and every workgroup of the launch is at this point at the same
-// time), the payload while SiLU is evaluated and the records are made.  The register budget is 128, so that all four
+// The payload of the first tile is requested BEFORE z is built, so that weights are in flight
+// while G and U are read and SiLU is evaluated -- of ONE tile: loads return in the order they
+// were asked for, so the rows of G and U wait behind whatever payload was requested first, and
+// every workgroup of the launch is at this point at the same time (two tiles ahead of z: the down
+// kernel 5 to 7 % slower on 128 experts at 8 and 64 tokens and on 64 experts at 16 tokens, 3 % on
+// 512 experts at 256 tokens; none: 2 to 6 % slower).  The second tile is requested when z is
+// done; afterwards the tiles stream through two register buffers, one tile ahead of the one
+// being computed.  The register budget is 128, so that all four
 // workgroups of a CU -- on the 64-token benchmark layer the whole grid -- are resident at once:
 // what only the epilogue needs (rank and multiplier of the rows, token and weight of the
-// assignments) waits in LDS (`rows` takes the place of the wavefront's z stage).
-template <int W, bool ZREADY, class AS>
+// assignments) waits in LDS, and z is built two assignment rows at a time.
+// ZREADY: `G` holds Z (16-bit operands, [A, I]) and `U` holds Zsum ([A, n_tiles] fp32) as written by
+// gateup_walk_z_item: the z phase is a copy into LDS instead of two fp32 reads and a SiLU per element.
+// Otherwise G and U are the first of `n_part` partial results, part_stride floats apart, that are added up.
+// ZR: assignment rows whose G / U loads are in flight together while z is built (one memory round trip per ZR
+// rows: the pass is latency-bound; more rows need more registers).
+// ZBY: z is built a row per wavefront (see there); a variant of its own, chosen by the launcher for batches of several
+// assignments per expert -- in one kernel with the column-wise form either is slowed down by the other's registers.
+template <int W, bool ZREADY, int ZR, bool ZBY, class AS>
 __device__ __forceinline__ void down_wave(gptr<uint32_t> payload, gptr<__half> scale, gptr<__half> svec, gptr<int32_t> rank_idx,
                                  const FastSlab fs, const float* __restrict__ G, const float* __restrict__ U, int n_part,
                                  int64_t part_stride, const AS& as,
                                  int a_begin, int a_end, int T, int I, int tb, int nt, int rank_out,
-                                 float* __restrict__ rank_accum, unsigned char* __restrict__ zrec, uint16_t* __restrict__ stage,
-                                 int2* __restrict__ assigns, int z_turn, int lane_in) {
+                                 float* __restrict__ rank_accum, uint16_t* __restrict__ z, int z_stride, float* __restrict__ zsum,
+                                 int2* __restrict__ rows, int2* __restrict__ assigns, int tid, int lane) {
+    const int n = lane & 15, kg = lane >> 4, g4 = kg * 4;
+    using I0 = std::integral_constant<int, 0>;
+    using I1 = std::integral_constant<int, 1>;
+    using I2 = std::integral_constant<int, 2>;
     constexpr int WL = W == 0 ? 2 : W;
-    constexpr int NBUF = WL == 2 ? DOWN_RING2 : WL == 3 ? DOWN_RING3 : DOWN_RING4;
-    int2* __restrict__ rows = reinterpret_cast<int2*>(stage);
     for (int a0 = a_begin; a0 < a_end; a0 += MAX_A) {
         const int n_a = min(MAX_A, a_end - a0);
         int chunk_zero = 0;
         asm volatile("" : "+s"(chunk_zero));   // keeps this chunk's address arithmetic inside the loop
-        int lane = lane_in;
-        asm volatile("" : "+v"(lane));         // (and what is derived from the lane: held across the loop it is spilled)
-        const int n = lane & 15, kg = lane >> 4, g4 = kg * 4;
-        Block16 buf[NBUF];
-        u32x2 sc[NBUF];       // the lane's four scales of the tile (f16, converted where they are used)
+        Block16 buf[2];
+        float sc[2][4];
         f32x4 acc[4];
+#pragma unroll
+        for (int nb = 0; nb < 4; ++nb) acc[nb] = f32x4{0, 0, 0, 0};
         // the workgroup's tiles are tb .. tb + nt - 1; `i` counts from 0
         auto issue = [&](auto b_c, int i) {
             constexpr int B = decltype(b_c)::value;
-            const int t = tb + i + chunk_zero;
-            load_block_role1<WL>(payload + (uint32_t)(fs.pack_off + t * block_words(WL)), lane, buf[B]);
-            sc[B] = *reinterpret_cast<gptr_u32x2>(scale + (uint32_t)(fs.scale_off + t * SLAB_ROWS + 4 * n));
+            const int t = tb + i;
+            load_block_role1<WL>(payload + (uint32_t)(fs.pack_off + (t + chunk_zero) * (WL == 3 ? R1W3_BLOCK_WORDS : 256 * WL)), lane,
+                                 buf[B]);
+            gptr<__half> sp = scale + (uint32_t)(fs.scale_off + t * SLAB_ROWS + n);
+#pragma unroll
+            for (int nb = 0; nb < 4; ++nb) sc[B][nb] = gload_half(sp + 16 * nb);
         };
         auto compute = [&](auto b_c, int i) {
             constexpr int B = decltype(b_c)::value;
-            const u32x4* zp = reinterpret_cast<const u32x4*>(zrec + i * ZB_BYTES) + lane;
-            const ZRecord rec = {zp[0], zp[64], zp[128], zp[192], zp[256]};
-            const uint32_t s01 = sc[B][0], s23 = sc[B][1];
-            const h2 a = __builtin_bit_cast(h2, s01), b = __builtin_bit_cast(h2, s23);
-            const float s[4] = {(float)a[0], (float)a[1], (float)b[0], (float)b[1]};
-            const ZOperand z = z_operand_of(rec);
-            down_block<WL>(buf[B], z, down_constant<WL>(z), [&](int nb, f32x4 t) { acc[nb] += t * s[nb]; });
+            u32x4 az[4];
+            const uint16_t* zp = z + n * z_stride + i * N_TILE + 8 * kg;      // (z holds this workgroup's tiles only)
+#pragma unroll
+            for (int m = 0; m < 4; ++m) az[m] = *reinterpret_cast<const u32x4*>(zp + 32 * m);
+            f32x4 corr;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) corr[j] = zsum[(g4 + j) * ZSUM_STRIDE + tb + i] * (1.5f * (float)(1 << WL));
+            down_block<WL>(buf[B], az, sc[B], corr, acc);
         };
-        // logical rank and multiplier of the slab's row `lane`, token id and routing weight of assignment `lane` of the
-        // chunk: needed by the epilogue only, kept in LDS until then (a wavefront's own 64 entries: no barrier involved; every
-        // wavefront writes the same sixteen assignments)
+        // logical rank and multiplier of the slab's row `lane`: needed by the epilogue only, kept
+        // in LDS until then (one wavefront's own 64 entries: no barrier involved)
         int row_rank = -1;
         float row_s = 0.0f;
         if constexpr (W != 0) {
+            issue(I0{}, 0);      // (ONE tile ahead of z: see above)
             row_rank = rank_idx[fs.rank_off + lane];
             row_s = gload_half(svec + fs.rank_off + lane);
         }
+        // token ids and routing weights of the chunk (lane a holds assignment a): for the epilogue,
+        // kept in LDS until then (every wavefront writes the same sixteen entries)
         const int tok_lane = as.token_if(a0 + lane, lane < n_a);
         const float rw_lane = as.weight_if(a0 + lane, lane < n_a);
         __syncthreads();   // the previous chunk is done with z
-        build_z_records<ZREADY>(G, U, n_part, part_stride, as, a0, n_a, I, tb, nt, zrec, stage, z_turn, lane, [&] {
-            if constexpr (W != 0)      // (fewer tiles than buffers: the last again, so that every path requests as much)
-                static_for([&](auto bc) { issue(bc, min(decltype(bc)::value, nt - 1)); }, std::make_integer_sequence<int, NBUF>{});
-        });
+        if constexpr (ZREADY) {
+            const uint16_t* __restrict__ Zg = reinterpret_cast<const uint16_t*>(G);
+            const int pieces = nt * (N_TILE / 8);          // 16-byte pieces per row of this workgroup's tiles
+            const int total = n_a * pieces;
+            for (int idx0 = tid; idx0 < total; idx0 += 3 * 256) {      // (three loads in flight per thread)
+                u32x4 v[3];
+                int dst[3];
+#pragma unroll
+                for (int k = 0; k < 3; ++k) {
+                    const int idx = min(idx0 + 256 * k, total - 1);
+                    const int a = idx / pieces, p = idx - a * pieces;
+                    const int c = tb * N_TILE + 8 * p;
+                    v[k] = *reinterpret_cast<const u32x4*>(Zg + (int64_t)(a0 + a) * I + c);
+                    dst[k] = a * z_stride + 8 * p;
+                }
+#pragma unroll
+                for (int k = 0; k < 3; ++k)
+                    if (idx0 + 256 * k < total) *reinterpret_cast<u32x4*>(z + dst[k]) = v[k];
+            }
+            if (tid < n_a * nt) {
+                const int a = tid / nt, i = tid - a * nt;
+                zsum[a * ZSUM_STRIDE + tb + i] = U[(int64_t)(a0 + a) * (((I + N_TILE - 1) / N_TILE)) + tb + i];
+            }
+        } else if constexpr (ZBY) {
+            // z[a][c] = silu(G) * U as 16-bit operands for the rows a < n_a (other rows feed output rows that are never
+            // stored).  A wavefront takes whole rows -- w, w + 4, ... -- and a lane four neighbouring columns of each 256
+            // of the row, ZP such pieces of G and of U requested together: the rows of a chunk are ceil(n_a / 4) memory
+            // round trips, where four columns per thread over all rows, two at a time, were ceil(n_a / 2).
+            constexpr int ZP = ZR > ZROWS ? 6 : 3;
+            const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+            const int c_begin = tb * N_TILE, c_end = min((tb + nt) * N_TILE, I);
+            for (int a = wv; a < n_a; a += 4) {
+                const int64_t row_off = (int64_t)as.row(a0 + a) * I;
+                for (int p0 = c_begin; p0 < c_end; p0 += 256 * ZP) {
+                    f32x4 gv[ZP], uv[ZP];
+#pragma unroll
+                    for (int p = 0; p < ZP; ++p) {
+                        const int c = min(p0 + 256 * p + 4 * lane, c_end - 4);      // (a piece past the end repeats the last)
+                        gv[p] = *reinterpret_cast<const f32x4*>(G + row_off + c);
+                        uv[p] = *reinterpret_cast<const f32x4*>(U + row_off + c);
+                    }
+                    for (int q = 1; q < n_part; ++q) {
+#pragma unroll
+                        for (int p = 0; p < ZP; ++p) {
+                            const int c = min(p0 + 256 * p + 4 * lane, c_end - 4);
+                            gv[p] += *reinterpret_cast<const f32x4*>(G + row_off + c + q * part_stride);
+                            uv[p] += *reinterpret_cast<const f32x4*>(U + row_off + c + q * part_stride);
+                        }
+                    }
+#pragma unroll
+                    for (int p = 0; p < ZP; ++p) {
+                        const int c = p0 + 256 * p + 4 * lane;
+                        if (p0 + 256 * p >= c_end) break;      // (wave-uniform)
+                        const bool live = c < c_end;
+                        uint16_t zb[4];
+                        float part = 0.0f;      // sum of the four operands as rounded
+#pragma unroll
+                        for (int x = 0; x < 4; ++x) {
+                            zb[x] = z_operand(gv[p][x], uv[p][x]);
+                            part += __half2float(__ushort_as_half(zb[x]));
+                        }
+                        part = live ? part : 0.0f;
+                        if (live) {
+                            u32x2 packed;
+                            packed[0] = (uint32_t)zb[0] | ((uint32_t)zb[1] << 16);
+                            packed[1] = (uint32_t)zb[2] | ((uint32_t)zb[3] << 16);
+                            *reinterpret_cast<u32x2*>(z + a * z_stride + c - c_begin) = packed;
+                        }
+                        // the 32 lanes of a half wavefront hold one tile's 128 columns: their sum arrives in lanes 31 and 63
+                        part = dpp_add_f32<0x111>(part);
+                        part = dpp_add_f32<0x112>(part);
+                        part = dpp_add_f32<0x114>(part);
+                        part = dpp_add_f32<0x118>(part);
+                        part = dpp_add_f32<0x142, 0xa>(part);
+                        const int c_tile = p0 + 256 * p + 4 * (lane & 32);      // first column of this half's tile
+                        if ((lane & 31) == 31 && c_tile < c_end) zsum[a * ZSUM_STRIDE + c_tile / N_TILE] = part;
+                    }
+                }
+            }
+        } else
+        // z[a][c] = silu(G) * U as 16-bit operands for the rows a < n_a (other rows feed
+        // output rows that are never stored).  Each thread owns four neighbouring columns
+        // and walks the assignments ZR at a time, their vector loads issued together.
+        for (int c = tb * N_TILE + tid * 4; c < min((tb + nt) * N_TILE, I); c += 1024) {
+            for (int ab = 0; ab < n_a; ab += ZR) {
+                f32x4 gv[ZR], uv[ZR];
+#pragma unroll
+                for (int j = 0; j < ZR; ++j) {
+                    const int a = min(ab + j, n_a - 1);
+                    const int64_t gi = (int64_t)as.row(a0 + a) * I + c;
+                    gv[j] = *reinterpret_cast<const f32x4*>(G + gi);
+                    uv[j] = *reinterpret_cast<const f32x4*>(U + gi);
+                }
+                // (the gate/up kernel split the contraction: the sums are totals of partial results)
+                for (int p = 1; p < n_part; ++p) {
+#pragma unroll
+                    for (int j = 0; j < ZR; ++j) {
+                        const int a = min(ab + j, n_a - 1);
+                        const int64_t gi = (int64_t)as.row(a0 + a) * I + c + p * part_stride;
+                        gv[j] += *reinterpret_cast<const f32x4*>(G + gi);
+                        uv[j] += *reinterpret_cast<const f32x4*>(U + gi);
+                    }
+                }
+#pragma unroll
+                for (int j = 0; j < ZR; ++j) {
+                    if (ab + j < n_a) {
+                        uint16_t zb[4];
+                        float part = 0.0f;      // sum of the four operands as rounded
+#pragma unroll
+                        for (int x = 0; x < 4; ++x) {
+                            zb[x] = z_operand(gv[j][x], uv[j][x]);
+                            part += __half2float(__ushort_as_half(zb[x]));
+                        }
+                        u32x2 packed;
+                        packed[0] = (uint32_t)zb[0] | ((uint32_t)zb[1] << 16);
+                        packed[1] = (uint32_t)zb[2] | ((uint32_t)zb[3] << 16);
+                        *reinterpret_cast<u32x2*>(z + (ab + j) * z_stride + c - tb * N_TILE) = packed;
+                        // the 32 lanes of a half wavefront hold one tile's 128 columns: their sum
+                        // arrives in lanes 31 and 63 (whole rows of 16 lanes are active or not)
+                        part = dpp_add_f32<0x111>(part);
+                        part = dpp_add_f32<0x112>(part);
+                        part = dpp_add_f32<0x114>(part);
+                        part = dpp_add_f32<0x118>(part);
+                        part = dpp_add_f32<0x142, 0xa>(part);
+                        if ((lane & 31) == 31) zsum[(ab + j) * ZSUM_STRIDE + c / N_TILE] = part;
+                    }
+                }
+            }
+        }
         if constexpr (W != 0) rows[lane] = int2{row_rank, __float_as_int(row_s)};
         if (lane < MAX_A) assigns[lane] = int2{tok_lane, __float_as_int(rw_lane)};
-        barrier_lds();       // (the payload in flight is not waited for)
+        __syncthreads();
         if (a0 == a_begin) BITSMOE_TL_DOWN_STAMP(2);
-#pragma unroll
-        for (int nb = 0; nb < 4; ++nb) acc[nb] = f32x4{0, 0, 0, 0};
         if constexpr (W != 0) {
-            for (int i = 0; i < nt; i += NBUF)
-                static_for([&](auto bc) {
-                    const int j = i + decltype(bc)::value;
-                    if (j < nt) {
-                        compute(bc, j);
-                        if (j + NBUF < nt) issue(bc, j + NBUF);
-                    }
-                }, std::make_integer_sequence<int, NBUF>{});
+            if (nt > 1) issue(I1{}, 1);
+        }
+        if constexpr (W != 0) {
+            // two buffers, one tile ahead of the one being computed (two ahead through three buffers: 3 to 5 % slower at 8
+            // to 256 tokens on 64, 128 and 512 experts, 1 % faster at 64 tokens on 128)
+            for (int i = 0; i < nt; i += 2) {
+                compute(I0{}, i);
+                if (i + 1 < nt) {
+                    if (i + 2 < nt) issue(I0{}, i + 2);
+                    compute(I1{}, i + 1);
+                    if (i + 3 < nt) issue(I1{}, i + 3);
+                }
+            }
         }
         if (a0 == a_begin) BITSMOE_TL_DOWN_STAMP(3);
         if constexpr (W != 0) {

@@ -65,39 +65,33 @@ __device__ __forceinline__ void load_pair_role0(gptr<uint32_t> blk, int bits, ui
     }
 }
 
-// Workgroup barrier that waits for the wavefront's own LDS accesses but not for its loads in flight (__syncthreads does).
-__device__ __forceinline__ void barrier_lds() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
-// A vector the compiler knows nothing more about.  Neighbouring vectors of a structure that are taken apart right after they
-// are read are otherwise turned into one wider read of the structure, which then is no longer split into registers: it
-// ends in scratch memory.
-__device__ __forceinline__ u32x4 opaque(u32x4 v) {
-    asm("" : "+v"(v));
-    return v;
-}
-
-// Up to 16 payload words of one lane for one (slab, tile) block.
-struct Block16 {
-    u32x4 q0, q1, q2, q3;
+struct Block16 {   // up to 16 payload words of one lane for one (slab, tile) block
+    uint32_t w[16];
 };
-template <int J>
-__device__ __forceinline__ uint32_t block_word(u32x4 q0, u32x4 q1, u32x4 q2, u32x4 q3) {
-    return J < 4 ? q0[J & 3] : J < 8 ? q1[J & 3] : J < 12 ? q2[J & 3] : q3[J & 3];
-}
 
-// role 1 loads: the lane's 8, 12 or 16 words
+// role 1 loads: 2-bit 8 words [nb][h], 4-bit 16 words [nb][m], 3-bit 13 words (five code pairs each)
 template <int W>
 __device__ __forceinline__ void load_block_role1(gptr<uint32_t> blk, int lane, Block16& b) {
-    gptr_u32x4 p = reinterpret_cast<gptr_u32x4>(blk + (W == 3 ? lane * 4 : lane * 4 * W));
-    constexpr int STEP = W == 3 ? 64 : 1;      // (3-bit: 256 words from one of the lane's pieces to the next)
-    b.q0 = p[0];
-    b.q1 = p[STEP];
-    if constexpr (W >= 3) b.q2 = p[2 * STEP];
-    if constexpr (W >= 4) b.q3 = p[3 * STEP];
+    gptr_u32x4 p = reinterpret_cast<gptr_u32x4>(blk + (W == 4 ? lane * 16 : W == 3 ? lane * 4 : lane * 8));
+    u32x4 v0 = p[0], v1, v2 = {0, 0, 0, 0}, v3 = {0, 0, 0, 0};
+    if constexpr (W == 3) {
+        v1 = p[64];       // (+256 words)
+        v2 = p[128];
+        v3[0] = blk[768 + lane];
+    } else {
+        v1 = p[1];
+    }
+    if constexpr (W == 4) {
+        v2 = p[2];
+        v3 = p[3];
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        b.w[i] = v0[i];
+        b.w[4 + i] = v1[i];
+        b.w[8 + i] = v2[i];
+        b.w[12 + i] = v3[i];
+    }
 }
 
 }  // namespace bitsmoe

@@ -501,14 +501,14 @@ __global__ __launch_bounds__(256, 4) void k_gateup_walk(
 }
 
 // gateup_walk_z_item launched as a grid: grid.x = (expert coordinate) * n_tiles; 256 threads.  One
-// workgroup forms BOTH projections of its tile and writes Z and Zlow; it also clears `zero_out`.
+// workgroup forms BOTH projections of its tile and writes Z / Zsum; it also clears `zero_out`.
 template <bool BF16, int MODE, bool IDENT>
 __global__ __launch_bounds__(256, 4) void k_gateup_walk_z(
     const FastExpert* __restrict__ gate_fe, const FastSlab* __restrict__ gate_fs, const FastExpert* __restrict__ up_fe,
     const FastSlab* __restrict__ up_fs, int max_slabs, const uint16_t* __restrict__ h_gate,
     const uint16_t* __restrict__ h_up, int64_t ldg, int64_t ldu, const int32_t* __restrict__ token_indices,
     const int32_t* __restrict__ expert_offsets, int T, int A, int I, int E, int n_tiles, uint16_t* __restrict__ Z,
-    uint16_t* __restrict__ Zlow, float* __restrict__ zero_out, int64_t zero_n, const ExpertOrder order) {
+    float* __restrict__ Zsum, float* __restrict__ zero_out, int64_t zero_n, const ExpertOrder order) {
     const int bid = blockIdx.x;
     const int tid = threadIdx.x;
     {   // this workgroup's share of the accumulator (before any exit)
@@ -546,13 +546,14 @@ __global__ __launch_bounds__(256, 4) void k_gateup_walk_z(
 
     __shared__ __attribute__((aligned(16))) uint16_t hs_all[2 * MAX_A * GU_STRIDE];
     __shared__ float cterm_lds[2 * MAX_A];
+    __shared__ float zs_lds[4 * MAX_A];
 
     for (int a0 = a_begin; a0 < a_end; a0 += MAX_A) {
         const int n_a = min(MAX_A, a_end - a0);
         if (a0 != a_begin) __syncthreads();      // the previous chunk's readers of the LDS buffers are done
         auto run = [&](auto w_c) {
             gateup_walk_z_item<BF16, IDENT, decltype(w_c)::value>(mg, mu, token_indices, a0, n_a, A, T, I, n_tiles, t, n_groups, Z,
-                                                                  Zlow, hs_all, cterm_lds, tid);
+                                                                  Zsum, hs_all, cterm_lds, zs_lds, tid);
         };
         if (first_g.bits == 2)
             run(std::integral_constant<int, 2>{});
@@ -567,30 +568,55 @@ __global__ __launch_bounds__(256, 4) void k_gateup_walk_z(
 // per-tile sums of its rows, the epilogue's row and assignment records.
 // A workgroup takes four slabs of one expert and a run of tiles; with few active experts the
 // tiles are split over several workgroups (their partial sums meet in the atomics of the combine).
-// z = silu(G) * U as f16 [A, I], and the remainders, from the fp32 gate and up sums (the totals of `n_part` partial results): what the down
-// kernel's workgroups otherwise each form for themselves.  Worth a launch of its own where those workgroups hold full
-// 16-assignment chunks and many of them share a chunk.  A thread owns four columns.
+// z = silu(G) * U as 16-bit operands [A, I] and the per-tile sums of the rounded operands [A, n_tiles], from the fp32
+// gate and up sums (the totals of `n_part` partial results): what the down kernel's workgroups otherwise each form
+// for themselves, two rows per memory round trip.  Worth a launch of its own where those workgroups hold full
+// 16-assignment chunks and many of them share a chunk.  A thread owns four columns, 32 lanes one tile of one row.
 __global__ __launch_bounds__(256) void k_decode_silu(const float* __restrict__ G, const float* __restrict__ U, int n_part,
-                                                     int64_t part_stride, int64_t n4, uint16_t* __restrict__ Z, uint16_t* __restrict__ Zlow) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n4) return;
-    f32x4 gv = *reinterpret_cast<const f32x4*>(G + 4 * i), uv = *reinterpret_cast<const f32x4*>(U + 4 * i);
+                                                     int64_t part_stride, int A, int I, int n_tiles,
+                                                     uint16_t* __restrict__ Z, float* __restrict__ Zsum) {
+    const int64_t unit = ((int64_t)blockIdx.x * 256 + threadIdx.x) >> 5;      // (row, tile)
+    const int lane32 = threadIdx.x & 31;
+    const int a = (int)(unit / n_tiles), t = (int)(unit - (int64_t)a * n_tiles);
+    if (a >= A) return;                  // (whole half-wavefronts leave)
+    const int c = t * N_TILE + 4 * lane32;
+    const bool in = c < I;
+    const int64_t gi = (int64_t)a * I + (in ? c : 0);
+    f32x4 gv = *reinterpret_cast<const f32x4*>(G + gi), uv = *reinterpret_cast<const f32x4*>(U + gi);
     for (int p = 1; p < n_part; ++p) {
-        gv += *reinterpret_cast<const f32x4*>(G + 4 * i + p * part_stride);
-        uv += *reinterpret_cast<const f32x4*>(U + 4 * i + p * part_stride);
+        gv += *reinterpret_cast<const f32x4*>(G + gi + p * part_stride);
+        uv += *reinterpret_cast<const f32x4*>(U + gi + p * part_stride);
     }
-    const ZPair a = z_pair(gv[0], uv[0], gv[1], uv[1]), b = z_pair(gv[2], uv[2], gv[3], uv[3]);
-    *reinterpret_cast<u32x2*>(Z + 4 * i) = u32x2{a.hi, b.hi};
-    *reinterpret_cast<u32x2*>(Zlow + 4 * i) = u32x2{a.lo, b.lo};
+    uint16_t zb[4];
+    float part = 0.0f;      // sum of the four operands as rounded
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+        zb[x] = in ? z_operand(gv[x], uv[x]) : (uint16_t)0;
+        part += __half2float(__ushort_as_half(zb[x]));
+    }
+    if (in) {
+        u32x2 packed;
+        packed[0] = (uint32_t)zb[0] | ((uint32_t)zb[1] << 16);
+        packed[1] = (uint32_t)zb[2] | ((uint32_t)zb[3] << 16);
+        *reinterpret_cast<u32x2*>(Z + (int64_t)a * I + c) = packed;
+    }
+    part = dpp_add_f32<0x111>(part);
+    part = dpp_add_f32<0x112>(part);
+    part = dpp_add_f32<0x114>(part);
+    part = dpp_add_f32<0x118>(part);
+    part = dpp_add_f32<0x142, 0xa>(part);
+    if (lane32 == 31) Zsum[(int64_t)a * n_tiles + t] = part;
 }
 
-// ZREADY: G and U hold Z and Zlow written by k_gateup_walk_z or k_decode_silu instead of the fp32 gate and up sums.  Otherwise the
+// ZREADY: G / U hold Z / Zsum written by k_gateup_walk_z instead of the fp32 gate and up sums.  Otherwise the
 // sums are the totals of `n_part` partial results part_stride floats apart (k_gateup_walk).
 // ROUTED (GRID_EXPERTS or GRID_ACTIVE): no routing tables; the workgroup finds its expert's entries among the routed
 // ids itself, as the gate/up kernel did (same rows of the intermediates), and takes the routing weights
 // from `sel_weights` in entry order.
-template <int MODE, bool ZREADY, bool ROUTED>
-__global__ __launch_bounds__(256, 4) void k_down_decode(
+// ZR: rows of G / U in flight while z is built; more than the usual two only where z is so large that three
+// workgroups fit a CU, which leaves each of them more registers (launch bounds follow).
+template <int MODE, bool ZREADY, bool ROUTED, int ZR, bool ZBY = false>
+__global__ __launch_bounds__(256, ZR > ZROWS ? 3 : 4) void k_down_decode(
     const FastExpert* __restrict__ down_fe, const FastSlab* __restrict__ down_fs, int max_slabs,
     const float* __restrict__ G, const float* __restrict__ U, int n_part, int64_t part_stride,
     const float* __restrict__ route_w, const int32_t* __restrict__ token_indices,
@@ -689,28 +715,26 @@ __global__ __launch_bounds__(256, 4) void k_down_decode(
     gptr<__half> svec = as_global(fe.s);
     gptr<int32_t> rank_idx = as_global(fe.rank_idx);
     extern __shared__ __attribute__((aligned(16))) unsigned char dsmem[];
-    unsigned char* zrec = dsmem;
-    uint16_t* stage_all = reinterpret_cast<uint16_t*>(dsmem + (size_t)tiles_per_wg * ZB_BYTES);
-    uint16_t* stage = stage_all + wave * (ZUNITS * 256);      // this wavefront's own
-    int2* assigns = reinterpret_cast<int2*>(stage_all + DN_SLABS_PER_WG * (ZUNITS * 256));      // (token, routing weight) per assignment
-    static_assert(ZUNITS * 256 * sizeof(uint16_t) >= SLAB_ROWS * sizeof(int2), "the rows' records take the stage's place");
+    uint16_t* z = reinterpret_cast<uint16_t*>(dsmem);
+    const int z_stride = tiles_per_wg * N_TILE + 8;      // (the workgroup's own tiles)
+    float* zsum = reinterpret_cast<float*>(dsmem + (size_t)MAX_A * z_stride * 2);      // [assignment][tile]
+    int2* rows = reinterpret_cast<int2*>(zsum + MAX_A * ZSUM_STRIDE) + wave * SLAB_ROWS;     // this wavefront's (rank, multiplier) per row
+    int2* assigns = reinterpret_cast<int2*>(zsum + MAX_A * ZSUM_STRIDE) + DN_SLABS_PER_WG * SLAB_ROWS;    // (token, routing weight) per assignment
 
     // the four wavefronts may run four different instantiations; every one of them executes
     // the same two workgroup barriers per assignment chunk
-    // (neighbouring workgroups' first batches of z go to different SIMDs)
-    const int z_turn = (wave + k_in_xcd) & 3;
-    auto run = [&](auto w_c) {
-        down_wave<decltype(w_c)::value, ZREADY>(payload, scale, svec, rank_idx, fs, G, U, n_part, part_stride, as, a_begin, a_end, T, I,
-                                                tb, nt, rank_out, rank_accum, zrec, stage, assigns, z_turn, lane);
-    };
     if (fs.bits == 2)
-        run(std::integral_constant<int, 2>{});
+        down_wave<2, ZREADY, ZR, ZBY>(payload, scale, svec, rank_idx, fs, G, U, n_part, part_stride, as, a_begin, a_end, T, I, tb, nt,
+                           rank_out, rank_accum, z, z_stride, zsum, rows, assigns, tid, lane);
     else if (fs.bits == 3)
-        run(std::integral_constant<int, 3>{});
+        down_wave<3, ZREADY, ZR, ZBY>(payload, scale, svec, rank_idx, fs, G, U, n_part, part_stride, as, a_begin, a_end, T, I, tb, nt,
+                           rank_out, rank_accum, z, z_stride, zsum, rows, assigns, tid, lane);
     else if (fs.bits == 4)
-        run(std::integral_constant<int, 4>{});
+        down_wave<4, ZREADY, ZR, ZBY>(payload, scale, svec, rank_idx, fs, G, U, n_part, part_stride, as, a_begin, a_end, T, I, tb, nt,
+                           rank_out, rank_accum, z, z_stride, zsum, rows, assigns, tid, lane);
     else
-        run(std::integral_constant<int, 0>{});
+        down_wave<0, ZREADY, ZR, ZBY>(payload, scale, svec, rank_idx, fs, G, U, n_part, part_stride, as, a_begin, a_end, T, I, tb, nt,
+                           rank_out, rank_accum, z, z_stride, zsum, rows, assigns, tid, lane);
     BITSMOE_TL(g_tl_down, 6);
 }
 
@@ -727,7 +751,8 @@ static inline void record(bitsmoe_profile* p, int i, hipStream_t st) {
 
 bool decode_path_supported(const bitsmoe_matset* gate, const bitsmoe_matset* up, const bitsmoe_matset* down, int I) {
     const int n_tiles = (I + N_TILE - 1) / N_TILE;
-    return n_tiles <= MAX_DECODE_TILES && gate->role == ROLE_GATE_UP && up->role == ROLE_GATE_UP && down->role == ROLE_DOWN;
+    const size_t z_bytes = (size_t)MAX_A * (n_tiles * N_TILE + 8) * 2 + MAX_A * ZSUM_STRIDE * 4 + DN_SLABS_PER_WG * SLAB_ROWS * 8 + MAX_A * 8;
+    return n_tiles <= ZSUM_STRIDE && gate->role == ROLE_GATE_UP && up->role == ROLE_GATE_UP && down->role == ROLE_DOWN && z_bytes <= 65536;
 }
 
 // Can the decode kernels find their assignments among the routed ids themselves (no routing tables)?
@@ -771,7 +796,7 @@ int launch_forward_decode(const bitsmoe_matset* gate, const bitsmoe_matset* up, 
         if (rc != BITSMOE_OK) return rc;
         record(prof, 2, st);
         record(prof, 3, st);
-        rc = launch_wide_down(down, G, U, WIDE_Z_SUMS, 1, 2 * inter_floats, tok, off, rw, A, I, rank_out, rank_accum, st);
+        rc = launch_wide_down(down, G, U, false, 1, 2 * inter_floats, tok, off, rw, A, I, rank_out, rank_accum, st);
         if (rc != BITSMOE_OK) return rc;
         record(prof, 4, st);
         record(prof, 5, st);
@@ -899,10 +924,10 @@ int launch_forward_decode(const bitsmoe_matset* gate, const bitsmoe_matset* up, 
     auto launch_walk_z_mode = [&](auto bf16_c, auto mode_c) {
         auto kern = k_gateup_walk_z<decltype(bf16_c)::value, decltype(mode_c)::value, false>;
         if (gate->rank_identity && up->rank_identity) kern = k_gateup_walk_z<decltype(bf16_c)::value, decltype(mode_c)::value, true>;
-        // Z takes the place of G in the workspace, Zlow that of U
+        // Z takes the place of G in the workspace, Zsum that of U
         hipLaunchKernelGGL(kern, dim3((unsigned)(e_dim * n_tiles)), dim3(256), 0, st, gate->d_fast_experts, gate->d_fast_slabs,
                            up->d_fast_experts, up->d_fast_slabs, gate->prep_max_slabs, (const uint16_t*)h_gate, (const uint16_t*)h_up,
-                           ldg, ldu, tok, off, (int)T, (int)A, I, E, n_tiles, (uint16_t*)G, (uint16_t*)U, rank_accum,
+                           ldg, ldu, tok, off, (int)T, (int)A, I, E, n_tiles, (uint16_t*)G, U, rank_accum,
                            T * (int64_t)rank_out, gate_order);
     };
     if (fused_z) {
@@ -939,23 +964,23 @@ int launch_forward_decode(const bitsmoe_matset* gate, const bitsmoe_matset* up, 
     float* down_u = U;
     if (split_z) {
         uint16_t* Z = reinterpret_cast<uint16_t*>(G + parts_in * part_stride);
-        uint16_t* Zlow = reinterpret_cast<uint16_t*>(U + parts_in * part_stride);
-        const int64_t n4 = A * (int64_t)I / 4;
-        hipLaunchKernelGGL(k_decode_silu, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, st, G, U, parts_in, part_stride, n4, Z, Zlow);
+        float* Zsum = U + parts_in * part_stride;
+        const int64_t threads = A * (int64_t)n_tiles * 32;
+        hipLaunchKernelGGL(k_decode_silu, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st, G, U, parts_in, part_stride,
+                           (int)A, I, n_tiles, Z, Zsum);
         BITSMOE_HIP_TRY(hipGetLastError());
         down_g = reinterpret_cast<float*>(Z);
-        down_u = reinterpret_cast<float*>(Zlow);
+        down_u = Zsum;
     }
     record(prof, 3, st);      // (otherwise SiLU happens inside the down kernel)
     const int dn_groups = (down->prep_max_slabs + DN_SLABS_PER_WG - 1) / DN_SLABS_PER_WG;
-    int dn_tiles_per_wg = (n_tiles + policy::DOWN_DECODE_MAX_TILES - 1) / policy::DOWN_DECODE_MAX_TILES;      // (shares of a row)
-    dn_tiles_per_wg = (n_tiles + dn_tiles_per_wg - 1) / dn_tiles_per_wg;
+    int dn_tiles_per_wg = n_tiles;
     // (600 measured best on the 26-layer stack at 32 tokens against 300, 1200 and 2400: the kernel is bound by the
     // instructions a workgroup issues, and more, shorter workgroups add their fixed part)
     while (dn_tiles_per_wg > 1 &&
            units * dn_groups * ((n_tiles + dn_tiles_per_wg - 1) / dn_tiles_per_wg) < policy::DOWN_DECODE_MIN_WORKGROUPS)
         dn_tiles_per_wg = (dn_tiles_per_wg + 1) / 2;
-    const size_t z_bytes = (size_t)dn_tiles_per_wg * ZB_BYTES + DN_SLABS_PER_WG * (ZUNITS * 256) * 2 + MAX_A * 8;
+    const size_t z_bytes = (size_t)MAX_A * (dn_tiles_per_wg * N_TILE + 8) * 2 + MAX_A * ZSUM_STRIDE * 4 + DN_SLABS_PER_WG * SLAB_ROWS * 8 + MAX_A * 8;
     const int dn_tchunks = (n_tiles + dn_tiles_per_wg - 1) / dn_tiles_per_wg;
     auto launch_down = [&](auto kernel) {
         const int n_work = e_dim * dn_groups * dn_tchunks;
@@ -970,13 +995,33 @@ int launch_forward_decode(const bitsmoe_matset* gate, const bitsmoe_matset* up, 
     auto launch_down_mode = [&](auto zready_c, auto mode_c) {
         constexpr int M = decltype(mode_c)::value;
         constexpr bool Z = decltype(zready_c)::value;
+        // (z beyond 40 KB: at most three workgroups per CU fit the LDS, the kernel compiled for three takes more
+        // rows of G / U per round trip)
+        const bool wide = !Z && z_bytes > 40 * 1024;
         if constexpr (M != GRID_CHUNKS && !Z) {
             if (routed) {
-                launch_down(k_down_decode<M, Z, true>);
+                if (wide)
+                    launch_down(k_down_decode<M, Z, true, ZROWS_WIDE>);
+                else
+                    launch_down(k_down_decode<M, Z, true, ZROWS>);
                 return;
             }
         }
-        launch_down(k_down_decode<M, Z, false>);
+        if constexpr (!Z) {
+            if (wide) {
+                launch_down(k_down_decode<M, Z, false, ZROWS_WIDE>);
+                return;
+            }
+        }
+        // z a row per wavefront: from five assignments per expert on average (512-expert layer, 256 tokens, top-10: the
+        // kernel 5 % faster; 128 experts with four per expert: no difference; with one or two: slower)
+        if constexpr (!Z && M != GRID_CHUNKS) {
+            if (A >= policy::DOWN_Z_BY_ROWS_MIN_PER_EXPERT * (int64_t)E) {
+                launch_down(k_down_decode<M, Z, false, ZROWS, true>);
+                return;
+            }
+        }
+        launch_down(k_down_decode<M, Z, false, ZROWS>);
     };
     // (G and U are fp32 and the operands f16 whatever the activation type was)
     if (fused_z || split_z)
@@ -985,7 +1030,7 @@ int launch_forward_decode(const bitsmoe_matset* gate, const bitsmoe_matset* up, 
         with_mode(launch_down_mode, std::false_type{});
     BITSMOE_HIP_TRY(hipGetLastError());
     if (has_wide_rows(down)) {      // (behind the gate/up kernel, which cleared rank_accum)
-        const int rc = launch_wide_down(down, down_g, down_u, split_z ? WIDE_Z_F16 : WIDE_Z_SUMS, split_z ? 1 : parts_in, part_stride, tok, off, rw, A, I,
+        const int rc = launch_wide_down(down, down_g, down_u, split_z, split_z ? 1 : parts_in, part_stride, tok, off, rw, A, I,
                                         rank_out, rank_accum, st);
         if (rc != BITSMOE_OK) return rc;
     }

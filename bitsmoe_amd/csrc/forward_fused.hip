@@ -64,6 +64,7 @@ constexpr int FUSED_MAX_DOWN_SLABS = 64;       // per expert: 16 per wavefront
 template <int WD>
 struct DownRing {
     static constexpr int NB = WD == 2 ? 8 : WD == 3 ? 5 : 4;
+    static constexpr int BW = WD == 3 ? R1W3_BLOCK_WORDS : 256 * WD;
     // Which ring slot the walk's tail call k = 0 .. 15 fills (-1: none): call k comes when the k-th of the sixteen
     // slab buffers of the walk's last two groups has been multiplied, so the ring fills as those drain -- spread so
     // that the registers of both together stay inside the budget (2-bit: half of the ring per group; wider blocks:
@@ -91,16 +92,58 @@ template <int WD, int B>
 __device__ __forceinline__ void down_issue(DownRing<WD>& ring, const DownSource& src, int wave, uint32_t lane, int i) {
     const uint32_t si = (uint32_t)(wave + 4 * i);
     const uint32_t st = si * (uint32_t)src.n_tiles + (uint32_t)src.t;      // (slab, tile) index, wave-uniform
-    load_block_role1<WD>(src.payload + st * (uint32_t)block_words(WD), (int)lane, ring.buf[B]);
-    ring.sc[B] = (reinterpret_cast<gptr<uint16_t>>(src.scale) + st * (uint32_t)SLAB_ROWS)[r1_scale_pos((int)lane)];
+    gptr<uint32_t> blk = src.payload + st * (uint32_t)DownRing<WD>::BW;
+    gptr_u32x4 p = reinterpret_cast<gptr_u32x4>(blk + (WD == 4 ? lane * 16u : WD == 3 ? lane * 4u : lane * 8u));
+    u32x4 v0 = p[0], v1, v2 = {0, 0, 0, 0}, v3 = {0, 0, 0, 0};
+    if constexpr (WD == 3) {
+        v1 = p[64];       // (+256 words)
+        v2 = p[128];
+        v3[0] = blk[768u + lane];
+    } else {
+        v1 = p[1];
+    }
+    if constexpr (WD == 4) {
+        v2 = p[2];
+        v3 = p[3];
+    }
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+        ring.buf[B].w[x] = v0[x];
+        ring.buf[B].w[4 + x] = v1[x];
+        ring.buf[B].w[8 + x] = v2[x];
+        ring.buf[B].w[12 + x] = v3[x];
+    }
+    ring.sc[B] = (reinterpret_cast<gptr<uint16_t>>(src.scale) + st * (uint32_t)SLAB_ROWS)[lane];
     ring.sv[B] = (reinterpret_cast<gptr<uint16_t>>(src.svec) + si * (uint32_t)SLAB_ROWS)[lane];
     ring.rk[B] = (src.rank_idx + si * (uint32_t)SLAB_ROWS)[lane];
+}
+
+// One (slab, tile) block of a down matrix without its scale: 4 row blocks x 4 k-steps; acc[nb][j] = sum over the
+// tile's columns of level[16 nb + n, c] * z[4 kg + j, c] (the constant term of the 2^W + code operands removed).
+template <int W>
+__device__ __forceinline__ void down_block_raw(const Block16& b, const u32x4 (&az)[4], f32x4 corr, f32x4 (&acc)[4]) {
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb) {
+        f32x4 t = {0, 0, 0, 0};
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+            u32x4 bw;
+            if constexpr (W == 2)
+                bw = decode_fields2<2, false>(b.w[nb * 2 + (m >> 1)], 8 * (m & 1));
+            else if constexpr (W == 4)
+                bw = decode_fields4<false>(b.w[nb * 4 + m]);
+            else
+                bw = decode_r1w3<false>(b.w, nb, m);
+            t = mfma16<false>(az[m], bw, t);
+        }
+        acc[nb] = t - corr;
+    }
 }
 
 // z of the workgroup's tile from the gate and up sums in registers, then the down projection of that tile.
 //   g, u       the lane's sums: rows a = 4*kg + j of columns 32*wave + 16*nbl + n
 //   n_pre      blocks of the ring that have been requested already (by the walk's tail)
-//   z_lds      2 x 16 x FZ_STRIDE 16-bit; assigns 16 x (token or -1, routing weight)
+//   z_lds      16 x FZ_STRIDE 16-bit; zs_lds 4 x 16 floats; assigns 16 x (token or -1, routing weight)
 //   tbuf_all   LDS the gate / up walks are done with: 4 x 16 x FT_STRIDE floats, one buffer per wavefront
 // The combine goes through a transposition in LDS: the MFMA leaves a lane with four assignments of four rows; the
 // wavefront writes its 16 x 64 block and reads it back with lane = row, so that one atomic instruction per REAL
@@ -109,7 +152,7 @@ template <int WD, class AS>
 __device__ __forceinline__ void fused_z_down(DownRing<WD>& ring, int n_pre, const f32x4 (&g)[2], const f32x4 (&u)[2],
                                              const DownSource& src, const AS& as, int a0, int n_a, int T, int rank_out,
                                              float* __restrict__ rank_accum, uint16_t* __restrict__ z_lds,
-                                             int2* __restrict__ assigns,
+                                             float* __restrict__ zs_lds, int2* __restrict__ assigns,
                                              float* __restrict__ tbuf_all, int tid, bool stamp) {
     constexpr int NB = DownRing<WD>::NB;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -126,38 +169,45 @@ __device__ __forceinline__ void fused_z_down(DownRing<WD>& ring, int n_pre, cons
     const int tok_lane = as.token_if(a0 + lane, lane < n_a);
     const float rw_lane = as.weight_if(a0 + lane, lane < n_a);
 
-    // z = silu(G) * U as f16 values, and their remainders behind them
+    // z = silu(G) * U as 16-bit operands, and the sums of the rounded operands per assignment row
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const int a = g4 + j;
-        ZPair z = z_pair(g[0][j], u[0][j], g[1][j], u[1][j]);
-        if (a >= n_a) z = ZPair{0, 0};      // (rows without an assignment hold whatever LDS held)
-        uint16_t* at = z_lds + a * FZ_STRIDE + 32 * wave + n;
-        at[0] = (uint16_t)z.hi;
-        at[16] = (uint16_t)(z.hi >> 16);
-        at[MAX_A * FZ_STRIDE] = (uint16_t)z.lo;
-        at[MAX_A * FZ_STRIDE + 16] = (uint16_t)(z.lo >> 16);
+        float v = 0.0f;
+#pragma unroll
+        for (int nbl = 0; nbl < 2; ++nbl) {
+            uint16_t zb = z_operand(g[nbl][j], u[nbl][j]);
+            if (a >= n_a) zb = 0;      // (rows without an assignment hold whatever LDS held)
+            z_lds[a * FZ_STRIDE + 32 * wave + 16 * nbl + n] = zb;
+            v += __half2float(__ushort_as_half(zb));
+        }
+        v = dpp_add_f32<0x111>(v);
+        v = dpp_add_f32<0x112>(v);
+        v = dpp_add_f32<0x114>(v);
+        v = dpp_add_f32<0x118>(v);
+        if (n == 15) zs_lds[wave * MAX_A + a] = v;
     }
     if (tid < MAX_A) assigns[tid] = int2{(tok_lane >= 0 && tok_lane < T) ? tok_lane : -1, __float_as_int(rw_lane)};
-    __syncthreads();      // z and the assignment records are complete
+    __syncthreads();      // z, its sums and the assignment records are complete
     if (stamp) BITSMOE_STAMP(4);
 
-    // the operand and the constant term are the same for every slab; every wavefront makes the tile's records for itself, a lane
-    // the one of row n and columns 32 kg .. +31 that it feeds to the MFMA
-    ZOperand zo;
+    // the operand and the constant term are the same for every slab
+    u32x4 az[4];
     {
-        const uint16_t* zp = z_lds + n * FZ_STRIDE + Z_BLOCK * kg;
-        const u32x4* zv = reinterpret_cast<const u32x4*>(zp);
-        const u32x4* zw = reinterpret_cast<const u32x4*>(zp + MAX_A * FZ_STRIDE);
-        float none;
-        const ZRecord rec = z_record<false>(F16x32{zv[0], zv[1], zv[2], zv[3]}, F16x32{zw[0], zw[1], zw[2], zw[3]}, none);
-        zo = z_operand_of(rec);
+        const uint16_t* zp = z_lds + n * FZ_STRIDE + 8 * kg;
+#pragma unroll
+        for (int m = 0; m < 4; ++m) az[m] = *reinterpret_cast<const u32x4*>(zp + 32 * m);
     }
-    const f32x4 c0 = down_constant<WD>(zo);
+    f32x4 corr;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int a = g4 + j;
+        corr[j] = (zs_lds[a] + zs_lds[MAX_A + a] + zs_lds[2 * MAX_A + a] + zs_lds[3 * MAX_A + a]) * (1.5f * (float)(1 << WD));
+    }
     auto compute = [&](auto b_c) {
         constexpr int B = decltype(b_c)::value;
         f32x4 acc[4];
-        down_block<WD>(ring.buf[B], zo, c0, [&](int nb, f32x4 t) { acc[nb] = t; });
+        down_block_raw<WD>(ring.buf[B], az, corr, acc);
 #pragma unroll
         for (int nb = 0; nb < 4; ++nb)
 #pragma unroll
@@ -448,7 +498,8 @@ __global__ __launch_bounds__(256, 3) void k_decode_fused(
     // (the operand buffers of the gate / up walks; the down phase transposes its results there)
     __shared__ __attribute__((aligned(16))) uint16_t hs_all[2 * MAX_A * GU_STRIDE];
     __shared__ float cterm_lds[2 * MAX_A];
-    __shared__ __attribute__((aligned(16))) uint16_t z_lds[2 * MAX_A * FZ_STRIDE];
+    __shared__ __attribute__((aligned(16))) uint16_t z_lds[MAX_A * FZ_STRIDE];
+    __shared__ float zs_lds[4 * MAX_A];
     __shared__ int2 assigns[MAX_A];
     static_assert(sizeof(uint16_t) * 2 * MAX_A * GU_STRIDE >= sizeof(float) * 4 * MAX_A * FT_STRIDE,
                   "the down phase's transposition buffers must fit the operand buffers");
@@ -484,7 +535,7 @@ __global__ __launch_bounds__(256, 3) void k_decode_fused(
                                                                  }
                                                              });
                 if (first_chunk) BITSMOE_STAMP(3);
-                fused_z_down<W>(ring, DownRing<W>::NB, g, u, dsrc, as, a0, n_a, T, rank_out, rank_accum, z_lds,
+                fused_z_down<W>(ring, DownRing<W>::NB, g, u, dsrc, as, a0, n_a, T, rank_out, rank_accum, z_lds, zs_lds,
                                 assigns, tbuf_all, tid_c, first_chunk);
             };
             if (wd == 2)
@@ -515,7 +566,7 @@ __global__ __launch_bounds__(256, 3) void k_decode_fused(
             auto down = [&](auto w_c) {
                 constexpr int WD = decltype(w_c)::value;
                 DownRing<WD> ring;
-                fused_z_down<WD>(ring, 0, g, u, dsrc, as, a0, n_a, T, rank_out, rank_accum, z_lds, assigns, tbuf_all, tid_c,
+                fused_z_down<WD>(ring, 0, g, u, dsrc, as, a0, n_a, T, rank_out, rank_accum, z_lds, zs_lds, assigns, tbuf_all, tid_c,
                                  first_chunk);
             };
             if (wd == 2)

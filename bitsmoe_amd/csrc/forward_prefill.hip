@@ -7,27 +7,26 @@
 //                    token_start = exclusive scan of the per-token assignment counts
 //   k_bf16_to_f16 /  activations as f16, read through the token index by the GEMM kernel, or
 //   k_pregather      Hs[a, k] = f16( h[tok_a, rank_idx[k]] ) in expert-sorted assignment order
-//   k_gateup_mfma    G = Hs_gate . W_gate, U = Hs_up . W_up as f16;  k_silu_records: z = silu(G) * U as records of fp6 planes
+//   k_gateup_mfma    G = Hs_gate . W_gate, U = Hs_up . W_up as f16;  k_silu_mul_f16: z = silu(G) * U
 //   k_down_mfma      y[a, r] = s[r] * sum_c W_down[r, c] z[a, c] as f16, and the per-token lists
 //   k_combine_tokens rank_accum[t, rank_idx[r]] = sum over the assignments of t of route_w * y
 //
-// The gate/up kernel uses 16x16x32 f16 MFMA with four wavefronts of 128 rows x 64 columns per
+// Both GEMM kernels use 16x16x32 f16 MFMA with four wavefronts of 128 rows x 64 columns per
 // workgroup.  Activations, payload words and scales come straight from global memory into a ring of LDS stages; every lane
 // takes its words of the prepared payload (wave_layout.h) from there and expands them to packed f16 pairs
 // (2^w + code) with a rotate and an and-or; a packed add and a packed multiply turn the pair
-// into (code - 2^(w-1)) * scale * s (folded once at prepare time) -- the same
+// into (code - 2^(w-1)) * scale (gate/up: scale * s, folded once at prepare time) -- the same
 // "weight rounded to half" operand the reference's tensor-core path builds
-// (bitsmoe/algorithms/cpp/mlp_forward.cu:691-751).  Its operands are f16 for f16 and bf16 inputs alike (f16 keeps more mantissa
-// than bf16).  The down kernel multiplies the codes themselves with z's planes (z_planes.h).  The top-k combine is a gather
+// (bitsmoe/algorithms/cpp/mlp_forward.cu:691-751, 1554-1694).  The top-k combine is a gather
 // per token instead of the reference's fp32 atomics (mlp_forward.cu:2036-2066): its result
 // does not depend on the order in which workgroups finish.
+// Operands are f16 for f16 and bf16 inputs alike (f16 keeps more mantissa than bf16).
 #include <algorithm>
 #include <type_traits>
 
 #include "fast_helpers.h"
 #include "launch_policy.h"
 #include "mtiles.h"
-#include "z_planes.h"
 
 // ---- optional in-kernel time stamps (timeline build: -DBITSMOE_TIMELINE) of k_gateup_mfma / k_down_mfma: thread 0 of a
 // workgroup writes the 100 MHz wall clock at: 0 entry, 1 tile record and tables at hand, 2 first pieces landed (before the
@@ -49,6 +48,13 @@ __device__ unsigned long long g_tl_pf_down[TLP_MAX_WG * TLP_STAMPS];
 #endif
 
 namespace bitsmoe {
+
+// -(1.5 * 2^W) as a packed f16 pair: times the scale it is the constant that turns
+// (2^W + code) * scale into (code - 2^(W-1)) * scale.
+template <int W>
+__device__ inline uint32_t neg_offset_pair() {
+    return Codec<W, false>::CORR | 0x80008000u;
+}
 
 // ------------------------------------------------------------------------------ schedule
 // slot[a] = how many assignments of the same token were counted before a (any order);
@@ -248,6 +254,9 @@ template <int N>
 __device__ __forceinline__ void wait_vmcnt() {
     __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N >> 4) << 14) | 0x0F70);
 }
+// s_waitcnt lgkmcnt(0) alone: every LDS read of the wavefront has returned (the vector-memory and
+// export counters are left at their maxima).
+__device__ __forceinline__ void wait_lds_reads() { __builtin_amdgcn_s_waitcnt(0xC07F); }
 // Workgroup barrier without the wait for outstanding loads that __syncthreads implies.  The empty
 // asm statements keep the compiler from moving LDS accesses across it (the bare instruction is no
 // memory fence for the compiler).
@@ -569,7 +578,7 @@ __device__ __forceinline__ void gateup_tile_body(const FastExpert fe, const Fast
 // grid.x = 32 * ceil(max_mtiles / 32) * (2 or 1 projections) * ceil(n_tiles / 2), 256 threads; G and U are f16 [A, I].
 // PFM: assignments per tile at most.  With 128 the ring takes 78 KB of LDS and a wavefront up to 247 registers: two workgroups
 // per CU.  With 64 (53 KB, 145 registers: three) a short tile's step -- a quarter or half of the MFMAs behind the same loads,
-// waits and barrier -- is hidden by one more workgroup (rule and measurements: launch_policy.h).
+// waits and barrier -- is hidden by one more workgroup (rule and measurements: launch_policy.h); k_down_mfma likewise.
 template <bool DIRECT, int PFM, bool FUSE>
 __global__ __launch_bounds__(256, PFM == 128 ? 2 : 3) void k_gateup_mfma(
     const FastExpert* __restrict__ gate_fe, const FastSlab* __restrict__ gate_fs, int gate_max_slabs,
@@ -643,174 +652,224 @@ __global__ __launch_bounds__(256, PFM == 128 ? 2 : 3) void k_gateup_mfma(
     BITSMOE_TLP(g_tl_pf_gateup, 6);
 }
 
-// z = f16( silu(G) * U ) as the records the down kernel multiplies (z_planes.h), written over the sums: the records of a
-// (row, tile of 128 columns) take the tile's 256 bytes of the row of G (pieces 0 to 3 of the four records, piece-major) and
-// the first 64 bytes of the tile in the row of U (piece 4).  A wavefront makes the 64 records of sixteen neighbouring (row, tile)s:
-// 4 KB of G and of U, read and written a KB at a time and turned in LDS of its own (a lane's record is 64 bytes of a row: read
-// as they lie, 16 bytes from every 64, the pass over 4096 tokens' sums takes 32 us).  It has read all of its sums before it
-// stores the first piece.
-// `plain`: G holds z already (the up launch's epilogue formed it), U is not read.
-__global__ __launch_bounds__(256) void k_silu_records(uint16_t* G, uint16_t* U, int64_t n_units, int plain) {
-    __shared__ __attribute__((aligned(16))) u32x4 turn_all[4 * 512];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    u32x4* turn = turn_all + wave * 512;
-    u32x4* turn_low = turn + 256;
-    const int64_t u0 = ((int64_t)blockIdx.x * 4 + wave) * 16;      // first (row, tile) of this wavefront
-    if (u0 >= n_units) return;                      // (nobody waits for the whole workgroup)
-    const int n_pieces = (int)min((int64_t)16, n_units - u0) * 16;
-    u32x4* g = reinterpret_cast<u32x4*>(G) + u0 * 16;
-    u32x4* u = reinterpret_cast<u32x4*>(U) + u0 * 16;
-    // (slots of a unit permuted by the unit: neither pass meets a bank twice)
-    auto slot = [](int unit, int p) { return unit * 16 + (p ^ unit); };
+// z = f16( silu(G) * U ), written over G; 8 elements per thread and iteration.
+__global__ __launch_bounds__(256) void k_silu_mul_f16(uint16_t* __restrict__ G, const uint16_t* __restrict__ U, int64_t n8) {
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n8; i += (int64_t)gridDim.x * blockDim.x) {
+        const u32x4 g = *reinterpret_cast<const u32x4*>(G + i * 8);
+        const u32x4 u = *reinterpret_cast<const u32x4*>(U + i * 8);
+        u32x4 o;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const int p = 64 * k + lane;
-        const int at = min(p, n_pieces - 1);        // (past the end: the last piece again)
-        u32x4 z = g[at], low = {0, 0, 0, 0};
-        if (!plain) {
-            const u32x4 v = u[at];
-#pragma unroll
-            for (int x = 0; x < 4; ++x) {
-                const uint32_t gw = z[x], uw = v[x];
-                const h2 g2 = __builtin_bit_cast(h2, gw), u2 = __builtin_bit_cast(h2, uw);
-                const ZPair r = z_pair((float)g2[0], (float)u2[0], (float)g2[1], (float)u2[1]);
-                z[x] = r.hi;
-                low[x] = r.lo;
-            }
+        for (int k = 0; k < 4; ++k) {
+            const float g0 = __half2float(__ushort_as_half((uint16_t)(g[k] & 0xFFFFu)));
+            const float g1 = __half2float(__ushort_as_half((uint16_t)(g[k] >> 16)));
+            const float u0 = __half2float(__ushort_as_half((uint16_t)(u[k] & 0xFFFFu)));
+            const float u1 = __half2float(__ushort_as_half((uint16_t)(u[k] >> 16)));
+            const uint32_t lo = z_operand(g0, u0);
+            const uint32_t hi = z_operand(g1, u1);
+            o[k] = lo | (hi << 16);
         }
-        turn[slot(p >> 4, p & 15)] = z;
-        turn_low[slot(p >> 4, p & 15)] = low;
+        *reinterpret_cast<u32x4*>(G + i * 8) = o;
     }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
-    __builtin_amdgcn_wave_barrier();
-    const int unit = lane >> 2, kg = lane & 3;
-    auto values = [&](const u32x4* t) {
-        return F16x32{t[slot(unit, 4 * kg)], t[slot(unit, 4 * kg + 1)], t[slot(unit, 4 * kg + 2)], t[slot(unit, 4 * kg + 3)]};
-    };
-    float sum;
-    ZRecord rec = z_record<true>(values(turn), values(turn_low), sum);
-    rec.e[3] = __float_as_uint(quad_sum(sum));
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
-    __builtin_amdgcn_wave_barrier();
-    turn[slot(unit, kg)] = rec.a;
-    turn[slot(unit, 4 + kg)] = rec.b;
-    turn[slot(unit, 8 + kg)] = rec.c;
-    turn[slot(unit, 12 + kg)] = rec.d;
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
-    __builtin_amdgcn_wave_barrier();
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const int p = 64 * k + lane;
-        if (p < n_pieces) g[p] = turn[slot(p >> 4, p & 15)];
-    }
-    if (unit * 16 < n_pieces) u[unit * 16 + kg] = rec.e;
 }
 
 // ----------------------------------------------------------------------------------- down
 constexpr int DN_SLABS_MFMA = 4;   // slabs (64 output rows each) per workgroup: one per wavefront
-constexpr int DN_ROWS = 64;        // assignments per workgroup
-constexpr int DN_MB = DN_ROWS / 16;
-constexpr int DN_STAGE = DN_MB * ZB_BYTES;      // bytes of one tile's z records of the workgroup's rows
 
-// LDS place of the 16-byte piece `p` (0..4) of the record (row n, 32-column block kg) of a 16-row block's records of a tile: the
-// pieces 0 to 3 as [row][16 slots], the pieces 4 behind them as [row][4 slots], the slots of a row permuted by the row
-// so that the sixteen rows an operand load touches fall into different banks.
-__device__ __forceinline__ int z_piece_at(int n, int kg, int p) {
-    return p < 4 ? n * 256 + (((4 * p + kg) ^ n) << 4) : 4096 + n * 64 + ((kg ^ ((n >> 2) & 3)) << 4);
-}
-
-// One (slab, tile) block against the workgroup's rows: acc[mb][nb] += scale * (codes x z - 2^(W-1) sum z).  The codes are the
-// MFMA's first operand: a lane holds, of assignment 16 mb + lane % 16, outputs 16 nb + 4 (lane / 16) + j.  `next()` requests the
-// block behind this one into the same registers, once the operands have been made.
-template <int W, int NMB, class Next>
-__device__ __forceinline__ void down_mfma_block(const Block16& blk, u32x4 sc0, u32x4 sc1, const unsigned char* stage, int lane,
-                                                f32x4 (&acc)[DN_MB][4], Next&& next) {
-    using F = CodeFormat<W>;
-    const u32x4 q0 = opaque(blk.q0), q1 = opaque(blk.q1), q2 = W >= 3 ? opaque(blk.q2) : q0, q3 = W >= 4 ? opaque(blk.q3) : q0;
+// Half a tile (64 columns = micro-tiles 2*HH, 2*HH+1) of one (slab, tile) block for a
+// wavefront's 128 assignments x 64 output rows.  scp: this lane's row scale in both halves of a
+// pair, per 16-row block.  The weight operand is (code - 2^(W-1)) * scale rounded once to f16,
+// the operand the reference builds (bitsmoe/algorithms/cpp/mlp_forward.cu:1554-1694).
+template <int HH, int NMB>
+__device__ __forceinline__ void down_half_mfma(int bits, const uint16_t* stage, const Block16& blk,
+                                      const uint32_t (&scp)[4], int lane, f32x4 (&acc)[NMB][4]) {
     const int n = lane & 15, kg = lane >> 4;
-    auto record = [&](int mb) {
-        auto piece = [&](int p) { return *reinterpret_cast<const u32x4*>(stage + mb * ZB_BYTES + z_piece_at(n, kg, p)); };
-        return ZRecord{piece(0), piece(1), piece(2), piece(3), piece(4)};
-    };
-    // the row blocks NA, NA + 1 (and two more: N == 4) against all rows
-    auto rows_by = [&](auto n_c, auto na_c) {
-        constexpr int N = decltype(n_c)::value, NA = decltype(na_c)::value;
-        i32x8 lo[N], hi[N];
-        static_for([&](auto xc) {
-            constexpr int x = decltype(xc)::value;
-            code_operands<W, NA + x>(q0, q1, q2, q3, lo[x], hi[x]);
-        }, std::make_integer_sequence<int, N>{});
-        if constexpr (NA + N == 4) next();
-        ZRecord rec = record(0);
-        static_for([&](auto mc) {
-            constexpr int mb = decltype(mc)::value;
-            const ZOperand z = z_operand_of(rec);
-            const float c0 = __uint_as_float(rec.e[3]) * (-0.5f * (float)(1 << W));
-            if constexpr (mb + 1 < NMB) rec = record(mb + 1);      // (behind this one's MFMAs)
-            f32x4 t[N];
-            static_for([&](auto xc) { t[decltype(xc)::value] = f32x4{c0, c0, c0, c0}; }, std::make_integer_sequence<int, N>{});
-            static_for([&](auto pc) {
-                constexpr int P = decltype(pc)::value;
-                static_for([&](auto xc) {
-                    constexpr int x = decltype(xc)::value;
-                    t[x] = mfma_plane<F::FMT, P, true>(z, lo[x], F::SCALE, t[x]);
-                    if constexpr (W == 4) t[x] = mfma_plane<F::FMT, P, true>(z, hi[x], W_SCALE_FP4_HI, t[x]);
-                }, std::make_integer_sequence<int, N>{});
-            }, std::make_integer_sequence<int, 3>{});
-            // (the lane's sixteen scales come as [row 4 kg + j][nb], r1_scale_pos: word 2 (j % 2) + nb / 2 of piece j / 2)
-            static_for([&](auto xc) {
-                constexpr int x = decltype(xc)::value, NB = NA + x;
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const uint32_t s2 = (j < 2 ? sc0 : sc1)[2 * (j & 1) + NB / 2];
-                    acc[mb][NB][j] += t[x][j] * (float)__builtin_bit_cast(h2, s2)[NB & 1];
-                }
-            }, std::make_integer_sequence<int, N>{});
-            __builtin_amdgcn_sched_barrier(0);
-        }, std::make_integer_sequence<int, NMB>{});
-    };
-    if constexpr (W != 4) {
-        rows_by(std::integral_constant<int, 4>{}, std::integral_constant<int, 0>{});
-    } else {      // (low and high operands take the registers of two: two row blocks at a time, the records read twice)
-        rows_by(std::integral_constant<int, 2>{}, std::integral_constant<int, 0>{});
-        rows_by(std::integral_constant<int, 2>{}, std::integral_constant<int, 2>{});
+    for (int km = 0; km < 2; ++km) {
+        const int m = 2 * HH + km;
+        u32x4 a[NMB];
+#pragma unroll
+        for (int mb = 0; mb < NMB; ++mb)
+            a[mb] = *reinterpret_cast<const u32x4*>(stage + dma_chunk_off(16 * mb + n, 4 * km + kg));
+#pragma unroll
+        for (int nb = 0; nb < 4; ++nb) {
+            // the width switch wraps one operand only: accumulators that flow through alternative
+            // paths multiply the register demand
+            u32x4 b;
+            uint32_t off;
+            if (bits == 2) {
+                b = decode_fields2<2, false>(blk.w[nb * 2 + HH], 8 * km);
+                off = neg_offset_pair<2>();
+            } else if (bits == 4) {
+                b = decode_fields4<false>(blk.w[nb * 4 + m]);
+                off = neg_offset_pair<4>();
+            } else {
+                b = decode_r1w3<false>(blk.w, nb, m);
+                off = neg_offset_pair<3>();
+            }
+            for (int i = 0; i < 4; ++i) b[i] = pk_mul_f16(pk_add_f16(b[i], off), scp[nb]);
+#pragma unroll
+            for (int mb = 0; mb < NMB; ++mb) acc[mb][nb] = mfma16<false>(b, a[mb], acc[mb][nb]);
+        }
     }
 }
 
-// Workgroup = (64 rows of an assignment tile, group of four slabs): wavefront w = the 64 assignments x the 64 output rows of slab
-// 4*group + w.  grid.x = 32 * ceil(max_mtiles / 32) * (tile rows / 64) * n_groups.
-// Output: y[a, r] = s[r] * sum_tiles scale[tile, r] * sum_{c in tile} level[r, c] z[a, c] as f16, r in the expert's own row order,
-// and the per-token assignment lists token_list[token_start[tok_a] + slot[a]] = (a, expert) that k_combine_tokens walks.
-// A step is one tile of 128 columns: its z records go from global memory straight into LDS (two stages in turn, shared by the
-// workgroup; a wavefront fetches 16 rows), the wavefront's payload and scales into registers, both a step
-// ahead of the MFMAs; one full wait and one barrier per step.  Tiles of 64 rows whatever the tile list has: the codes cost one mask
-// or shift per four weights, so that making them again for every 64 rows is nothing beside the MFMAs, and 128 rows' sums would leave
-// no registers for the next block.  (z kept in LDS for all slabs, wavefronts without barriers and 32 rows of two slabs each: 338 us
-// where this takes 129 -- payload one step of 48 MFMAs ahead arrives too late.)
+constexpr int DN_WBUF = 1024;    // 32-bit words: the payload block of one (slab, tile) as its wavefront fetches it
+constexpr int DN_SBUF = 64;      // 16-bit scales of one (slab, tile) block
+
+// The column loop of one wavefront (fs.bits == 0: no slab, the wavefront only helps to stage).
+// Everything comes straight from global memory into LDS (LDS-direct loads, no registers in
+// between): the pieces of z (128 assignments x 64 columns, chunk order of dma_chunk_off) into a
+// ring of three stages shared by the workgroup, two pieces ahead of the MFMAs; the payload block
+// and scales of the wavefront's next tile into a buffer of its own, from where they are taken
+// into registers when the tile begins.  The loads of a wavefront complete in order and every
+// wavefront issues the same number per step (four 16-byte payload loads whatever the width:
+// narrower blocks repeat an address), so "piece h + 1 has landed" is a count of outstanding
+// loads, waited for with a bare s_waitcnt before a bare barrier.
+template <int NMB>
+__device__ __forceinline__ void down_tile_loop(const uint32_t* __restrict__ payload, const __half* __restrict__ scale,
+                                      const FastSlab fs, const uint16_t* __restrict__ z, int I, int n_tiles, int a_begin, int rows,
+                                      uint16_t* st0, uint16_t* st1, uint16_t* st2, uint32_t* wbuf_all,
+                                      uint16_t* sbuf_all, int tid, int lane, f32x4 (&acc)[NMB][4]) {
+    constexpr int NJ = (NMB + 1) / 2;      // 32-row groups that hold assignments
+    constexpr int NP = 5;                  // payload and scale load instructions per tile
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n = lane & 15;
+    const int W = fs.bits;
+    uint32_t* wbuf = wbuf_all + wave * DN_WBUF;
+    uint16_t* sbuf = sbuf_all + wave * DN_SBUF;
+    // this lane lands in row r0 + 32*j, chunk position tid % 8 of a stage and fetches the chunk
+    // that belongs there
+    const int r0 = tid >> 3;
+    const int cpos = (tid & 7) ^ ((r0 >> 1) & 7);
+    uint32_t rowbase[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+        rowbase[j] = (uint32_t)(a_begin + min(r0 + 32 * j, rows - 1)) * (uint32_t)I + (uint32_t)(8 * cpos);
+    auto request_z = [&](uint16_t* st, int h) {
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+            load_to_lds16(z + (rowbase[j] + (uint32_t)(64 * h)), st + j * 2048 + wave * 512);
+    };
+    // role 1 block: 2-bit 8 words per lane, 4-bit 16, 3-bit 13 (three regions of four words per lane, the
+    // thirteenth in a region of its own: four lanes fetch the same 16 bytes and each keeps its word)
+    // (fast_helpers.h, wave_layout.h); load i fills words 4i .. 4i+3 of every lane's sixteen
+    const uint32_t lane_words = (uint32_t)lane * (W == 4 ? 16u : W == 2 ? 8u : 4u);
+    auto request_b = [&](int t) {
+        const uint32_t base = W != 0 ? (uint32_t)(fs.pack_off + t * block_words(ROLE_DOWN, W)) : 0u;
+        const uint32_t o0 = base + lane_words;
+        const uint32_t o1 = W == 3 ? o0 + 256u : W != 0 ? o0 + 4u : o0;
+        const uint32_t o2 = W == 4 ? o0 + 8u : W == 3 ? o0 + 512u : o0;
+        const uint32_t o3 = W == 4 ? o0 + 12u : W == 3 ? base + 768u + (uint32_t)(lane & ~3) : o0;
+        load_to_lds16(payload + o0, wbuf);
+        load_to_lds16(payload + o1, wbuf + 256);
+        load_to_lds16(payload + o2, wbuf + 512);
+        load_to_lds16(payload + o3, wbuf + 768);
+        const uint32_t so = W != 0 ? (uint32_t)(fs.scale_off + t * SLAB_ROWS) : 0u;
+        if (lane < 8) load_to_lds16(scale + (so + (uint32_t)lane * 8u), sbuf);
+    };
+    Block16 blk;
+    uint32_t scp[4];
+    auto take_b = [&]() {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const u32x4 v = *reinterpret_cast<const u32x4*>(wbuf + i * 256 + lane * 4);
+            blk.w[4 * i] = v[0];
+            blk.w[4 * i + 1] = v[1];
+            blk.w[4 * i + 2] = v[2];
+            blk.w[4 * i + 3] = v[3];
+        }
+        if (W == 3) {      // the thirteenth word: this lane's of the four its load brought
+            const int k = lane & 3;
+            blk.w[12] = k == 0 ? blk.w[12] : k == 1 ? blk.w[13] : k == 2 ? blk.w[14] : blk.w[15];
+        }
+#pragma unroll
+        for (int nb = 0; nb < 4; ++nb) scp[nb] = (uint32_t)sbuf[16 * nb + n] * 0x10001u;
+        // the buffer is requested again right away: its reads must have returned
+        wait_lds_reads();
+        asm volatile("" ::: "memory");
+    };
+    const int n_halves = 2 * n_tiles;      // at least two
+    request_z(st0, 0);
+    request_b(0);
+    request_z(st1, 1);
+    wait_vmcnt<NJ>();                      // block 0 and piece 0 have landed
+    barrier_no_drain();
+    BITSMOE_TLP(g_tl_pf_down, 2);
+    // step h (h % 3 == U, h % 2 == HH): (first half of a tile) the tile's block taken into
+    // registers; piece h + 2 requested into the stage piece h - 1 used, then (first half) the next
+    // tile's block; piece h multiplied
+    auto step = [&](auto u_c, auto hh_c, int h) {
+        constexpr int U = decltype(u_c)::value;
+        constexpr int HH = decltype(hh_c)::value;
+        // (the stages are named statically, so that the compiler can tell the stage being read
+        // from the ones being loaded)
+        uint16_t* cur = U == 0 ? st0 : U == 1 ? st1 : st2;
+        uint16_t* nxt = U == 0 ? st2 : U == 1 ? st0 : st1;
+        const bool more = h + 2 < n_halves;
+        if (HH == 0) take_b();
+        if (more) {
+            request_z(nxt, h + 2);
+            if (HH == 0) request_b((h >> 1) + 1);      // h + 2 < n_halves: there is a next tile
+        }
+        if (W != 0) down_half_mfma<HH, NMB>(W, cur, blk, scp, lane, acc);
+        asm volatile("" ::: "memory");
+        // piece h + 1 (and, after a second half, the next tile's block) must have landed; what this
+        // step requested may still be in flight
+        if (!more)
+            wait_vmcnt<0>();
+        else if (HH == 0)
+            wait_vmcnt<NJ + NP>();
+        else
+            wait_vmcnt<NJ>();
+        barrier_no_drain();
+    };
+    using I0 = std::integral_constant<int, 0>;
+    using I1 = std::integral_constant<int, 1>;
+    using I2 = std::integral_constant<int, 2>;
+    for (int h0 = 0; h0 < n_halves; h0 += 6) {
+        step(I0{}, I0{}, h0);
+        step(I1{}, I1{}, h0 + 1);
+        if (h0 + 2 < n_halves) {
+            step(I2{}, I0{}, h0 + 2);
+            step(I0{}, I1{}, h0 + 3);
+        }
+        if (h0 + 4 < n_halves) {
+            step(I1{}, I0{}, h0 + 4);
+            step(I2{}, I1{}, h0 + 5);
+        }
+    }
+}
+
+// grid.x = 32 * ceil(max_mtiles / 32) * n_groups; workgroup = (assignment tile, group of four
+// slabs): wavefront w = all 128 assignments x the 64 output rows of slab 4*group + w.
+// Output: y[a, r] = s[r] * sum_c W_down[r, c] z[a, c] as f16, r in the expert's own row order, and the per-token
+// assignment lists
+// token_list[token_start[tok_a] + slot[a]] = (a, expert) that k_combine_tokens walks.
 template <int PFM>
-__global__ __launch_bounds__(256, 2) void k_down_mfma(const FastExpert* __restrict__ down_fe,
+__global__ __launch_bounds__(256, PFM == 128 ? 2 : 3) void k_down_mfma(const FastExpert* __restrict__ down_fe,
                                                       const FastSlab* __restrict__ down_fs, int max_slabs,
-                                                      const uint16_t* __restrict__ zg, const uint16_t* __restrict__ zu,
-                                                      const MTile* __restrict__ mtiles,
+                                                      const uint16_t* __restrict__ z, const MTile* __restrict__ mtiles,
                                                       const int32_t* __restrict__ n_mtiles,
                                                       const int32_t* __restrict__ token_indices,
                                                       const int32_t* __restrict__ slot,
                                                       const int32_t* __restrict__ token_start,
-                                                      int2* __restrict__ token_list, int I, int n_tiles,
+                                                      int2* __restrict__ token_list, int A, int I, int n_tiles,
                                                       int n_groups, _Float16* __restrict__ y, int ldy) {
-    // two stages of z records, which the epilogue uses again: 128 bytes per row and wavefront
-    __shared__ __attribute__((aligned(16))) unsigned char lds[2 * DN_STAGE];
-    static_assert(sizeof(lds) >= 4 * dma_stage(DN_ROWS) * sizeof(uint16_t), "the epilogue's space");
-    constexpr int HALVES = PFM / DN_ROWS;
+    // three stages of z and the wavefronts' payload buffers, which the epilogue uses again: 128 bytes per row and wavefront
+    __shared__ __attribute__((aligned(16))) uint16_t lds[3 * dma_stage(PFM) + 2 * 4 * DN_WBUF];
+    constexpr int STAGE = dma_stage(PFM);
+    static_assert(sizeof(lds) >= 4 * STAGE * sizeof(uint16_t), "the epilogue's space");
+    uint16_t *sz0 = lds, *sz1 = lds + STAGE, *sz2 = lds + 2 * STAGE;
+    uint32_t* wbuf = reinterpret_cast<uint32_t*>(lds + 3 * STAGE);
+    __shared__ __attribute__((aligned(16))) uint16_t sbuf[4 * DN_SBUF];
     BITSMOE_TLP(g_tl_pf_down, 0);
-    const int logical = xcd_logical(blockIdx.x, __builtin_amdgcn_readfirstlane(*n_mtiles), n_groups * HALVES);
+    const int logical = xcd_logical(blockIdx.x, __builtin_amdgcn_readfirstlane(*n_mtiles), n_groups);
     if (logical < 0) return;
-    const int mt_i = logical / (n_groups * HALVES), unit = logical - mt_i * (n_groups * HALVES);
-    const int half = unit / n_groups, grp = unit - half * n_groups;
+    const int mt_i = logical / n_groups, grp = logical - mt_i * n_groups;
     const i32x4 tv = *reinterpret_cast<const i32x4*>(mtiles + mt_i);
     const int e = __builtin_amdgcn_readfirstlane(tv[0]);
-    const int a_begin = __builtin_amdgcn_readfirstlane(tv[1]) + half * DN_ROWS;
-    const int rows = min(__builtin_amdgcn_readfirstlane(tv[2]) - half * DN_ROWS, DN_ROWS);
+    const int a_begin = __builtin_amdgcn_readfirstlane(tv[1]);
+    const int rows = __builtin_amdgcn_readfirstlane(tv[2]);
     if (e < 0 || rows <= 0) return;
     const int tid = threadIdx.x;
     if (grp == 0 && tid < rows) {
@@ -829,92 +888,44 @@ __global__ __launch_bounds__(256, 2) void k_down_mfma(const FastExpert* __restri
     if (si < nslabs) fs = load_fast_slab(down_fs + (int64_t)e * max_slabs, si);
     BITSMOE_TLP(g_tl_pf_down, 1);
 
-    // This wavefront fetches rows 16 wave .. +15 (past the tile's: its last row again).  Pieces 0 to 3: a load covers four rows
-    // of 256 bytes, lane = 16 * row + slot; piece 4: all sixteen rows, lane = 4 * row + slot.  (Offsets in 16-byte pieces.)
-    const int z_rows = min(rows - 16 * wave, 16);
-    auto z_off = [&](int r) { return (uint32_t)(a_begin + 16 * wave + min(r, max(z_rows, 1) - 1)) * (uint32_t)(I / 8); };
-    uint32_t g_off[4], u_off;
+    // tiles of at most 32 / 64 / 96 assignments run a body with a quarter / half / three quarters of
+    // the accumulators and MFMAs: complete bodies, so that no accumulator lives across the choice
+    auto run = [&](auto nmb_c) {
+        constexpr int NMB = decltype(nmb_c)::value;
+        f32x4 acc[NMB][4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) g_off[j] = z_off(4 * j + (lane >> 4)) + (uint32_t)((lane & 15) ^ (4 * j + (lane >> 4)));
-    u_off = z_off(lane >> 2) + (uint32_t)((lane & 3) ^ ((lane >> 4) & 3));
-    const u32x4* zg_p = reinterpret_cast<const u32x4*>(zg);
-    const u32x4* zu_p = reinterpret_cast<const u32x4*>(zu);
-    auto request_z = [&](unsigned char* st, int t) {
-        if (z_rows <= 0) return;
-        unsigned char* at = st + wave * ZB_BYTES;
+        for (int i = 0; i < NMB; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) load_to_lds16(zg_p + (g_off[j] + (uint32_t)(16 * t)), at + 1024 * j);
-        load_to_lds16(zu_p + (u_off + (uint32_t)(16 * t)), at + 4096);
-    };
-    f32x4 acc[DN_MB][4];
-#pragma unroll
-    for (int i = 0; i < DN_MB; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0, 0, 0, 0};
-    // (the loop compiled per width; wavefronts without a slab only fetch z; all execute the same barriers)
-    auto columns = [&](auto w_c, auto nmb_c) {
-        constexpr int W = decltype(w_c)::value;
-        constexpr int WL = W == 0 ? 2 : W;
-        gptr<uint32_t> payload = as_global(fe.payload);
-        gptr<__half> scale = as_global(fe.scale);
-        Block16 blk;
-        u32x4 sc0, sc1;
-        auto request_b = [&](int t) {
-            if constexpr (W != 0) {
-                load_block_role1<WL>(payload + (uint32_t)(fs.pack_off + t * block_words(WL)), lane, blk);
-                gptr<__half> sp = scale + (uint32_t)(fs.scale_off + t * SLAB_ROWS + 16 * kg);
-                sc0 = *reinterpret_cast<gptr_u32x4>(sp);
-                sc1 = *reinterpret_cast<gptr_u32x4>(sp + 8);
-            }
-        };
-        request_z(lds, 0);
-        request_b(0);
-#pragma unroll 1
-        for (int t = 0; t < n_tiles; ++t) {
-            unsigned char* cur = lds + (t & 1) * DN_STAGE;
-            wait_vmcnt<0>();         // tile t has landed (this wavefront's part of it)
-            barrier_no_drain();      // ... everyone's; and everyone is done with the other stage
-            if (t == 0) BITSMOE_TLP(g_tl_pf_down, 2);
-            if (t + 1 < n_tiles) request_z(lds + ((t & 1) ^ 1) * DN_STAGE, t + 1);
-            if constexpr (W != 0)
-                down_mfma_block<WL, decltype(nmb_c)::value>(blk, sc0, sc1, cur, lane, acc, [&] { request_b(min(t + 1, n_tiles - 1)); });
-            asm volatile("" ::: "memory");
-        }
-    };
-    auto by_rows = [&](auto w_c) {
-        if (rows <= 16)
-            columns(w_c, std::integral_constant<int, 1>{});
-        else if (rows <= 32)
-            columns(w_c, std::integral_constant<int, 2>{});
-        else
-            columns(w_c, std::integral_constant<int, DN_MB>{});
-    };
-    if (fs.bits == 2)
-        by_rows(std::integral_constant<int, 2>{});
-    else if (fs.bits == 3)
-        by_rows(std::integral_constant<int, 3>{});
-    else if (fs.bits == 4)
-        by_rows(std::integral_constant<int, 4>{});
-    else
-        columns(std::integral_constant<int, 0>{}, std::integral_constant<int, 1>{});
-    wait_vmcnt<0>();
-    barrier_no_drain();      // (every wavefront has read its last records: the epilogue takes their place)
-    BITSMOE_TLP(g_tl_pf_down, 3);
-    if (fs.bits == 0) return;
+            for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0, 0, 0, 0};
+        // wavefronts without a slab skip the MFMAs; all execute the same barriers
+        down_tile_loop<NMB>(fe.payload, fe.scale, fs, z, I, n_tiles, a_begin, rows, sz0, sz1, sz2, wbuf, sbuf, tid, lane, acc);
+        BITSMOE_TLP(g_tl_pf_down, 3);
+        if (fs.bits == 0) return;
 
-    // the rows' multipliers s[r] go into y here, so that the combine reads one operand per assignment
+        // the rows' multipliers s[r] go into y here, so that the combine reads one operand per assignment
 #pragma unroll
-    for (int nb = 0; nb < 4; ++nb) {
-        const u32x2 sw = *reinterpret_cast<const u32x2*>(fe.s + fs.rank_off + 16 * nb + 4 * kg);
-        const h2 s01 = __builtin_bit_cast(h2, (uint32_t)sw[0]), s23 = __builtin_bit_cast(h2, (uint32_t)sw[1]);
-        const f32x4 srow = {(float)s01[0], (float)s01[1], (float)s23[0], (float)s23[1]};
+        for (int nb = 0; nb < 4; ++nb) {
+            const u32x2 sw = *reinterpret_cast<const u32x2*>(fe.s + fs.rank_off + 16 * nb + 4 * kg);
+            const h2 s01 = __builtin_bit_cast(h2, (uint32_t)sw[0]), s23 = __builtin_bit_cast(h2, (uint32_t)sw[1]);
+            const f32x4 srow = {(float)s01[0], (float)s01[1], (float)s23[0], (float)s23[1]};
 #pragma unroll
-        for (int mb = 0; mb < DN_MB; ++mb) acc[mb][nb] *= srow;
+            for (int mb = 0; mb < NMB; ++mb) acc[mb][nb] *= srow;
+        }
+        _Float16* block = y + (int64_t)a_begin * ldy + fs.rank_off;
+        store_turned<NMB>(lds + wave * STAGE, rows, lane, acc, [&](int row, int c, u32x4 v) {
+            *reinterpret_cast<u32x4*>(block + (int64_t)row * ldy + 8 * c) = v;
+        });
+    };
+    if (rows <= 32)
+        run(std::integral_constant<int, 2>{});
+    else if (rows <= 64)
+        run(std::integral_constant<int, 4>{});
+    else if constexpr (PFM > 64) {
+        if (rows <= 96)
+            run(std::integral_constant<int, 6>{});
+        else
+            run(std::integral_constant<int, 8>{});
     }
-    _Float16* block = y + (int64_t)a_begin * ldy + fs.rank_off;
-    store_turned<DN_MB>(reinterpret_cast<uint16_t*>(lds) + wave * dma_stage(DN_ROWS), rows, lane, acc, [&](int row, int c, u32x4 v) {
-        *reinterpret_cast<u32x4*>(block + (int64_t)row * ldy + 8 * c) = v;
-    });
     BITSMOE_TLP(g_tl_pf_down, 6);
 }
 
@@ -1270,18 +1281,19 @@ int launch_forward_mfma(const bitsmoe_matset* gate, const bitsmoe_matset* up, co
                 if (rc != BITSMOE_OK) return rc;
             }
             record(prof, 2, st);
+            const int64_t n8 = A * (int64_t)I / 8;
+            hipLaunchKernelGGL(k_silu_mul_f16, dim3((unsigned)std::min<int64_t>((n8 + 255) / 256, 4096)), dim3(256), 0, st, z,
+                               Ubuf, n8);
+            BITSMOE_HIP_TRY(hipGetLastError());
         }
-        const int64_t n_units = A * (int64_t)n_tiles;
-        hipLaunchKernelGGL(k_silu_records, dim3((unsigned)((n_units + 63) / 64)), dim3(256), 0, st, z, Ubuf, n_units, split ? 1 : 0);
-        BITSMOE_HIP_TRY(hipGetLastError());
     }
     record(prof, 3, st);
     {
-        const int n_groups = (down->prep_max_slabs + DN_SLABS_MFMA - 1) / DN_SLABS_MFMA;
-        const int64_t wgs = (max_mtiles + 31) / 32 * 32 * (tile_rows / DN_ROWS) * n_groups;
+        const int n_pairs = (down->prep_max_slabs + DN_SLABS_MFMA - 1) / DN_SLABS_MFMA;
+        const int64_t wgs = (max_mtiles + 31) / 32 * 32 * n_pairs;
         hipLaunchKernelGGL((tile_rows == PF_M ? k_down_mfma<PF_M> : k_down_mfma<PF_M / 2>), dim3((unsigned)wgs), dim3(256), 0, st,
-                           down->d_fast_experts, down->d_fast_slabs, down->prep_max_slabs, z, Ubuf, mtiles, n_mtiles, tok, slot, token_start,
-                           token_list, I, n_tiles, n_groups, y, ldy);
+                           down->d_fast_experts, down->d_fast_slabs, down->prep_max_slabs, z, mtiles, n_mtiles, tok, slot, token_start, token_list, (int)A, I, n_tiles,
+                           n_pairs, y, ldy);
         record(prof, 4, st);
         // (wide rows add to the fp32 sums behind the combine)
         const bool to_cast = cast && !has_wide_rows(down) && rank_out % 8 == 0 && cast->ld % 8 == 0 && ((uintptr_t)cast->out & 15) == 0;
@@ -1292,7 +1304,7 @@ int launch_forward_mfma(const bitsmoe_matset* gate, const bitsmoe_matset* up, co
         if (to_cast) cast->done = true;
         BITSMOE_HIP_TRY(hipGetLastError());
         if (has_wide_rows(down)) {      // (behind the combine, which writes every element of rank_accum)
-            const int rc = launch_wide_down(down, z, reinterpret_cast<const float*>(Ubuf), WIDE_Z_RECORDS, 1, 0, tok, off, rw, A, I, rank_out, rank_accum, st);
+            const int rc = launch_wide_down(down, z, nullptr, true, 1, 0, tok, off, rw, A, I, rank_out, rank_accum, st);
             if (rc != BITSMOE_OK) return rc;
         }
     }

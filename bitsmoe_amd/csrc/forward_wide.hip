@@ -221,9 +221,8 @@ __global__ __launch_bounds__(256) void k_wide_gateup(WideSet gate, WideSet up, c
 // slab (64 output rows: wavefront w owns rows 16w .. 16w + 15) for the rows m0 = 64 * slot, ... of its expert,
 // contracting over its chunk of column tiles, WD_TC tiles at a time, and adds s'[r] * route_w[a] * sum into
 // rank_accum[tok[a], rank'[r]] by atomics.
-// ZSRC: WIDE_Z_F16 `g` holds z = silu(G) * U as f16 [A, I]; WIDE_Z_RECORDS g / u hold z's records where the grouped GEMM's
-// SiLU pass leaves them (k_silu_records); WIDE_Z_SUMS g / u hold n_part fp32 partial sums part_stride apart.
-template <int ZSRC, bool ROUTED>
+// ZF16: `g` holds z = silu(G) * U as f16 [A, I]; otherwise g / u hold n_part fp32 partial sums part_stride apart.
+template <bool ZF16, bool ROUTED>
 __global__ __launch_bounds__(256) void k_wide_down(WideSet down, int max_slabs, const void* __restrict__ g,
                                                    const float* __restrict__ u, int n_part, int64_t part_stride,
                                                    const int32_t* __restrict__ tok, const int32_t* __restrict__ off,
@@ -285,17 +284,7 @@ __global__ __launch_bounds__(256) void k_wide_down(WideSet down, int max_slabs, 
                 for (int c = 0; c < 4; ++c) zp[q][c] = u32x4{0u, 0u, 0u, 0u};
                 if (my_a < 0 || tb + q >= t1) continue;
                 const int64_t at = (int64_t)my_a * I + (tb + q) * N_TILE + sc0;
-                if constexpr (ZSRC == WIDE_Z_RECORDS) {
-                    const unsigned char* gb = reinterpret_cast<const unsigned char*>(g) + 2 * (at - sc0);
-                    const unsigned char* ub = reinterpret_cast<const unsigned char*>(u) + 2 * (at - sc0);
-                    const int kg = tid & 3;
-                    auto piece = [&](const unsigned char* p) { return *reinterpret_cast<const u32x4*>(p + 16 * kg); };
-                    const F16x32 zv = z_from_record(ZRecord{piece(gb), piece(gb + 64), piece(gb + 128), piece(gb + 192), piece(ub)});
-                    zp[q][0] = zv.a;
-                    zp[q][1] = zv.b;
-                    zp[q][2] = zv.c;
-                    zp[q][3] = zv.d;
-                } else if constexpr (ZSRC == WIDE_Z_F16) {
+                if constexpr (ZF16) {
                     const u32x4* src = reinterpret_cast<const u32x4*>(reinterpret_cast<const uint16_t*>(g) + at);
 #pragma unroll
                     for (int c = 0; c < 4; ++c) zp[q][c] = src[c];
@@ -457,7 +446,7 @@ static int wide_gateup_impl(const bitsmoe_matset* gate, const bitsmoe_matset* up
     return BITSMOE_OK;
 }
 
-static int wide_down_impl(const bitsmoe_matset* down, const void* g_or_z, const float* u, int z_source, int n_part,
+static int wide_down_impl(const bitsmoe_matset* down, const void* g_or_z, const float* u, bool z_f16, int n_part,
                           int64_t part_stride, const int32_t* tok, const int32_t* off, const float* rw, const WideRouted* routed,
                           int64_t A, int I, int rank_out, float* rank_accum, hipStream_t st) {
     const int max_slabs = max_wide_slabs(down);
@@ -476,14 +465,12 @@ static int wide_down_impl(const bitsmoe_matset* down, const void* g_or_z, const 
         hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, wide_set_of(down), max_slabs, g_or_z, u, parts, stride, tok, off, rw, ra,
                            I, n_tiles, tiles_per_wg, n_tchunks, n_slots, uniform, rank_out, rank_accum);
     };
-    if (z_source == WIDE_Z_RECORDS)
-        launch(k_wide_down<WIDE_Z_RECORDS, false>, 1, (int64_t)0);
-    else if (z_source == WIDE_Z_F16)
-        launch(k_wide_down<WIDE_Z_F16, false>, 1, (int64_t)0);
+    if (z_f16)
+        launch(k_wide_down<true, false>, 1, (int64_t)0);
     else if (routed)
-        launch(k_wide_down<WIDE_Z_SUMS, true>, n_part, part_stride);
+        launch(k_wide_down<false, true>, n_part, part_stride);
     else
-        launch(k_wide_down<WIDE_Z_SUMS, false>, n_part, part_stride);
+        launch(k_wide_down<false, false>, n_part, part_stride);
     BITSMOE_HIP_TRY(hipGetLastError());
     return BITSMOE_OK;
 }
@@ -497,12 +484,12 @@ int launch_wide_gateup(const bitsmoe_matset* gate, const bitsmoe_matset* up, con
                             0, st);
 }
 
-int launch_wide_down(const bitsmoe_matset* down, const void* g_or_z, const float* u, int z_source, int n_part,
+int launch_wide_down(const bitsmoe_matset* down, const void* g_or_z, const float* u, bool z_f16, int n_part,
                      int64_t part_stride, const int32_t* tok, const int32_t* off, const float* rw, int64_t A, int I,
                      int rank_out, float* rank_accum, hipStream_t st) {
     if (!has_wide_rows(down) || A <= 0) return BITSMOE_OK;
     BITSMOE_REQUIRE(tok && off && rw, "the wide rows of this matrix set need the routing tables");
-    return wide_down_impl(down, g_or_z, u, z_source, n_part, part_stride, tok, off, rw, nullptr, A, I, rank_out, rank_accum, st);
+    return wide_down_impl(down, g_or_z, u, z_f16, n_part, part_stride, tok, off, rw, nullptr, A, I, rank_out, rank_accum, st);
 }
 
 bool wide_routed_possible(const bitsmoe_matset* gate, const bitsmoe_matset* up, const bitsmoe_matset* down, int64_t T, int top_k) {
@@ -532,7 +519,7 @@ int launch_forward_wide_routed(const bitsmoe_matset* gate, const bitsmoe_matset*
     if (rc != BITSMOE_OK) return rc;
     if (prof) (void)hipEventRecord(prof->ev[2], st);
     if (prof) (void)hipEventRecord(prof->ev[3], st);
-    rc = wide_down_impl(down, G, U, WIDE_Z_SUMS, 1, 0, nullptr, nullptr, nullptr, &ra, n_flat, I, rank_out, rank_accum, st);
+    rc = wide_down_impl(down, G, U, false, 1, 0, nullptr, nullptr, nullptr, &ra, n_flat, I, rank_out, rank_accum, st);
     if (rc != BITSMOE_OK) return rc;
     if (prof) {
         (void)hipEventRecord(prof->ev[4], st);

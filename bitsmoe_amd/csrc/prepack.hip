@@ -13,9 +13,9 @@ __device__ inline void run_element(int role, int nb, int kg, int n, int x, int* 
     if (role == ROLE_GATE_UP) {          // 16 rows 16*kg + x, column 16*nb + n
         *row = 16 * kg + x;
         *col = 16 * nb + n;
-    } else {                              // row 16*nb + n, columns 32*kg + x
+    } else {                              // row 16*nb + n, columns 32*(x/8) + 8*kg + x%8
         *row = 16 * nb + n;
-        *col = 32 * kg + x;
+        *col = 32 * (x >> 3) + 8 * kg + (x & 7);
     }
 }
 
@@ -60,26 +60,26 @@ __global__ __launch_bounds__(256) void k_prepack(const MatView* __restrict__ src
     const FastSlab fs = fslabs[(int64_t)task.expert * max_slabs + ps];
     const int w = fs.bits;
     const int32_t* __restrict__ row_src = ps_tab.row_src + (fe.rank_idx - ps_tab.rank_base);
-    uint32_t* __restrict__ out = const_cast<uint32_t*>(fe.payload) + fs.pack_off + t * block_words(w);
+    uint32_t* __restrict__ out = const_cast<uint32_t*>(fe.payload) + fs.pack_off + t * block_words(role, w);
     auto code_at = [&](int row, int col) { return (uint32_t)(source_level(mv, row_src, ps, row, t, col) + level_offset(w)); };
-    const int n_words = block_words(w);
+    const int nbs = (role == ROLE_GATE_UP) ? 8 : 4;        // output blocks per lane
+    const int run = (role == ROLE_GATE_UP) ? 16 : 32;      // contraction indices per (lane, nb)
+    const int n_words = block_words(role, w);
     for (int idx = threadIdx.x; idx < n_words; idx += blockDim.x) {
         uint32_t word = 0;
-        if (role == ROLE_DOWN) {
-            // the codes with a bit in this word: of one row block, or (3-bit) of the two of a pair
-            const int l = w == 3 ? (idx & 255) >> 2 : idx / (4 * w);
-            const int j = w == 3 ? (idx >> 8) * 4 + (idx & 3) : idx % (4 * w);
-            const int per = w == 3 ? 6 : w;                  // words of a row block or pair
-            const int first_bit = 32 * (j % per);
-            for (int half = 0; half < (w == 3 ? 2 : 1); ++half) {
-                const int nb = w == 3 ? 2 * (j / per) + half : j / per;
-                for (int e = 0; e < 32; ++e) {
-                    const int at = r1_code_bit(w, nb, e) - first_bit;
-                    if (at <= -w || at >= 32) continue;
+        if (w == 3 && role == ROLE_DOWN) {
+            // whole 3-bit fields, five pairs of neighbouring codes per word (wave_layout.h)
+            const int l = idx < 768 ? (idx & 255) >> 2 : idx - 768;
+            const int j = idx < 768 ? (idx >> 8) * 4 + (idx & 3) : 12;
+            const int n = l & 15, kg = l >> 4;
+            for (int sl = 0; sl < 5; ++sl) {
+                const int P = 5 * j + sl;
+                if (P >= 64) break;
+                const int nb = P >> 4, m = (P >> 2) & 3, i = P & 3;
+                for (int odd = 0; odd < 2; ++odd) {
                     int row, col;
-                    run_element(role, nb, l >> 4, l & 15, e, &row, &col);
-                    const uint32_t u = code_at(row, col);
-                    word |= at >= 0 ? u << at : u >> -at;
+                    run_element(role, nb, kg, n, 8 * m + 2 * i + odd, &row, &col);
+                    word |= (code_at(row, col) & 7u) << (r1w3_slot_pos(sl) + 16 * odd);
                 }
             }
             out[idx] = word;
@@ -88,36 +88,51 @@ __global__ __launch_bounds__(256) void k_prepack(const MatView* __restrict__ src
         if (w == 3 && idx >= 512) {
             // third bit of the 3-bit codes
             const int j = idx - 512;
-            // (j = hi_index0(kg, n8, nb), shared by lanes n8 and n8 + 8)
-            const int q = (j >> 1) & 31;
-            const int nb = 2 * (j >> 6) + (j & 1), n8 = q & 7, kg = q >> 3;
-            for (int upper = 0; upper < 2; ++upper)
-                for (int x = 0; x < 16; ++x) {
-                    int row, col;
-                    run_element(role, nb, kg, n8 + 8 * upper, x, &row, &col);
-                    word |= ((code_at(row, col) >> 2) & 1u) << pos1s(x, upper);
-                }
+            if (role == ROLE_GATE_UP) {   // j = hi_index0(kg, n8, nb), shared by lanes n8 and n8 + 8
+                const int q = (j >> 1) & 31;
+                const int nb = 2 * (j >> 6) + (j & 1), n8 = q & 7, kg = q >> 3;
+                for (int upper = 0; upper < 2; ++upper)
+                    for (int x = 0; x < 16; ++x) {
+                        int row, col;
+                        run_element(role, nb, kg, n8 + 8 * upper, x, &row, &col);
+                        word |= ((code_at(row, col) >> 2) & 1u) << pos1s(x, upper);
+                    }
+            }
             out[idx] = word;
             continue;
         }
-        // two-bit / four-bit field words: one or two words per (lane, nb), idx / per = idx2_role0(nb, l)
+        // two-bit / four-bit field words: words per (lane, nb) = run * fieldbits / 32
         const int fb = (w == 4) ? 4 : 2;
-        const int per = fb / 2;
-        const int sub = idx % per, i2 = idx / per;
-        const int nb = 2 * (i2 >> 7) + (i2 & 1), l = (i2 >> 1) & 63;
+        const int per = run * fb / 32;                   // role0: 1 (w=2,3) or 2 (w=4); role1: 2 or 4
+        const int sub = idx % per;
+        int nb, l;
+        if (role == ROLE_GATE_UP) {      // idx / per = idx2_role0(nb, l)
+            const int i2 = idx / per;
+            nb = 2 * (i2 >> 7) + (i2 & 1);
+            l = (i2 >> 1) & 63;
+        } else {
+            nb = (idx / per) % nbs;
+            l = idx / (per * nbs);
+        }
+        const int n = l & 15, kg = l >> 4;
         const int codes = 32 / fb;                       // codes per word
         for (int i = 0; i < codes; ++i) {
+            const int x = sub * codes + i;
             int row, col;
-            run_element(role, nb, l >> 4, l & 15, sub * codes + i, &row, &col);
+            run_element(role, nb, kg, n, x, &row, &col);
             const uint32_t u = code_at(row, col);
-            // staggered fields; one may wrap around bit 31
-            word |= rotl32(fb == 4 ? (u & 15u) : (u & 3u), fb == 4 ? pos4s(i) : pos2s(w, i));
+            if (role == ROLE_GATE_UP)      // staggered fields; one may wrap around bit 31
+                word |= rotl32(fb == 4 ? (u & 15u) : (u & 3u), fb == 4 ? pos4s(i) : pos2s(w, i));
+            else if (fb == 4)
+                word |= (u & 15u) << pos4(i);
+            else
+                word |= (u & 3u) << pos2(i);
         }
         out[idx] = word;
     }
 }
 
-// The per-row tables of the prepared copy: s' (multiplier), scale' [(slab, tile)][64] (down sets: in the order of r1_scale_pos) and, for gate/up
+// The per-row tables of the prepared copy: s' (multiplier), scale' [(slab, tile)][64] and, for gate/up
 // sets, scale_s' = scale * s * stagger factor of the row at the PREPARED slab's width (a power of two: the
 // decoded weight carries its inverse), each rounded once to fp16.  Padding rows get zeros, so whatever
 // the kernels read for them contributes nothing.  grid (prepared slab tasks, tiles), 64 threads.
@@ -139,7 +154,7 @@ __global__ __launch_bounds__(64) void k_prepare_rows(const MatView* __restrict__
         sc = __half2float(mv.scale[mv.tile_meta[(mv.slab_meta[s * 4 + 3] + t) * 3 + 1] + r]);
     }
     const int out_sc = fs.scale_off + t * SLAB_ROWS + row;
-    const_cast<__half*>(fe.scale)[fe.scale_s ? out_sc : out_sc - row + r1_scale_pos(row)] = __float2half(sc);
+    const_cast<__half*>(fe.scale)[out_sc] = __float2half(sc);
     if (fe.scale_s) const_cast<__half*>(fe.scale_s)[out_sc] = __float2half(sc * sv * (float)stagger_factor(fs.bits, row));
     if (t == 0) const_cast<__half*>(fe.s)[fs.rank_off + row] = __float2half(sv);
 }
@@ -200,7 +215,7 @@ __global__ __launch_bounds__(256) void k_dequant_prepared(MatView mv /* the call
     const int ps = blockIdx.x;
     const FastSlab fs = fs_row[ps];
     const int w = fs.bits;
-    const uint32_t* __restrict__ blk = fe.payload + fs.pack_off + (int)blockIdx.y * block_words(w);
+    const uint32_t* __restrict__ blk = fe.payload + fs.pack_off + (int)blockIdx.y * block_words(role, w);
     const int nbs = (role == ROLE_GATE_UP) ? 8 : 4;
     const int run = (role == ROLE_GATE_UP) ? 16 : 32;
     for (int idx = threadIdx.x; idx < SLAB_ROWS * N_TILE; idx += blockDim.x) {
@@ -212,25 +227,32 @@ __global__ __launch_bounds__(256) void k_dequant_prepared(MatView mv /* the call
         int row, col;
         run_element(role, nb, kg, n, x, &row, &col);
         uint32_t u;
-        if (role == ROLE_DOWN) {
-            const int bit = r1_code_bit(w, nb, x);
-            const int j = (w == 3 ? 6 * (nb >> 1) : w * nb) + (bit >> 5);
-            uint64_t two = blk[r1_word_index(w, l, j)];
-            if ((bit & 31) + w > 32) two |= (uint64_t)blk[r1_word_index(w, l, j + 1)] << 32;
-            u = (uint32_t)(two >> (bit & 31)) & ((1u << w) - 1u);
+        const int unit = (role == ROLE_GATE_UP) ? idx2_role0(nb, l) : (l * nbs + nb);
+        if (w == 3 && role == ROLE_DOWN) {
+            const int P = 16 * nb + 4 * (x >> 3) + ((x & 7) >> 1);
+            u = (blk[r1w3_word_index(l, P / 5)] >> (r1w3_slot_pos(P % 5) + 16 * (x & 1))) & 7u;
         } else if (w == 4) {
-            u = rotr32(blk[idx2_role0(nb, l) * 2 + (x >> 3)], pos4s(x & 7)) & 15u;
+            const int per = run / 8;
+            const uint32_t word = blk[unit * per + (x >> 3)];
+            u = (role == ROLE_GATE_UP ? rotr32(word, pos4s(x & 7)) : word >> pos4(x & 7)) & 15u;
         } else {
-            u = rotr32(blk[idx2_role0(nb, l)], pos2s(w, x)) & 3u;
-            if (w == 3) u |= ((blk[512 + hi_index0(kg, n, nb)] >> pos1s(x, n >> 3)) & 1u) << 2;
+            const int per = run / 16;
+            const uint32_t word = blk[unit * per + (x >> 4)];
+            u = (role == ROLE_GATE_UP ? rotr32(word, pos2s(w, x & 15)) : word >> pos2(x & 15)) & 3u;
+            if (w == 3) {
+                uint32_t hi;
+                int p;
+                hi = blk[512 + hi_index0(kg, n, nb)];      // (role 0: role 1 took the branch above)
+                p = pos1s(x, n >> 3);
+                u |= ((hi >> p) & 1u) << 2;
+            }
         }
         const int c = blockIdx.y * N_TILE + col;
         const int src = row_src[ps * SLAB_ROWS + row];
         if (c < I && src >= 0) {
             const int local_row = mv.slab_meta[(src >> 8) * 4 + 2] + (src & 255);
             const float q = (float)((int)u - level_offset(w));
-            out[(int64_t)local_row * I + c] = q * __half2float(fe.scale[fs.scale_off + (int)blockIdx.y * SLAB_ROWS +
-                                                                           (role == ROLE_DOWN ? r1_scale_pos(row) : row)]);
+            out[(int64_t)local_row * I + c] = q * __half2float(fe.scale[fs.scale_off + (int)blockIdx.y * SLAB_ROWS + row]);
         }
     }
 }
@@ -353,7 +375,7 @@ static int prepare_impl(bitsmoe_matset* set, int32_t role, hipStream_t st) {
         for (int ps = 0; ps < n_ps[e]; ++ps) {
             BITSMOE_REQUIRE(words < ((int64_t)1 << 31) - (int64_t)n_tiles * 256 * 4, "expert %d: prepared payload exceeds int32 word offsets", e);
             fslabs[(size_t)e * pms + ps] = FastSlab{width[ps], (int32_t)words, ps * n_tiles * SLAB_ROWS, ps * SLAB_ROWS};
-            words += (int64_t)n_tiles * block_words(width[ps]);
+            words += (int64_t)n_tiles * block_words(role, width[ps]);
             tasks.push_back(SlabTask{e, ps});
         }
         pay_words += round_up(words, 64);      // keep every matrix 256-byte aligned

@@ -13,19 +13,18 @@
 //   role 0 (gate / up: contraction over rows, outputs are columns; nb = 0..7)
 //     output column 16*nb + n, rows 16*kg + e, e = 0..15              (16 codes)
 //   role 1 (down: contraction over columns, outputs are rows; nb = 0..3)
-//     output row 16*nb + n, columns 32*kg + e, e = 0..31               (32 codes)
+//     output row 16*nb + n, columns 32*m + 8*kg + e', m = 0..3, e' = 0..7   (32 codes)
 //
-//   Role 1 fields are those of the block-scaled MFMA's fp4 and fp6 operands (z_planes.h says why), so that masks make
-//   operands of the payload's words:
-//     2-bit codes: code e in word e/16 of the (lane, nb), bits 4*(e%8) + 2*((e/8)%2) -- the low halves of a word's nibbles
-//                  are one fp4 register, the high halves the next
-//     4-bit codes: code e in word e/8, bits 4*(e%8): the low and the high halves of the nibbles are two fp4 operands
-//     3-bit codes: the lane's four row blocks two by two; the 192 bits of a pair hold 32 6-bit fields, code e of the even
-//                  block in bits 6e .. 6e+2, of the odd one in 6e+3 .. 6e+5: each is an fp6 operand under its mask
+//   Role 1: a run of 16 codes with index x = 0..15 sits in a word, precisely:
+//     2-bit fields:  field LSB at  (x & ~1) + 16*(x & 1)
+//     4-bit fields:  8 codes per word, field LSB at 4*(x'/2) + 16*(x' & 1), x' = x % 8
+//     3-bit codes :  whole 3-bit fields, five PAIRS of neighbouring codes per word: pair P = 16*nb + 4*m + e'/2
+//                    of the lane (0..63) sits in word P/5 of the lane's thirteen, its two fields at bits
+//                    1 + 3*(P%5) and 17 + 3*(P%5) (832 words per block instead of 768)
+//   so that ONE rotate and ONE and-or turn a word into a packed pair of 16-bit floats
+//   (2^w + code) for two neighbouring contraction indices: the pair lives 16 bits apart.
 //
-//   Role 0: f16 operands.  ONE and-or (and a rotate) turns a word into a packed pair of 16-bit floats (2^w + code) for two
-//   neighbouring contraction indices: the pair lives 16 bits apart.
-//   It staggers the fields so that most rotates disappear.  The MFMA operand of one k-step
+//   Role 0 staggers the fields so that most rotates disappear.  The MFMA operand of one k-step
 //   is four registers i = 0..3 (contraction indices 2i, 2i+1 of the lane's run of eight).  The
 //   field of register i sits 2i bits (4-bit codes: 4*(i%2) bits) BELOW the place where it would
 //   read as 2^w + code in an f16 mantissa, so the four registers of a k-step come out of the
@@ -45,12 +44,12 @@
 //           w=2: word[idx2(nb, l)]   idx2 = ((nb/2)*64 + l)*2 + nb%2
 //           w=4: word[idx2(nb, l)*2 + j]
 //           w=3: low word[idx2(nb, l)], high word[512 + hi_index0(kg, n, nb)]
-//   role 1: w=2: word[(l*4 + nb)*2 + h]           w=4: word[(l*4 + nb)*4 + q]
-//           w=3: word j of lane l's twelve at (j/4)*256 + l*4 + j%4 (three 16-byte loads per lane), pair nb/2 in 6*(nb/2) ..
+//   role 1: w=2: word[(l*4 + nb)*2 + h]           w=4: word[(l*4 + nb)*4 + m]
+//           w=3: word j of lane l at (j/4)*256 + l*4 + j%4 for j < 12 (three 16-byte loads per lane), word 12 at 768 + l
 //
-// Decoded role 0 operands are (2^w + code), role 1's the codes; the true level is code - 2^(w-1), so every dot
-// product carries the constant 1.5 * 2^w (role 1: 2^(w-1)) times the sum of the other operand, which the
-// kernels remove.
+// Decoded operand value is (2^w + code); the true level is code - 2^(w-1), so every dot
+// product carries the constant 1.5 * 2^w times the sum of the other operand, which the
+// kernels remove with one extra MFMA against a constant operand.
 #pragma once
 
 #include <cstdint>
@@ -69,17 +68,19 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
-// role 1: the first bit of code e (0..31) of row block nb among the lane's words of the row block (2- and 4-bit: 2 and 4 words;
-// 3-bit: the six words of the pair of row blocks)
-__host__ __device__ inline int r1_code_bit(int w, int nb, int e) {
-    return w == 2 ? 32 * (e >> 4) + 4 * (e & 7) + 2 * ((e >> 3) & 1) : w == 4 ? 4 * e : 6 * e + 3 * (nb & 1);
-}
-// role 1: word j of lane l's 4 w words of a block (j = 0..4w-1; 3-bit: the even pair's six, then the odd pair's)
-__host__ __device__ inline int r1_word_index(int w, int l, int j) { return w == 3 ? (j >> 2) * 256 + l * 4 + (j & 3) : l * 4 * w + j; }
-// role 1: place of row r's scale among the 64 of a (slab, tile): the four rows 16 nb + n of a lane side by side (one 8-byte load)
-__host__ __device__ inline int r1_scale_pos(int r) { return (r & 15) * 4 + (r >> 4); }
-// words of one (slab, tile) block
-__host__ __device__ inline int block_words(int w) { return 256 * w; }
+// position of the field LSB for index x (0..15) of a run of 16 two-bit fields
+__host__ __device__ inline int pos2(int x) { return (x & ~1) + 16 * (x & 1); }
+// index x' (0..7) of a run of 8 four-bit fields
+__host__ __device__ inline int pos4(int x) { return 4 * (x >> 1) + 16 * (x & 1); }
+// index y (0..31) of a run of 32 single bits (role 1) / (0..15) + 8*upper (role 0)
+__host__ __device__ inline int pos1(int y) { return (y >> 1) + 16 * (y & 1); }
+
+// role 1, 3-bit: words of one (slab, tile) block, the place of word j (0..12) of lane l, the low-half bit offset of
+// slot sl (0..4) of a word, and the words of a block of either role and width
+constexpr int R1W3_BLOCK_WORDS = 13 * 64;
+__host__ __device__ inline int r1w3_word_index(int l, int j) { return j < 12 ? (j >> 2) * 256 + l * 4 + (j & 3) : 768 + l; }
+__host__ __device__ inline int r1w3_slot_pos(int sl) { return 1 + 3 * sl; }
+__host__ __device__ inline int block_words(int role, int w) { return (role == 1 && w == 3) ? R1W3_BLOCK_WORDS : 256 * w; }
 
 // role 0 (staggered): field LSB of code x (0..15) of a run in a two-bit field word, w = 2 or 3
 __host__ __device__ inline int pos2s(int w, int x) {
@@ -143,6 +144,58 @@ typedef const u32x4 __attribute__((address_space(1)))* gptr_u32x4;
 __device__ inline uint32_t vreg(uint32_t c) {
     asm("" : "+v"(c));
     return c;
+}
+
+// Four packed registers (8 values = one MFMA k-step) from two-bit fields: `first` is the
+// run index of the first of the 8 codes (0 or 8).
+template <int W, bool BF16>
+__device__ inline u32x4 decode_fields2(uint32_t z, int first) {
+    using C = Codec<W, BF16>;
+    u32x4 r;
+    const uint32_t m = vreg(C::FMASK_2BIT);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r[i] = (rotr32(z, first + 2 * i - C::POS) & m) | C::MAGIC;
+    return r;
+}
+
+template <bool BF16>
+__device__ inline u32x4 decode_fields4(uint32_t z) {
+    using C = Codec<4, BF16>;
+    u32x4 r;
+    const uint32_t m = vreg(C::FMASK_4BIT);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r[i] = (rotr32(z, 4 * i - C::POS) & m) | C::MAGIC;
+    return r;
+}
+
+// 3-bit: two-bit fields from `z`, third bit from `hi`; `hi_first` = position of the bit of
+// the first of the 8 codes inside `hi` (pos1 of its run index, plus 8 for an upper lane).
+template <bool BF16>
+__device__ inline u32x4 decode_fields3(uint32_t z, int first, uint32_t hi, int hi_first) {
+    using C = Codec<3, BF16>;
+    u32x4 r;
+    const uint32_t m = vreg(C::FMASK_2BIT), mh = vreg(C::FMASK_HIBIT);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t lo = (rotr32(z, first + 2 * i - C::POS) & m) | C::MAGIC;
+        r[i] = (rotr32(hi, hi_first + i - (C::POS + 2)) & mh) | lo;
+    }
+    return r;
+}
+
+// role 1, 3-bit: the four registers of k-step m of row block nb from the lane's thirteen words (indices fold to
+// constants where nb and m are unrolled).  One rotate (none for the slot that already sits in place) and one and-or each.
+template <bool BF16>
+__device__ __forceinline__ u32x4 decode_r1w3(const uint32_t (&w)[16], int nb, int m) {
+    using C = Codec<3, BF16>;
+    const uint32_t mask = vreg((7u << C::POS) * 0x10001u);
+    u32x4 r;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int P = 16 * nb + 4 * m + i;
+        r[i] = (rotr32(w[P / 5], r1w3_slot_pos(P % 5) - C::POS) & mask) | C::MAGIC;
+    }
+    return r;
 }
 
 // ---- role 0 (staggered fields, f16 operands) ----
