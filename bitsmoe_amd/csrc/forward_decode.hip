@@ -960,6 +960,7 @@ int launch_forward_decode(const bitsmoe_matset* gate, const bitsmoe_matset* up, 
     const bool split_z_possible = !fused_z && !routed && (walk ? n_part : 1) < part_capacity && I % 4 == 0;
     const bool split_z = split_z_possible && (split_z_env >= 0 ? split_z_env > 0 : mode == GRID_CHUNKS);
     const int parts_in = walk && !fused_z ? n_part : 1;
+    const bool z_ready = fused_z || split_z;      // z is at hand as f16 [A, I]; otherwise the fp32 gate and up sums are
     float* down_g = G;
     float* down_u = U;
     if (split_z) {
@@ -985,7 +986,7 @@ int launch_forward_decode(const bitsmoe_matset* gate, const bitsmoe_matset* up, 
     auto launch_down = [&](auto kernel) {
         const int n_work = e_dim * dn_groups * dn_tchunks;
         hipLaunchKernelGGL(kernel, dim3((unsigned)((e_dim + 7) / 8 * 8 * dn_groups * dn_tchunks)), dim3(256), z_bytes, st, down->d_fast_experts,
-                           down->d_fast_slabs, down->prep_max_slabs, down_g, down_u, split_z ? 1 : parts_in, part_stride, rw, tok, off,
+                           down->d_fast_slabs, down->prep_max_slabs, down_g, down_u, z_ready ? 1 : parts_in, part_stride, rw, tok, off,
                            (int)T, (int)A, I, E, n_tiles, dn_groups, dn_tchunks, dn_tiles_per_wg, n_work, rank_out, rank_accum,
                            routed ? routed->selected : nullptr, routed ? routed->ids_are_i64 : 0, routed ? (int)A : 0,
                            routed ? routed->top_k : 1, routed ? routed->local_to_global : nullptr,
@@ -1024,13 +1025,13 @@ int launch_forward_decode(const bitsmoe_matset* gate, const bitsmoe_matset* up, 
         launch_down(k_down_decode<M, Z, false, ZROWS>);
     };
     // (G and U are fp32 and the operands f16 whatever the activation type was)
-    if (fused_z || split_z)
+    if (z_ready)
         with_mode(launch_down_mode, std::true_type{});
     else
         with_mode(launch_down_mode, std::false_type{});
     BITSMOE_HIP_TRY(hipGetLastError());
     if (has_wide_rows(down)) {      // (behind the gate/up kernel, which cleared rank_accum)
-        const int rc = launch_wide_down(down, down_g, down_u, split_z, split_z ? 1 : parts_in, part_stride, tok, off, rw, A, I,
+        const int rc = launch_wide_down(down, down_g, down_u, z_ready, z_ready ? 1 : parts_in, part_stride, tok, off, rw, A, I,
                                         rank_out, rank_accum, st);
         if (rc != BITSMOE_OK) return rc;
     }

@@ -133,6 +133,23 @@ def test_forward_dense_experts_as_16_bit_sets(cuda_device, path_name, tokens):
     print(f"dense experts {tokens} tokens {path_name}: err {err:.2e}")
 
 
+@pytest.mark.parametrize("option", ["decode_fused_z", "decode_split_z"])
+@pytest.mark.parametrize("tokens", [1, 5, 40])      # active experts, experts, chunks
+def test_wide_down_rows_read_z_that_is_made_already(cuda_device, tokens, option, lib_option):
+    """z = silu(G) * U in the place of the fp32 sums, made by the gate/up kernel or by a launch of its own: the wide rows of a down set
+    read it there too."""
+    e, k, rank, dim = 3, 2, 1024, 384
+    lib_option(option, 1)
+
+    def make(rng):
+        gate, up = [[helpers.make_matrix(rng, rank, dim, [(2, (0, rank))]) for _ in range(e)] for _ in range(2)]
+        down = [helpers.make_matrix(rng, 256, dim, [(16, (0, 64)), (8, (64, 100)), (2, (100, 256))]) for _ in range(e)]
+        return gate, up, down
+
+    sets, err = _case(cuda_device, 900 + tokens, e, tokens, k, rank, 256, dim, "bf16", _paths()["decode"], make)
+    assert sets[2].wide_slabs > 0 and sets[0].wide_slabs == sets[1].wide_slabs == 0
+
+
 def test_wide_rows_only_in_some_experts_and_some_projections(cuda_device):
     """Wide rows in the down matrices of two experts only, and in one expert's gate matrix: the side kernels' lists
     of experts differ per projection; experts nobody routed to are skipped."""
