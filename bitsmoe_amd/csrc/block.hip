@@ -14,11 +14,6 @@ static inline size_t align256(size_t v) { return (v + 255) / 256 * 256; }
 // Rows that the few-rows kernel takes: a call of more ends with the projection's operand (and super_out), in the caller's memory.
 constexpr int64_t PROJECT_OUT_MAX_ROWS = 64;
 
-// Rows that go into the output projection as the operator's fp32 sums (layers without a shared expert): no pass that rounds them, but
-// twice the bytes of x for every workgroup of the projection.  Graph of four 128-expert layers, us per layer, pass -> fp32 rows:
-// 20 tokens 70.5 -> 68.7, 32 tokens 72.9 -> 71.1, 48 tokens 78.4 either way, 64 tokens 83.8 -> 84.7.
-constexpr int F32_ROWS_MAX = 32;
-
 // Where the intermediates of a call sit in the workspace.
 struct BlockWorkspace {
     size_t selected, weights, rank_accum, operand, forward, forward_bytes, super_forward, super_bytes, super_out, total;
@@ -114,8 +109,7 @@ extern "C" int bitsmoe_block_forward(const bitsmoe_block_plan* p, const void* x,
     float* rank_accum = (float*)(ws + w.rank_accum);
     // what the output projection reads: the cast sums beside the shared expert's activations; a few fp32 rows without a
     // shared expert go into it as they are
-    const bool f32_rows = project_out && p->shared_intermediate == 0 && n_tokens <= F32_ROWS_MAX &&
-                          skinny_f32_rows_possible(n_tokens, p->rank_out, p->w_out_prepared);
+    const bool f32_rows = project_out && p->shared_intermediate == 0 && skinny_f32_rows_possible(n_tokens, p->rank_out, p->w_out_prepared);
     void* operand = project_out ? (void*)(ws + w.operand) : out;
     const int k_out = p->rank_out + p->shared_intermediate;
     CastRows cast = {operand, k_out, false};
@@ -140,7 +134,7 @@ extern "C" int bitsmoe_block_forward(const bitsmoe_block_plan* p, const void* x,
     if (project_out)
         BITSMOE_TRY(skinny_linear(f32_rows ? (const void*)rank_accum : operand, p->act_dtype, f32_rows ? 1 : 0, k_out, p->w_out,
                                   p->w_out_prepared, n_tokens, k_out, p->hidden, out, p->hidden, super ? sup : nullptr, p->hidden,
-                                  F32_ROWS_MAX, stream));
+                                  stream));
 #undef BITSMOE_TRY
     return BITSMOE_OK;
 }

@@ -189,10 +189,10 @@ int forward_routed_cast(const bitsmoe_matset* gate, const bitsmoe_matset* up, co
 int block_finish(const float* rank_accum, int64_t n_tokens, int32_t rank_out, const void* shared_gate_out, const void* shared_up_out,
                  int64_t ld_shared, int32_t shared_intermediate, const void* shared_gate_logit, int64_t ld_gate_logit, int32_t act_dtype,
                  void* out, int64_t ld_out, bool shared_only, void* stream);
-// bitsmoe_skinny_linear; fp32 rows up to `f32_rows` of them where skinny_f32_rows_possible says so.
+// bitsmoe_skinny_linear; fp32 rows where skinny_f32_rows_possible says so.
 int skinny_linear(const void* x, int32_t dtype, int32_t x_is_f32, int64_t ld_x, const void* weight, int32_t weight_is_prepared,
                   int64_t n_rows, int32_t in_features, int32_t out_features, void* out, int64_t ld_out, const float* addend,
-                  int64_t ld_addend, int f32_rows, void* stream);
+                  int64_t ld_addend, void* stream);
 bool skinny_f32_rows_possible(int64_t n_rows, int32_t in_features, int32_t weight_is_prepared);
 
 // bf16 -> f16, eight elements at a time: group `i` of `total = T * (ld / 8)` groups of one projection.

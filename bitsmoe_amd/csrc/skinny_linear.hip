@@ -239,21 +239,30 @@ extern "C" int bitsmoe_prepare_linear_weight(const void* weight, int32_t in_feat
 extern "C" int bitsmoe_skinny_linear(const void* x, int32_t dtype, int32_t x_is_f32, int64_t ld_x, const void* weight,
                                      int32_t weight_is_prepared, int64_t n_rows, int32_t in_features, int32_t out_features,
                                      void* out, int64_t ld_out, const float* addend, int64_t ld_addend, void* stream) {
+    BITSMOE_REQUIRE(!x_is_f32 || n_rows <= 16, "n_rows must be in [0, 64] (fp32 rows: [0, 16])");
     return bitsmoe::skinny_linear(x, dtype, x_is_f32, ld_x, weight, weight_is_prepared, n_rows, in_features, out_features, out, ld_out,
-                                  addend, ld_addend, 16, stream);
+                                  addend, ld_addend, stream);
 }
 
-// More than sixteen fp32 rows: prepared weights and four wavefronts (their pieces of x fill the LDS).
+// Up to sixteen rows always; seventeen to 32 with prepared weights of up to 1536 features (shares of up to twelve steps).  Instead of a
+// pass that rounds them, every workgroup fetches twice the bytes of x, which shows from 2048 features on.  Graph of four layers of a
+// block, us per layer, pass -> fp32 rows, at 17, 20, 26 and 32 tokens (runs of one side differ by 0.3 us):
+//   1024 features:  34.2 -> 33.3  34.3 -> 33.4  45.1 -> 44.4  46.5 -> 45.7
+//   1536 features:  42.4 -> 41.7  43.3 -> 42.4  44.0 -> 43.1  42.6 -> 41.9
+//   2048 features, 32 experts:  51.1 -> 50.8  53.5 -> 53.2  53.9 -> 53.6  56.0 -> 55.5
+//   2048 features, 128 experts:  67.1 -> 66.9  68.4 -> 68.3  (32 tokens) 72.5 -> 72.5  (48) 78.2 -> 79.8  (64) 83.1 -> 85.9
+//   2560 features:  70.0 -> 70.7  72.2 -> 72.7  74.9 -> 75.6  73.7 -> 74.6
 bool bitsmoe::skinny_f32_rows_possible(int64_t n_rows, int32_t in_features, int32_t weight_is_prepared) {
-    return n_rows <= 16 || (n_rows <= 64 && weight_is_prepared != 0 && in_features <= 80 * 32);
+    return n_rows <= 16 || (n_rows <= 32 && weight_is_prepared != 0 && in_features <= 48 * 32);
 }
 
 int bitsmoe::skinny_linear(const void* x, int32_t dtype, int32_t x_is_f32, int64_t ld_x, const void* weight, int32_t weight_is_prepared,
                            int64_t n_rows, int32_t in_features, int32_t out_features, void* out, int64_t ld_out, const float* addend,
-                           int64_t ld_addend, int f32_rows, void* stream) {
+                           int64_t ld_addend, void* stream) {
     BITSMOE_REQUIRE(dtype == BITSMOE_DT_F16 || dtype == BITSMOE_DT_BF16, "dtype must be f16 (0) or bf16 (1)");
-    BITSMOE_REQUIRE(n_rows >= 0 && n_rows <= (x_is_f32 ? f32_rows : 64), "n_rows must be in [0, 64] (fp32 rows: [0, %d])", f32_rows);
-    BITSMOE_REQUIRE(!x_is_f32 || skinny_f32_rows_possible(n_rows, in_features, weight_is_prepared), "fp32 rows past 16 need prepared weights");
+    BITSMOE_REQUIRE(n_rows >= 0 && n_rows <= 64, "n_rows must be in [0, 64] (fp32 rows: [0, 16])");
+    BITSMOE_REQUIRE(!x_is_f32 || skinny_f32_rows_possible(n_rows, in_features, weight_is_prepared),
+                    "more than 16 fp32 rows: at most 32, and prepared weights of at most 1536 features");
     BITSMOE_REQUIRE(in_features >= 128 && in_features % 128 == 0, "in_features must be a positive multiple of 128");
     BITSMOE_REQUIRE(out_features >= 2 && out_features % 2 == 0, "out_features must be even");
     BITSMOE_REQUIRE(ld_x >= in_features && ld_x % (x_is_f32 ? 4 : 8) == 0,
@@ -296,11 +305,9 @@ int bitsmoe::skinny_linear(const void* x, int32_t dtype, int32_t x_is_f32, int64
     auto by_share = [&](auto bf_c, auto nmb_c, auto xf_c, auto turn_c) {
         constexpr bool twenty = !(decltype(xf_c)::value && !decltype(turn_c)::value);      // (fp32 operands of twenty steps do not fit the registers)
         constexpr bool many_f32 = decltype(xf_c)::value && decltype(nmb_c)::value > 1;
-        if constexpr (many_f32) {       // (prepared, four wavefronts: skinny_f32_rows_possible)
+        if constexpr (many_f32) {       // (prepared, four wavefronts, up to twelve steps: skinny_f32_rows_possible)
             if (share <= 8) run(bf_c, nmb_c, W4{}, S8{}, xf_c, Yes{}, turn_c);
-            else if (share <= 12) run(bf_c, nmb_c, W4{}, S12{}, xf_c, Yes{}, turn_c);
-            else if (share <= 16) run(bf_c, nmb_c, W4{}, S16{}, xf_c, Yes{}, turn_c);
-            else run(bf_c, nmb_c, W4{}, S20{}, xf_c, Yes{}, turn_c);
+            else run(bf_c, nmb_c, W4{}, S12{}, xf_c, Yes{}, turn_c);
         } else if (!weight_is_prepared) {      // (in passes of sixteen steps: the same sums in the same order)
             if (nw == 8) run(bf_c, nmb_c, W8{}, S16{}, xf_c, No{}, turn_c); else run(bf_c, nmb_c, W4{}, S16{}, xf_c, No{}, turn_c);
         } else if (nw == 8) {
@@ -322,9 +329,7 @@ int bitsmoe::skinny_linear(const void* x, int32_t dtype, int32_t x_is_f32, int64
         if (n_rows <= 4 && x_is_f32 && share <= 16) by_share(bf_c, One{}, Yes{}, No{});
         else if (n_rows <= 4 && !x_is_f32) by_share(bf_c, One{}, No{}, No{});
         else if (x_is_f32 && nmb == 1) by_share(bf_c, One{}, Yes{}, Yes{});
-        else if (x_is_f32 && nmb == 2) by_share(bf_c, integral_constant<int, 2>{}, Yes{}, Yes{});
-        else if (x_is_f32 && nmb == 3) by_share(bf_c, integral_constant<int, 3>{}, Yes{}, Yes{});
-        else if (x_is_f32) by_share(bf_c, integral_constant<int, 4>{}, Yes{}, Yes{});
+        else if (x_is_f32) by_share(bf_c, integral_constant<int, 2>{}, Yes{}, Yes{});
         else if (nmb == 1) by_share(bf_c, One{}, No{}, Yes{});
         else if (nmb == 2) by_share(bf_c, integral_constant<int, 2>{}, No{}, Yes{});
         else if (nmb == 3) by_share(bf_c, integral_constant<int, 3>{}, No{}, Yes{});

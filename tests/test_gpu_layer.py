@@ -372,6 +372,51 @@ def test_block_sums_reach_the_output_projection_in_the_activation_type(cuda_devi
     assert float((got - apart).abs().max()) <= 1e-2 * float(apart.abs().max())
 
 
+def _between_the_projections(block, x, stages):
+    """One call of the block's plan on x -> (what it writes, the operator's fp32 sums from the same projections and picks, the output
+    projection's weights as the plan keeps them)."""
+    import torch
+
+    from bitsmoe_amd.algorithms import mlp_forward_cuda as hip
+
+    with torch.no_grad():
+        block(x[None])
+    plan = next(v for v in block._basis_cache.values() if isinstance(v, dict) and "native" in v)
+    native, r, t = plan["native"][0], int(block.shared_u_down.shape[1]), x.shape[0]
+    proj = x @ plan["w_in"].T
+    selected = torch.empty((t, block.top_k), dtype=torch.int64, device=x.device)
+    weights = torch.empty((t, block.top_k), dtype=torch.float32, device=x.device)
+    project_out = stages & hip.BLOCK_PROJECT_OUT
+    out = torch.empty((t, plan["w_out"].shape[0 if project_out else 1]), dtype=x.dtype, device=x.device)
+    hip.block_forward(native, x, proj, stages, out, selected, weights)
+    lo, hi = plan["ranges"]["h_gate"], plan["ranges"]["h_up"]
+    sums = hip.moe_forward_routed(proj[:, lo[0]:lo[1]], proj[:, hi[0]:hi[1]], selected, weights, block._packed_global_to_local,
+                                  block._packed_local_to_global, *block._ensure_matsets(), r, block._packed_intermediate_size)
+    return out, sums, plan.get("w_out_prepared")
+
+
+# a block of sixteen rows, the second block's first and last row, and one more (rounded by a pass); shares of up to eight and twelve
+# steps, whole and not, and widths past them (more than sixteen rows rounded by a pass).  Two experts that take every token: the
+# grouped GEMM, whose sums are the same from call to call
+@pytest.mark.parametrize("tokens", [16, 17, 32, 33])
+@pytest.mark.parametrize("width", [128, 640, 1024, 1152, 1536, 1664, 2048])
+@pytest.mark.parametrize("dtype_name", ["bfloat16", "float16"])
+def test_fp32_rows_into_the_output_projection_equal_rounded_rows(cuda_device, dtype_name, width, tokens):
+    """Bit for bit: the block's output is the few-rows kernel's on the operator's sums rounded to the activation type."""
+    import torch
+
+    from bitsmoe_amd.algorithms import mlp_forward_cuda as hip
+    from bitsmoe_amd.synth import make_layer
+
+    dtype = getattr(torch, dtype_name)
+    spec = _small_spec("qwen3moe", num_experts=2, hidden_size=width)
+    block = make_layer(spec, device=cuda_device, dtype=dtype, seed=61, basis_seed=7, s_mode="rand").eval()
+    block.prepare_runtime_fastpath(warmup=True)
+    x = torch.randn((tokens, width), generator=torch.Generator().manual_seed(tokens)).to(dtype).to(cuda_device)
+    out, sums, w_out = _between_the_projections(block, x, hip.BLOCK_PROJECT_OUT)
+    assert torch.equal(out, hip.skinny_linear(sums.to(dtype), w_out))
+
+
 def test_block_plan_made_twice_at_once(cuda_device, monkeypatch):
     """Two first forwards of one block at the same time may each make a native plan: both get both projections' weights
     (the second forward runs here in the middle of the first, where a thread switch would put it, and on its stream: what other
