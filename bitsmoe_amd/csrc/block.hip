@@ -61,6 +61,8 @@ extern "C" int bitsmoe_block_forward(const bitsmoe_block_plan* p, const void* x,
     if (n_tokens == 0) return BITSMOE_OK;
     BITSMOE_REQUIRE(x && proj && out, "null pointer");
     BITSMOE_REQUIRE(p->router_form != BITSMOE_ROUTER_CALLER || (selected && weights), "the caller's routing is missing");
+    // (here, not only in the closing pass: the grouped GEMM's combine writes rows of rank_out before that, rank_out + this apart)
+    BITSMOE_REQUIRE(p->shared_intermediate >= 0, "negative size");
     const bool project_in = (stages & BITSMOE_BLOCK_PROJECT_IN) != 0, project_out = (stages & BITSMOE_BLOCK_PROJECT_OUT) != 0;
     BITSMOE_REQUIRE(!project_out || n_tokens <= PROJECT_OUT_MAX_ROWS, "the output projection takes at most 64 tokens");
     const bool super = p->super_gate != nullptr;

@@ -168,7 +168,7 @@ int route_with_jobs(const void* selected, int32_t ids_are_i64, const float* weig
                     int32_t* expert_offsets, float* route_flat, void* workspace, size_t workspace_bytes,
                     const RouteSideJobs* jobs, int* jobs_done, hipStream_t st);
 // Where a caller that only goes on with the sums rounded to the activation dtype takes them: rows of `rank_out` 16-bit values, `ld`
-// apart.  The grouped GEMM's combine then writes these instead of rank_accum and says so (`done`).
+// (at least rank_out) apart.  The grouped GEMM's combine then writes these instead of rank_accum and says so (`done`).
 struct CastRows {
     void* out;
     int64_t ld;

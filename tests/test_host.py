@@ -75,6 +75,20 @@ def test_c_abi_rejects_bad_arguments_without_gpu():
     assert lib.bitsmoe_route_workspace_bytes(32768, 128) >= 32768 * 4
 
 
+def test_block_call_refuses_a_negative_shared_size_first():
+    """The operand's rows would overlap, and the last ones reach past its end: refused before sizes are made of it or anything is
+    launched."""
+    from bitsmoe_amd.algorithms import _capi
+
+    lib = _capi.load()
+    some = ctypes.create_string_buffer(1 << 16)      # (not read: it is the address of everything the call checks for null)
+    at = ctypes.addressof(some)
+    plan = _capi.BlockPlan(gate=at, up=at, down=at, global_to_local=at, local_to_global=at, top_k=2, n_global=1, rank_out=64,
+                           hidden=128, intermediate_size=128, shared_intermediate=-8)
+    rc = lib.bitsmoe_block_forward(ctypes.addressof(plan), at, 128, 100, at, 0, None, None, at, None, None, 0, None, None)
+    assert (rc, lib.bitsmoe_last_error()) == (-1, b"negative size")
+
+
 def _state_dict_for(mats_by_mtype, prefix, scheme):
     sd = {}
     for mtype, m in mats_by_mtype.items():
