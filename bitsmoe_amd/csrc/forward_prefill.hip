@@ -939,8 +939,8 @@ constexpr int CB_SORT = 256;     // list entries ordered at a time
 // thread keeps its eight columns in registers; otherwise the row is accumulated in LDS, one
 // assignment after the other.
 // `cast`: the sums go there, rounded to bf16 (cast_bf16) or f16, eight columns at a time, and not into rank_accum: a block's output
-// projection reads them in the activation dtype (at 4096 tokens of 2048 ranks: 34 MB less written here, and no
-// pass that reads 34 MB and writes 17: the 128-expert layer 558 -> 541 us).
+// projection reads them in the activation dtype (at 4096 tokens of 2048 ranks: 17 MB written here instead of 34, and no
+// pass that reads 34 MB and writes 17: graph of four 128-expert layers, 549 -> 525 us per layer; at 1024 tokens 215.6 -> 207.3).
 template <bool IDENTITY>
 __global__ __launch_bounds__(256) void k_combine_tokens(const FastExpert* __restrict__ down_fe, int max_slabs,
                                                         const _Float16* __restrict__ y, int ldy,

@@ -417,6 +417,25 @@ def test_fp32_rows_into_the_output_projection_equal_rounded_rows(cuda_device, dt
     assert torch.equal(out, hip.skinny_linear(sums.to(dtype), w_out))
 
 
+@pytest.mark.parametrize("hidden", [128, 2176])      # one round of the combine's 2048 columns, and a second of 128
+@pytest.mark.parametrize("layout", ["uniform", "checkpoint"])
+@pytest.mark.parametrize("family,kw", [("qwen3moe", {}), ("qwen3next", {"shared_intermediate": 128})])
+@pytest.mark.parametrize("dtype_name", ["bfloat16", "float16"])
+def test_combine_rounds_the_sums_to_nearest(cuda_device, dtype_name, family, kw, layout, hidden):
+    """Bit for bit: the operand that a larger call ends with holds the operator's sums as the framework's cast rounds them."""
+    import torch
+
+    from bitsmoe_amd.synth import make_layer
+
+    dtype = getattr(torch, dtype_name)
+    spec = _small_spec(family, hidden_size=hidden, **kw)
+    block = make_layer(spec, device=cuda_device, dtype=dtype, seed=62, basis_seed=7, s_mode="rand", layout=layout).eval()
+    block.prepare_runtime_fastpath(warmup=True)
+    x = torch.randn((150, hidden), generator=torch.Generator().manual_seed(3)).to(dtype).to(cuda_device)
+    out, sums, _ = _between_the_projections(block, x, 0)
+    assert torch.equal(out[:, : sums.shape[1]], sums.to(dtype))
+
+
 def test_block_plan_made_twice_at_once(cuda_device, monkeypatch):
     """Two first forwards of one block at the same time may each make a native plan: both get both projections' weights
     (the second forward runs here in the middle of the first, where a thread switch would put it, and on its stream: what other
