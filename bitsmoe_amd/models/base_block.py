@@ -514,8 +514,8 @@ class BitsMoE_BaseSparseMoeBlock(nn.Module):
     # the operator and the router kernel read their operands as column ranges of its output.  Everything that
     # is projected back to hidden space -- rank_accum @ shared_u_down.T (bitsmoe/models/base_block.py:414) and the
     # shared expert's down projection -- is ONE GEMM against the column-stacked weights, its operand written by
-    # one elementwise pass (bitsmoe_block_finish).  Beside the operator's own launches a block forward is then
-    # four launches instead of ten to twenty framework ops.
+    # one elementwise pass (bitsmoe_block_finish) or, at prefill sizes, by the operator's last kernel.  Beside the
+    # operator's own launches a block forward is then four launches instead of ten to twenty framework ops.
     _FUSED_BLOCK = _os.environ.get("BITSMOE_FUSED_BLOCK", "1") != "0"
 
     @staticmethod
