@@ -418,7 +418,8 @@ def test_fp32_rows_into_the_output_projection_equal_rounded_rows(cuda_device, dt
 
 
 @pytest.mark.parametrize("hidden", [128, 2176])      # one round of the combine's 2048 columns, and a second of 128
-@pytest.mark.parametrize("layout", ["uniform", "checkpoint", "scattered"])      # output ranks in order; the last ones dropped; in no order (the row summed in LDS)
+# output ranks in order; the last ones dropped; in no order (the row summed in LDS)
+@pytest.mark.parametrize("layout", ["uniform", "checkpoint", "scattered"])
 @pytest.mark.parametrize("family,kw", [("qwen3moe", {}), ("qwen3next", {"shared_intermediate": 128})])
 @pytest.mark.parametrize("dtype_name", ["bfloat16", "float16"])
 def test_combine_rounds_the_sums_to_nearest(cuda_device, dtype_name, family, kw, layout, hidden):
