@@ -803,8 +803,8 @@ __device__ __forceinline__ void gateup_walk_z_item(const WalkMatrix& mg, const W
 
 // ----------------------------------------------------------------------------------- down
 // One (slab, tile) block of a down matrix: 4 row blocks x 4 k-steps (micro-tiles).
-// `corr`: 1.5 * 2^W times the sum of the tile's z over its 128 columns, per assignment row of the
-// lane (the constant term of the decoded operands 2^W + code; the z rows are summed once, when z
+// `corr`: down_offset times the sum of the tile's z over its 128 columns, per assignment row of the
+// lane (the constant term of the decoded operands; the z rows are summed once, when z
 // is built, instead of by four more MFMAs per block).
 template <int W>
 __device__ __forceinline__ void down_block(const Block16& b, const u32x4 (&az)[4], const float (&sc)[4], f32x4 corr, f32x4 (&acc)[4]) {
@@ -815,7 +815,7 @@ __device__ __forceinline__ void down_block(const Block16& b, const u32x4 (&az)[4
         for (int m = 0; m < 4; ++m) {
             u32x4 bw;
             if constexpr (W == 2)
-                bw = decode_fields2<2, false>(b.w[nb * 2 + (m >> 1)], 8 * (m & 1));
+                bw = decode_r1w2(b.w[nb * 2 + (m >> 1)], m & 1);
             else if constexpr (W == 4)
                 bw = decode_fields4<false>(b.w[nb * 4 + m]);
             else
@@ -885,7 +885,7 @@ __device__ __forceinline__ void down_wave(gptr<uint32_t> payload, gptr<__half> s
             for (int m = 0; m < 4; ++m) az[m] = *reinterpret_cast<const u32x4*>(zp + 32 * m);
             f32x4 corr;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) corr[j] = zsum[(g4 + j) * ZSUM_STRIDE + tb + i] * (1.5f * (float)(1 << WL));
+            for (int j = 0; j < 4; ++j) corr[j] = zsum[(g4 + j) * ZSUM_STRIDE + tb + i] * down_offset<WL>();
             down_block<WL>(buf[B], az, sc[B], corr, acc);
         };
         // logical rank and multiplier of the slab's row `lane`: needed by the epilogue only, kept

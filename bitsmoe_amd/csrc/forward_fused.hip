@@ -119,7 +119,7 @@ __device__ __forceinline__ void down_issue(DownRing<WD>& ring, const DownSource&
 }
 
 // One (slab, tile) block of a down matrix without its scale: 4 row blocks x 4 k-steps; acc[nb][j] = sum over the
-// tile's columns of level[16 nb + n, c] * z[4 kg + j, c] (the constant term of the 2^W + code operands removed).
+// tile's columns of level[16 nb + n, c] * z[4 kg + j, c] (the constant term of the decoded operands removed).
 template <int W>
 __device__ __forceinline__ void down_block_raw(const Block16& b, const u32x4 (&az)[4], f32x4 corr, f32x4 (&acc)[4]) {
 #pragma unroll
@@ -129,7 +129,7 @@ __device__ __forceinline__ void down_block_raw(const Block16& b, const u32x4 (&a
         for (int m = 0; m < 4; ++m) {
             u32x4 bw;
             if constexpr (W == 2)
-                bw = decode_fields2<2, false>(b.w[nb * 2 + (m >> 1)], 8 * (m & 1));
+                bw = decode_r1w2(b.w[nb * 2 + (m >> 1)], m & 1);
             else if constexpr (W == 4)
                 bw = decode_fields4<false>(b.w[nb * 4 + m]);
             else
@@ -202,7 +202,7 @@ __device__ __forceinline__ void fused_z_down(DownRing<WD>& ring, int n_pre, cons
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const int a = g4 + j;
-        corr[j] = (zs_lds[a] + zs_lds[MAX_A + a] + zs_lds[2 * MAX_A + a] + zs_lds[3 * MAX_A + a]) * (1.5f * (float)(1 << WD));
+        corr[j] = (zs_lds[a] + zs_lds[MAX_A + a] + zs_lds[2 * MAX_A + a] + zs_lds[3 * MAX_A + a]) * down_offset<WD>();
     }
     auto compute = [&](auto b_c) {
         constexpr int B = decltype(b_c)::value;

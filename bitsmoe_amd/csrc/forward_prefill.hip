@@ -697,8 +697,8 @@ __device__ __forceinline__ void down_half_mfma(int bits, const uint16_t* stage, 
             u32x4 b;
             uint32_t off;
             if (bits == 2) {
-                b = decode_fields2<2, false>(blk.w[nb * 2 + HH], 8 * km);
-                off = neg_offset_pair<2>();
+                b = decode_r1w2(blk.w[nb * 2 + HH], km);
+                off = 0xC000C000u;      // -2
             } else if (bits == 4) {
                 b = decode_fields4<false>(blk.w[nb * 4 + m]);
                 off = neg_offset_pair<4>();

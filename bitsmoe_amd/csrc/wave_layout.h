@@ -16,12 +16,14 @@
 //     output row 16*nb + n, columns 32*m + 8*kg + e', m = 0..3, e' = 0..7   (32 codes)
 //
 //   Role 1: a run of 16 codes with index x = 0..15 sits in a word, precisely:
-//     2-bit fields:  field LSB at  (x & ~1) + 16*(x & 1)
+//     2-bit codes :  field LSB at  4*(x % 8) + 2*(x / 8): a nibble holds code j of the run's first k-step in its low two bits
+//                    and code j of the second in its high two, so (word >> 2*ks) & 0x33333333 is a k-step's eight codes as
+//                    E2M1 numbers (0, 1/2, 1, 3/2), a pair to a byte: one conversion per pair (decode_r1w2)
 //     4-bit fields:  8 codes per word, field LSB at 4*(x'/2) + 16*(x' & 1), x' = x % 8
 //     3-bit codes :  whole 3-bit fields, five PAIRS of neighbouring codes per word: pair P = 16*nb + 4*m + e'/2
 //                    of the lane (0..63) sits in word P/5 of the lane's thirteen, its two fields at bits
 //                    1 + 3*(P%5) and 17 + 3*(P%5) (832 words per block instead of 768)
-//   so that ONE rotate and ONE and-or turn a word into a packed pair of 16-bit floats
+//   so that ONE rotate and ONE and-or turn a 3- or 4-bit word into a packed pair of 16-bit floats
 //   (2^w + code) for two neighbouring contraction indices: the pair lives 16 bits apart.
 //
 //   Role 0 staggers the fields so that most rotates disappear.  The MFMA operand of one k-step
@@ -47,9 +49,9 @@
 //   role 1: w=2: word[(l*4 + nb)*2 + h]           w=4: word[(l*4 + nb)*4 + m]
 //           w=3: word j of lane l at (j/4)*256 + l*4 + j%4 for j < 12 (three 16-byte loads per lane), word 12 at 768 + l
 //
-// Decoded operand value is (2^w + code); the true level is code - 2^(w-1), so every dot
-// product carries the constant 1.5 * 2^w times the sum of the other operand, which the
-// kernels remove with one extra MFMA against a constant operand.
+// Decoded operand value is (2^w + code), of 2-bit role 1 codes the code itself; the true level is code - 2^(w-1), so every dot
+// product carries the constant 1.5 * 2^w (2-bit role 1: 2) times the sum of the other operand, which the
+// kernels remove.
 #pragma once
 
 #include <cstdint>
@@ -68,12 +70,10 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
-// position of the field LSB for index x (0..15) of a run of 16 two-bit fields
-__host__ __device__ inline int pos2(int x) { return (x & ~1) + 16 * (x & 1); }
+// role 1: position of the field LSB for index x (0..15) of a run of 16 two-bit codes
+__host__ __device__ inline int pos2(int x) { return 4 * (x & 7) + 2 * (x >> 3); }
 // index x' (0..7) of a run of 8 four-bit fields
 __host__ __device__ inline int pos4(int x) { return 4 * (x >> 1) + 16 * (x & 1); }
-// index y (0..31) of a run of 32 single bits (role 1) / (0..15) + 8*upper (role 0)
-__host__ __device__ inline int pos1(int y) { return (y >> 1) + 16 * (y & 1); }
 
 // role 1, 3-bit: words of one (slab, tile) block, the place of word j (0..12) of lane l, the low-half bit offset of
 // slot sl (0..4) of a word, and the words of a block of either role and width
@@ -120,9 +120,7 @@ template <int W, bool BF16>
 struct Codec {
     static constexpr int POS = FloatFmt<BF16>::MANT - W;                              // field LSB in each half
     static constexpr uint32_t MAGIC = (uint32_t)((FloatFmt<BF16>::BIAS + W) << FloatFmt<BF16>::MANT) * 0x10001u;  // 2^W
-    static constexpr uint32_t FMASK_2BIT = (3u << POS) * 0x10001u;
     static constexpr uint32_t FMASK_4BIT = (15u << POS) * 0x10001u;
-    static constexpr uint32_t FMASK_HIBIT = (1u << (POS + 2)) * 0x10001u;                  // bit 2 of a 3-bit code
     // 1.5 * 2^W: exponent BIAS + W, top mantissa bit set
     static constexpr uint32_t CORR =
         (uint32_t)(((FloatFmt<BF16>::BIAS + W) << FloatFmt<BF16>::MANT) | (1 << (FloatFmt<BF16>::MANT - 1))) * 0x10001u;
@@ -146,17 +144,22 @@ __device__ inline uint32_t vreg(uint32_t c) {
     return c;
 }
 
-// Four packed registers (8 values = one MFMA k-step) from two-bit fields: `first` is the
-// run index of the first of the 8 codes (0 or 8).
-template <int W, bool BF16>
-__device__ inline u32x4 decode_fields2(uint32_t z, int first) {
-    using C = Codec<W, BF16>;
+// role 1, 2-bit: the four registers (8 values = one MFMA k-step) of k-step ks from a lane's word: the codes themselves, 0 to 3.
+// The nibbles are E2M1 numbers of half that value, doubled by the conversion's scale (exact): one mask for four registers and
+// one instruction per register, where fields 16 bits apart took a rotate and an and-or per register (down kernel under the tracer,
+// us: 128 experts at 64 tokens 27.7 -> 26.8, four layers of a graph at 32 tokens 21.6 -> 20.9, 512 experts at 256 tokens 55.2 -> 53.1).
+__device__ __forceinline__ u32x4 decode_r1w2(uint32_t z, int ks) {
+    const uint32_t codes = (ks ? z >> 2 : z) & 0x33333333u;
     u32x4 r;
-    const uint32_t m = vreg(C::FMASK_2BIT);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) r[i] = (rotr32(z, first + 2 * i - C::POS) & m) | C::MAGIC;
+    r[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(codes, 2.0f, 0));
+    r[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(codes, 2.0f, 1));
+    r[2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(codes, 2.0f, 2));
+    r[3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(codes, 2.0f, 3));
     return r;
 }
+// What a decoded role 1 value is above its level: every dot product carries it times the sum of the other operand.
+template <int W>
+__host__ __device__ constexpr float down_offset() { return W == 2 ? 2.0f : 1.5f * (float)(1 << W); }
 
 template <bool BF16>
 __device__ inline u32x4 decode_fields4(uint32_t z) {
@@ -165,21 +168,6 @@ __device__ inline u32x4 decode_fields4(uint32_t z) {
     const uint32_t m = vreg(C::FMASK_4BIT);
 #pragma unroll
     for (int i = 0; i < 4; ++i) r[i] = (rotr32(z, 4 * i - C::POS) & m) | C::MAGIC;
-    return r;
-}
-
-// 3-bit: two-bit fields from `z`, third bit from `hi`; `hi_first` = position of the bit of
-// the first of the 8 codes inside `hi` (pos1 of its run index, plus 8 for an upper lane).
-template <bool BF16>
-__device__ inline u32x4 decode_fields3(uint32_t z, int first, uint32_t hi, int hi_first) {
-    using C = Codec<3, BF16>;
-    u32x4 r;
-    const uint32_t m = vreg(C::FMASK_2BIT), mh = vreg(C::FMASK_HIBIT);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const uint32_t lo = (rotr32(z, first + 2 * i - C::POS) & m) | C::MAGIC;
-        r[i] = (rotr32(hi, hi_first + i - (C::POS + 2)) & mh) | lo;
-    }
     return r;
 }
 
