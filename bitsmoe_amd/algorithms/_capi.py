@@ -44,6 +44,8 @@ EXPORTED_SYMBOLS = (
     "bitsmoe_skinny_linear",
     "bitsmoe_prepared_linear_weight_elements",
     "bitsmoe_prepare_linear_weight",
+    "bitsmoe_tiled_linear",
+    "bitsmoe_tiled_linear_pays",
     "bitsmoe_forward_workspace_bytes",
     "bitsmoe_forward_workspace_bytes_sets",
     "bitsmoe_moe_forward",
@@ -56,6 +58,7 @@ EXPORTED_SYMBOLS = (
     "bitsmoe_forward_decode_is_fused",
     "bitsmoe_block_workspace_bytes",
     "bitsmoe_block_forward",
+    "bitsmoe_block_forward_tiled",
     "bitsmoe_profile_create",
     "bitsmoe_profile_destroy",
     "bitsmoe_profile_read",
@@ -85,7 +88,7 @@ class MatrixDesc(Structure):
 
 
 ROUTER_LOGITS, ROUTER_LINEAR, ROUTER_CALLER = 0, 1, 2
-BLOCK_PROJECT_IN, BLOCK_PROJECT_OUT = 1, 2
+BLOCK_PROJECT_IN, BLOCK_PROJECT_OUT, BLOCK_PROJECT_IN_TILED, BLOCK_PROJECT_OUT_TILED = 1, 2, 4, 8
 
 
 class BlockPlan(Structure):
@@ -95,7 +98,7 @@ class BlockPlan(Structure):
             "w_in_prepared", "w_out_prepared", "act_dtype", "hidden", "in_features", "rank_gate", "rank_up", "rank_out",
             "intermediate_size", "super_intermediate", "top_k", "n_global", "router_form", "renormalize", "round_dtype",
             "col_gate", "col_up", "col_logits", "col_shared_gate", "col_shared_up", "col_shared_logit",
-            "shared_intermediate")] + [("weight_scale", c_float)]
+            "shared_intermediate")] + [("weight_scale", c_float), ("w_in_rows", c_void_p), ("w_out_rows", c_void_p)]
 
 
 _lib = None
@@ -152,6 +155,11 @@ def load() -> ctypes.CDLL:
     lib.bitsmoe_prepared_linear_weight_elements.argtypes = [c_int32, c_int32]
     lib.bitsmoe_prepare_linear_weight.restype = c_int32
     lib.bitsmoe_prepare_linear_weight.argtypes = [c_void_p, c_int32, c_int32, c_void_p, c_void_p]
+    lib.bitsmoe_tiled_linear.restype = c_int32
+    lib.bitsmoe_tiled_linear.argtypes = [c_void_p, c_int32, c_int64, c_void_p, c_int64, c_int32, c_int32, c_void_p, c_int64, c_void_p,
+                                         c_int64, c_void_p]
+    lib.bitsmoe_tiled_linear_pays.restype = c_int32
+    lib.bitsmoe_tiled_linear_pays.argtypes = [c_int64, c_int32, c_int32]
     lib.bitsmoe_block_finish.restype = c_int32
     lib.bitsmoe_block_finish.argtypes = [c_void_p, c_int64, c_int32, c_void_p, c_void_p, c_int64, c_int32, c_void_p, c_int64,
                                          c_int32, c_void_p, c_int64, c_void_p]
@@ -194,6 +202,9 @@ def load() -> ctypes.CDLL:
     ]
     lib.bitsmoe_block_workspace_bytes.restype = c_size_t
     lib.bitsmoe_block_workspace_bytes.argtypes = [c_void_p, c_int64]
+    lib.bitsmoe_block_forward_tiled.restype = c_int32
+    lib.bitsmoe_block_forward_tiled.argtypes = [c_void_p, c_void_p, c_int64, c_int64, c_void_p, c_int32, c_void_p, c_void_p, c_void_p,
+                                                c_void_p, c_void_p, c_void_p, c_size_t, c_void_p, c_void_p]
     lib.bitsmoe_block_forward.restype = c_int32
     lib.bitsmoe_block_forward.argtypes = [c_void_p, c_void_p, c_int64, c_int64, c_void_p, c_int32, c_void_p, c_void_p, c_void_p,
                                           c_void_p, c_void_p, c_size_t, c_void_p, c_void_p]

@@ -13,6 +13,7 @@ bitsmoe/algorithms/cpp/mlp_forward.cu:2464-2503), `route`, `dequant_matrix`.
 from __future__ import annotations
 
 import ctypes
+import functools
 import operator
 import os
 from collections import OrderedDict
@@ -661,6 +662,7 @@ def prepared_linear_weight_of(owner, weight: torch.Tensor) -> "PreparedLinearWei
 SKINNY_LINEAR_MAX_ROWS = 64
 ROUTER_LOGITS, ROUTER_LINEAR, ROUTER_CALLER = _capi.ROUTER_LOGITS, _capi.ROUTER_LINEAR, _capi.ROUTER_CALLER
 BLOCK_PROJECT_IN, BLOCK_PROJECT_OUT = _capi.BLOCK_PROJECT_IN, _capi.BLOCK_PROJECT_OUT
+BLOCK_PROJECT_IN_TILED, BLOCK_PROJECT_OUT_TILED = _capi.BLOCK_PROJECT_IN_TILED, _capi.BLOCK_PROJECT_OUT_TILED
 
 
 class PreparedLinearWeight:
@@ -729,6 +731,47 @@ def skinny_linear(x: torch.Tensor, weight, addend: Optional[torch.Tensor] = None
     return out
 
 
+TILED_LINEAR_MAX_STRIDE = 1 << 22      # elements between rows of x (a tile's rows are addressed by 32 bits of byte offset)
+
+
+@functools.lru_cache(maxsize=1024)
+def tiled_linear_pays(rows: int, in_features: int, out_features: int) -> bool:
+    """Is tiled_linear measured to be faster than the framework's GEMM at this size (and possible at all)?"""
+    return bool(_lib.bitsmoe_tiled_linear_pays(rows, in_features, out_features))
+
+
+def tiled_linear_possible(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Can tiled_linear take these tensors?  (x [T, K] and a contiguous weight [N, K] of one 16-bit dtype on one GPU, x with unit
+    column stride and 16-byte aligned rows, K a multiple of 128, N of 8.)"""
+    if not (x.is_cuda and x.dim() == 2 and weight.dim() == 2 and x.device == weight.device and x.dtype == weight.dtype
+            and x.dtype in (torch.float16, torch.bfloat16) and weight.is_contiguous() and x.stride(1) == 1):
+        return False
+    t, k = int(x.shape[0]), int(x.shape[1])
+    n = int(weight.shape[0])
+    return (t >= 1 and int(weight.shape[1]) == k and 128 <= k <= TILED_LINEAR_MAX_STRIDE and k % 128 == 0 and n >= 8 and n % 8 == 0
+            and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0
+            and (t <= 1 or (int(x.stride(0)) % 8 == 0 and k <= int(x.stride(0)) <= TILED_LINEAR_MAX_STRIDE)))
+
+
+def tiled_linear(x: torch.Tensor, weight: torch.Tensor, addend: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """x @ weight.T for any number of rows (a bias-free linear layer from decode batches of tens of tokens up to prompts): fp32
+    sums in a fixed order, result in the weight's dtype.  `addend`: fp32 [T, N] added to the sums before the result is rounded."""
+    _check(tiled_linear_possible(x, weight), "tiled_linear: unsupported shapes, dtypes or alignment")
+    dev = x.device
+    t, k, n = int(x.shape[0]), int(x.shape[1]), int(weight.shape[0])
+    out = torch.empty((t, n), dtype=x.dtype, device=dev)
+    if addend is not None:
+        _check(addend.dtype == torch.float32 and tuple(addend.shape) == (t, n) and addend.stride(1) == 1 and addend.device == dev
+               and addend.data_ptr() % 16 == 0 and (t <= 1 or (int(addend.stride(0)) % 4 == 0 and int(addend.stride(0)) >= n)),
+               "tiled_linear: addend must be float32 [T, N] with unit column stride and 16-byte aligned rows on x's device")
+    with torch.cuda.device(dev):
+        _capi.check(_lib.bitsmoe_tiled_linear(x.data_ptr(), _capi.DT_F16 if x.dtype == torch.float16 else _capi.DT_BF16,
+                                              int(x.stride(0)) if t > 1 else k, weight.data_ptr(), t, k, n, out.data_ptr(), n,
+                                              None if addend is None else addend.data_ptr(),
+                                              0 if addend is None else (int(addend.stride(0)) if t > 1 else n), _stream_ptr(dev)))
+    return out
+
+
 def block_finish(rank_accum: torch.Tensor, dtype: torch.dtype, shared_gate_out: Optional[torch.Tensor] = None,
                  shared_up_out: Optional[torch.Tensor] = None, shared_gate_logit: Optional[torch.Tensor] = None) -> torch.Tensor:
     """[T, rank_out + I_sh] in `dtype`: rank_accum cast, beside it silu(gate_out) * up_out (* sigmoid(gate_logit)) of an
@@ -790,9 +833,9 @@ class BlockPlan:
         return all(ms._handle is h for ms, h in zip(self._sets, self._handles))
 
     def set_weight(self, name: str, weight) -> None:
-        """w_in / w_out / w_router: a tensor or a PreparedLinearWeight of it."""
+        """w_in / w_out / w_router: a tensor or a PreparedLinearWeight of it; w_in_rows / w_out_rows: a tensor."""
         prepared = isinstance(weight, PreparedLinearWeight)
-        if name != "w_router":
+        if name in ("w_in", "w_out"):
             setattr(self.c, name + "_prepared", 1 if prepared else 0)
         setattr(self.c, name, (weight.data if prepared else weight).data_ptr())
         self._weights[name] = weight
@@ -820,15 +863,15 @@ class BlockPlan:
 
 def block_forward(plan: BlockPlan, x: torch.Tensor, proj: torch.Tensor, stages: int, out: torch.Tensor,
                   selected: Optional[torch.Tensor] = None, weights: Optional[torch.Tensor] = None,
-                  super_out: Optional[torch.Tensor] = None, side_stream: int = 0) -> None:
-    """bitsmoe_block_forward on x's device and current stream (the tensors are the caller's to check)."""
+                  super_out: Optional[torch.Tensor] = None, side_stream: int = 0, operand: Optional[torch.Tensor] = None) -> None:
+    """bitsmoe_block_forward_tiled on x's device and current stream (the tensors are the caller's to check)."""
     dev = x.device
     n_tokens = x.shape[0]
     ws = _workspace(dev, plan.workspace_bytes(n_tokens))
-    _on(dev, _lib.bitsmoe_block_forward, plan.address, x.data_ptr(), x.stride(0) if n_tokens > 1 else x.shape[1], n_tokens,
+    _on(dev, _lib.bitsmoe_block_forward_tiled, plan.address, x.data_ptr(), x.stride(0) if n_tokens > 1 else x.shape[1], n_tokens,
         proj.data_ptr(), stages, None if selected is None else selected.data_ptr(), None if weights is None else weights.data_ptr(),
-        out.data_ptr(), None if super_out is None else super_out.data_ptr(), ws.data_ptr(), ws.numel(), side_stream,
-        _stream_ptr(dev))
+        None if operand is None else operand.data_ptr(), out.data_ptr(), None if super_out is None else super_out.data_ptr(),
+        ws.data_ptr(), ws.numel(), side_stream, _stream_ptr(dev))
 
 
 # ----------------------------------------------------------------------------------------

@@ -1,5 +1,5 @@
 // The block's forward as one call: everything between the hidden states and the block output that runs on this library's
-// kernels -- the few-rows projections, the router, the routed-expert operator, the super experts' operator call beside it, the
+// kernels -- the two projections, the router, the routed-expert operator, the super experts' operator call beside it, the
 // closing pass -- is launched from here, so that a forward costs its host one call instead of one per kernel.  At decode
 // sizes the kernels of a block take 30 to 100 us and the host work of launching them one by one from the framework took as
 // long or longer (128-expert layer, one token: 82 us per eager forward for 29 us of kernels).
@@ -11,7 +11,7 @@ using namespace bitsmoe;
 
 static inline size_t align256(size_t v) { return (v + 255) / 256 * 256; }
 
-// Rows that the few-rows kernel takes: a call of more ends with the projection's operand (and super_out), in the caller's memory.
+// Rows that the few-rows kernel takes: a call of more ends with the projection's operand (and super_out) in the caller's memory.
 constexpr int64_t PROJECT_OUT_MAX_ROWS = 64;
 
 // Where the intermediates of a call sit in the workspace.
@@ -56,6 +56,13 @@ static int stream_after(hipStream_t later, hipStream_t earlier) {
 extern "C" int bitsmoe_block_forward(const bitsmoe_block_plan* p, const void* x, int64_t ld_x, int64_t n_tokens, void* proj,
                                      int32_t stages, void* selected, float* weights, void* out, float* super_out, void* workspace,
                                      size_t workspace_bytes, void* side_stream, void* stream) {
+    return bitsmoe_block_forward_tiled(p, x, ld_x, n_tokens, proj, stages, selected, weights, nullptr, out, super_out, workspace,
+                                       workspace_bytes, side_stream, stream);
+}
+
+extern "C" int bitsmoe_block_forward_tiled(const bitsmoe_block_plan* p, const void* x, int64_t ld_x, int64_t n_tokens, void* proj,
+                                           int32_t stages, void* selected, float* weights, void* operand, void* out, float* super_out,
+                                           void* workspace, size_t workspace_bytes, void* side_stream, void* stream) {
     BITSMOE_REQUIRE(p && p->gate && p->up && p->down && p->global_to_local && p->local_to_global, "null pointer in the block's plan");
     BITSMOE_REQUIRE(n_tokens >= 0 && p->top_k > 0, "n_tokens must be >= 0 and top_k > 0");
     if (n_tokens == 0) return BITSMOE_OK;
@@ -63,10 +70,15 @@ extern "C" int bitsmoe_block_forward(const bitsmoe_block_plan* p, const void* x,
     BITSMOE_REQUIRE(p->router_form != BITSMOE_ROUTER_CALLER || (selected && weights), "the caller's routing is missing");
     // (here, not only in the closing pass: the grouped GEMM's combine writes rows of rank_out before that, rank_out + this apart)
     BITSMOE_REQUIRE(p->shared_intermediate >= 0, "negative size");
-    const bool project_in = (stages & BITSMOE_BLOCK_PROJECT_IN) != 0, project_out = (stages & BITSMOE_BLOCK_PROJECT_OUT) != 0;
-    BITSMOE_REQUIRE(!project_out || n_tokens <= PROJECT_OUT_MAX_ROWS, "the output projection takes at most 64 tokens");
+    const bool tiled_in = (stages & BITSMOE_BLOCK_PROJECT_IN_TILED) != 0, tiled_out = (stages & BITSMOE_BLOCK_PROJECT_OUT_TILED) != 0;
+    const bool few_in = (stages & BITSMOE_BLOCK_PROJECT_IN) != 0, few_out = (stages & BITSMOE_BLOCK_PROJECT_OUT) != 0;
+    const bool project_out = few_out || tiled_out;
+    BITSMOE_REQUIRE(!(few_in && tiled_in) && !(few_out && tiled_out), "one kernel per projection");
+    BITSMOE_REQUIRE(!few_out || n_tokens <= PROJECT_OUT_MAX_ROWS, "the output projection takes at most 64 tokens");
     const bool super = p->super_gate != nullptr;
-    BITSMOE_REQUIRE(!super || project_out || super_out, "super_out must not be null where the caller projects");
+    const bool in_workspace = project_out && n_tokens <= PROJECT_OUT_MAX_ROWS;
+    BITSMOE_REQUIRE(!tiled_out || operand || in_workspace, "more than 64 tokens: the operand's memory is the caller's");
+    BITSMOE_REQUIRE(!super || in_workspace || super_out, "super_out must not be null where the caller projects");
     const BlockWorkspace w = carve(p, n_tokens);
     if (workspace == nullptr || workspace_bytes < w.total) {
         set_error("workspace too small: need %zu bytes, got %zu", w.total, workspace_bytes);
@@ -83,7 +95,9 @@ extern "C" int bitsmoe_block_forward(const bitsmoe_block_plan* p, const void* x,
         if (_rc != BITSMOE_OK) return _rc;     \
     } while (0)
 
-    if (project_in)
+    if (tiled_in)
+        BITSMOE_TRY(bitsmoe_tiled_linear(x, p->act_dtype, ld_x, p->w_in_rows, n_tokens, p->hidden, p->in_features, proj, ld, nullptr, 0, stream));
+    if (few_in)
         BITSMOE_TRY(bitsmoe_skinny_linear(x, p->act_dtype, 0, ld_x, p->w_in, p->w_in_prepared, n_tokens, p->hidden, p->in_features,
                                           proj, ld, nullptr, 0, stream));
     if (!selected) selected = ws + w.selected;
@@ -111,8 +125,9 @@ extern "C" int bitsmoe_block_forward(const bitsmoe_block_plan* p, const void* x,
     float* rank_accum = (float*)(ws + w.rank_accum);
     // what the output projection reads: the cast sums beside the shared expert's activations; a few fp32 rows without a
     // shared expert go into it as they are
-    const bool f32_rows = project_out && p->shared_intermediate == 0 && skinny_f32_rows_possible(n_tokens, p->rank_out, p->w_out_prepared);
-    void* operand = project_out ? (void*)(ws + w.operand) : out;
+    const bool f32_rows = few_out && p->shared_intermediate == 0 && skinny_f32_rows_possible(n_tokens, p->rank_out, p->w_out_prepared);
+    if (!project_out) operand = out;
+    else if (few_out || !operand) operand = ws + w.operand;
     const int k_out = p->rank_out + p->shared_intermediate;
     CastRows cast = {operand, k_out, false};
     const int rc = forward_routed_cast(p->gate, p->up, p->down, big + p->col_gate, big + p->col_up, p->act_dtype, n_tokens, p->rank_gate,
@@ -133,7 +148,10 @@ extern "C" int bitsmoe_block_forward(const bitsmoe_block_plan* p, const void* x,
     BITSMOE_TRY(finish_rc);
     BITSMOE_TRY(super_rc);
     if (super && !side_stream) BITSMOE_TRY(run_super(st));
-    if (project_out)
+    if (tiled_out)
+        BITSMOE_TRY(bitsmoe_tiled_linear(operand, p->act_dtype, k_out, p->w_out_rows, n_tokens, k_out, p->hidden, out, p->hidden,
+                                         super ? sup : nullptr, p->hidden, stream));
+    if (few_out)
         BITSMOE_TRY(skinny_linear(f32_rows ? (const void*)rank_accum : operand, p->act_dtype, f32_rows ? 1 : 0, k_out, p->w_out,
                                   p->w_out_prepared, n_tokens, k_out, p->hidden, out, p->hidden, super ? sup : nullptr, p->hidden,
                                   stream));

@@ -56,9 +56,9 @@ def _super_via_operator() -> bool:
 # shapes of hidden sizes 1024 to 2048 with and without shared experts: up to 32 rows it is the faster one at all of them (at 32:
 # 2048 -> 4224 features 9.0 vs 11.9, 2048 -> 9728 13.0 vs 14.4, 4864 -> 2048 10.3 vs 13.8, 4352 -> 1536 9.7 vs 12.6); from 33 to 48 at
 # all but one (at 48: 10.3 vs 12.3, 15.2 vs 15.5, 13.4 vs 13.9; but 4352 -> 1536 12.9 vs 12.6).  Every workgroup reads all
-# rows of x, so from 49 to 64 rows only GEMMs of about one workgroup per CU and a contraction of at most 4096 take it (at 64: 2048 -> 2048
-# 7.4 vs 11.6, 2560 -> 2048 8.4 vs 13.6, 2048 -> 4224 12.4 vs 12.5); 2048 -> 9728 17.6 vs 15.5 and, at 56, 4864 -> 2048 15.4 vs 13.8,
-# 4352 -> 1536 14.8 vs 12.6.
+# rows of x: from 49 rows on the many-rows kernel takes over wherever it can (at 64: 2048 -> 4224 12.4 vs 9.6, 2048 -> 2048 7.4 vs 5.5,
+# 4864 -> 2048 15.8 vs 13.8), and what that cannot take runs here up to 64 rows at GEMMs of about one workgroup per CU and a
+# contraction of at most 4096 (at 64 against the framework: 2048 -> 2048 7.4 vs 11.6, 2560 -> 2048 8.4 vs 13.6; but 2048 -> 9728 17.6 vs 15.5).
 # BITSMOE_BLOCK_SKINNY_ROWS caps the rows, 0 switches the kernel off.
 _SKINNY_ROWS = int(_os.environ.get("BITSMOE_BLOCK_SKINNY_ROWS", "64"))
 _SKINNY_MOST_ROWS = 64            # that the kernel takes at all
@@ -76,6 +76,20 @@ def _few_rows(rows: int, n_in: int, n_out: int) -> bool:
     """Does the few-rows kernel run this GEMM?  (It takes contractions of whole 128 and an even number of outputs.)"""
     return (0 < rows <= min(_SKINNY_ROWS, _SKINNY_MOST_ROWS) and n_in % 128 == 0 and n_out % 2 == 0 and (
         rows <= _SKINNY_ANY_SHAPE_ROWS or (n_in <= _SKINNY_SHORT_CONTRACTION and n_out <= _SKINNY_NARROW_FEATURES)))
+
+
+def _tiled(rows: int, weight: torch.Tensor) -> bool:
+    """Does the library's many-rows kernel run this GEMM?  (Where it is measured to be faster than the framework's; the rows are 16-byte
+    aligned, the stacked weights contiguous.)"""
+    if rows <= _SKINNY_ANY_SHAPE_ROWS:
+        return False
+    n_out, n_in = weight.shape
+    return mlp_forward_cuda.tiled_linear_pays(rows, n_in, n_out)
+
+
+def _differentiated(x: torch.Tensor) -> bool:
+    """Does autograd follow x, in either direction?  (The router's logits are among a block's results.)"""
+    return (x.requires_grad and torch.is_grad_enabled()) or torch.autograd.forward_ad.unpack_dual(x).tangent is not None
 
 
 _SIDE_STREAMS: Dict[int, "torch.cuda.Stream"] = {}
@@ -615,6 +629,8 @@ class BitsMoE_BaseSparseMoeBlock(nn.Module):
             col_gate=rng["h_gate"][0], col_up=rng["h_up"][0], col_logits=rng.get("logits", (0,))[0],
             col_shared_gate=rng.get("sh_gate", (0,))[0], col_shared_up=rng.get("sh_up", (0,))[0],
             col_shared_logit=rng.get("sh_logit", (-1,))[0], shared_intermediate=plan["i_sh"])
+        native.set_weight("w_in_rows", plan["w_in"])
+        native.set_weight("w_out_rows", plan["w_out"])
         if router_weight is not None:
             native.set_weight("w_router", router_weight)
         plan["native"] = (native, stamp)
@@ -678,7 +694,10 @@ class BitsMoE_BaseSparseMoeBlock(nn.Module):
         w_in, w_out = plan["w_in"], plan["w_out"]
         dev = x.device
         stages = 0
-        if _few_rows(rows, hidden, w_in.shape[0]):
+        if _tiled(rows, w_in) and x.stride(0) <= mlp_forward_cuda.TILED_LINEAR_MAX_STRIDE and not _differentiated(x):
+            proj = torch.empty((rows, w_in.shape[0]), dtype=dtype, device=dev)
+            stages |= mlp_forward_cuda.BLOCK_PROJECT_IN_TILED
+        elif _few_rows(rows, hidden, w_in.shape[0]):
             native = self._few_rows_weight(plan, native, "w_in")
             proj = torch.empty((rows, w_in.shape[0]), dtype=dtype, device=dev)
             stages |= mlp_forward_cuda.BLOCK_PROJECT_IN
@@ -695,19 +714,26 @@ class BitsMoE_BaseSparseMoeBlock(nn.Module):
         if super_modules and selected is None:
             selected = torch.empty((rows, self.top_k), dtype=torch.int64, device=dev)
             weights = torch.empty((rows, self.top_k), dtype=torch.float32, device=dev)
-        if _few_rows(rows, w_out.shape[1], hidden):
+        operand = None
+        if _tiled(rows, w_out):
+            out = torch.empty((rows, hidden), dtype=dtype, device=dev)
+            stages |= mlp_forward_cuda.BLOCK_PROJECT_OUT_TILED
+            if rows > _SKINNY_MOST_ROWS:      # (up to that many the library's workspace has room)
+                operand = torch.empty((rows, w_out.shape[1]), dtype=dtype, device=dev)
+        elif _few_rows(rows, w_out.shape[1], hidden):
             native = self._few_rows_weight(plan, native, "w_out")
             out = torch.empty((rows, hidden), dtype=dtype, device=dev)
             stages |= mlp_forward_cuda.BLOCK_PROJECT_OUT
         else:
             out = torch.empty((rows, w_out.shape[1]), dtype=dtype, device=dev)
-            if self._super_expert_items and not super_modules:
-                sup = torch.empty((rows, hidden), dtype=torch.float32, device=dev)
+        projected = bool(stages & (mlp_forward_cuda.BLOCK_PROJECT_OUT | mlp_forward_cuda.BLOCK_PROJECT_OUT_TILED))
+        if self._super_expert_items and not super_modules and (operand is not None or not projected):
+            sup = torch.empty((rows, hidden), dtype=torch.float32, device=dev)
         # The super experts' operator call needs the router's output and the hidden states only: it runs on a side
         # stream beside the packed experts' call (its small launches fill what the packed kernels leave idle).
         side = _side_stream(dev).cuda_stream if self._super_expert_items and _SUPER_SIDE_STREAM and not super_modules else 0
-        mlp_forward_cuda.block_forward(native, x, proj, stages, out, selected, weights, sup, side)
-        if not stages & mlp_forward_cuda.BLOCK_PROJECT_OUT:
+        mlp_forward_cuda.block_forward(native, x, proj, stages, out, selected, weights, sup, side, operand)
+        if not projected:
             out = out @ w_out.T
             if sup is not None:
                 out.add_(sup)

@@ -199,6 +199,16 @@ int bitsmoe_prepare_linear_weight(const void* weight, int32_t in_features, int32
                                   void* stream);
 
 /*
+ * The same product for many rows: out [n_rows, out_features] = x [n_rows, in_features] * weight [out_features, in_features]^T, weight
+ * in the framework's layout, 16-bit x / weight / out of one dtype, fp32 sums (+ addend as above, 16-byte aligned, ld_addend a multiple of 4).
+ * in_features a multiple of 128, out_features of 8; ld_x and ld_out multiples of 8, all pointers 16-byte aligned.
+ * bitsmoe_tiled_linear_pays: 1 where that is measured to be faster than the framework's GEMM (0: slower, or not possible).
+ */
+int bitsmoe_tiled_linear(const void* x, int32_t dtype, int64_t ld_x, const void* weight, int64_t n_rows, int32_t in_features,
+                         int32_t out_features, void* out, int64_t ld_out, const float* addend, int64_t ld_addend, void* stream);
+int32_t bitsmoe_tiled_linear_pays(int64_t n_rows, int32_t in_features, int32_t out_features);
+
+/*
  * The block's closing elementwise pass: one row of the operand of the output GEMM in the activation dtype,
  *   out[t, 0 .. rank_out)                      = rank_accum[t, :]  (fp32 -> 16 bit; bitsmoe/models/base_block.py:414 casts
  *                                                 with a framework op)
@@ -323,7 +333,11 @@ int bitsmoe_moe_forward_routed(const bitsmoe_matset* gate, const bitsmoe_matset*
  *   selected int64 / weights fp32 [T, top_k]: given with BITSMOE_ROUTER_CALLER, else written (may then be null).
  *   out: with BITSMOE_BLOCK_PROJECT_OUT the block output [T, hidden], else the output projection's operand
  *   [T, rank_out + shared_intermediate]; super experts' share: in the output, or (fp32 [T, hidden]) in super_out.
- *   The projections run here at up to 64 tokens; a larger call's workspace has no room for their operand and is refused.
+ *   The few-rows projections run here at up to 64 tokens; a larger call's workspace has no room for their operand and is refused.
+ *   BITSMOE_BLOCK_PROJECT_IN_TILED / _OUT_TILED: the same two projections by bitsmoe_tiled_linear, at any number of tokens, from the
+ *   weights in the framework's layout (w_in_rows, w_out_rows: read with these stages only).  With the latter `operand`
+ *   [T, rank_out + shared_intermediate] in act_dtype (bitsmoe_block_forward_tiled; null: no more than 64 tokens) takes the place of
+ *   `out`, which is the block output, and super_out is needed where there are super experts (null: no more than 64 tokens).
  *   side_stream (may be null): a stream for the super experts' call beside the packed experts'; joined before the call ends.
  */
 #define BITSMOE_ROUTER_LOGITS 0     /* softmax and top-k of proj's logits columns */
@@ -331,6 +345,8 @@ int bitsmoe_moe_forward_routed(const bitsmoe_matset* gate, const bitsmoe_matset*
 #define BITSMOE_ROUTER_CALLER 2
 #define BITSMOE_BLOCK_PROJECT_IN 1
 #define BITSMOE_BLOCK_PROJECT_OUT 2
+#define BITSMOE_BLOCK_PROJECT_IN_TILED 4
+#define BITSMOE_BLOCK_PROJECT_OUT_TILED 8
 typedef struct {
     const bitsmoe_matset *gate, *up, *down;
     const int32_t *global_to_local, *local_to_global;
@@ -342,11 +358,15 @@ typedef struct {
     int32_t top_k, n_global, router_form, renormalize, round_dtype;
     int32_t col_gate, col_up, col_logits, col_shared_gate, col_shared_up, col_shared_logit, shared_intermediate;
     float weight_scale;
+    const void *w_in_rows, *w_out_rows;
 } bitsmoe_block_plan;
 size_t bitsmoe_block_workspace_bytes(const bitsmoe_block_plan* plan, int64_t n_tokens);
 int bitsmoe_block_forward(const bitsmoe_block_plan* plan, const void* x, int64_t ld_x, int64_t n_tokens, void* proj,
                           int32_t stages, void* selected, float* weights, void* out, float* super_out, void* workspace,
                           size_t workspace_bytes, void* side_stream, void* stream);
+int bitsmoe_block_forward_tiled(const bitsmoe_block_plan* plan, const void* x, int64_t ld_x, int64_t n_tokens, void* proj,
+                                int32_t stages, void* selected, float* weights, void* operand, void* out, float* super_out,
+                                void* workspace, size_t workspace_bytes, void* side_stream, void* stream);
 
 /*
  * The forward for callers that cannot allocate device memory (code under HIP graph capture,

@@ -750,3 +750,33 @@ def test_block_workspace_holds_no_projection_past_the_few_rows_kernel(cuda_devic
         hip.block_forward(native, x, proj, hip.BLOCK_PROJECT_OUT, out)
     torch.cuda.synchronize()
     assert bool((out == 3.0).all())
+
+
+# the few-rows kernel's last size, the many-rows kernel with what the workspace holds and with the caller's memory, a grouped-GEMM size
+@pytest.mark.parametrize("tokens", [48, 49, 64, 65, 200])
+@pytest.mark.parametrize("family,shared,super_experts", [("qwen3moe", 0, ()), ("qwen3moe", 0, (1, 6)), ("qwen3next", 128, ()),
+                                                         ("deepseekv2", 256, ())])
+def test_block_projections_by_the_many_rows_kernel(cuda_device, monkeypatch, family, shared, super_experts, tokens):
+    """Equal to the block between the framework's GEMMs up to the roundings that the sums' order may move: projected activations, the
+    output projection's operand and the output are bf16 (2^-8 each), three of them in a row on independent elements."""
+    import torch
+
+    from bitsmoe_amd.models import base_block
+    from bitsmoe_amd.synth import make_layer
+
+    spec = _small_spec(family, shared_intermediate=shared)
+    block = make_layer(spec, device=cuda_device, dtype=torch.bfloat16, seed=71, super_experts=super_experts).eval()
+    block.prepare_runtime_fastpath(warmup=True)
+    x = torch.randn((1, tokens, spec.hidden_size), generator=torch.Generator().manual_seed(tokens)).to(torch.bfloat16).to(cuda_device)
+    as_tensor = lambda y: (y[0] if isinstance(y, tuple) else y).float()
+    with torch.no_grad():
+        out = as_tensor(block(x))
+        monkeypatch.setattr(base_block, "_tiled", lambda rows, weight: False)
+        monkeypatch.setattr(base_block, "_SKINNY_ROWS", 0)
+        ref = as_tensor(block(x))
+    assert float((out - ref).norm() / ref.norm()) <= 3 * 2.0 ** -8
+    wanted = x.clone().requires_grad_(True)
+    monkeypatch.undo()
+    if family != "deepseekv2" and tokens > 64:      # (the logits stay differentiable where they were)
+        logits = block(wanted)[1]
+        assert logits.requires_grad

@@ -796,3 +796,39 @@ def test_router_rounds_with_ties_and_masked_logits(cuda_device, n_experts, top_k
         assert list(sel[t][:len(order)]) == order and not sel[t][len(order):].any()
         # (each weight: one exponential, one division, a sum of at most 64 terms in fp32)
         assert np.allclose(w[t][:len(order)], p / p.sum(), rtol=1e-5, atol=0) and not w[t][len(order):].any()
+
+
+@pytest.mark.parametrize("dtype_name", ["bf16", "f16"])
+@pytest.mark.parametrize("rows,k,n", [(1, 128, 8), (70, 256, 200), (130, 1024, 4232), (100, 256, 5640), (257, 384, 2056), (100, 384, 9736),
+                                      (800, 128, 2056), (250, 640, 9736), (1300, 256, 2056), (500, 1024, 9736), (2040, 128, 4232),
+                                      (1500, 2048, 4160), (1030, 256, 9720)])
+def test_tiled_linear_matches_float64(cuda_device, rows, k, n, dtype_name):
+    """Every tile of the rule, with row and column remainders, rings longer than the contraction, strided x and the fp32 addend.  A sum of k
+    exact products in fp32 is off by less than k 2^-23 of the sum of magnitudes; then one rounding to 16 bits."""
+    import torch
+
+    hip = _hip()
+    dt = {"bf16": torch.bfloat16, "f16": torch.float16}[dtype_name]
+    g = torch.Generator().manual_seed(rows * 7 + n)
+    x = (torch.randn((rows, k), generator=g) * 0.5).to(dt)
+    w = (torch.randn((n, k), generator=g) / k ** 0.5).to(dt)
+    add = torch.randn((rows, n), generator=g)
+    xd, wd = x.to(cuda_device), w.to(cuda_device)
+    exact = xd.double() @ wd.double().T
+    magnitude = xd.double().abs() @ wd.double().abs().T
+    unit = 2.0 ** -8 if dt == torch.bfloat16 else 2.0 ** -11
+    tiny = 2.0 ** -25          # (half of f16's smallest step)
+    out = hip.tiled_linear(xd, wd)
+    assert ((out.double() - exact).abs() <= (1 + unit) * k * 2.0 ** -23 * magnitude + unit * exact.abs() + tiny).all()
+    assert torch.equal(hip.tiled_linear(xd, wd), out)
+    wide = torch.full((rows, k + 24), float("nan"), dtype=dt, device=cuda_device)
+    wide[:, 16:16 + k] = xd
+    assert torch.equal(hip.tiled_linear(wide[:, 16:16 + k], wd), out)
+    added = hip.tiled_linear(xd, wd, add.to(cuda_device))
+    total = exact + add.to(cuda_device).double()
+    bound = (1 + unit) * (k + 1) * 2.0 ** -23 * (magnitude + add.to(cuda_device).double().abs()) + unit * total.abs() + tiny
+    assert ((added.double() - total).abs() <= bound).all()
+    xd[rows // 2, 3] = float("inf")
+    with_inf = hip.tiled_linear(xd, wd)
+    keep = torch.arange(rows, device=cuda_device) != rows // 2
+    assert torch.equal(with_inf[keep], out[keep]) and not torch.isfinite(with_inf[rows // 2]).all()
