@@ -207,6 +207,137 @@ __global__ __launch_bounds__(ROUTE_THREADS) void k_route_fused(
     }
 }
 
+// The whole routing of up to ROUTE_WHOLE_MAX entries in ONE launch, with nothing passed between workgroups: workgroup b places the
+// entries of chunk b, and to know where they go it counts ALL entries itself -- those of earlier chunks (`before`) and the rest
+// (`later`) per expert.  What bounds it: one trip for the ids (every workgroup reads them all, from L2) and the LDS atomics of the count, of
+// which a workgroup has n_flat / 1024 per thread.  Against the three launches below, which wait for each other (kernel times under the tracer, us; two gaps
+// between launches go as well): 1998 entries of 64 experts with the copy of 333 rows 5.8 + 7.0 + 4.7 -> 8.3; 32768 entries of 128 experts
+// 13.1 (with the copy of 4096 rows) + 9.4 + 5.7 -> 15.6 (without).  Whole passes: 333 tokens 123.3 -> 112.4, 512 experts at 256 tokens
+// 173.7 -> 165.0.
+// With side jobs: workgroup n_chunks builds the tile list and token_start, the ones past it copy the activations.
+constexpr int WHOLE_THREADS = 1024;
+constexpr int WHOLE_WAVES = WHOLE_THREADS / 64;
+constexpr int ROUTE_WHOLE_MAX = 32768;
+constexpr int ROUTE_WHOLE_MAX_EXPERTS = 512;
+constexpr int ROUTE_WHOLE_MAX_TOP_K = 64;
+
+template <typename IdT>
+__global__ __launch_bounds__(WHOLE_THREADS) void k_route_whole(
+    const IdT* __restrict__ selected, const float* __restrict__ weights, const int32_t* __restrict__ g2l, int n_global, int n_flat, int top_k,
+    int n_packed, int id_bits, int32_t* __restrict__ token_indices, int32_t* __restrict__ expert_offsets, float* __restrict__ route_flat,
+    int n_chunks, const RouteSideJobs jobs) {
+    extern __shared__ int lds[];
+    __shared__ MTileLds mt_lds;
+    __shared__ int wave_sums[WHOLE_WAVES];
+    __shared__ uint64_t kept[WHOLE_WAVES + 1];      // which entries of the 64 in front of the chunk and of the chunk have an expert here
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int b = blockIdx.x;
+    if (b > n_chunks) {
+        // the f16 copy of the activations, grid-stride over groups of eight
+        const int64_t n_g = jobs.T * (jobs.ldg >> 3), n_u = jobs.T * (jobs.ldu >> 3);
+        const int64_t step = (int64_t)(gridDim.x - n_chunks - 1) * WHOLE_THREADS;
+        for (int64_t i = (int64_t)(b - n_chunks - 1) * WHOLE_THREADS + tid; i < n_g + n_u; i += step) {
+            if (i < n_g)
+                convert_bf16_group(jobs.src_g, jobs.dst_g, jobs.sg, jobs.ldg, i);
+            else
+                convert_bf16_group(jobs.src_u, jobs.dst_u, jobs.su, jobs.ldu, i - n_g);
+        }
+        return;
+    }
+    int* offsets = lds;                          // [n_packed + 1]: `later`, then all, then the exclusive scan
+    int* before = lds + n_packed + 1;            // [n_packed]
+    int* tables = before + n_packed;             // [WHOLE_WAVES][n_packed]: entries of an expert in the chunk's wavefronts
+    int* map = tables + WHOLE_WAVES * n_packed;  // [n_global] when it fits
+    const bool map_in_lds = n_global <= ROUTE_G2L_LDS_MAX;
+    const bool places = b < n_chunks;
+    const int chunk = b * WHOLE_THREADS;
+    const int mine = chunk + tid, in_front = chunk - 64 + lane;
+    auto raw_id = [&](int i) -> int64_t { return i >= 0 && i < n_flat ? (int64_t)selected[i] : -1; };
+    const int64_t raw_mine = places ? raw_id(mine) : -1;
+    const int64_t raw_front = places && wave == 0 ? raw_id(in_front) : -1;
+    const float weight = places && mine < n_flat ? weights[mine] : 0.0f;
+    constexpr int AHEAD = 4;      // ids a thread has on their way at once
+    int64_t raw[AHEAD];
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j) raw[j] = raw_id(j * WHOLE_THREADS + tid);
+    for (int i = tid; i < (WHOLE_WAVES + 2) * n_packed + 1; i += WHOLE_THREADS) lds[i] = 0;
+    if (map_in_lds)
+        for (int i = tid; i < n_global; i += WHOLE_THREADS) map[i] = g2l[i];
+    __syncthreads();
+    auto local_of = [&](int64_t g) {
+        if (g < 0 || g >= n_global) return -1;
+        const int l = map_in_lds ? map[g] : g2l[g];
+        return l >= 0 && l < n_packed ? l : -1;
+    };
+    for (int at = 0; at < n_flat; at += AHEAD * WHOLE_THREADS) {
+        int64_t now[AHEAD];
+#pragma unroll
+        for (int j = 0; j < AHEAD; ++j) now[j] = raw[j];
+#pragma unroll
+        for (int j = 0; j < AHEAD; ++j) raw[j] = raw_id(at + (AHEAD + j) * WHOLE_THREADS + tid);
+#pragma unroll
+        for (int j = 0; j < AHEAD; ++j) {
+            const int l = local_of(now[j]);
+            if (l >= 0) atomicAdd((at + j * WHOLE_THREADS < chunk ? before : offsets) + l, 1);
+        }
+    }
+    const int id = local_of(raw_mine);
+    int rank = 0;
+    if (places) {
+        const uint64_t same = match_same_id(id, id_bits);
+        rank = __popcll(same & ((1ull << lane) - 1ull));
+        if (id >= 0 && lane == 63 - __clzll((long long)same)) tables[wave * n_packed + id] = __popcll(same);
+        const uint64_t k = __ballot(id >= 0);
+        if (lane == 0) kept[wave + 1] = k;
+        if (wave == 0) {
+            const uint64_t f = __ballot(local_of(raw_front) >= 0);
+            if (lane == 0) kept[0] = f;
+        }
+    }
+    __syncthreads();
+    for (int e = tid; e < n_packed; e += WHOLE_THREADS) {
+        int run = before[e];
+        offsets[e] += run;
+        if (places) {
+            for (int t = 0; t < WHOLE_WAVES; ++t) {
+                const int c = tables[t * n_packed + e];
+                tables[t * n_packed + e] = run;
+                run += c;
+            }
+        }
+    }
+    __syncthreads();
+    const int total = block_exclusive_scan(offsets, n_packed, wave_sums);
+    if (b == 0) {
+        for (int e = tid; e < n_packed; e += WHOLE_THREADS) expert_offsets[e] = offsets[e];
+        if (tid == 0) expert_offsets[n_packed] = total;
+    }
+    if (!places) {
+        if (tid == 0) offsets[n_packed] = total;
+        if (jobs.token_start != nullptr)
+            for (int64_t t = tid; t <= jobs.T; t += WHOLE_THREADS) jobs.token_start[t] = (int32_t)(t * top_k);
+        if (jobs.mtiles == nullptr) return;
+        __syncthreads();
+        build_mtile_list(offsets, n_packed, n_flat, jobs.mtile_rows, jobs.max_mtiles, jobs.mtiles, jobs.n_mtiles, jobs.gate_fe, jobs.up_fe, mt_lds);
+        return;
+    }
+    if (mine >= n_flat) return;
+    const int token = mine / top_k;
+    int earlier = 0;      // kept entries of the same token in front of this one (they are neighbours in the flat order)
+    if (jobs.slot != nullptr) {
+        const int nth = mine - token * top_k;      // < 64: at most this word of `kept` and the one in front of it
+        const uint64_t here = kept[wave + 1] & ((1ull << lane) - 1ull);
+        earlier = __popcll(lane >= nth ? here >> (lane - nth) : here);
+        if (lane < nth) earlier += __popcll(kept[wave] >> (64 - (nth - lane)));
+        if (nth == top_k - 1) jobs.token_count[token] = earlier + (id >= 0);
+    }
+    if (id < 0) return;
+    const int pos = offsets[id] + tables[wave * n_packed + id] + rank;
+    token_indices[pos] = token;
+    route_flat[pos] = weight;
+    if (jobs.slot != nullptr) jobs.slot[pos] = earlier;
+}
+
 // Multi-workgroup version: (1) per-chunk ranks + histograms, (2) scan, (3) scatter.
 template <typename IdT>
 __global__ __launch_bounds__(ROUTE_THREADS) void k_route_count(
@@ -352,6 +483,23 @@ static int route_impl(const IdT* selected, const float* weights, const int32_t* 
                            g2l, n_global, n_flat, top_k, n_packed, id_bits, token_indices, expert_offsets,
                            route_flat);
         BITSMOE_HIP_TRY(hipGetLastError());
+        return BITSMOE_OK;
+    }
+    if (n_flat <= ROUTE_WHOLE_MAX && n_packed <= ROUTE_WHOLE_MAX_EXPERTS && top_k <= ROUTE_WHOLE_MAX_TOP_K) {
+        const RouteSideJobs carried = jobs ? *jobs : RouteSideJobs{};
+        const int chunks = (int)((n_flat + WHOLE_THREADS - 1) / WHOLE_THREADS);
+        int64_t copy_blocks = 0;
+        if (carried.src_g != nullptr)
+            copy_blocks = std::min<int64_t>((carried.T * ((carried.ldg >> 3) + (carried.ldu >> 3)) + WHOLE_THREADS - 1) / WHOLE_THREADS, 1024);
+        const size_t bytes = ((size_t)(WHOLE_WAVES + 2) * n_packed + 1 + (n_global <= ROUTE_G2L_LDS_MAX ? n_global : 0)) * sizeof(int);
+        // (the tile list's workgroup also where there is no list to build: only the copies come behind it)
+        const int64_t grid = chunks + (carried.mtiles || carried.token_start || copy_blocks ? 1 : 0) + copy_blocks;
+        hipLaunchKernelGGL(k_route_whole<IdT>, dim3((unsigned)grid), dim3(WHOLE_THREADS), bytes, st, selected, weights, g2l, n_global, (int)n_flat,
+                           top_k, n_packed, id_bits, token_indices, expert_offsets, route_flat, chunks, carried);
+        BITSMOE_HIP_TRY(hipGetLastError());
+        if (jobs_done)
+            *jobs_done = (copy_blocks > 0 ? MFMA_FRONT_CONVERTED : 0) |
+                         (carried.slot && carried.token_start ? MFMA_FRONT_TOKEN_COUNTED : 0) | (carried.mtiles ? MFMA_FRONT_MTILES : 0);
         return BITSMOE_OK;
     }
     const int64_t n_chunks = (n_flat + ROUTE_CHUNK - 1) / ROUTE_CHUNK;
