@@ -97,15 +97,22 @@ extern "C" int bitsmoe_block_forward_tiled(const bitsmoe_block_plan* p, const vo
 
     if (tiled_in)
         BITSMOE_TRY(bitsmoe_tiled_linear(x, p->act_dtype, ld_x, p->w_in_rows, n_tokens, p->hidden, p->in_features, proj, ld, nullptr, 0, stream));
-    if (few_in)
-        BITSMOE_TRY(bitsmoe_skinny_linear(x, p->act_dtype, 0, ld_x, p->w_in, p->w_in_prepared, n_tokens, p->hidden, p->in_features,
-                                          proj, ld, nullptr, 0, stream));
     if (!selected) selected = ws + w.selected;
     if (!weights) weights = (float*)(ws + w.weights);
+    bool routed = false;
+    if (few_in && p->router_form == BITSMOE_ROUTER_LINEAR &&
+        skinny_linear_takes_router(n_tokens, p->hidden, p->w_in_prepared, p->n_global, p->top_k)) {
+        const RouterBeside router = {p->w_router, p->n_global, p->top_k, p->renormalize, p->round_dtype, p->weight_scale, (int64_t*)selected, weights};
+        BITSMOE_TRY(skinny_linear_with_router(x, p->act_dtype, ld_x, p->w_in, n_tokens, p->hidden, p->in_features, proj, ld, router, stream));
+        routed = true;
+    } else if (few_in) {
+        BITSMOE_TRY(bitsmoe_skinny_linear(x, p->act_dtype, 0, ld_x, p->w_in, p->w_in_prepared, n_tokens, p->hidden, p->in_features,
+                                          proj, ld, nullptr, 0, stream));
+    }
     if (p->router_form == BITSMOE_ROUTER_LOGITS)
         BITSMOE_TRY(bitsmoe_router_softmax_topk_strided(big + p->col_logits, p->act_dtype, ld, n_tokens, p->n_global, p->top_k,
                                                         p->renormalize, p->weight_scale, p->round_dtype, selected, 1, weights, stream));
-    else if (p->router_form == BITSMOE_ROUTER_LINEAR)
+    else if (p->router_form == BITSMOE_ROUTER_LINEAR && !routed)
         BITSMOE_TRY(bitsmoe_router_linear_topk(x, p->act_dtype, ld_x, p->w_router, 1, n_tokens, p->hidden, p->n_global, p->top_k,
                                                p->renormalize, p->weight_scale, p->round_dtype, selected, 1, weights, stream));
     // The super experts' operator call needs the router's output and the hidden states only: on the side stream it runs

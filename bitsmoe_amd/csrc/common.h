@@ -193,6 +193,18 @@ int block_finish(const float* rank_accum, int64_t n_tokens, int32_t rank_out, co
 int skinny_linear(const void* x, int32_t dtype, int32_t x_is_f32, int64_t ld_x, const void* weight, int32_t weight_is_prepared,
                   int64_t n_rows, int32_t in_features, int32_t out_features, void* out, int64_t ld_out, const float* addend,
                   int64_t ld_addend, void* stream);
+// The router's linear layer and top-k (bitsmoe_router_linear_topk, prepared weight, 64-bit ids) in the launch of a few-rows projection of the
+// same rows, which has no addend.
+struct RouterBeside {
+    const void* weight;
+    int32_t n_experts, top_k, renormalize, round_dtype;
+    float weight_scale;
+    int64_t* selected;
+    float* weights;
+};
+bool skinny_linear_takes_router(int64_t n_rows, int32_t in_features, int32_t weight_is_prepared, int32_t n_experts, int32_t top_k);
+int skinny_linear_with_router(const void* x, int32_t dtype, int64_t ld_x, const void* weight, int64_t n_rows, int32_t in_features,
+                              int32_t out_features, void* out, int64_t ld_out, const RouterBeside& router, void* stream);
 bool skinny_f32_rows_possible(int64_t n_rows, int32_t in_features, int32_t weight_is_prepared);
 
 // bf16 -> f16, eight elements at a time: group `i` of `total = T * (ld / 8)` groups of one projection.

@@ -21,6 +21,7 @@
 //   2048 -> 9728 features: 9.7 (15.9;  9.9), 11.1 (14.4; 12.6), 13.0 (14.4; 18.1), 15.2 (15.5; 23.5), 17.6 (15.5; 28.6)
 // (Shares that are no whole passes -- 4864 features are eight of nineteen steps -- pay for their selects: 0.5 to 1 us.)
 #include "common.h"
+#include "router_bodies.h"
 
 #include <algorithm>
 #include <type_traits>
@@ -44,10 +45,13 @@ __device__ __forceinline__ void static_for_pieces(F&& f, std::integer_sequence<i
 // [k-step of 32][lane][8 values], so that a wavefront's load is 1 KB of consecutive memory instead of sixteen 64-byte
 // pieces of sixteen rows.
 // TURN: x by way of LDS; else (a few rows: nothing to gain from whole lines) every step's operand straight from x.
+template <int NMB, int NW, bool XF32, bool TURN>
+constexpr int SKINNY_LDS_BYTES = std::max(TURN ? NW * 16 * NMB * 32 * (NMB <= (XF32 ? 1 : 2) ? 4 : 2) * (XF32 ? 4 : 2) : 0, NW * NMB * 16 * 17 * 4);
+
 template <bool BF16, int NMB, int NW, int MAXS, bool XF32, bool PREP, bool TURN, bool WHOLE>
-__global__ __launch_bounds__(64 * NW) void k_skinny_linear(const void* __restrict__ x, int64_t ld_x, const uint16_t* __restrict__ w,
-                                                           int T, int K, int N, uint16_t* __restrict__ out, int64_t ld_out,
-                                                           const float* __restrict__ addend, int64_t ld_add) {
+__device__ __forceinline__ void skinny_body(const void* __restrict__ x, int64_t ld_x, const uint16_t* __restrict__ w, int T, int K, int N,
+                                            uint16_t* __restrict__ out, int64_t ld_out, const float* __restrict__ addend, int64_t ld_add,
+                                            int column_block, unsigned char* lds, unsigned char* zero_piece) {
     static_assert(TURN || NMB == 1, "few rows: one block of 16 rows");
     constexpr int G = NMB <= (XF32 ? 1 : 2) ? 4 : 2;   // k-steps per piece of x
     static_assert(MAXS % G == 0, "whole pieces");
@@ -57,12 +61,11 @@ __global__ __launch_bounds__(64 * NW) void k_skinny_linear(const void* __restric
     constexpr int NI = 16 * NMB / RPI;                 // load instructions per piece
     constexpr int PIECE = TURN ? 16 * NMB * CPR * 16 : 0;      // bytes
     constexpr int PART = NW * NMB * 16 * 17 * 4;
-    __shared__ __attribute__((aligned(16))) unsigned char lds[NW * PIECE > PART ? NW * PIECE : PART];
-    __shared__ __attribute__((aligned(16))) unsigned char zero_piece[16];
+    static_assert((NW * PIECE > PART ? NW * PIECE : PART) == SKINNY_LDS_BYTES<NMB, NW, XF32, TURN>, "the kernel's LDS");
     const int lane = threadIdx.x & 63;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n = lane & 15, kg = lane >> 4;
-    const int n0 = blockIdx.x * 16;
+    const int n0 = column_block * 16;
     if (TURN && lane == 0) *reinterpret_cast<sk_u32x4*>(zero_piece) = sk_u32x4{0u, 0u, 0u, 0u};      // (by every wavefront: no barrier)
     const int steps = K >> 5;
     const int first = wv * steps / NW, end = (wv + 1) * steps / NW;
@@ -75,7 +78,7 @@ __global__ __launch_bounds__(64 * NW) void k_skinny_linear(const void* __restric
         const int r = i * RPI + lane / CPR;
         xrow[i] = (const unsigned char*)x + (int64_t)min(r, T - 1) * ld_x * EB + ((lane % CPR) ^ swz(r)) * 16;
     }
-    const uint16_t* wp = PREP ? w + ((int64_t)blockIdx.x * steps) * 512 + lane * 8 : w + (int64_t)min(n0 + n, N - 1) * K + kg * 8;
+    const uint16_t* wp = PREP ? w + ((int64_t)column_block * steps) * 512 + lane * 8 : w + (int64_t)min(n0 + n, N - 1) * K + kg * 8;
     sk_f32x4 acc[NMB];
 #pragma unroll
     for (int mb = 0; mb < NMB; ++mb) acc[mb] = sk_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -196,6 +199,37 @@ __global__ __launch_bounds__(64 * NW) void k_skinny_linear(const void* __restric
         }
         *reinterpret_cast<uint32_t*>(out + (int64_t)row * ld_out + n0 + c) = round16(v0) | (round16(v1) << 16);
     }
+}
+
+template <bool BF16, int NMB, int NW, int MAXS, bool XF32, bool PREP, bool TURN, bool WHOLE>
+__global__ __launch_bounds__(64 * NW) void k_skinny_linear(const void* __restrict__ x, int64_t ld_x, const uint16_t* __restrict__ w,
+                                                           int T, int K, int N, uint16_t* __restrict__ out, int64_t ld_out,
+                                                           const float* __restrict__ addend, int64_t ld_add) {
+    __shared__ __attribute__((aligned(16))) unsigned char lds[SKINNY_LDS_BYTES<NMB, NW, XF32, TURN>];
+    __shared__ __attribute__((aligned(16))) unsigned char zero_piece[16];
+    skinny_body<BF16, NMB, NW, MAXS, XF32, PREP, TURN, WHOLE>(x, ld_x, w, T, K, N, out, ld_out, addend, ld_add, blockIdx.x, lds, zero_piece);
+}
+
+// The input projection and, in its first `router_blocks` workgroups, the router's linear layer and top-k of four tokens each: both read
+// the hidden states only.  What bounds the router is what one CU can fetch (256 KB of gate weight at 64 experts and a hidden size of 2048), so
+// on its own it takes about as long as the projection, on a card that is idle but for one workgroup per sixteen tokens; here
+// it is over before the projection is.  ROUTER_BESIDE_FIGURES
+constexpr int ROUTER_BESIDE_NB = 4;      // 16-expert blocks
+template <bool BF16, int NMB, int MAXS, bool TURN>
+__global__ __launch_bounds__(256) void k_skinny_linear_router(const void* __restrict__ x, int64_t ld_x, const uint16_t* __restrict__ w, int T,
+                                                              int K, int N, uint16_t* __restrict__ out, int64_t ld_out, int router_blocks,
+                                                              const RouterBeside r) {
+    using RouterLds = RouterLinearLds<ROUTER_BESIDE_NB, 4>;
+    constexpr int BYTES = std::max((int)sizeof(RouterLds), SKINNY_LDS_BYTES<NMB, 4, false, TURN>);
+    __shared__ __attribute__((aligned(16))) unsigned char lds[BYTES];
+    __shared__ __attribute__((aligned(16))) unsigned char zero_piece[16];
+    if ((int)blockIdx.x < router_blocks)
+        router_linear_body<BF16, ROUTER_BESIDE_NB, 4, true, 4>((const uint16_t*)x, ld_x, (const uint16_t*)r.weight, T, K, r.n_experts, r.top_k,
+                                                               r.weight_scale, r.renormalize, r.round_dtype, nullptr, r.selected, r.weights,
+                                                               blockIdx.x * 4, *reinterpret_cast<RouterLds*>(lds));
+    else
+        skinny_body<BF16, NMB, 4, MAXS, false, true, TURN, true>(x, ld_x, w, T, K, N, out, ld_out, nullptr, 0, blockIdx.x - router_blocks, lds,
+                                                                 zero_piece);
 }
 
 // W [N, K] -> [ceil(N / 16)][K / 32][64 lanes][8]: lane = 16 * (k % 32 / 8) + n % 16 holds W[n][32 ks + 8 (lane / 16) .. + 7];
@@ -336,6 +370,47 @@ int bitsmoe::skinny_linear(const void* x, int32_t dtype, int32_t x_is_f32, int64
         else by_share(bf_c, integral_constant<int, 4>{}, No{}, Yes{});
     };
     if (dtype == BITSMOE_DT_BF16) by_rows(Yes{}); else by_rows(No{});
+    BITSMOE_HIP_TRY(hipGetLastError());
+    return BITSMOE_OK;
+}
+
+// Prepared weights whose contraction is four whole shares of the few-rows kernel (hidden sizes 1024, 1536, 2048 and 2560), up to 64 experts.
+bool bitsmoe::skinny_linear_takes_router(int64_t n_rows, int32_t in_features, int32_t weight_is_prepared, int32_t n_experts, int32_t top_k) {
+    return n_rows >= 1 && n_rows <= 48 && weight_is_prepared != 0 && n_experts >= 1 && n_experts <= 16 * ROUTER_BESIDE_NB && top_k >= 1 && top_k <= n_experts &&
+           (in_features == 1024 || in_features == 1536 || in_features == 2048 || in_features == 2560);
+}
+
+int bitsmoe::skinny_linear_with_router(const void* x, int32_t dtype, int64_t ld_x, const void* weight, int64_t n_rows, int32_t in_features,
+                                       int32_t out_features, void* out, int64_t ld_out, const RouterBeside& router, void* stream) {
+    BITSMOE_REQUIRE(dtype == BITSMOE_DT_F16 || dtype == BITSMOE_DT_BF16, "dtype must be f16 (0) or bf16 (1)");
+    BITSMOE_REQUIRE(skinny_linear_takes_router(n_rows, in_features, 1, router.n_experts, router.top_k), "not a shape of the joint launch");
+    BITSMOE_REQUIRE(out_features >= 2 && out_features % 2 == 0, "out_features must be even");
+    BITSMOE_REQUIRE(ld_x >= in_features && ld_x % 8 == 0, "ld_x must be at least in_features and a multiple of 8");
+    BITSMOE_REQUIRE(ld_out >= out_features && ld_out % 2 == 0, "ld_out must be at least out_features and even");
+    BITSMOE_REQUIRE(router.round_dtype >= -1 && router.round_dtype <= 1, "round_dtype must be -1 (none), 0 (fp16) or 1 (bf16)");
+    BITSMOE_REQUIRE(x && weight && out && router.weight && router.selected && router.weights, "null pointer");
+    BITSMOE_REQUIRE((((uintptr_t)x | (uintptr_t)weight | (uintptr_t)router.weight) & 15) == 0 && ((uintptr_t)out & 3) == 0,
+                    "x and the weights must be 16-byte aligned, out 4-byte aligned");
+    const int router_blocks = (int)((n_rows + 3) / 4);
+    const dim3 grid((unsigned)(router_blocks + (out_features + 15) / 16));
+    auto run = [&](auto bf_c, auto nmb_c, auto s_c, auto turn_c) {
+        hipLaunchKernelGGL((k_skinny_linear_router<decltype(bf_c)::value, decltype(nmb_c)::value, decltype(s_c)::value, decltype(turn_c)::value>), grid,
+                           dim3(256), 0, (hipStream_t)stream, x, ld_x, (const uint16_t*)weight, (int)n_rows, in_features, out_features,
+                           (uint16_t*)out, ld_out, router_blocks, router);
+    };
+    auto by_share = [&](auto bf_c, auto nmb_c, auto turn_c) {
+        if (in_features == 1024) run(bf_c, nmb_c, std::integral_constant<int, 8>{}, turn_c);
+        else if (in_features == 1536) run(bf_c, nmb_c, std::integral_constant<int, 12>{}, turn_c);
+        else if (in_features == 2048) run(bf_c, nmb_c, std::integral_constant<int, 16>{}, turn_c);
+        else run(bf_c, nmb_c, std::integral_constant<int, 20>{}, turn_c);
+    };
+    auto by_rows = [&](auto bf_c) {
+        if (n_rows <= 4) by_share(bf_c, std::integral_constant<int, 1>{}, std::false_type{});
+        else if (n_rows <= 16) by_share(bf_c, std::integral_constant<int, 1>{}, std::true_type{});
+        else if (n_rows <= 32) by_share(bf_c, std::integral_constant<int, 2>{}, std::true_type{});
+        else by_share(bf_c, std::integral_constant<int, 3>{}, std::true_type{});
+    };
+    if (dtype == BITSMOE_DT_BF16) by_rows(std::true_type{}); else by_rows(std::false_type{});
     BITSMOE_HIP_TRY(hipGetLastError());
     return BITSMOE_OK;
 }

@@ -780,3 +780,41 @@ def test_block_projections_by_the_many_rows_kernel(cuda_device, monkeypatch, fam
     if family != "deepseekv2" and tokens > 64:      # (the logits stay differentiable where they were)
         logits = block(wanted)[1]
         assert logits.requires_grad
+
+
+# one to four tokens per router workgroup, all forms of the few-rows kernel (operands straight from memory, one to three blocks of rows) and
+# the first size past it; all hidden sizes the joint launch takes and one it does not; whole and partial 16-expert blocks
+@pytest.mark.parametrize("tokens", [1, 4, 5, 16, 17, 33, 48, 49])
+@pytest.mark.parametrize("hidden,experts", [(1024, 64), (1536, 8), (2048, 40), (2560, 64), (640, 64), (1024, 72)])
+@pytest.mark.parametrize("dtype_name", ["bfloat16", "float16"])
+def test_router_beside_the_input_projection(cuda_device, monkeypatch, dtype_name, hidden, experts, tokens):
+    """The block's picks are the router kernel's on its own (logits in another order of fp32 sums: a pick may only change where two logits are
+    closer than that), its projected rows the projection's on its own, bit for bit."""
+    import torch
+
+    from bitsmoe_amd.algorithms import mlp_forward_cuda as hip
+    from bitsmoe_amd.synth import make_layer
+
+    dtype = getattr(torch, dtype_name)
+    spec = _small_spec("deepseekv2", num_experts=experts, top_k=6, hidden_size=hidden, intermediate_size=128)
+    block = make_layer(spec, device=cuda_device, dtype=dtype, seed=81, basis_seed=7).eval()
+    block.prepare_runtime_fastpath(warmup=True)
+    x = torch.randn((1, tokens, hidden), generator=torch.Generator().manual_seed(tokens + experts)).to(dtype).to(cuda_device)
+    real, seen = hip.block_forward, {}
+
+    def spy(native, x, proj, stages, out, selected, weights, *rest):
+        selected = torch.full((tokens, 6), -1, dtype=torch.int64, device=cuda_device)
+        weights = torch.full((tokens, 6), float("nan"), device=cuda_device)
+        real(native, x, proj, stages, out, selected, weights, *rest)
+        seen.update(native=native, x=x, proj=proj, stages=stages, selected=selected, weights=weights)
+
+    monkeypatch.setattr(hip, "block_forward", spy)
+    with torch.no_grad():
+        block(x)
+    c, kept = seen["native"].c, seen["native"]._weights
+    sel, wt = hip.router_linear_topk(seen["x"], kept["w_router"], 6, bool(c.renormalize), weight_scale=float(c.weight_scale),
+                                     round_dtype={-1: None, 0: torch.float16, 1: torch.bfloat16}[c.round_dtype])
+    assert torch.equal(seen["selected"], sel)
+    assert torch.allclose(seen["weights"], wt, rtol=1e-5, atol=0)
+    if seen["stages"] & hip.BLOCK_PROJECT_IN:
+        assert torch.equal(seen["proj"], hip.skinny_linear(seen["x"], kept["w_in"]))
