@@ -214,17 +214,16 @@ __global__ __launch_bounds__(64 * NW) void k_skinny_linear(const void* __restric
 // the hidden states only.  What bounds the router is what one CU can fetch (256 KB of gate weight at 64 experts and a hidden size of 2048), so
 // on its own it takes about as long as the projection, on a card that is idle but for one workgroup per sixteen tokens; here
 // it is over before the projection is.  ROUTER_BESIDE_FIGURES
-constexpr int ROUTER_BESIDE_NB = 4;      // 16-expert blocks
-template <bool BF16, int NMB, int MAXS, bool TURN>
+template <bool BF16, int NMB, int MAXS, bool TURN, int NB>      // NB: 16-expert blocks
 __global__ __launch_bounds__(256) void k_skinny_linear_router(const void* __restrict__ x, int64_t ld_x, const uint16_t* __restrict__ w, int T,
                                                               int K, int N, uint16_t* __restrict__ out, int64_t ld_out, int router_blocks,
                                                               const RouterBeside r) {
-    using RouterLds = RouterLinearLds<ROUTER_BESIDE_NB, 4>;
+    using RouterLds = RouterLinearLds<NB, 4>;
     constexpr int BYTES = std::max((int)sizeof(RouterLds), SKINNY_LDS_BYTES<NMB, 4, false, TURN>);
     __shared__ __attribute__((aligned(16))) unsigned char lds[BYTES];
     __shared__ __attribute__((aligned(16))) unsigned char zero_piece[16];
     if ((int)blockIdx.x < router_blocks)
-        router_linear_body<BF16, ROUTER_BESIDE_NB, 4, true, 4>((const uint16_t*)x, ld_x, (const uint16_t*)r.weight, T, K, r.n_experts, r.top_k,
+        router_linear_body<BF16, NB, 4, true, 4>((const uint16_t*)x, ld_x, (const uint16_t*)r.weight, T, K, r.n_experts, r.top_k,
                                                                r.weight_scale, r.renormalize, r.round_dtype, nullptr, r.selected, r.weights,
                                                                blockIdx.x * 4, *reinterpret_cast<RouterLds*>(lds));
     else
@@ -374,9 +373,9 @@ int bitsmoe::skinny_linear(const void* x, int32_t dtype, int32_t x_is_f32, int64
     return BITSMOE_OK;
 }
 
-// Prepared weights whose contraction is four whole shares of the few-rows kernel (hidden sizes 1024, 1536, 2048 and 2560), up to 64 experts.
+// Prepared weights whose contraction is four whole shares of the few-rows kernel (hidden sizes 1024, 1536, 2048 and 2560), up to 128 experts.
 bool bitsmoe::skinny_linear_takes_router(int64_t n_rows, int32_t in_features, int32_t weight_is_prepared, int32_t n_experts, int32_t top_k) {
-    return n_rows >= 1 && n_rows <= 48 && weight_is_prepared != 0 && n_experts >= 1 && n_experts <= 16 * ROUTER_BESIDE_NB && top_k >= 1 && top_k <= n_experts &&
+    return n_rows >= 1 && n_rows <= 48 && weight_is_prepared != 0 && n_experts >= 1 && n_experts <= 128 && top_k >= 1 && top_k <= 64 && top_k <= n_experts &&
            (in_features == 1024 || in_features == 1536 || in_features == 2048 || in_features == 2560);
 }
 
@@ -393,10 +392,14 @@ int bitsmoe::skinny_linear_with_router(const void* x, int32_t dtype, int64_t ld_
                     "x and the weights must be 16-byte aligned, out 4-byte aligned");
     const int router_blocks = (int)((n_rows + 3) / 4);
     const dim3 grid((unsigned)(router_blocks + (out_features + 15) / 16));
-    auto run = [&](auto bf_c, auto nmb_c, auto s_c, auto turn_c) {
-        hipLaunchKernelGGL((k_skinny_linear_router<decltype(bf_c)::value, decltype(nmb_c)::value, decltype(s_c)::value, decltype(turn_c)::value>), grid,
-                           dim3(256), 0, (hipStream_t)stream, x, ld_x, (const uint16_t*)weight, (int)n_rows, in_features, out_features,
+    auto run_nb = [&](auto bf_c, auto nmb_c, auto s_c, auto turn_c, auto nb_c) {
+        hipLaunchKernelGGL((k_skinny_linear_router<decltype(bf_c)::value, decltype(nmb_c)::value, decltype(s_c)::value, decltype(turn_c)::value,
+                                                   decltype(nb_c)::value>), grid, dim3(256), 0, (hipStream_t)stream, x, ld_x, (const uint16_t*)weight, (int)n_rows, in_features, out_features,
                            (uint16_t*)out, ld_out, router_blocks, router);
+    };
+    auto run = [&](auto bf_c, auto nmb_c, auto s_c, auto turn_c) {
+        if (router.n_experts <= 64) run_nb(bf_c, nmb_c, s_c, turn_c, std::integral_constant<int, 4>{});
+        else run_nb(bf_c, nmb_c, s_c, turn_c, std::integral_constant<int, 8>{});
     };
     auto by_share = [&](auto bf_c, auto nmb_c, auto turn_c) {
         if (in_features == 1024) run(bf_c, nmb_c, std::integral_constant<int, 8>{}, turn_c);

@@ -785,7 +785,7 @@ def test_block_projections_by_the_many_rows_kernel(cuda_device, monkeypatch, fam
 # one to four tokens per router workgroup, all forms of the few-rows kernel (operands straight from memory, one to three blocks of rows) and
 # the first size past it; all hidden sizes the joint launch takes and one it does not; whole and partial 16-expert blocks
 @pytest.mark.parametrize("tokens", [1, 4, 5, 16, 17, 33, 48, 49])
-@pytest.mark.parametrize("hidden,experts", [(1024, 64), (1536, 8), (2048, 40), (2560, 64), (640, 64), (1024, 72)])
+@pytest.mark.parametrize("hidden,experts", [(1024, 64), (1536, 8), (2048, 40), (2560, 64), (640, 64), (1024, 72), (2048, 128), (1024, 136)])
 @pytest.mark.parametrize("dtype_name", ["bfloat16", "float16"])
 def test_router_beside_the_input_projection(cuda_device, monkeypatch, dtype_name, hidden, experts, tokens):
     """The block's picks are the router kernel's on its own (logits in another order of fp32 sums: a pick may only change where two logits are
