@@ -478,14 +478,18 @@ static int route_impl(const IdT* selected, const float* weights, const int32_t* 
                                                    ? ((size_t)ROUTE_ROUNDS * (ROUTE_THREADS / 64) * n_packed +
                                                       (n_global <= ROUTE_G2L_LDS_MAX ? n_global : 0)) * sizeof(int)
                                                    : 0);
-    if (n_flat <= ROUTE_CHUNK) {
+    const bool whole = n_flat <= ROUTE_WHOLE_MAX && n_packed <= ROUTE_WHOLE_MAX_EXPERTS && top_k <= ROUTE_WHOLE_MAX_TOP_K;
+    // (tables alone, 72 entries of 64 experts: 4.6 us by the one workgroup of 256 threads, 5.3 by the other kernel's 1024; but with the grouped
+    // GEMM's front end that one saves three launches: operator, us, 32 experts top-4 128 tokens 74.8 -> 66.8, 64 top-6 160 tokens 108.3 -> 98.9,
+    // 48 top-8 100 tokens 72.7 -> 63.0, 32 top-8 60 tokens 80.9 -> 73.3)
+    if (n_flat <= ROUTE_CHUNK && !(whole && jobs != nullptr)) {
         hipLaunchKernelGGL(k_route_fused<IdT>, dim3(1), dim3(ROUTE_THREADS), lds_rank_bytes, st, selected, weights,
                            g2l, n_global, n_flat, top_k, n_packed, id_bits, token_indices, expert_offsets,
                            route_flat);
         BITSMOE_HIP_TRY(hipGetLastError());
         return BITSMOE_OK;
     }
-    if (n_flat <= ROUTE_WHOLE_MAX && n_packed <= ROUTE_WHOLE_MAX_EXPERTS && top_k <= ROUTE_WHOLE_MAX_TOP_K) {
+    if (whole) {
         const RouteSideJobs carried = jobs ? *jobs : RouteSideJobs{};
         const int chunks = (int)((n_flat + WHOLE_THREADS - 1) / WHOLE_THREADS);
         int64_t copy_blocks = 0;
