@@ -132,10 +132,10 @@ inline int decode_part_capacity(int64_t n_assign) { return n_assign <= 1024 ? 4 
 bool mfma_path_supported(const bitsmoe_matset* gate, const bitsmoe_matset* up, const bitsmoe_matset* down, int I);
 size_t mfma_workspace_bytes(const bitsmoe_matset* gate, const bitsmoe_matset* up, const bitsmoe_matset* down, int64_t T,
                             int64_t A, int I);
-// Work of the grouped-GEMM path's front end that the routing launches can carry, so that a forward from the
-// router's output needs fewer launches: the f16 copy of bf16 activations rides in extra workgroups of the
-// counting launch, the scan also builds the tile list (it has the expert offsets at hand) and the scatter also
-// writes every assignment's slot within its token and the per-token counts.  The per-token lists then have a
+// Work of the grouped-GEMM path's front end that the routing launch (past its limits: the three routing launches) can carry, so that a
+// forward from the router's output needs fewer launches: the f16 copy of bf16 activations rides in extra workgroups, the
+// one that has the expert offsets also builds the tile list, and those that place the entries also
+// write every assignment's slot within its token and the per-token counts.  The per-token lists then have a
 // fixed stride: token t's list starts at t * top_k (token_start), its length is token_count[t].
 struct MTile;
 struct RouteSideJobs {

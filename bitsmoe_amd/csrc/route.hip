@@ -212,7 +212,7 @@ __global__ __launch_bounds__(ROUTE_THREADS) void k_route_fused(
 // (`later`) per expert.  What bounds it: one trip for the ids (every workgroup reads them all, from L2) and the LDS atomics of the count, of
 // which a workgroup has n_flat / 1024 per thread.  Against the three launches below, which wait for each other (kernel times under the tracer, us; two gaps
 // between launches go as well): 1998 entries of 64 experts with the copy of 333 rows 5.8 + 7.0 + 4.7 -> 8.3; 32768 entries of 128 experts
-// 13.1 (with the copy of 4096 rows) + 9.4 + 5.7 -> 15.6 (without).  Whole passes: 333 tokens 123.3 -> 112.4, 512 experts at 256 tokens
+// with the copy of 4096 rows 13.1 + 9.4 + 5.7 -> 19.4 (without it 15.6).  Whole passes: 333 tokens 123.3 -> 112.4, 512 experts at 256 tokens
 // 173.7 -> 165.0.
 // With side jobs: workgroup n_chunks builds the tile list and token_start, the ones past it copy the activations.
 constexpr int WHOLE_THREADS = 1024;

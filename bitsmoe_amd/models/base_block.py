@@ -56,9 +56,10 @@ def _super_via_operator() -> bool:
 # shapes of hidden sizes 1024 to 2048 with and without shared experts: up to 32 rows it is the faster one at all of them (at 32:
 # 2048 -> 4224 features 9.0 vs 11.9, 2048 -> 9728 13.0 vs 14.4, 4864 -> 2048 10.3 vs 13.8, 4352 -> 1536 9.7 vs 12.6); from 33 to 48 at
 # all but one (at 48: 10.3 vs 12.3, 15.2 vs 15.5, 13.4 vs 13.9; but 4352 -> 1536 12.9 vs 12.6).  Every workgroup reads all
-# rows of x: from 49 rows on the many-rows kernel takes over wherever it can (at 64: 2048 -> 4224 12.4 vs 9.6, 2048 -> 2048 7.4 vs 5.5,
-# 4864 -> 2048 15.8 vs 13.8), and what that cannot take runs here up to 64 rows at GEMMs of about one workgroup per CU and a
-# contraction of at most 4096 (at 64 against the framework: 2048 -> 2048 7.4 vs 11.6, 2560 -> 2048 8.4 vs 13.6; but 2048 -> 9728 17.6 vs 15.5).
+# rows of x, so from 49 to 64 rows only GEMMs of about one workgroup per CU and a contraction of at most 4096 take it (at 64: 2048 -> 2048
+# 7.4 vs 11.6, 2560 -> 2048 8.4 vs 13.6, 2048 -> 4224 12.4 vs 12.5; 2048 -> 9728 17.6 vs 15.5).  What it does not take goes to the many-rows
+# kernel.  (That one is the faster one there too, 5.5 and 9.6 us at 64 rows, but eager blocks with dense experts beside the packed ones came
+# out slower with it, 104 -> 115 us at 64 tokens, where a graph of them gained 105 -> 102.)
 # BITSMOE_BLOCK_SKINNY_ROWS caps the rows, 0 switches the kernel off.
 _SKINNY_ROWS = int(_os.environ.get("BITSMOE_BLOCK_SKINNY_ROWS", "64"))
 _SKINNY_MOST_ROWS = 64            # that the kernel takes at all
@@ -694,13 +695,13 @@ class BitsMoE_BaseSparseMoeBlock(nn.Module):
         w_in, w_out = plan["w_in"], plan["w_out"]
         dev = x.device
         stages = 0
-        if _tiled(rows, w_in) and x.stride(0) <= mlp_forward_cuda.TILED_LINEAR_MAX_STRIDE and not _differentiated(x):
-            proj = torch.empty((rows, w_in.shape[0]), dtype=dtype, device=dev)
-            stages |= mlp_forward_cuda.BLOCK_PROJECT_IN_TILED
-        elif _few_rows(rows, hidden, w_in.shape[0]):
+        if _few_rows(rows, hidden, w_in.shape[0]):
             native = self._few_rows_weight(plan, native, "w_in")
             proj = torch.empty((rows, w_in.shape[0]), dtype=dtype, device=dev)
             stages |= mlp_forward_cuda.BLOCK_PROJECT_IN
+        elif _tiled(rows, w_in) and x.stride(0) <= mlp_forward_cuda.TILED_LINEAR_MAX_STRIDE and not _differentiated(x):
+            proj = torch.empty((rows, w_in.shape[0]), dtype=dtype, device=dev)
+            stages |= mlp_forward_cuda.BLOCK_PROJECT_IN_TILED
         else:
             proj = x @ w_in.T
         selected = weights = sup = None
@@ -714,19 +715,19 @@ class BitsMoE_BaseSparseMoeBlock(nn.Module):
         if super_modules and selected is None:
             selected = torch.empty((rows, self.top_k), dtype=torch.int64, device=dev)
             weights = torch.empty((rows, self.top_k), dtype=torch.float32, device=dev)
-        operand = None
-        if _tiled(rows, w_out):
+        operand, projected = None, True
+        if _few_rows(rows, w_out.shape[1], hidden):
+            native = self._few_rows_weight(plan, native, "w_out")
+            out = torch.empty((rows, hidden), dtype=dtype, device=dev)
+            stages |= mlp_forward_cuda.BLOCK_PROJECT_OUT
+        elif _tiled(rows, w_out):
             out = torch.empty((rows, hidden), dtype=dtype, device=dev)
             stages |= mlp_forward_cuda.BLOCK_PROJECT_OUT_TILED
             if rows > _SKINNY_MOST_ROWS:      # (up to that many the library's workspace has room)
                 operand = torch.empty((rows, w_out.shape[1]), dtype=dtype, device=dev)
-        elif _few_rows(rows, w_out.shape[1], hidden):
-            native = self._few_rows_weight(plan, native, "w_out")
-            out = torch.empty((rows, hidden), dtype=dtype, device=dev)
-            stages |= mlp_forward_cuda.BLOCK_PROJECT_OUT
         else:
             out = torch.empty((rows, w_out.shape[1]), dtype=dtype, device=dev)
-        projected = bool(stages & (mlp_forward_cuda.BLOCK_PROJECT_OUT | mlp_forward_cuda.BLOCK_PROJECT_OUT_TILED))
+            projected = False
         if self._super_expert_items and not super_modules and (operand is not None or not projected):
             sup = torch.empty((rows, hidden), dtype=torch.float32, device=dev)
         # The super experts' operator call needs the router's output and the hidden states only: it runs on a side
