@@ -736,7 +736,7 @@ TILED_LINEAR_MAX_STRIDE = 1 << 22      # elements between rows of x (a tile's ro
 
 @functools.lru_cache(maxsize=1024)
 def tiled_linear_pays(rows: int, in_features: int, out_features: int) -> bool:
-    """Is tiled_linear measured to be faster than the framework's GEMM at this size (and possible at all)?"""
+    """Is tiled_linear expected to be faster than the framework's GEMM at this size (and possible at all)?"""
     return bool(_lib.bitsmoe_tiled_linear_pays(rows, in_features, out_features))
 
 

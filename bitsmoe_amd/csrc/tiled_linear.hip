@@ -13,7 +13,7 @@
 //   2048 -> 4224       13.0 ->  9.6  15.0 -> 12.2  23.8 -> 14.8  23.3 -> 20.8  31.6 -> 29.3  80.6 -> 68.1
 //   2048 -> 2048        8.9 ->  5.5   8.8 ->  5.7  10.1 ->  7.7  11.2 ->  9.2  18.6 -> 17.1  34.1 -> 31.8
 //   2048 -> 9728       16.4 -> 14.6  18.2 -> 16.4  27.2 -> 21.1  30.2 -> 29.7  (library)    163 -> 148
-//   4864 -> 2048       16.7 -> 13.8  14.9 -> 13.8  19.3 -> 19.4  24.9 -> 24.1  (library)    73.8 -> 66.0
+//   4864 -> 2048       16.7 -> 13.8  14.9 -> 13.8  (library)     24.9 -> 24.1  (library)    73.8 -> 66.0
 #include "common.h"
 #include "lds_direct.h"
 
@@ -221,12 +221,19 @@ struct Tile {
     double one, more;
     bool shared;      // several workgroups per CU
     bool single;      // only in launches of at most one round (128 x 192 in two rounds: 2048 -> 5640 at 2048 rows 53.2 us, library 50.3)
+    // Where the tile is the faster one, next to the framework's GEMM (tiled_linear_pays below): contractions of up to `k_filled` in one round
+    // that takes at least `filled` of the CUs, of up to `k_emptier` in an emptier one, of up to `k_more` in more than one round (`shared` only).
+    double filled;
+    int k_filled, k_emptier, k_more;
 };
+constexpr int ANY_K = 1 << 22;
 constexpr Tile TILES[] = {
-    {256, 160, 1.15, 1.15, false, false}, {256, 128, 0.90, 0.90, false, false}, {192, 192, 1.06, 1.06, false, false},
-    {128, 192, 0.84, 0.84, false, true},  {128, 128, 0.62, 0.62, false, false}, {128, 96, 0.60, 0.60, false, false},
-    {128, 64, 0.52, 0.55, true, false},   {64, 96, 0.46, 0.46, false, false},   {64, 64, 0.41, 0.40, true, false},
-    {64, 32, 0.36, 0.30, true, false},    {32, 32, 0.31, 0.20, true, false},
+    {256, 160, 1.15, 1.15, false, false, 0.75, ANY_K, 0, 0},   {256, 128, 0.90, 0.90, false, false, 0.75, ANY_K, 0, 0},
+    {192, 192, 1.06, 1.06, false, false, 0.70, ANY_K, 0, 0},   {128, 192, 0.84, 0.84, false, true, 0.80, ANY_K, 2048, 0},
+    {128, 128, 0.62, 0.62, false, false, 0.80, ANY_K, 2048, 0}, {128, 96, 0.60, 0.60, false, false, 0.70, ANY_K, 0, 0},
+    {128, 64, 0.52, 0.55, true, false, 0.80, ANY_K, 1536, 1024}, {64, 96, 0.46, 0.46, false, false, 0.60, ANY_K, 0, 0},
+    {64, 64, 0.41, 0.40, true, false, 0.0, 6144, 0, 1536},     {64, 32, 0.36, 0.30, true, false, 0.0, 4096, 0, 4096},
+    {32, 32, 0.31, 0.20, true, false, 0.60, ANY_K, 5120, 5120},
 };
 constexpr int N_TILES_KNOWN = sizeof(TILES) / sizeof(TILES[0]);
 constexpr int CUS = 256;
@@ -249,17 +256,30 @@ int best_tile(int64_t rows, int out_features) {
 }
 }  // namespace
 
-// Is this kernel the faster one, next to the framework's GEMM?  Up to 512 rows at all but a few of the eight shapes measured (0.5 to 1.03 of
-// its time).  Above that where the tiles fill the CUs: the framework's GEMM splits long contractions and cuts its tiles to
-// fit.  One round three quarters full (K up to 2048; longer ones four fifths): 0.77 to 0.95 of its time; emptier 0.82 to 1.15.  Several
-// rounds: 0.84 to 0.93 when the last is nearly full, 0.96 to 1.27 when 86 or 89 % of the places are taken.
+// Is this kernel the faster one, next to the framework's GEMM?  That one may split the contraction, cuts its tiles to fit and has
+// tiles of 256 x 256; this one does neither, so it depends on the tile, on the share of the CUs' places that a launch takes and, in
+// emptier launches, on the contraction.  Time over the framework's, medians over cold weights, 5980 shapes of 49 to 8192
+// rows, 128 to 8192 and 64 to 12288 features (means of a band; of the 4946 shapes that get a yes 65 are above 1.03, the worst 1.23; of
+// the others the worst 1.68):
+//   32 x 32, less than 0.6 of the CUs:  up to 5120 in features 0.3 to 0.9, from 6144 on 1.03 to 1.16;  fuller: 0.5 to 0.96 at all
+//   64 x 32:  up to 4096 0.6 to 0.93, 5120 0.94 to 1.02, longer 0.9 to 1.09
+//   64 x 64:  one round 0.6 to 0.98 up to 6144; two: 1024 0.75, 1536 0.78, 2048 0.94 (up to 272 tiles 0.89, 288 1.01), 2560 0.99, 4096 1.01
+//   128 x 64: one round of 0.8 or more 0.6 to 1.0 at all, emptier 0.7 to 0.8 up to 1536 and 1.06 to 1.13 longer; two: 1024 0.88, 2048 0.97
+//             (0.83 to 1.37), longer 1.07 to 1.17
+//   128 x 128, 128 x 192: 0.8 or more 0.65 to 0.99, emptier 0.74 to 0.97 up to 2048 and 0.95 to 1.07 longer
+//   the others in one round 0.6 to 0.98
+// Several rounds of a tile that a CU holds one of: 0.5 to 1.02 where at least 0.93 of the last one is taken, 0.96 to 1.27 when 0.86 or 0.89
+// are; but 1.04 to 1.2 where tiles of 256 x 256 fill the CUs about as well (4096 x 7168, 3546 x 4608, 3909 x 4096).
 extern "C" int32_t bitsmoe_tiled_linear_pays(int64_t n_rows, int32_t in_features, int32_t out_features) {
     if (n_rows <= 0 || in_features < 128 || in_features > (1 << 22) || in_features % 128 != 0 || out_features < 8 || out_features % 8 != 0) return 0;
-    if (n_rows <= 512) return 1;
     const Tile& t = TILES[best_tile(n_rows, out_features)];
+    auto taken = [](int64_t tiles) { return (double)tiles / (double)((tiles + CUS - 1) / CUS * CUS); };
     const int64_t tiles = tiles_of(t, n_rows, out_features);
-    const double filled = (double)tiles / (double)((tiles + CUS - 1) / CUS * CUS);
-    return filled >= (tiles > CUS ? 0.93 : in_features <= 2048 ? 0.75 : 0.80);
+    if (tiles <= CUS) return in_features <= (taken(tiles) >= t.filled ? t.k_filled : t.k_emptier);
+    // (64 x 64 with at most a sixteenth more than one round: up to 2048)
+    if (t.shared) return in_features <= (t.rows == 64 && t.cols == 64 && tiles <= CUS + CUS / 16 ? 2048 : t.k_more);
+    const int64_t of_256 = ((n_rows + 255) / 256) * ((out_features + 255) / 256);
+    return taken(tiles) >= 0.93 && taken(of_256) < 0.85;
 }
 
 extern "C" int bitsmoe_tiled_linear(const void* x, int32_t dtype, int64_t ld_x, const void* weight, int64_t n_rows, int32_t in_features,

@@ -80,7 +80,7 @@ def _few_rows(rows: int, n_in: int, n_out: int) -> bool:
 
 
 def _tiled(rows: int, weight: torch.Tensor) -> bool:
-    """Does the library's many-rows kernel run this GEMM?  (Where it is measured to be faster than the framework's; the rows are 16-byte
+    """Does the library's many-rows kernel run this GEMM?  (Where its rule expects it to be faster than the framework's; the rows are 16-byte
     aligned, the stacked weights contiguous.)"""
     if rows <= _SKINNY_ANY_SHAPE_ROWS:
         return False

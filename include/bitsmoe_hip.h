@@ -202,7 +202,8 @@ int bitsmoe_prepare_linear_weight(const void* weight, int32_t in_features, int32
  * The same product for many rows: out [n_rows, out_features] = x [n_rows, in_features] * weight [out_features, in_features]^T, weight
  * in the framework's layout, 16-bit x / weight / out of one dtype, fp32 sums (+ addend as above, 16-byte aligned, ld_addend a multiple of 4).
  * in_features a multiple of 128, out_features of 8; ld_x and ld_out multiples of 8, all pointers 16-byte aligned.
- * bitsmoe_tiled_linear_pays: 1 where that is measured to be faster than the framework's GEMM (0: slower, or not possible).
+ * bitsmoe_tiled_linear_pays: 1 where that is expected to be faster than the framework's GEMM, by a rule on the tile it would take and the
+ * contraction that measurements of both support (0: slower, or not possible).
  */
 int bitsmoe_tiled_linear(const void* x, int32_t dtype, int64_t ld_x, const void* weight, int64_t n_rows, int32_t in_features,
                          int32_t out_features, void* out, int64_t ld_out, const float* addend, int64_t ld_addend, void* stream);

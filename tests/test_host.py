@@ -89,6 +89,25 @@ def test_block_call_refuses_a_negative_shared_size_first():
     assert (rc, lib.bitsmoe_last_error()) == (-1, b"negative size")
 
 
+# us per launch, framework's GEMM and this kernel, weights from memory
+@pytest.mark.parametrize("rows,k,n,framework,kernel", [
+    # few tiles and a contraction that only splitting shortens
+    (64, 8192, 256, 12.0, 20.1), (256, 7168, 256, 12.0, 17.9), (128, 8192, 1024, 15.8, 20.8), (256, 8192, 2048, 27.9, 32.1),
+    (130, 4864, 2048, 19.4, 20.5),
+    # an emptier round, a second round of a few tiles
+    (768, 2048, 2048, 15.7, 18.0), (225, 2048, 4608, 17.5, 19.5), (384, 3072, 5640, 30.7, 39.5), (317, 2048, 5640, 19.4, 25.3),
+    (1500, 2048, 7168, 50.4, 57.6),
+    # tiles of 256 x 256 fit as well
+    (4096, 2048, 7168, 97.4, 111.1), (3909, 2048, 4096, 53.1, 62.1),
+    (64, 2048, 4224, 14.3, 11.6), (64, 4864, 2048, 18.1, 15.2), (256, 2048, 5640, 26.0, 16.4), (256, 2560, 2048, 15.9, 13.7),
+    (1500, 2048, 4224, 33.1, 30.6), (1500, 2048, 2048, 23.0, 21.5), (4096, 2048, 4224, 79.5, 69.4), (4096, 4864, 2048, 75.3, 67.0),
+])
+def test_many_rows_kernel_where_it_is_the_faster_one(rows, k, n, framework, kernel):
+    from bitsmoe_amd.algorithms import mlp_forward_cuda as hip
+
+    assert hip.tiled_linear_pays(rows, k, n) == (kernel < framework)
+
+
 def _state_dict_for(mats_by_mtype, prefix, scheme):
     sd = {}
     for mtype, m in mats_by_mtype.items():
