@@ -46,6 +46,7 @@ EXPORTED_SYMBOLS = (
     "bitsmoe_prepare_linear_weight",
     "bitsmoe_tiled_linear",
     "bitsmoe_tiled_linear_pays",
+    "bitsmoe_tiled_linear_tile",
     "bitsmoe_forward_workspace_bytes",
     "bitsmoe_forward_workspace_bytes_sets",
     "bitsmoe_moe_forward",
@@ -160,6 +161,8 @@ def load() -> ctypes.CDLL:
                                          c_int64, c_void_p]
     lib.bitsmoe_tiled_linear_pays.restype = c_int32
     lib.bitsmoe_tiled_linear_pays.argtypes = [c_int64, c_int32, c_int32]
+    lib.bitsmoe_tiled_linear_tile.restype = c_int32
+    lib.bitsmoe_tiled_linear_tile.argtypes = [c_int64, c_int32, c_void_p, c_void_p]
     lib.bitsmoe_block_finish.restype = c_int32
     lib.bitsmoe_block_finish.argtypes = [c_void_p, c_int64, c_int32, c_void_p, c_void_p, c_int64, c_int32, c_void_p, c_int64,
                                          c_int32, c_void_p, c_int64, c_void_p]

@@ -740,6 +740,12 @@ def tiled_linear_pays(rows: int, in_features: int, out_features: int) -> bool:
     return bool(_lib.bitsmoe_tiled_linear_pays(rows, in_features, out_features))
 
 
+def tiled_linear_tile(rows: int, out_features: int) -> Optional[Tuple[int, int]]:
+    """(rows, columns) of the tile that tiled_linear takes at this size; None where it takes none."""
+    r, c = ctypes.c_int32(), ctypes.c_int32()
+    return (r.value, c.value) if _lib.bitsmoe_tiled_linear_tile(rows, out_features, ctypes.byref(r), ctypes.byref(c)) else None
+
+
 def tiled_linear_possible(x: torch.Tensor, weight: torch.Tensor) -> bool:
     """Can tiled_linear take these tensors?  (x [T, K] and a contiguous weight [N, K] of one 16-bit dtype on one GPU, x with unit
     column stride and 16-byte aligned rows, K a multiple of 128, N of 8.)"""

@@ -282,6 +282,15 @@ extern "C" int32_t bitsmoe_tiled_linear_pays(int64_t n_rows, int32_t in_features
     return taken(tiles) >= 0.93 && taken(of_256) < 0.85;
 }
 
+// The tile that the rule takes: its rows and columns (0: no size of the kernel's).
+extern "C" int32_t bitsmoe_tiled_linear_tile(int64_t n_rows, int32_t out_features, int32_t* tile_rows, int32_t* tile_cols) {
+    if (n_rows <= 0 || out_features < 8 || out_features % 8 != 0 || !tile_rows || !tile_cols) return 0;
+    const Tile& t = TILES[best_tile(n_rows, out_features)];
+    *tile_rows = t.rows;
+    *tile_cols = t.cols;
+    return 1;
+}
+
 extern "C" int bitsmoe_tiled_linear(const void* x, int32_t dtype, int64_t ld_x, const void* weight, int64_t n_rows, int32_t in_features,
                                     int32_t out_features, void* out, int64_t ld_out, const float* addend, int64_t ld_addend, void* stream) {
     BITSMOE_REQUIRE(dtype == BITSMOE_DT_F16 || dtype == BITSMOE_DT_BF16, "dtype must be f16 (0) or bf16 (1)");

@@ -204,10 +204,12 @@ int bitsmoe_prepare_linear_weight(const void* weight, int32_t in_features, int32
  * in_features a multiple of 128, out_features of 8; ld_x and ld_out multiples of 8, all pointers 16-byte aligned.
  * bitsmoe_tiled_linear_pays: 1 where that is expected to be faster than the framework's GEMM, by a rule on the tile it would take and the
  * contraction that measurements of both support (0: slower, or not possible).
+ * bitsmoe_tiled_linear_tile: the rows and columns of that tile (returns 0, and writes nothing, where the kernel does not take the size).
  */
 int bitsmoe_tiled_linear(const void* x, int32_t dtype, int64_t ld_x, const void* weight, int64_t n_rows, int32_t in_features,
                          int32_t out_features, void* out, int64_t ld_out, const float* addend, int64_t ld_addend, void* stream);
 int32_t bitsmoe_tiled_linear_pays(int64_t n_rows, int32_t in_features, int32_t out_features);
+int32_t bitsmoe_tiled_linear_tile(int64_t n_rows, int32_t out_features, int32_t* tile_rows, int32_t* tile_cols);
 
 /*
  * The block's closing elementwise pass: one row of the operand of the output GEMM in the activation dtype,

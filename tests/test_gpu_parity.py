@@ -801,13 +801,16 @@ def test_router_rounds_with_ties_and_masked_logits(cuda_device, n_experts, top_k
         assert np.allclose(w[t][:len(order)], p / p.sum(), rtol=1e-5, atol=0) and not w[t][len(order):].any()
 
 
+_TILED_SIZES = [(1, 128, 8), (70, 256, 200), (130, 1024, 4232), (100, 256, 5640), (257, 384, 2056), (100, 384, 9736),
+                (800, 128, 2056), (250, 640, 9736), (1300, 256, 2056), (500, 1024, 9736), (2040, 128, 4232),
+                (1500, 2048, 4160), (1030, 256, 9720), (1000, 128, 9720), (1490, 256, 2040), (250, 384, 2040), (250, 128, 2040)]
+
+
 @pytest.mark.parametrize("dtype_name", ["bf16", "f16"])
-@pytest.mark.parametrize("rows,k,n", [(1, 128, 8), (70, 256, 200), (130, 1024, 4232), (100, 256, 5640), (257, 384, 2056), (100, 384, 9736),
-                                      (800, 128, 2056), (250, 640, 9736), (1300, 256, 2056), (500, 1024, 9736), (2040, 128, 4232),
-                                      (1500, 2048, 4160), (1030, 256, 9720), (1000, 128, 9720)])
+@pytest.mark.parametrize("rows,k,n", _TILED_SIZES)
 def test_tiled_linear_matches_float64(cuda_device, rows, k, n, dtype_name):
-    """Every tile of the rule, with row and column remainders, rings longer than the contraction, strided x and the fp32 addend.  A sum of k
-    exact products in fp32 is off by less than k 2^-23 of the sum of magnitudes; then one rounding to 16 bits."""
+    """Every tile of the rule (test_host.py looks after that), with row and column remainders, rings longer than the contraction, strided x
+    and the fp32 addend.  A sum of k exact products in fp32 is off by less than k 2^-23 of the sum of magnitudes; then one rounding to 16 bits."""
     import torch
 
     hip = _hip()

@@ -108,6 +108,17 @@ def test_many_rows_kernel_where_it_is_the_faster_one(rows, k, n, framework, kern
     assert hip.tiled_linear_pays(rows, k, n) == (kernel < framework)
 
 
+def test_many_rows_kernel_sizes_of_the_numerics_test_reach_every_tile():
+    """Also with rows and columns that are no whole tiles (one row of tiles or columns at least ends early)."""
+    from bitsmoe_amd.algorithms import mlp_forward_cuda as hip
+    from test_gpu_parity import _TILED_SIZES
+
+    rule = {hip.tiled_linear_tile(int(48 * 1.04 ** i), n) for i in range(130) for n in range(8, 16000, 104)}
+    ragged = {hip.tiled_linear_tile(rows, n) for rows, _, n in _TILED_SIZES
+              if rows % hip.tiled_linear_tile(rows, n)[0] and n % hip.tiled_linear_tile(rows, n)[1]}
+    assert ragged == rule and len(rule) == 11
+
+
 def _state_dict_for(mats_by_mtype, prefix, scheme):
     sd = {}
     for mtype, m in mats_by_mtype.items():
