@@ -37,6 +37,7 @@ EXPORTED_SYMBOLS = (
     "bitsmoe_dequant_matrix_prepared",
     "bitsmoe_route_workspace_bytes",
     "bitsmoe_route",
+    "bitsmoe_route_is_one_launch",
     "bitsmoe_router_softmax_topk",
     "bitsmoe_router_softmax_topk_strided",
     "bitsmoe_router_linear_topk",
@@ -135,6 +136,8 @@ def load() -> ctypes.CDLL:
     lib.bitsmoe_dequant_matrix_prepared.argtypes = [c_void_p, c_int32, c_void_p, c_void_p]
     lib.bitsmoe_route_workspace_bytes.restype = c_size_t
     lib.bitsmoe_route_workspace_bytes.argtypes = [c_int64, c_int32]
+    lib.bitsmoe_route_is_one_launch.restype = c_int32
+    lib.bitsmoe_route_is_one_launch.argtypes = [c_int64, c_int32, c_int32, c_int32]
     lib.bitsmoe_route.restype = c_int32
     lib.bitsmoe_route.argtypes = [
         c_void_p, c_int32, c_void_p, c_void_p, c_int32, c_int64, c_int32, c_int32,

@@ -207,7 +207,7 @@ __global__ __launch_bounds__(ROUTE_THREADS) void k_route_fused(
     }
 }
 
-// The whole routing of up to ROUTE_WHOLE_MAX entries in ONE launch, with nothing passed between workgroups: workgroup b places the
+// The whole routing in ONE launch (where: route_whole_pays), with nothing passed between workgroups: workgroup b places the
 // entries of chunk b, and to know where they go it counts ALL entries itself -- those of earlier chunks (`before`) and the rest
 // (`later`) per expert.  What bounds it: one trip for the ids (every workgroup reads them all, from L2) and the LDS atomics of the count, of
 // which a workgroup has n_flat / 1024 per thread.  Against the three launches below, which wait for each other (kernel times under the tracer, us; two gaps
@@ -220,6 +220,25 @@ constexpr int WHOLE_WAVES = WHOLE_THREADS / 64;
 constexpr int ROUTE_WHOLE_MAX = 32768;
 constexpr int ROUTE_WHOLE_MAX_EXPERTS = 512;
 constexpr int ROUTE_WHOLE_MAX_TOP_K = 64;
+
+// Is the one launch the faster form?  Its time grows with the entries, which every workgroup counts, and where picks crowd: lanes of
+// a wavefront that count for the same expert take turns.  A token picks an expert once, so at most 64 / top_k of them do, whatever the routing:
+// the lines keep even a routing in which every token picks the same experts from being slower than the three launches, whose time
+// hardly depends on the entries and grows with the experts.  us, three launches -> one, uniform picks (all tokens the same ones), graph:
+//   tables   8 experts top-2    8192 entries 10.1 ->  7.8 (10.0 ->  9.3), 16384 10.2 ->  9.8 (10.1 -> 12.8), 32768 10.4 -> 13.6 (10.4 -> 20.1)
+//           64 experts top-1    4096 10.8 ->  6.7 (10.6 ->  9.0), 8192 11.0 ->  7.7 (10.6 -> 12.7), 32768 11.8 -> 12.2 (11.5 -> 33.8)
+//           64 experts top-8   24576 11.6 -> 10.7 (11.2 -> 10.7), 32768 11.9 -> 12.2 (11.6 -> 12.2)
+//          128 experts top-8   32768 13.0 -> 12.6 (12.5 -> 12.3)
+//          512 experts top-2   16384 15.6 -> 10.2 (15.1 -> 13.4), 32768 18.4 -> 13.2 (17.9 -> 20.7)
+//   with the grouped GEMM's front end beside it (operator, small matrices):
+//            8 experts top-1    8192 71.4 -> 66.0 (71.5 -> 71.5), 16384 96.3 -> 93.0 (98.0 -> 103.8); top-2 16384 82.4 -> 78.3 (81.0 -> 80.8)
+//           64 experts top-6   32766 107.3 -> 104.1 (108.1 -> 105.9)
+static bool route_whole_pays(int64_t n_flat, int top_k, int n_packed, bool front_end) {
+    if (n_flat > ROUTE_WHOLE_MAX || n_packed > ROUTE_WHOLE_MAX_EXPERTS || top_k > ROUTE_WHOLE_MAX_TOP_K || top_k < 1) return false;
+    const int64_t crowded = n_flat * ((64 + top_k - 1) / top_k);      // entries times the most turns a wavefront may take for one
+    if (front_end) return crowded <= 1 << 19;
+    return n_flat <= 16384 + 128 * n_packed && crowded <= (1 << 18) + 512 * n_packed;
+}
 
 template <typename IdT>
 __global__ __launch_bounds__(WHOLE_THREADS) void k_route_whole(
@@ -478,7 +497,7 @@ static int route_impl(const IdT* selected, const float* weights, const int32_t* 
                                                    ? ((size_t)ROUTE_ROUNDS * (ROUTE_THREADS / 64) * n_packed +
                                                       (n_global <= ROUTE_G2L_LDS_MAX ? n_global : 0)) * sizeof(int)
                                                    : 0);
-    const bool whole = n_flat <= ROUTE_WHOLE_MAX && n_packed <= ROUTE_WHOLE_MAX_EXPERTS && top_k <= ROUTE_WHOLE_MAX_TOP_K;
+    const bool whole = route_whole_pays(n_flat, top_k, n_packed, jobs != nullptr);
     // (tables alone, 72 entries of 64 experts: 4.6 us by the one workgroup of 256 threads, 5.3 by the other kernel's 1024; but with the grouped
     // GEMM's front end that one saves three launches: operator, us, 32 experts top-4 128 tokens 74.8 -> 66.8, 64 top-6 160 tokens 108.3 -> 98.9,
     // 48 top-8 100 tokens 72.7 -> 63.0, 32 top-8 60 tokens 80.9 -> 73.3)
@@ -544,6 +563,12 @@ extern "C" size_t bitsmoe_route_workspace_bytes(int64_t n_flat, int32_t n_packed
     if (n_flat <= ROUTE_CHUNK || n_packed <= 0) return 256;
     const int64_t n_chunks = (n_flat + ROUTE_CHUNK - 1) / ROUTE_CHUNK;
     return (size_t)(((n_flat + 63) / 64) * 64 + n_chunks * (int64_t)n_packed) * sizeof(int32_t) + 256;
+}
+
+extern "C" int32_t bitsmoe_route_is_one_launch(int64_t n_tokens, int32_t top_k, int32_t n_packed, int32_t front_end) {
+    if (n_tokens <= 0 || top_k <= 0 || n_packed <= 0) return 0;
+    const int64_t n_flat = n_tokens * top_k;
+    return (n_flat <= ROUTE_CHUNK && !front_end) || route_whole_pays(n_flat, top_k, n_packed, front_end != 0);
 }
 
 extern "C" int bitsmoe_route(const void* selected, int32_t ids_are_i64, const float* weights,

@@ -136,6 +136,8 @@ int bitsmoe_route(const void* selected, int32_t ids_are_i64, const float* weight
                   int32_t top_k, int32_t n_packed, int32_t* token_indices,
                   int32_t* expert_offsets, float* route_flat, void* workspace,
                   size_t workspace_bytes, void* stream);
+/* 1 where that is one launch, 0 where it is three (front_end: as bitsmoe_moe_forward_routed calls it at grouped-GEMM sizes). */
+int32_t bitsmoe_route_is_one_launch(int64_t n_tokens, int32_t top_k, int32_t n_packed, int32_t front_end);
 
 /*
  * Router front end in one kernel.  Replaces the framework-op chain of the reference's Qwen

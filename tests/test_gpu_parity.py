@@ -45,7 +45,9 @@ def test_dequant_bit_exact_all_bitwidths(cuda_device, rank, dim):
     (1, 8, 128, 0), (64, 8, 128, 0), (7, 6, 64, 2), (256, 10, 512, 0), (4096, 8, 128, 1), (333, 3, 9, 0), (128, 8, 128, 0),
     # one launch (1025 to 32768 entries) with a last chunk of one entry, top_k that straddles chunks, the most experts and choices it takes;
     # three launches past each of its limits
-    (205, 5, 7, 0), (4096, 8, 512, 3), (1024, 64, 66, 1), (350, 6, 513, 0), (20, 65, 70, 2), (4097, 8, 130, 2), (50000, 1, 64, 1)])
+    (205, 5, 7, 0), (4096, 8, 512, 3), (1024, 64, 66, 1), (350, 6, 513, 0), (20, 65, 70, 2), (4097, 8, 130, 2), (50000, 1, 64, 1),
+    # both sides of where crowded picks and many entries of few experts end it
+    (4608, 1, 64, 0), (4609, 1, 64, 0), (2304, 8, 16, 0), (2305, 8, 16, 0)])
 @pytest.mark.parametrize("i64", [True, False])
 def test_routing_tables_bit_exact(cuda_device, tokens, top_k, n_global, n_super, i64):
     import torch

@@ -87,6 +87,16 @@ def test_forward_from_router_output(cuda_device, n_global, n_super, tokens, top_
     assert inline == expect_inline
 
 
+@pytest.mark.parametrize("tokens,dtype_name", [(8192, "bf16"), (8193, "bf16"), (8193, "f16")])
+def test_forward_from_router_output_most_single_picks(cuda_device, tokens, dtype_name):
+    """The most entries of one pick per token whose routing is one launch with the grouped GEMM's front end in it, and one more."""
+    from bitsmoe_amd.algorithms import _capi
+
+    assert bool(_capi.load().bitsmoe_route_is_one_launch(tokens, 1, 8, 1)) == (tokens == 8192)
+    _, inline = _case(cuda_device, 95, 8, 0, tokens, 1, 128, 128, True, dtype_name)
+    assert not inline
+
+
 @pytest.mark.parametrize("dtype_name,choices", [("bf16", (2,)), ("f16", (2, 2, 2, 3, 4))])
 def test_forward_from_router_output_more_items_than_workgroup_slots(cuda_device, dtype_name, choices):
     """More (expert, tile, projection) items than the chip holds workgroups at once (128 experts x 5 tiles x 2);

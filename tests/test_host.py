@@ -89,6 +89,22 @@ def test_block_call_refuses_a_negative_shared_size_first():
     assert (rc, lib.bitsmoe_last_error()) == (-1, b"negative size")
 
 
+# us, three launches and one: where every token picks the same experts the one launch's count takes turns (the slower of this and
+# uniform picks is stated)
+@pytest.mark.parametrize("entries,top_k,experts,front_end,three,one", [
+    (32768, 1, 8, 0, 10.1, 33.5), (8192, 1, 64, 0, 10.6, 12.7), (16384, 2, 16, 0, 10.3, 12.8), (32768, 4, 64, 0, 11.6, 14.0),
+    (32768, 8, 32, 0, 10.8, 12.2), (16384, 2, 256, 0, 12.7, 13.2), (32768, 2, 512, 0, 17.9, 20.7),
+    (16384, 1, 8, 1, 98.0, 103.8), (24576, 2, 64, 1, 103.0, 105.8),
+    (4096, 1, 8, 0, 10.0, 8.8), (8192, 2, 16, 0, 10.2, 9.3), (16384, 4, 32, 0, 10.6, 9.9), (20480, 8, 32, 0, 10.8, 9.9),
+    (32768, 8, 128, 0, 12.5, 12.3), (16384, 2, 512, 0, 15.1, 13.4), (32768, 4, 512, 0, 17.9, 14.7),
+    (4096, 1, 64, 1, 56.5, 52.0), (16384, 2, 8, 1, 81.0, 80.8), (32768, 4, 128, 1, 108.0, 106.7),
+])
+def test_routing_in_one_launch_where_that_is_faster(entries, top_k, experts, front_end, three, one):
+    from bitsmoe_amd.algorithms import _capi
+
+    assert bool(_capi.load().bitsmoe_route_is_one_launch(entries // top_k, top_k, experts, front_end)) == (one < three)
+
+
 # us per launch, framework's GEMM and this kernel, weights from memory
 @pytest.mark.parametrize("rows,k,n,framework,kernel", [
     # few tiles and a contraction that only splitting shortens
