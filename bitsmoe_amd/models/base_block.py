@@ -56,16 +56,16 @@ def _super_via_operator() -> bool:
 # shapes of hidden sizes 1024 to 2048 with and without shared experts: up to 32 rows it is the faster one at all of them (at 32:
 # 2048 -> 4224 features 9.0 vs 11.9, 2048 -> 9728 13.0 vs 14.4, 4864 -> 2048 10.3 vs 13.8, 4352 -> 1536 9.7 vs 12.6); from 33 to 48 at
 # all but one (at 48: 10.3 vs 12.3, 15.2 vs 15.5, 13.4 vs 13.9; but 4352 -> 1536 12.9 vs 12.6).  Every workgroup reads all
-# rows of x, so from 49 to 64 rows only GEMMs of about one workgroup per CU and a contraction of at most 4096 take it (at 64: 2048 -> 2048
-# 7.4 vs 11.6, 2560 -> 2048 8.4 vs 13.6, 2048 -> 4224 12.4 vs 12.5; 2048 -> 9728 17.6 vs 15.5).  What it does not take goes to the many-rows
-# kernel.  (That one is the faster one there too, 5.5 and 9.6 us at 64 rows, but eager blocks with dense experts beside the packed ones came
-# out slower with it, 104 -> 115 us at 64 tokens, where a graph of them gained 105 -> 102.)
-# BITSMOE_BLOCK_SKINNY_ROWS caps the rows, 0 switches the kernel off.
-_SKINNY_ROWS = int(_os.environ.get("BITSMOE_BLOCK_SKINNY_ROWS", "64"))
+# rows of x, so past 48 rows the many-rows kernel takes over: at 49 to 64 rows of 346 shapes up to 4096 -> 4352 it needs 0.78 to
+# 0.89 of the few-rows kernel's time on average and 1.09 at most (weights from memory, at 64: 2048 -> 2048 8.5 vs 8.8, 2048 -> 4224 11.6 vs
+# 14.1, 2560 -> 1536 10.6 vs 9.8), at larger ones far less.  Blocks of 128 experts,
+# six runs of each in turn, few rows -> many rows: graph, 52 tokens 79.4 -> 76.4, 64 tokens 81.2 -> 78.9, with two dense experts 103.5 ->
+# 100.4; eager 77.7..79.0 -> 74.7..76.1, 79.4..81.2 -> 77.2..78.6, with the dense experts, whose two streams overlap now more, now less,
+# 110.8..126.7 -> 97.1..124.1.
+# BITSMOE_BLOCK_SKINNY_ROWS sets the rows (at most 64, what the kernel takes), 0 switches the kernel off.
+_SKINNY_ROWS = int(_os.environ.get("BITSMOE_BLOCK_SKINNY_ROWS", "48"))
 _SKINNY_MOST_ROWS = 64            # that the kernel takes at all
-_SKINNY_ANY_SHAPE_ROWS = 48
-_SKINNY_NARROW_FEATURES = 4352    # output features, and
-_SKINNY_SHORT_CONTRACTION = 4096  # input features up to which 49 to 64 rows take it
+_MANY_ROWS = 49                   # from which the many-rows kernel is measured
 # BITSMOE_BLOCK_SKINNY_PREPARED=0: the few-rows kernel reads the stacked weights in the framework's layout (no extra copy)
 _SKINNY_PREPARED = _os.environ.get("BITSMOE_BLOCK_SKINNY_PREPARED", "1") != "0"
 
@@ -75,14 +75,13 @@ _FEW_ROWS_LOCK = _threading.Lock()      # (held while a layer's copy is made or 
 
 def _few_rows(rows: int, n_in: int, n_out: int) -> bool:
     """Does the few-rows kernel run this GEMM?  (It takes contractions of whole 128 and an even number of outputs.)"""
-    return (0 < rows <= min(_SKINNY_ROWS, _SKINNY_MOST_ROWS) and n_in % 128 == 0 and n_out % 2 == 0 and (
-        rows <= _SKINNY_ANY_SHAPE_ROWS or (n_in <= _SKINNY_SHORT_CONTRACTION and n_out <= _SKINNY_NARROW_FEATURES)))
+    return 0 < rows <= min(_SKINNY_ROWS, _SKINNY_MOST_ROWS) and n_in % 128 == 0 and n_out % 2 == 0
 
 
 def _tiled(rows: int, weight: torch.Tensor) -> bool:
     """Does the library's many-rows kernel run this GEMM?  (Where its rule expects it to be faster than the framework's; the rows are 16-byte
     aligned, the stacked weights contiguous.)"""
-    if rows <= _SKINNY_ANY_SHAPE_ROWS:
+    if rows < _MANY_ROWS:
         return False
     n_out, n_in = weight.shape
     return mlp_forward_cuda.tiled_linear_pays(rows, n_in, n_out)

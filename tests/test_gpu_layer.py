@@ -752,28 +752,47 @@ def test_block_workspace_holds_no_projection_past_the_few_rows_kernel(cuda_devic
     assert bool((out == 3.0).all())
 
 
-# the few-rows kernel's last size, the many-rows kernel with what the workspace holds and with the caller's memory, a grouped-GEMM size
+def _stages_of(monkeypatch):
+    """The stage bits of the block calls from here on, in order."""
+    from bitsmoe_amd.algorithms import mlp_forward_cuda as hip
+
+    seen, real = [], hip.block_forward
+
+    def spy(native, x, proj, stages, *rest):
+        seen.append(stages)
+        return real(native, x, proj, stages, *rest)
+
+    monkeypatch.setattr(hip, "block_forward", spy)
+    return seen
+
+
+# the few-rows kernel's last size, the many-rows kernel with what the workspace holds and with the caller's memory, a grouped-GEMM size;
+# stacked GEMMs of a narrow layer and of 1024 -> 7744 and 3840 -> 1024 features
 @pytest.mark.parametrize("tokens", [48, 49, 64, 65, 200])
-@pytest.mark.parametrize("family,shared,super_experts", [("qwen3moe", 0, ()), ("qwen3moe", 0, (1, 6)), ("qwen3next", 128, ()),
-                                                         ("deepseekv2", 256, ())])
-def test_block_projections_by_the_many_rows_kernel(cuda_device, monkeypatch, family, shared, super_experts, tokens):
+@pytest.mark.parametrize("family,hidden,shared,super_experts", [
+    ("qwen3moe", 128, 0, ()), ("qwen3moe", 128, 0, (1, 6)), ("qwen3next", 128, 128, ()), ("deepseekv2", 128, 256, ()),
+    ("deepseekv2", 1024, 2816, ()), ("deepseekv2", 1024, 2816, (1, 6))])
+def test_block_projections_by_the_many_rows_kernel(cuda_device, monkeypatch, family, hidden, shared, super_experts, tokens):
     """Equal to the block between the framework's GEMMs up to the roundings that the sums' order may move: projected activations, the
     output projection's operand and the output are bf16 (2^-8 each), three of them in a row on independent elements."""
     import torch
 
+    from bitsmoe_amd.algorithms import mlp_forward_cuda as hip
     from bitsmoe_amd.models import base_block
     from bitsmoe_amd.synth import make_layer
 
-    spec = _small_spec(family, shared_intermediate=shared)
+    spec = _small_spec(family, hidden_size=hidden, shared_intermediate=shared)
     block = make_layer(spec, device=cuda_device, dtype=torch.bfloat16, seed=71, super_experts=super_experts).eval()
     block.prepare_runtime_fastpath(warmup=True)
     x = torch.randn((1, tokens, spec.hidden_size), generator=torch.Generator().manual_seed(tokens)).to(torch.bfloat16).to(cuda_device)
     as_tensor = lambda y: (y[0] if isinstance(y, tuple) else y).float()
+    stages = _stages_of(monkeypatch)
     with torch.no_grad():
         out = as_tensor(block(x))
         monkeypatch.setattr(base_block, "_tiled", lambda rows, weight: False)
         monkeypatch.setattr(base_block, "_SKINNY_ROWS", 0)
         ref = as_tensor(block(x))
+    assert stages == [hip.BLOCK_PROJECT_IN | hip.BLOCK_PROJECT_OUT if tokens <= 48 else hip.BLOCK_PROJECT_IN_TILED | hip.BLOCK_PROJECT_OUT_TILED, 0]
     assert float((out - ref).norm() / ref.norm()) <= 3 * 2.0 ** -8
     wanted = x.clone().requires_grad_(True)
     monkeypatch.undo()
