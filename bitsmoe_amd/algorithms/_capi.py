@@ -59,6 +59,7 @@ EXPORTED_SYMBOLS = (
     "bitsmoe_forward_routed_is_inline",
     "bitsmoe_forward_decode_is_fused",
     "bitsmoe_block_workspace_bytes",
+    "bitsmoe_block_router_is_beside",
     "bitsmoe_block_forward",
     "bitsmoe_block_forward_tiled",
     "bitsmoe_profile_create",
@@ -208,6 +209,8 @@ def load() -> ctypes.CDLL:
     ]
     lib.bitsmoe_block_workspace_bytes.restype = c_size_t
     lib.bitsmoe_block_workspace_bytes.argtypes = [c_void_p, c_int64]
+    lib.bitsmoe_block_router_is_beside.restype = c_int32
+    lib.bitsmoe_block_router_is_beside.argtypes = [c_void_p, c_int64, c_int32]
     lib.bitsmoe_block_forward_tiled.restype = c_int32
     lib.bitsmoe_block_forward_tiled.argtypes = [c_void_p, c_void_p, c_int64, c_int64, c_void_p, c_int32, c_void_p, c_void_p, c_void_p,
                                                 c_void_p, c_void_p, c_void_p, c_size_t, c_void_p, c_void_p]

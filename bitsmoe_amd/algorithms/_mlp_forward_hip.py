@@ -867,6 +867,11 @@ class BlockPlan:
         return n
 
 
+def block_router_is_beside(plan: BlockPlan, n_tokens: int, stages: int) -> bool:
+    """Would a block call run its gate's linear layer and top-k in the input projection's launch?"""
+    return bool(_lib.bitsmoe_block_router_is_beside(plan.address, n_tokens, stages))
+
+
 def block_forward(plan: BlockPlan, x: torch.Tensor, proj: torch.Tensor, stages: int, out: torch.Tensor,
                   selected: Optional[torch.Tensor] = None, weights: Optional[torch.Tensor] = None,
                   super_out: Optional[torch.Tensor] = None, side_stream: int = 0, operand: Optional[torch.Tensor] = None) -> None:

@@ -53,6 +53,11 @@ static int stream_after(hipStream_t later, hipStream_t earlier) {
     return BITSMOE_OK;
 }
 
+extern "C" int32_t bitsmoe_block_router_is_beside(const bitsmoe_block_plan* p, int64_t n_tokens, int32_t stages) {
+    return p && (stages & BITSMOE_BLOCK_PROJECT_IN) != 0 && p->router_form == BITSMOE_ROUTER_LINEAR &&
+           skinny_linear_takes_router(n_tokens, p->hidden, p->w_in_prepared, p->n_global, p->top_k);
+}
+
 extern "C" int bitsmoe_block_forward(const bitsmoe_block_plan* p, const void* x, int64_t ld_x, int64_t n_tokens, void* proj,
                                      int32_t stages, void* selected, float* weights, void* out, float* super_out, void* workspace,
                                      size_t workspace_bytes, void* side_stream, void* stream) {
@@ -99,12 +104,10 @@ extern "C" int bitsmoe_block_forward_tiled(const bitsmoe_block_plan* p, const vo
         BITSMOE_TRY(bitsmoe_tiled_linear(x, p->act_dtype, ld_x, p->w_in_rows, n_tokens, p->hidden, p->in_features, proj, ld, nullptr, 0, stream));
     if (!selected) selected = ws + w.selected;
     if (!weights) weights = (float*)(ws + w.weights);
-    bool routed = false;
-    if (few_in && p->router_form == BITSMOE_ROUTER_LINEAR &&
-        skinny_linear_takes_router(n_tokens, p->hidden, p->w_in_prepared, p->n_global, p->top_k)) {
+    const bool routed = bitsmoe_block_router_is_beside(p, n_tokens, stages) != 0;
+    if (routed) {
         const RouterBeside router = {p->w_router, p->n_global, p->top_k, p->renormalize, p->round_dtype, p->weight_scale, (int64_t*)selected, weights};
         BITSMOE_TRY(skinny_linear_with_router(x, p->act_dtype, ld_x, p->w_in, n_tokens, p->hidden, p->in_features, proj, ld, router, stream));
-        routed = true;
     } else if (few_in) {
         BITSMOE_TRY(bitsmoe_skinny_linear(x, p->act_dtype, 0, ld_x, p->w_in, p->w_in_prepared, n_tokens, p->hidden, p->in_features,
                                           proj, ld, nullptr, 0, stream));

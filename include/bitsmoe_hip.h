@@ -366,6 +366,8 @@ typedef struct {
     const void *w_in_rows, *w_out_rows;
 } bitsmoe_block_plan;
 size_t bitsmoe_block_workspace_bytes(const bitsmoe_block_plan* plan, int64_t n_tokens);
+/* 1 where a linear-layer router runs in the launch of the few-rows input projection, not behind it. */
+int32_t bitsmoe_block_router_is_beside(const bitsmoe_block_plan* plan, int64_t n_tokens, int32_t stages);
 int bitsmoe_block_forward(const bitsmoe_block_plan* plan, const void* x, int64_t ld_x, int64_t n_tokens, void* proj,
                           int32_t stages, void* selected, float* weights, void* out, float* super_out, void* workspace,
                           size_t workspace_bytes, void* side_stream, void* stream);

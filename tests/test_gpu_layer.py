@@ -801,23 +801,38 @@ def test_block_projections_by_the_many_rows_kernel(cuda_device, monkeypatch, fam
         assert logits.requires_grad
 
 
+@pytest.fixture(scope="module")
+def gate_layers():
+    """Layers with a gate of their own, made once per shape."""
+    from bitsmoe_amd.synth import make_layer
+
+    made = {}
+
+    def layer(device, dtype, hidden, experts):
+        if (dtype, hidden, experts) not in made:
+            spec = _small_spec("deepseekv2", num_experts=experts, top_k=6, hidden_size=hidden, intermediate_size=128)
+            made[dtype, hidden, experts] = make_layer(spec, device=device, dtype=dtype, seed=81, basis_seed=7).eval()
+            made[dtype, hidden, experts].prepare_runtime_fastpath(warmup=True)
+        return made[dtype, hidden, experts]
+
+    yield layer
+    made.clear()
+
+
 # one to four tokens per router workgroup, all forms of the few-rows kernel (operands straight from memory, one to three blocks of rows) and
 # the first size past it; all hidden sizes the joint launch takes and one it does not; whole and partial 16-expert blocks
 @pytest.mark.parametrize("tokens", [1, 4, 5, 16, 17, 33, 48, 49])
 @pytest.mark.parametrize("hidden,experts", [(1024, 64), (1536, 8), (2048, 40), (2560, 64), (640, 64), (1024, 72), (2048, 128), (1024, 136)])
 @pytest.mark.parametrize("dtype_name", ["bfloat16", "float16"])
-def test_router_beside_the_input_projection(cuda_device, monkeypatch, dtype_name, hidden, experts, tokens):
+def test_router_beside_the_input_projection(cuda_device, gate_layers, monkeypatch, dtype_name, hidden, experts, tokens):
     """The block's picks are the router kernel's on its own (logits in another order of fp32 sums: a pick may only change where two logits are
     closer than that), its projected rows the projection's on its own, bit for bit."""
     import torch
 
     from bitsmoe_amd.algorithms import mlp_forward_cuda as hip
-    from bitsmoe_amd.synth import make_layer
 
     dtype = getattr(torch, dtype_name)
-    spec = _small_spec("deepseekv2", num_experts=experts, top_k=6, hidden_size=hidden, intermediate_size=128)
-    block = make_layer(spec, device=cuda_device, dtype=dtype, seed=81, basis_seed=7).eval()
-    block.prepare_runtime_fastpath(warmup=True)
+    block = gate_layers(cuda_device, dtype, hidden, experts)
     x = torch.randn((1, tokens, hidden), generator=torch.Generator().manual_seed(tokens + experts)).to(dtype).to(cuda_device)
     real, seen = hip.block_forward, {}
 
@@ -830,6 +845,8 @@ def test_router_beside_the_input_projection(cuda_device, monkeypatch, dtype_name
     monkeypatch.setattr(hip, "block_forward", spy)
     with torch.no_grad():
         block(x)
+    beside = hip.block_router_is_beside(seen["native"], tokens, seen["stages"])
+    assert beside == (tokens <= 48 and hidden != 640 and experts <= 128)
     c, kept = seen["native"].c, seen["native"]._weights
     sel, wt = hip.router_linear_topk(seen["x"], kept["w_router"], 6, bool(c.renormalize), weight_scale=float(c.weight_scale),
                                      round_dtype={-1: None, 0: torch.float16, 1: torch.bfloat16}[c.round_dtype])
