@@ -10,6 +10,8 @@
 #include <cstdint>
 #include <cstdio>
 #include <string>
+#include <type_traits>
+#include <utility>
 #include <vector>
 
 #include "../../include/bitsmoe_hip.h"
@@ -21,6 +23,13 @@ constexpr int K_STAGE = 16;   // rows per stage inside a slab
 constexpr int N_TILE = 128;   // columns per tile
 constexpr int N_MICRO = 32;   // columns per plane word
 constexpr int MICROS = N_TILE / N_MICRO;
+
+// Calls f(integral_constant<int, 0>) ... f(integral_constant<int, N-1>): an unrolled loop whose
+// index is a compile-time constant (register-array indices must be static).
+template <class F, int... Q>
+__device__ __forceinline__ void static_for(F&& f, std::integer_sequence<int, Q...>) {
+    (f(std::integral_constant<int, Q>{}), ...);
+}
 
 // One packed expert matrix as the kernels see it.
 struct MatView {

@@ -18,13 +18,6 @@ __device__ inline float gload_half(gptr<__half> p) {
     return __half2float(__ushort_as_half(bits));
 }
 
-// Calls f(integral_constant<int, 0>) ... f(integral_constant<int, N-1>): an unrolled loop whose
-// index is a compile-time constant (register-array indices must be static).
-template <class F, int... Q>
-__device__ inline void static_for(F&& f, std::integer_sequence<int, Q...>) {
-    (f(std::integral_constant<int, Q>{}), ...);
-}
-
 // The index is wave-uniform at every call site; readfirstlane tells the compiler so (scalar
 // registers, scalar branches, scalar-base addressing downstream).
 __device__ inline FastSlab load_fast_slab(const FastSlab* __restrict__ tab, int idx) {

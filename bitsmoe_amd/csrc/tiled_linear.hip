@@ -24,11 +24,6 @@
 
 namespace bitsmoe {
 
-template <class F, int... P>
-__device__ __forceinline__ void static_for(F&& f, std::integer_sequence<int, P...>) {
-    (f(std::integral_constant<int, P>{}), ...);
-}
-
 typedef float tl_f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t tl_u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t tl_u32x2 __attribute__((ext_vector_type(2)));
