@@ -156,7 +156,7 @@ def run_workload(blocks, spec, tokens, steps, warmup, seed=42, use_graph=True, l
         side = None
         if st.has_super:
             # the dense experts' matrix sets: a second call of the operator (output in hidden space), on a side stream
-            # beside the packed experts' call, as the block runs it
+            # beside the packed experts' call, as the block runs it where there is enough to run (at small sizes on one stream)
             from bitsmoe_amd.models.base_block import _side_stream
 
             cur = torch.cuda.current_stream(dev)

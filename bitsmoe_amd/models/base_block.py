@@ -32,7 +32,7 @@ import os as _os
 import threading as _threading
 
 _CHECK_VERSIONS = _os.environ.get("BITSMOE_BLOCK_CHECK_VERSIONS", "0") == "1"
-# BITSMOE_SUPER_SIDE_STREAM=0: the super experts' operator call on the caller's stream, after the packed experts'
+# BITSMOE_SUPER_SIDE_STREAM=0: the super experts' operator call on the caller's stream, after the packed experts', at all sizes
 _SUPER_SIDE_STREAM = _os.environ.get("BITSMOE_SUPER_SIDE_STREAM", "1") != "0"
 
 
@@ -93,6 +93,26 @@ def _differentiated(x: torch.Tensor) -> bool:
 
 
 _SIDE_STREAMS: Dict[int, "torch.cuda.Stream"] = {}
+
+
+# A second stream costs an eager block two waits between hardware queues, which the kernels of a small call do not cover: its host then
+# takes 90 to 140 us, differently from run to run.  Products of a matrix (routed entries x hidden x intermediate size) from which it is the faster
+# form, eager and captured (a graph has no host to wait for); us per block with two dense experts, one stream -> two:
+#   128 experts top-8, 2048 x 768    eager 1 token 54 -> 87..113, 64 101 -> 116..121, 128 119 -> 122..128, 256 200 -> 170, 4096 727 -> 652
+#                                    graph 1 token 39 -> 47, 32 94 -> 93, 128 121 -> 114, 256 202 -> 165
+#   64 experts top-4, 1024 x 512     eager 64 68 -> 125, 512 115 -> 132, 1024 169 -> 157;   graph 64 60 -> 63, 256 80 -> 81, 512 115 -> 99
+#   64 experts top-6, 2048 x 1408    eager 64 130 -> 140, 128 151 -> 147, 256 283 -> 248;   graph 4 66 -> 70, 16 94 -> 91, 64 130 -> 122
+#   32 experts top-2, 2048 x 1408    eager 128 97 -> 140, 256 143 -> 141..153, 512 232 -> 184;   graph 4 48 -> 57, 16 75 -> 74, 64 90 -> 88
+_BESIDE_PRODUCTS = 1 << 31
+_BESIDE_PRODUCTS_CAPTURED = 1 << 28
+
+
+def _beside(products: int, device: torch.device) -> bool:
+    """Do the super experts run on a stream of their own?"""
+    if not _BESIDE_PRODUCTS_CAPTURED <= products < _BESIDE_PRODUCTS:
+        return products >= _BESIDE_PRODUCTS
+    with torch.cuda.device(device):
+        return torch.cuda.is_current_stream_capturing()
 
 
 def _side_stream(device: torch.device) -> "torch.cuda.Stream":
@@ -731,7 +751,11 @@ class BitsMoE_BaseSparseMoeBlock(nn.Module):
             sup = torch.empty((rows, hidden), dtype=torch.float32, device=dev)
         # The super experts' operator call needs the router's output and the hidden states only: it runs on a side
         # stream beside the packed experts' call (its small launches fill what the packed kernels leave idle).
-        side = _side_stream(dev).cuda_stream if self._super_expert_items and _SUPER_SIDE_STREAM and not super_modules else 0
+        # (where there is enough to run beside: _beside)
+        side = 0
+        if self._super_expert_items and _SUPER_SIDE_STREAM and not super_modules and _beside(
+                rows * self.top_k * hidden * int(self._packed_intermediate_size), dev):
+            side = _side_stream(dev).cuda_stream
         mlp_forward_cuda.block_forward(native, x, proj, stages, out, selected, weights, sup, side, operand)
         if not projected:
             out = out @ w_out.T

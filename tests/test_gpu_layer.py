@@ -801,6 +801,43 @@ def test_block_projections_by_the_many_rows_kernel(cuda_device, monkeypatch, fam
         assert logits.requires_grad
 
 
+def test_super_experts_beside_the_packed_ones_where_there_is_enough_to_run(cuda_device, monkeypatch):
+    """Eager from 2^31 products on, captured from 2^28 on, before that on the caller's stream: the same block either way, up to the order of
+    fp32 sums in front of the output's rounding (bf16: 2^-8)."""
+    import torch
+
+    from bitsmoe_amd.algorithms import mlp_forward_cuda as hip
+    from bitsmoe_amd.models import base_block
+    from bitsmoe_amd.synth import make_layer
+
+    sides, real = [], hip.block_forward
+    monkeypatch.setattr(hip, "block_forward", lambda *a: (sides.append(a[8] != 0), real(*a))[1])
+    block = make_layer(_small_spec("qwen3moe"), device=cuda_device, dtype=torch.bfloat16, seed=91, super_experts=(1, 6)).eval()
+    block.prepare_runtime_fastpath(warmup=True)
+    x = torch.randn((1, 70, 128), generator=torch.Generator().manual_seed(3)).to(torch.bfloat16).to(cuda_device)
+    per_token = 2 * 128 * 256
+    with torch.no_grad():
+        ref = block(x)[0].float()
+        close = lambda y: float((y.float() - ref).abs().max()) <= 2.0 ** -7 * float(ref.abs().max())
+        for most in (70 * per_token, 70 * per_token + 1):
+            monkeypatch.setattr(base_block, "_BESIDE_PRODUCTS", most)
+            assert close(block(x)[0])
+        assert sides == [False, True, False]
+        monkeypatch.setattr(base_block, "_BESIDE_PRODUCTS_CAPTURED", 70 * per_token)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            y = block(x)[0]
+        assert sides == [False, True, False, True]
+        for _ in range(3):
+            y.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert close(y) and close(block(x)[0])
+    monkeypatch.undo()
+    on_card = torch.device(cuda_device)
+    assert [base_block._beside(n, on_card) for n in ((1 << 28), (1 << 31) - 1, 1 << 31)] == [False, False, True]
+
+
 @pytest.fixture(scope="module")
 def gate_layers():
     """Layers with a gate of their own, made once per shape."""
