@@ -209,7 +209,7 @@ __global__ __launch_bounds__(64 * NW) void k_skinny_linear(const void* __restric
 // the hidden states only.  What bounds the router is what one CU can fetch (256 KB of gate weight at 64 experts and a hidden size of 2048), so
 // on its own it takes about as long as the projection, on a card that is idle but for one workgroup per sixteen tokens; here
 // it is over before the projection is.  us, projection + router -> joint, 64 experts: 12 rows 11.1 + 10.2 -> 12.8; blocks in a graph at 1, 12 and
-// 40 tokens 36.6 -> 32.8, 72.8 -> 63.7, 91.7 -> 79.9; 128 experts at 12 and 40 tokens 70.9 -> 60.9, 105.4 -> 88.7.  Blocks of 8 to 128
+// 40 tokens 36.6 -> 32.1, 72.8 -> 63.7, 91.7 -> 79.9; 128 experts at 12 and 40 tokens 70.9 -> 61.4, 105.4 -> 88.5.  Blocks of 8 to 128
 // experts, hidden sizes 1024 to 2560, 1 to 48 tokens: 0.85 of the time on average, none of 385 slower.  Contractions that are no
 // four whole shares (3072, 4096, 5120) and more than 128 experts have no joint form built: they run the two launches.
 template <bool BF16, int NMB, int MAXS, bool TURN, int NB>      // NB: 16-expert blocks

@@ -146,8 +146,8 @@ __device__ inline uint32_t vreg(uint32_t c) {
 
 // role 1, 2-bit: the four registers (8 values = one MFMA k-step) of k-step ks from a lane's word: the codes themselves, 0 to 3.
 // The nibbles are E2M1 numbers of half that value, doubled by the conversion's scale (exact): one mask for four registers and
-// one instruction per register, where fields 16 bits apart took a rotate and an and-or per register (down kernel under the tracer,
-// us: 128 experts at 64 tokens 27.7 -> 26.8, four layers of a graph at 32 tokens 21.6 -> 20.9, 512 experts at 256 tokens 55.2 -> 53.1).
+// one instruction per register, where fields 16 bits apart took a rotate and an and-or per register (down kernel under the tracer, before and
+// after on one card, us: 128 experts at 64 tokens 27.7 -> 26.8, four layers of a graph at 32 tokens 21.6 -> 20.9, 512 experts at 256 tokens 55.2 -> 53.1).
 __device__ __forceinline__ u32x4 decode_r1w2(uint32_t z, int ks) {
     const uint32_t codes = (ks ? z >> 2 : z) & 0x33333333u;
     u32x4 r;
